@@ -346,7 +346,9 @@ __global__ __launch_bounds__(256) void norm_rope_kernel(NormRopeArgs a) {
                            a.rope_style);
 }
 
-// The same for many rows (a prefill chunk): one workgroup per ROWS_PAIRS (row, head) pairs.
+// The same for many rows (a prefill chunk) of heads that norm_rope_wave_kernel below does not
+// serve (head_dim or rotated halves not in whole 16-byte units, unaligned rows): one workgroup
+// per ROWS_PAIRS (row, head) pairs.
 // Their raw values are staged in LDS with coalesced loads (pair stride head_dim + 1: lane i
 // walking pair i is conflict-free), lane i of the first wavefront takes the sum of squares of
 // pair i in index order, exactly as above, and all threads then produce the outputs with
@@ -446,10 +448,183 @@ __global__ __launch_bounds__(256) void norm_rope_rows_kernel(NormRopeArgs a) {
     }
 }
 
+// The same for heads of whole 16-byte units: one wavefront, alone in its workgroup, per few
+// (row, head) pairs. The pairs' values, weights and rotations come in one trip to memory and
+// stay in registers; values and squares go to LDS once; lane p adds up the squares of pair p in
+// index order with 16-byte LDS reads, the next 32 on their way while 32 are added; the outputs
+// come from the registers, the rotation's other half from LDS. Bound by latency: the launch, one
+// trip to memory, head_dim dependent additions at 4 cycles each, the stores; no barrier, no
+// second pass. Kernel times on one MI355X, in us, the workgroup-wide kernel above (4-byte
+// LDS reads, the squares taken inside the chain, three phases between barriers) first:
+// 512 rows of 32 x 128 11.6 -> 6.4, of 8 x 128 8.3 -> 4.6, of 16 x 256 12.3 -> 7.0, of 2 x 256
+// 9.4 -> 4.8; 6 rows of 16 x 256 8.7 -> 4.2; 2048 rows of 32 x 128 28.4 -> 18.0; 1 row of 32 x 128
+// (one workgroup per pair) 4.2 -> 3.8.
+// U: 16-byte units a lane holds. HD4: units of the widest head served; EXACT: head_dim is it.
+template <int HD4, int U, bool EXACT>
+__global__ __launch_bounds__(64) void norm_rope_wave_kernel(NormRopeArgs a) {
+#pragma clang fp contract(off)
+    typedef __attribute__((ext_vector_type(4))) float f4;
+    constexpr int PAIRS = U * 64 / HD4;
+    // values and their squares; a unit of padding: lanes on different rows, different banks
+    __shared__ f4 raw[PAIRS * (HD4 + 1)], sqs[PAIRS * (HD4 + 1)];
+    const int lane = threadIdx.x;
+    const int hd4 = EXACT ? HD4 : a.head_dim >> 2;
+    const int pair0 = (int)blockIdx.x * PAIRS;
+    const int here = min(PAIRS, a.n_rows * a.heads - pair0);
+    const long row_elems = (long)a.heads * a.head_dim;
+    const int hstride = a.x_head_stride > 0 ? a.x_head_stride : a.head_dim;
+    const int half4 = a.rope_dims >> 3, rope4 = a.rope_dims >> 2;
+    const int row0 = pair0 / a.heads, head0 = pair0 - row0 * a.heads;
+
+    // unit u of a lane: pair pr (past the end: the last one again, not stored), dims 4*c4 .. +3
+    int pr[U], c4[U];
+    bool mine[U];
+    f4 x[U], w[U], ow[U], r0[U], r1[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        if constexpr (EXACT) {
+            pr[u] = (lane + u * 64) / HD4;
+            c4[u] = (lane & (HD4 - 1)) + ((u * 64) & (HD4 - 1));
+        } else {
+            pr[u] = (int)__umulhi((unsigned)(lane + u * 64), a.hd4_magic);
+            c4[u] = lane + u * 64 - pr[u] * hd4;
+        }
+        mine[u] = pr[u] < here;
+        pr[u] = min(pr[u], here - 1);
+        const int at = head0 + pr[u];
+        const int r = a.heads > 1 ? (int)__umulhi((unsigned)at, a.heads_magic) : at;
+        const int row = row0 + r, h = at - r * a.heads;
+        x[u] = *reinterpret_cast<const f4 *>(a.x + row * row_elems + (long)h * hstride + c4[u] * 4);
+        const bool rotated = a.rope && c4[u] < rope4;
+        // the rotation's partner unit (halves) and the first of the unit's pairs
+        const int oc4 = c4[u] < half4 ? c4[u] + half4 : c4[u] - half4;
+        w[u] = ow[u] = f4{1.0f, 1.0f, 1.0f, 1.0f};
+        if (a.weight) {
+            w[u] = *reinterpret_cast<const f4 *>(a.weight + c4[u] * 4);
+            if (rotated) ow[u] = *reinterpret_cast<const f4 *>(a.weight + oc4 * 4);
+        }
+        r0[u] = r1[u] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (rotated) {
+            const float *rt = a.rope + (long)row * a.rope_dims;
+            if (a.rope_style == 1) {
+                r0[u] = *reinterpret_cast<const f4 *>(rt + c4[u] * 4);
+            } else {
+                const int b = min(c4[u], oc4);
+                r0[u] = *reinterpret_cast<const f4 *>(rt + b * 8);
+                r1[u] = *reinterpret_cast<const f4 *>(rt + b * 8 + 4);
+            }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (mine[u]) {
+            raw[pr[u] * (HD4 + 1) + c4[u]] = x[u];
+            sqs[pr[u] * (HD4 + 1) + c4[u]] = x[u] * x[u];
+        }
+    __syncthreads();
+    float inv = 1.0f;
+    if (a.weight && lane < here) {
+        const f4 *row = sqs + lane * (HD4 + 1);
+        constexpr int R = 8; // units per round
+        float sum = 0.0f;
+        auto add = [&](const f4 &v) __attribute__((always_inline)) {
+#pragma clang fp contract(off)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum = sum + v[e];
+        };
+        f4 cur[R], nxt[R];
+        const int full = hd4 / R;
+        if (full > 0) {
+#pragma unroll
+            for (int i = 0; i < R; ++i) cur[i] = row[i];
+        }
+        for (int k = 0; k < full; ++k) {
+            const int at = min(k + 1, full - 1) * R;
+#pragma unroll
+            for (int i = 0; i < R; ++i) nxt[i] = row[at + i];
+#pragma unroll
+            for (int i = 0; i < R; ++i) add(cur[i]);
+#pragma unroll
+            for (int i = 0; i < R; ++i) cur[i] = nxt[i];
+        }
+        for (int i = full * R; i < hd4; ++i) add(row[i]);
+        const float mean_square = sum / (float)a.head_dim;
+        inv = 1.0f / sqrtf(mean_square + a.eps);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const float iv = __shfl(inv, pr[u], 64);
+        f4 n = x[u] * iv;
+        n = n * w[u];
+        if (a.rope && c4[u] < rope4) {
+            if (a.rope_style == 1) {
+                const float a0 = n[0] * r0[u][0], b0 = n[1] * r0[u][1], c0 = n[0] * r0[u][1], d0 = n[1] * r0[u][0];
+                const float a1 = n[2] * r0[u][2], b1 = n[3] * r0[u][3], c1 = n[2] * r0[u][3], d1 = n[3] * r0[u][2];
+                n = f4{a0 - b0, c0 + d0, a1 - b1, c1 + d1};
+            } else {
+                const bool is_first = c4[u] < half4;
+                const int oc4 = is_first ? c4[u] + half4 : c4[u] - half4;
+                f4 o = raw[pr[u] * (HD4 + 1) + oc4] * iv;
+                o = o * ow[u];
+                const float cs[4] = {r0[u][0], r0[u][2], r1[u][0], r1[u][2]};
+                const float sn[4] = {r0[u][1], r0[u][3], r1[u][1], r1[u][3]};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float nc = n[e] * cs[e], os = o[e] * sn[e];
+                    n[e] = is_first ? nc - os : os + nc;
+                }
+            }
+        }
+        if (mine[u])
+            *reinterpret_cast<f4 *>(a.out + ((long)(pair0 + pr[u]) * hd4 + c4[u]) * 4) = n;
+    }
+}
+
+// Whether the wavefront kernel serves these heads: whole 16-byte units everywhere, rotated
+// halves of whole units, quotients of the small products below 2^32.
+static bool norm_rope_wave_fits(const NormRopeArgs &a) {
+    const auto ok = [](const void *p) { return ((uintptr_t)p & 15) == 0; };
+    const int rot = a.rope ? a.rope_dims : 0;
+    return a.head_dim % 4 == 0 && a.head_dim >= 8 && a.heads <= 16384 && a.x_head_stride % 4 == 0 &&
+           rot % (a.rope_style == 1 ? 4 : 8) == 0 && ok(a.x) && ok(a.out) && ok(a.weight) && ok(a.rope) &&
+           (long)a.n_rows * a.heads < (1l << 30);
+}
+
+template <int HD4, int U>
+static void launch_norm_rope_wave_u(const NormRopeArgs &a, hipStream_t s) {
+    constexpr int PAIRS = U * 64 / HD4;
+    const long n_pairs = (long)a.n_rows * a.heads;
+    const dim3 grid((unsigned)((n_pairs + PAIRS - 1) / PAIRS));
+    if (a.head_dim == HD4 * 4) hipLaunchKernelGGL((norm_rope_wave_kernel<HD4, U, true>), grid, dim3(64), 0, s, a);
+    else hipLaunchKernelGGL((norm_rope_wave_kernel<HD4, U, false>), grid, dim3(64), 0, s, a);
+}
+
+// Two units a lane: short chains of loads and stores, and more wavefronts to overlap them. Four on
+// heads above 128 once two would make 4096 wavefronts and more, whose ordered sums then use one or
+// two lanes each (512 rows of 8 x 512 9.2 -> 7.9 us, 4096 rows of 16 x 256 33.8 -> 31.1; 32 x 128 is better
+// with two at any number of rows: 18.0 against 18.9 for 2048). Eight: 22.2 for those 2048 rows.
+template <int HD4> // widest head_dim / 4 served
+static hipError_t launch_norm_rope_wave(const NormRopeArgs &a, hipStream_t s) {
+    constexpr int PAIRS2 = 2 * 64 / HD4;
+    if (HD4 >= 64 && (long)a.n_rows * a.heads >= 4096l * PAIRS2) launch_norm_rope_wave_u<HD4, 4>(a, s);
+    else launch_norm_rope_wave_u<HD4, 2>(a, s);
+    return hipGetLastError();
+}
+
 hipError_t launch_norm_rope(const NormRopeArgs &a, hipStream_t s) {
     if (a.heads <= 0 || a.head_dim <= 0 || a.head_dim > 512) return hipErrorInvalidValue;
     const int rows = a.n_rows > 0 ? a.n_rows : 1;
     if (rows > 65535) return hipErrorInvalidValue;
+    if (norm_rope_wave_fits(a)) {
+        NormRopeArgs b = a;
+        b.n_rows = rows;
+        b.hd4_magic = (unsigned)(0xffffffffu / (unsigned)(a.head_dim / 4)) + 1u;
+        b.heads_magic = (unsigned)(0xffffffffu / (unsigned)a.heads) + 1u;
+        if (a.head_dim <= 64) return launch_norm_rope_wave<16>(b, s);
+        if (a.head_dim <= 128) return launch_norm_rope_wave<32>(b, s);
+        if (a.head_dim <= 256) return launch_norm_rope_wave<64>(b, s);
+        return launch_norm_rope_wave<128>(b, s);
+    }
     if (rows >= 4) {
         const int pairs = a.head_dim <= 128 ? 16 : 8;
         const int rows_per_wg = std::min(rows, (pairs + a.heads - 1) / a.heads + 1);

@@ -178,6 +178,7 @@ struct NormRopeArgs {
     // several rows at consecutive positions (grid y): row r of x and out is heads * head_dim
     // further (contiguous rows) and uses the rotation of the position r further in the table
     int n_rows;
+    unsigned hd4_magic, heads_magic; // wavefront kernel: floor(2^32 / d) + 1 of head_dim / 4 and heads (set by the launcher)
 };
 
 // out[h][c] = ctx[h][c] * sigmoid(gate[h * gate_head_stride + c])

@@ -93,6 +93,43 @@ def test_rms_norm_rope_rows_is_bit_exact(state, heads, head_dim, rope_dims, thet
     rope.close()
 
 
+@pytest.mark.parametrize("heads,head_dim,rope_dims,rows,style,norm,pad", [
+    (12, 96, 96, 7, 0, True, 0),      # heads narrower than the kernel's, rows not a multiple of its pairs
+    (3, 8, 8, 5, 0, True, 0),         # two units a head
+    (5, 80, 40, 9, 0, True, 0),       # partial rotation, a remainder behind the rounds of the ordered sum
+    (2, 260, 256, 3, 0, True, 0),     # just above a power of two
+    (8, 512, 512, 513, 0, True, 0),   # four units a lane, an odd row at the end
+    (16, 256, 64, 515, 0, False, 0),  # four units a lane, rotation only
+    (7, 128, 0, 11, 0, True, 0),      # norm only
+    (4, 64, 12, 6, 1, True, 0),       # interleaved, rotated dims of three units
+    (4, 64, 12, 6, 0, True, 0),       # halves of one and a half units: the general kernel
+    (8, 128, 128, 6, 0, True, 1),     # rows at an odd address: the general kernel
+])
+def test_rms_norm_rope_rows_wavefront_kernel_edges(state, heads, head_dim, rope_dims, rows, style, norm, pad):
+    """Bit for bit at the edges of the wavefront kernel's range, in place as well."""
+    rng = np.random.default_rng(heads * head_dim + rows)
+    x = rng.standard_normal((rows, heads * head_dim), dtype=np.float32) * 2
+    w = (0.5 + rng.random(head_dim, dtype=np.float32)).astype(np.float32)
+    offset = 3
+    rope = state.rope_table(offset + rows, rope_dims, 1.0e6, style=style) if rope_dims else None
+    buf = torch.zeros(x.size + pad, device="cuda")
+    xd = buf[pad:]
+    xd.copy_(torch.from_numpy(x.reshape(-1)))
+    wd = _dev(w)
+    state.encode_rms_norm_rope_rows(_stream(), rope, offset, xd.data_ptr(), wd.data_ptr() if norm else None, rows,
+                                    heads, head_dim, 1e-6, xd.data_ptr())
+    st = oracle.ROPE_INTERLEAVED if style else oracle.ROPE_HALVES
+    if norm and rope is None:  # position 0 rotates by nothing
+        want = np.stack([oracle.rms_norm_rope_heads_at(r, heads, head_dim, 2, w, 1e-6, 1.0e6, 0)[0] for r in x])
+    elif norm:
+        want = oracle.rms_norm_rope_heads_at(x, heads, head_dim, rope_dims, w, 1e-6, 1.0e6, offset, style=st)
+    else:
+        want = oracle.apply_rope_heads_at(x, heads, head_dim, rope_dims, 1.0e6, offset, style=st)
+    assert np.array_equal(xd.cpu().numpy().view(np.uint32), want.reshape(-1).view(np.uint32))
+    if rope is not None:
+        rope.close()
+
+
 def test_rms_norm_rope_decode_errors(state):
     x, w = np.zeros(16, np.float32), np.ones(8, np.float32)
     with pytest.raises(skv.DimensionError):
