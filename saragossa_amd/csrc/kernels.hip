@@ -24,9 +24,13 @@ __device__ __forceinline__ float bf16_to_f32(uint16_t b) {
 // dims and writes the 16 contiguous bytes they occupy in the tile.
 // Stands in for copy_at_f32_to_bf16 (src/decode_resident/kernels.rs:1036-1044).
 // ------------------------------------------------------------------------------------
+// 8-dim groups of a row: those of head_dim (a layer's pools are zero in the padding from the start),
+// in pages without a table, which are scratch, those of the padding too.
+__host__ __device__ inline int append_groups(const AppendArgs &a) { return a.table ? (a.g.head_dim + 7) >> 3 : a.g.P >> 3; }
+
 __global__ __launch_bounds__(256) void append_kernel(AppendArgs a) {
     const Geom g = a.g;
-    const int groups = (g.head_dim + 7) >> 3;
+    const int groups = append_groups(a);
     const long per_row = (long)g.kv_heads * groups;
     const long page0 = a.first_pos >> 4; // first page of positions the batch touches
     const long n_blk = ((a.first_pos + a.n_rows + 15) >> 4) - page0;
@@ -46,7 +50,7 @@ __global__ __launch_bounds__(256) void append_kernel(AppendArgs a) {
             const int db = rem >> 4, c = rem & 15;
             const int row0 = a.v_grp_first + grp4 * 4;
             const long slot = slot_of(a.first_pos + row0, g.ring_rows); // a multiple of 4
-            const int page = a.table[slot >> 4];
+            const int page = a.table ? a.table[slot >> 4] : (int)(slot >> 4);
             const long tile = (long)page * g.page_elems + (long)kvh * g.tile_elems;
             const int d0 = db * 32 + c, d1 = d0 + 16;
             const float *vs = a.v_src + (long)row0 * kv_dim + kvh * g.head_dim;
@@ -80,7 +84,7 @@ __global__ __launch_bounds__(256) void append_kernel(AppendArgs a) {
             grp = rem - kvh * groups;
         }
         const long slot = slot_of(a.first_pos + row, g.ring_rows);
-        const int page = a.table[slot >> 4];
+        const int page = a.table ? a.table[slot >> 4] : (int)(slot >> 4);
         const int r = (int)(slot & 15);
         const long tile = (long)page * g.page_elems + (long)kvh * g.tile_elems;
         const float *ks = a.k_src + (long)row * kv_dim + kvh * g.head_dim + grp * 8;
@@ -104,7 +108,7 @@ __global__ __launch_bounds__(256) void append_kernel(AppendArgs a) {
 }
 
 hipError_t launch_append(const AppendArgs &a, hipStream_t s) {
-    const int groups = (a.g.head_dim + 7) >> 3;
+    const int groups = append_groups(a);
     const long n_blk = ((a.first_pos + a.n_rows + 15) >> 4) - (a.first_pos >> 4);
     const long row_items = a.by_page ? n_blk * 16 : (long)a.n_rows;
     const long total = (long)a.g.kv_heads * groups * row_items +

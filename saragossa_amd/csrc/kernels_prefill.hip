@@ -1,5 +1,7 @@
 // gfx950 kernels of the KV hot path, part 3: chunked prefill over the paged cache, the one
 // matrix-core-bound kernel of the path.
+#include <type_traits>
+
 #include "skv_internal.h"
 
 namespace skv {
@@ -7,15 +9,16 @@ namespace skv {
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) short short4_t;
 typedef __attribute__((ext_vector_type(4))) float float4_t;
+typedef __attribute__((ext_vector_type(4))) unsigned int u4;
 
 namespace {
 
-__device__ __forceinline__ uint16_t bf16_bits(float v) {
-    uint32_t b = __float_as_uint(v);
-    uint32_t lsb = (b >> 16) & 1u;
-    return (uint16_t)((b + 0x7fffu + lsb) >> 16);
+// two values rounded to bf16 (nearest even), the first in the low half: one instruction
+__device__ __forceinline__ uint32_t bf16_pair(float x, float y) {
+    typedef __attribute__((ext_vector_type(2))) float f2;
+    typedef __attribute__((ext_vector_type(2))) __bf16 b2;
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{x, y}, b2));
 }
-__device__ __forceinline__ float bf16_to_f32(uint16_t b) { return __uint_as_float(((uint32_t)b) << 16); }
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 } // namespace
@@ -23,113 +26,123 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // ------------------------------------------------------------------------------------
 // Many query rows over the cache (cached_attention_prefill_rows,
 // src/decoder/attention_ops.rs:976-1017, as one launch): query slot (i, g) = new row i,
-// head g of the kv head's group, attends positions up to len - n_queries + i through the
-// layer's window.
+// head g of the kv head's group, attends positions up to q_pos0 + i through the layer's window.
 //
-// One workgroup = 8 wavefronts = 8 * TILES tiles of 16 query slots of one kv head, and a
-// range of the context's pages (split). The workgroup walks its pages once: all threads
-// copy PG pages' K and V tiles (already in matrix-operand order) from memory to LDS, double
-// buffered, and every wavefront multiplies them with its own query tiles, which it holds in
-// registers as bf16 hi + lo halves (pre-scaled by log2(e)/sqrt(head_dim)). So a K/V byte is
-// fetched from memory once per 128 * TILES query slots instead of once per 16. Pages are
-// consumed in pairs: S^T = K . Q^T per page (16 keys x 16 slots, 16x16x32 over the head
-// dims), one online-softmax step in base 2 over the pair's 32 keys on the accumulator
-// registers, then O^T += V^T . P^T as 16x16x32 products over those 32 keys with P split
-// hi + lo. There is no merge inside the workgroup (every wavefront owns its slots); with
-// several splits the (o, m, l) partials go to merge_rows_kernel.
+// One workgroup = WAVES wavefronts of TILES tiles of 16 query slots of one kv head, and a range
+// of the pages any of them attends (split). The workgroup walks its pages once, in pairs: all
+// threads copy the pages' K and V tiles (already in matrix-operand order) from memory to LDS,
+// double buffered, and every wavefront multiplies them with its own query tiles, which it holds
+// in registers as bf16 hi + lo halves (pre-scaled by log2(e)/sqrt(head_dim)). Per pair:
+//   window 1: S^T(p+1) = K . Q^T of the NEXT pair (16x16x32 products over the head dims) with the
+//             exponentials and the hi + lo split of this pair's probabilities between the products;
+//   window 2: O^T += V^T . P^T(p), 16x16x32 products over the pair's 32 keys.
+// A product occupies the matrix pipe for 16 cycles and its wavefront for 4; the vector work of
+// the softmax therefore costs nothing where it is issued between products that do not depend on
+// it, and a pair's softmax never depends on the next pair's scores. (With the softmax between the
+// two products of the same pair, the two wavefronts of a SIMD, which a barrier keeps in step,
+// were in their vector phases at the same time: four pairs at head_dim 128 took 4.4 us by
+// time stamps where they take 3.4 now, of which the products are 1.75.)
+//
+// The softmax runs in base 2 against a base m per slot that is not the running maximum but
+// within 2^8 of it: the score accumulators start at -m, so the products deliver s - m and the
+// exponential needs no subtraction, and only a score above m + 8 makes the wavefront move the
+// bases and rescale its sums. Probabilities stay below 2^8 and are split relatively, so
+// nothing is lost; partials carry (o, base, l) and any base serves the merge.
+// With HALVES = 2 the wavefronts are two halves that hold the same slots and take the page pairs in
+// turn; the second half's (o, m, l) join the first's through LDS at the end. Otherwise there is
+// no merge inside the workgroup; with several splits the partials go to merge_rows_kernel.
+// The copies go straight from memory to LDS. 512 rows as one call (append, attention, merge), in us
+// on one MI355X, against the kernel that ran scores, softmax and accumulation of a pair one after
+// the other and copied through registers: q32/kv8/hd128 over 0, 1536, 4700, 16384 rows 34.5 -> 21.7,
+// 57.2 -> 41.1, 106 -> 86.5, 256 -> 225; q16/kv2/hd256 40.0 -> 24.3, 55.7 -> 50.5, 97.9 -> 89.0, 247 -> 225 (where
+// the matrix pipes alone need 130).
 // ------------------------------------------------------------------------------------
-// Copies of PG pages (K tile then V tile each) of one kv head: memory -> registers -> LDS.
-template <int P, int PG, int THREADS>
-__device__ __forceinline__ void fetch_step(uint4 (&stage)[PG][(2 * (P / 32) * 64 + THREADS - 1) / THREADS], const DecodeArgs &a,
-                                           int pb0, int step, int n_it, int kvh, int tid) {
-    constexpr int TILE_U4 = (P / 32) * 64;
-    constexpr int LOAD_U = (2 * TILE_U4 + THREADS - 1) / THREADS;
-#pragma unroll
-    for (int pg = 0; pg < PG; ++pg) {
-        // past the end: a page again, unused; always a page the layer holds
-        const int it = max(min(step * PG + pg, n_it - 1), 0);
-        const int page = a.table[min(pb0 + it, a.page_first + a.n_pages - 1)]; // uniform: a scalar load
-        const long tile = (long)page * a.g.page_elems + (long)kvh * a.g.tile_elems;
-        const uint4 *kp = reinterpret_cast<const uint4 *>(a.k_pool + tile);
-        const uint4 *vp = reinterpret_cast<const uint4 *>(a.v_pool + tile);
-#pragma unroll
-        for (int u = 0; u < LOAD_U; ++u) {
-            // unconditional (a thread past the end re-reads the last unit and drops it)
-            const int i = min(tid + u * THREADS, 2 * TILE_U4 - 1);
-            const uint4 *src = i < TILE_U4 ? kp + i : vp + (i - TILE_U4);
-            stage[pg][u] = *src;
-        }
+
+// Entry e of the launch's page list: where its tiles lie (of the workgroup's kv head, in 16-byte
+// units from its pool's start), which position its first row has, and the first and last
+// position whose rows it may speak for. On full layers entry e is logical page e.
+template <bool RING>
+__device__ __forceinline__ uint32_t entry_tile(const DecodeArgs &a, const ChunkPages &c, int e, int kvh) {
+    int page;
+    if constexpr (RING) {
+        int at = c.start + min(e, c.n_old - 1);
+        if (at >= c.ring_pages) at -= c.ring_pages;
+        page = e < c.n_old ? a.table[max(at, 0)] : e - c.n_old;
+    } else {
+        page = a.table[e];
     }
+    return (uint32_t)page * (uint32_t)(a.g.page_elems >> 3) + (uint32_t)kvh * (uint32_t)(a.g.tile_elems >> 3);
 }
-// LDS order of a step: [PG/2 pairs][K tile of page A | K tile of page B | V tiles of both].
-// The K tiles are copied verbatim. The two V tiles of a pair are interleaved in 8-byte
-// halves, unit (kk, h, lane) = {page A's four keys, page B's four keys} of dim tile h, so
-// that one 16-byte read is the 32-key operand of the PV product as it stands.
+template <bool RING>
+__device__ __forceinline__ int entry_pos(const ChunkPages &c, int e) {
+    if constexpr (!RING) return e * 16;
+    return e < c.n_old ? c.first_pos + e * 16 : c.new_first + (e - c.n_old) * 16;
+}
+template <bool RING>
+__device__ __forceinline__ int entry_lo(const ChunkPages &c, int e) {
+    return !RING || e < c.n_old ? INT32_MIN : c.new_pos0;
+}
+template <bool RING>
+__device__ __forceinline__ int entry_hi(const ChunkPages &c, int e) {
+    return !RING || e >= c.n_old ? INT32_MAX : c.new_pos0 - 1;
+}
+// The entries [e0, e1) of [first, last) all of whose rows lie in [lo, hi] and are the entry's to
+// speak for, as two ranges: old entries, new ones.
+struct Inner {
+    int o0, o1, n0, n1;
+};
+template <bool RING>
+__device__ __forceinline__ Inner inner_entries(const ChunkPages &c, int first, int last, int lo, int hi) {
+    Inner r;
+    if constexpr (!RING) {
+        r.o0 = max(first, (lo + 15) >> 4);
+        r.o1 = min(last, (hi - 15 >= 0 ? (hi - 15) >> 4 : -1) + 1);
+        r.n0 = r.n1 = 0;
+    } else {
+        r.o0 = max(first, (lo - c.first_pos + 15) >> 4);
+        r.o1 = min(min(last, c.n_old), ((min(hi, c.new_pos0 - 1) - 15 - c.first_pos) >> 4) + 1);
+        r.n0 = max(max(first, c.n_old), c.n_old + ((max(lo, c.new_pos0) - c.new_first + 15) >> 4));
+        r.n1 = min(last, c.n_old + ((hi - 15 - c.new_first) >> 4) + 1);
+    }
+    return r;
+}
+
+// 64 x 16 bytes straight from memory to LDS, lane l's to lds + 16 l (`lds` the same in every lane), no
+// register in between. In assembly because the compiler, which cannot tell the two halves of the
+// double buffer apart, would make every LDS read wait for a copy it knows of; the kernel
+// waits for all of them itself (copies_landed) in front of the barrier that hands the buffer over.
+__device__ __forceinline__ void copy_to_lds(const void *base, uint32_t lane_offset, uint32_t lds) {
+    // (both are the same in every lane: said so, whatever the compiler can prove)
+    const uint64_t b = reinterpret_cast<uint64_t>(base);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
+    const uint64_t from = ((uint64_t)hi << 32) | lo;
+    const uint32_t to = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(lane_offset), "s"(from) : "m0");
+}
+__device__ __forceinline__ void copies_landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// LDS order of a step, SP pairs: [SP][K tile of page A | K tile of page B], then V the same way, tiles
+// as they are in memory.
 //
 // Keys that no query slot of the workgroup attends (rows at or past the cache's length after a
 // rollback, ring rows not valid, rows before every slot's window, the stand-in page past the
-// end of a split) get zero probability, but 0 x NaN is NaN: on the pages at the edges of the
-// attended range [ws_lo, lim_hi] (and on ring pages) their V values are cleared on the way
-// into LDS, so the bits of such a row never reach a context (the reference never reads those
-// rows, src/decode_resident/kernels.rs:11-88).
-template <int P, int PG, int THREADS>
-__device__ __forceinline__ void store_step(const uint4 (&stage)[PG][(2 * (P / 32) * 64 + THREADS - 1) / THREADS], uint4 *buf,
-                                           int tid, const DecodeArgs &a, int pb0, int step, int n_it, int ws_lo,
-                                           int lim_hi) {
-    constexpr int TILE_U4 = (P / 32) * 64;
-    constexpr int LOAD_U = (2 * TILE_U4 + THREADS - 1) / THREADS;
-    static_assert(PG % 2 == 0, "pages are consumed in pairs");
-#pragma unroll
-    for (int pg = 0; pg < PG; ++pg) {
-        uint4 *pair = buf + (pg >> 1) * 4 * TILE_U4;
-        const int it = step * PG + pg;
-        const int slot_a = (pb0 + it) * 16; // first cache slot of the page
-        const bool inside = it < n_it && a.g.ring_rows == 0 && slot_a >= ws_lo && slot_a + 15 <= lim_hi;
-#pragma unroll
-        for (int u = 0; u < LOAD_U; ++u) {
-            const int i = tid + u * THREADS;
-            if (2 * TILE_U4 < THREADS && i >= 2 * TILE_U4) continue;
-            uint4 x = stage[pg][u];
-            if (i < TILE_U4) {
-                pair[(pg & 1) * TILE_U4 + i] = x;
-            } else {
-                const int iv = i - TILE_U4;
-                if (!inside) {
-                    // the unit holds keys 4rq .. 4rq+3 of two dim tiles: (x, y) and (z, w), two keys a word
-                    const int rq = (iv >> 4) & 3;
-                    uint32_t keep[2] = {0u, 0u};
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int slot = slot_a + rq * 4 + r;
-                        int pos = slot;
-                        if (a.g.ring_rows > 0)
-                            pos = slot <= a.ring_t ? a.ring_base + slot : a.ring_base - a.g.ring_rows + slot;
-                        if (it < n_it && pos >= ws_lo && pos <= lim_hi) keep[r >> 1] |= 0xffffu << ((r & 1) * 16);
-                    }
-                    x.x &= keep[0];
-                    x.z &= keep[0];
-                    x.y &= keep[1];
-                    x.w &= keep[1];
-                }
-                uint2 *dst = reinterpret_cast<uint2 *>(pair + 2 * TILE_U4 + (iv >> 6) * 128 + (iv & 63)) + (pg & 1);
-                dst[0] = make_uint2(x.x, x.y);
-                dst[128] = make_uint2(x.z, x.w); // dim tile 1: 64 units of 16 bytes further
-            }
-        }
-    }
-}
-
-// PG: pages copied and consumed per barrier step (the copies of step i+1 are in flight while
-// step i is multiplied, so a step must hold about a memory latency's worth of work).
-template <int P, int TILES, int PG, int WAVES>
-__global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a) {
+// end of a split) get zero probability, but 0 x NaN is NaN: in steps that touch the edges of the
+// attended range their V values are cleared in LDS, behind a barrier of its own, so the bits of
+// such a row never reach a context (the reference never reads those rows,
+// src/decode_resident/kernels.rs:11-88).
+template <int P, int TILES, int SP, int WAVES, int HALVES, bool RING>
+__global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, ChunkPages c) {
     constexpr int THREADS = WAVES * 64;
     constexpr int KK = P / 32;
     constexpr int NT = P / 16;
-    constexpr int TILE_U4 = KK * 64;                       // 16-byte units of one K (or V) tile
-    constexpr int LOAD_U = (2 * TILE_U4 + THREADS - 1) / THREADS;
-    extern __shared__ __attribute__((aligned(16))) uint4 kv_lds[]; // [2 buffers][PG][K tile | V tile]
-    constexpr int BUF_U4 = PG * 2 * TILE_U4;
+    constexpr int TILE_U4 = KK * 64;                           // 16-byte units of one K (or V) tile
+    constexpr int GP = 2 * HALVES;                             // pages of a group: a pair for each half
+    constexpr int CU = SP * GP * TILE_U4 / THREADS;            // units of K, and of V, a thread copies per step
+    static_assert(SP * GP * TILE_U4 % THREADS == 0 && TILE_U4 % 64 == 0, "a wavefront copies whole KiB of one page");
+    extern __shared__ __attribute__((aligned(16))) u4 kv_lds[]; // [2 buffers][K of SP pairs | V of SP pairs]
+    constexpr int HALF_U4 = SP * GP * TILE_U4;
+    constexpr int BUF_U4 = 2 * HALF_U4;
 
     const Geom g = a.g;
     const int tid = threadIdx.x;
@@ -140,42 +153,120 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a) 
     const int split = blockIdx.x;
     const int kvh = blockIdx.y;
     const int G = g.gqa;
-    const int C = a.n_queries;
-    const int n_slots = C * G;
-    const int wg_slot0 = blockIdx.z * (WAVES * TILES * 16);
-    const int wg_slot1 = min(n_slots, wg_slot0 + WAVES * TILES * 16) - 1; // last slot of the workgroup
+    const int n_slots = a.n_queries * G;
+    constexpr int TW = WAVES / HALVES;                         // wavefronts of a half, TILES slot tiles each
+    const int half = HALVES > 1 ? wave / TW : 0;
+    const int tw = HALVES > 1 ? wave % TW : wave;
+    const int wg_slot0 = blockIdx.z * (TW * TILES * 16);
+    const int wg_slot1 = min(n_slots, wg_slot0 + TW * TILES * 16) - 1; // last slot of the workgroup
 
-    // query slot -> position of its row, last position it attends, first position it attends
-    auto pos_of = [&](int slot) { return a.q_pos0 + slot / G; };
-    auto limit_of = [&](int slot) { return min(pos_of(slot), a.limit_cap); };
-    auto ws_of = [&](int slot) { return a.window > 0 ? max(a.window_start, pos_of(slot) + 1 - a.window) : a.window_start; };
+    // query slot -> position of its row (the last it attends), first position it attends
+    auto limit_of = [&](int slot) { return a.q_pos0 + slot / G; };
+    auto ws_of = [&](int slot) { return a.window > 0 ? max(a.window_start, limit_of(slot) + 1 - a.window) : a.window_start; };
 
-    // pages any slot of the workgroup can see, divided among the splits
+    // entries of the page list any slot of the workgroup can see, divided among the splits
     const int wg_ws_lo = ws_of(wg_slot0);
     const int wg_lim_hi = limit_of(wg_slot1);
-    const int page_lo = g.ring_rows > 0 ? 0 : wg_ws_lo >> 4;
-    const int page_hi = g.ring_rows > 0 ? a.n_pages : (wg_lim_hi >> 4) + 1;
-    const unsigned span = (unsigned)(page_hi - page_lo);
-    const int pb0 = page_lo + (int)(((unsigned)split * span) / (unsigned)a.splits);
-    const int pb1 = page_lo + (int)(((unsigned)(split + 1) * span) / (unsigned)a.splits);
+    auto entry_of = [&](int pos) {
+        if (!RING) return pos >> 4;
+        return pos < c.new_pos0 ? max((pos - c.first_pos) >> 4, 0) : c.n_old + ((pos - c.new_first) >> 4);
+    };
+    const int e_lo = entry_of(wg_ws_lo);
+    const int e_hi = entry_of(wg_lim_hi) + 1;
+    const unsigned span = (unsigned)(e_hi - e_lo);
+    const int pb0 = e_lo + (int)(((unsigned)split * span) / (unsigned)a.splits);
+    const int pb1 = e_lo + (int)(((unsigned)(split + 1) * span) / (unsigned)a.splits);
     const int n_it = pb1 - pb0;
+    const int n_groups = (n_it + GP - 1) / GP;
 
+    // ---- page copies, memory -> LDS. K runs one group ahead of V: step s brings K of the groups
+    // SP*s + 1 .. and V of the groups SP*s ..
+    auto entry = [&](int it) { return min(pb0 + it, e_hi - 1); }; // past the end: a page again, unused
+    // Places of the next copy's tiles, one per lane, asked for a step ahead and read with
+    // v_readlane: a scalar read of the table in front of the loads would make the wavefront wait
+    // for it and, the two being counted together, for every LDS read in flight (512 rows of
+    // q16/kv2/hd256 over 16384 rows: 285 us against 265).
+    uint32_t ids;
+    auto ask_ids = [&](int it) __attribute__((always_inline)) { ids = entry_tile<RING>(a, c, entry(it + lane), kvh); };
+    // tile of page it0 + d, it0 being the page that lane 0's entry belongs to
+    auto tile_of = [&](int it0, int d, bool v) __attribute__((always_inline)) {
+        const uint16_t *pool = v ? a.v_pool : a.k_pool;
+        if (RING && entry(it0 + d) >= c.n_old) pool = v ? c.v_new : c.k_new;
+        return reinterpret_cast<const u4 *>(pool) + (uint32_t)__builtin_amdgcn_readlane(ids, d);
+    };
+    ask_ids(0);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)kv_lds;
+    const uint32_t lane_at = (uint32_t)(tid & (TILE_U4 - 1)) * 16; // where in its page a lane's units lie, in bytes
+    // unit u of a step's K (v = false) or V into the buffer half at unit `dst` of LDS; it0: see tile_of
+    auto copy_unit = [&](int u, bool v, int it0, int dst) __attribute__((always_inline)) {
+        const int i0 = wave * 64 + u * THREADS; // the wavefront's first unit
+        const int pg = i0 / TILE_U4;
+        const uint32_t off = THREADS % TILE_U4 == 0 ? lane_at : lane_at + (uint32_t)((u * THREADS) & (TILE_U4 - 1)) * 16;
+        copy_to_lds(tile_of(it0, v ? pg : pg + GP, v), off, lds0 + (uint32_t)(dst + i0) * 16);
+    };
+    // The copies of a step are spread over the K-steps of the first half of its products (512 rows of
+    // q16/kv2/hd256 over 16384 rows: 243 us against 265 with all of them in front of one window; 223
+    // with copies straight to LDS instead of through registers, which took stores besides).
+    constexpr int COPY_SPAN = KK * SP;
+    auto copy_slot = [&](int slot, int step) __attribute__((always_inline)) {
+        const int it0 = (step + 1) * SP * GP; // first page of the V copy, a group before the K copy's
+        const int dst = ((step + 1) & 1) * BUF_U4;
+#pragma unroll
+        for (int i = 0; i < 2 * CU; ++i)
+            if (i * COPY_SPAN / (2 * CU) == slot) {
+                if (i < CU) copy_unit(i, false, it0, dst);
+                else copy_unit(i - CU, true, it0, dst + HALF_U4);
+                if (i == 2 * CU - 1) ask_ids((step + 2) * SP * GP);
+            }
+    };
+    // V rows of the pages from first_page on that nobody attends, cleared in the buffer half at `v`
+    const Inner wg_in = inner_entries<RING>(c, pb0, pb1, wg_ws_lo, wg_lim_hi);
+    auto clear_v = [&](int first_page, u4 *v) __attribute__((always_inline)) {
+        const int e0 = pb0 + first_page, e1 = e0 + SP * GP;
+        if ((e0 >= wg_in.o0 && e1 <= wg_in.o1) || (RING && e0 >= wg_in.n0 && e1 <= wg_in.n1)) return; // uniform
+        for (int i = tid; i < SP * GP * TILE_U4; i += THREADS) {
+            const int it = first_page + i / TILE_U4;
+            const int e = entry(it);
+            const int pos0 = entry_pos<RING>(c, e) + ((i >> 4) & 3) * 4; // unit: keys 4rq .. 4rq+3 of two dims
+            const int lo = max(wg_ws_lo, entry_lo<RING>(c, e)), hi = min(wg_lim_hi, entry_hi<RING>(c, e));
+            uint32_t keep[2] = {0u, 0u};
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (it < n_it && pos0 + r >= lo && pos0 + r <= hi) keep[r >> 1] |= 0xffffu << ((r & 1) * 16);
+            v[i] &= u4{keep[0], keep[1], keep[0], keep[1]};
+        }
+        __syncthreads();
+    };
+
+    // the first group's K (into the second buffer) and the first step's pages are on their way while
+    // the queries are prepared
+#pragma unroll
+    for (int u = 0; u < (GP * TILE_U4 + THREADS - 1) / THREADS; ++u) {
+        const int i0 = wave * 64 + u * THREADS;
+        if (GP * TILE_U4 % THREADS == 0 || i0 < GP * TILE_U4)
+            copy_to_lds(tile_of(0, i0 / TILE_U4, false),
+                        THREADS % TILE_U4 == 0 ? lane_at : lane_at + (uint32_t)((u * THREADS) & (TILE_U4 - 1)) * 16,
+                        lds0 + (uint32_t)(BUF_U4 + i0) * 16);
+    }
+#pragma unroll
+    for (int u = 0; u < CU; ++u) {
+        copy_unit(u, false, 0, 0);
+        copy_unit(u, true, 0, HALF_U4);
+    }
     // ---- this wavefront's query tiles ------------------------------------------------
     int my_limit[TILES], my_ws[TILES];
-    int t_ws_hi[TILES], t_lim_lo[TILES], t_ws_lo[TILES], t_lim_hi[TILES]; // per tile extremes
+    int t_ws_hi[TILES], t_lim_lo[TILES]; // per tile extremes
     bool t_on[TILES];
     bf16x8_t qh[TILES][KK], ql[TILES][KK];
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
-        const int s0 = wg_slot0 + (wave * TILES + t) * 16;
+        const int s0 = wg_slot0 + (tw * TILES + t) * 16;
         t_on[t] = s0 < n_slots;
         const int s_last = min(s0 + 15, n_slots - 1);
         const int my_slot = min(s0 + n, n_slots - 1);
         my_limit[t] = limit_of(my_slot);
         my_ws[t] = ws_of(my_slot);
         t_lim_lo[t] = limit_of(min(s0, n_slots - 1));
-        t_lim_hi[t] = limit_of(s_last);
-        t_ws_lo[t] = ws_of(min(s0, n_slots - 1));
         t_ws_hi[t] = ws_of(s_last);
         const float *qrow = a.q + ((long)(my_slot / G) * g.q_heads + kvh * G + my_slot % G) * g.head_dim;
         // eight consecutive dims of the slot's row per k-step: all loads first (two 16-byte
@@ -205,191 +296,194 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a) 
         for (int kk = 0; kk < KK; ++kk) {
             const int d0 = kk * 32 + j * 8;
             uint32_t hi[4], lo[4];
+            // (with 16-byte loads head_dim is a multiple of 8: the lane's eight dims are all inside or all padding)
+            const float scale = !a.q_vec || d0 < g.head_dim ? a.qscale : 0.0f;
 #pragma unroll
             for (int e2 = 0; e2 < 4; ++e2) {
-                uint32_t h2 = 0, l2 = 0;
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const float v = d0 + e2 * 2 + h < g.head_dim ? qv[kk][e2 * 2 + h] * a.qscale : 0.0f;
-                    const uint16_t hb = bf16_bits(v);
-                    const uint16_t lb = bf16_bits(v - bf16_to_f32(hb));
-                    h2 |= (uint32_t)hb << (16 * h);
-                    l2 |= (uint32_t)lb << (16 * h);
+                float x0 = qv[kk][e2 * 2] * scale, x1 = qv[kk][e2 * 2 + 1] * scale;
+                if (!a.q_vec) {
+                    x0 = d0 + e2 * 2 < g.head_dim ? x0 : 0.0f;
+                    x1 = d0 + e2 * 2 + 1 < g.head_dim ? x1 : 0.0f;
                 }
-                hi[e2] = h2;
-                lo[e2] = l2;
+                hi[e2] = bf16_pair(x0, x1);
+                lo[e2] = bf16_pair(x0 - __uint_as_float(hi[e2] << 16), x1 - __uint_as_float(hi[e2] & 0xffff0000u));
             }
-            qh[t][kk] = __builtin_bit_cast(bf16x8_t, make_uint4(hi[0], hi[1], hi[2], hi[3]));
-            ql[t][kk] = __builtin_bit_cast(bf16x8_t, make_uint4(lo[0], lo[1], lo[2], lo[3]));
+            qh[t][kk] = __builtin_bit_cast(bf16x8_t, u4{hi[0], hi[1], hi[2], hi[3]});
+            ql[t][kk] = __builtin_bit_cast(bf16x8_t, u4{lo[0], lo[1], lo[2], lo[3]});
         }
     }
+    ask_ids(SP * GP);
 
     float4_t o[TILES][NT];
-    float m_run[TILES], l_run[TILES];
+    float4_t neg_m[TILES];             // -m in all four: what the score accumulators start from
+    float m_base[TILES], thr[TILES];   // base of the slot; a score above base + thr moves it (-inf: no key yet)
+    float l_run[TILES];                // this lane's share of the slot's sum
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
 #pragma unroll
-        for (int c = 0; c < NT; ++c) o[t][c] = float4_t{0.f, 0.f, 0.f, 0.f};
-        m_run[t] = -INFINITY;
+        for (int u = 0; u < NT; ++u) o[t][u] = float4_t{0.f, 0.f, 0.f, 0.f};
+        m_base[t] = 0.0f;
+        neg_m[t] = float4_t{0.f, 0.f, 0.f, 0.f};
+        thr[t] = -INFINITY;
         l_run[t] = 0.0f;
     }
 
-    // ---- page copies: memory -> registers -> LDS -------------------------------------
-    const int n_steps = (n_it + PG - 1) / PG;
-    constexpr int FETCH_PAIR = PG / 2 - 1; // in front of the step's last pair
-    uint4 stage[PG][LOAD_U];
-    // (a split without pages still reads one valid page, and writes empty partials below)
-    fetch_step<P, PG, THREADS>(stage, a, pb0, 0, n_it, kvh, tid);
-    store_step<P, PG, THREADS>(stage, kv_lds, tid, a, pb0, 0, n_it, wg_ws_lo, wg_lim_hi);
-    __syncthreads();
+    // S^T - m of a pair, eight scores a lane and tile: keys 4j .. 4j+3 of page A, then of page B
+    float4_t sa[TILES], sb[TILES];
+    // probabilities of the pair being accumulated, as two bf16 terms
+    bf16x8_t ph[TILES], pl[TILES];
+    constexpr int DEPTH = KK < 2 || TILES > 1 ? 1 : 2; // K-steps an operand is asked for ahead of its products
 
-    for (int step = 0; step < n_steps; ++step) {
-      // The next step's pages are asked for in front of the last pair of this step, not at its
-      // top: the copies still land before store_step needs them, and the staging registers are
-      // live for less of the step (a stream of calls, same box each: config 2 shape 450 against
-      // 466 us and 470.6 against 480.3; config 1 shape, four pairs per step, 56.8 in front of the
-      // last pair, 57.4 and 57.9 in front of the third and second, 57.75 at the top; inside the
-      // last pair, after its scores or its softmax, 481-483 against 475 at config 2 shape).
-      // Unconditional: after the last step this re-reads its pages into the idle buffer.
-      // Pages are consumed in pairs (A, B): the PV product then contracts over 32 keys with
-      // the k index of lane group j, element e meaning key 4j+e of page A (e < 4) or key
-      // 4j+e-4 of page B, which is exactly how the two S^T tiles and the two V tiles already
-      // sit in the lanes.
+    // the half's pairs are the page pairs HALVES * group + half.
+    // pairs whose keys every slot of the wavefront attends: [in0, in1) and, of new pages, [in2, in3)
+    int in0, in1, in2, in3;
+    {
+        int lo = t_ws_hi[0], hi = t_lim_lo[0];
 #pragma unroll
-      for (int pp = 0; pp < PG / 2; ++pp) {
-        if (pp == FETCH_PAIR) fetch_step<P, PG, THREADS>(stage, a, pb0, min(step + 1, n_steps - 1), n_it, kvh, tid);
-        const int it_a = step * PG + 2 * pp;
-        if (it_a >= n_it) continue;
-        const bool has_b = it_a + 1 < n_it;
-        const uint4 *kt_a = kv_lds + (step & 1) * BUF_U4 + pp * 4 * TILE_U4;
-        const uint4 *kt_b = kt_a + TILE_U4;
-        const uint4 *vt = kt_a + 2 * TILE_U4; // both pages' V tiles, interleaved (store_step)
-        const int slot_a = (pb0 + it_a) * 16; // first cache slot of page A; page B follows it
-
-        // which of the wavefront's tiles see the pair at all
-        bool use[TILES];
-        bool any = false;
+        for (int t = 1; t < TILES; ++t) {
+            lo = max(lo, t_ws_hi[t]);
+            hi = min(hi, t_lim_lo[t]);
+        }
+        const Inner r = inner_entries<RING>(c, pb0, pb1, lo, hi);
+        in0 = (r.o0 - pb0 + 1) >> 1;
+        in1 = (r.o1 - pb0) >> 1;
+        in2 = (r.n0 - pb0 + 1) >> 1;
+        in3 = (r.n1 - pb0) >> 1;
+    }
+    // scores of keys outside the slot's range become -inf; then, where a score passes the base by more
+    // than thr, the wavefront's bases move
+    auto settle = [&](int pair) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
-            use[t] = t_on[t] && (g.ring_rows > 0 || (slot_a <= t_lim_hi[t] && slot_a + 31 >= t_ws_lo[t]));
-            any = any || use[t];
+            if (!((pair >= in0 && pair < in1) || (RING && pair >= in2 && pair < in3))) { // uniform
+                const int it = 2 * pair;
+                const int ea = entry(it), eb = entry(it + 1);
+                const int pos_a = entry_pos<RING>(c, ea), pos_b = entry_pos<RING>(c, eb);
+                const int lo_a = max(my_ws[t], entry_lo<RING>(c, ea)), hi_a = min(my_limit[t], entry_hi<RING>(c, ea));
+                const int lo_b = max(my_ws[t], entry_lo<RING>(c, eb)), hi_b = min(my_limit[t], entry_hi<RING>(c, eb));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int pa = pos_a + j * 4 + e, pb = pos_b + j * 4 + e;
+                    sa[t][e] = it < n_it && pa >= lo_a && pa <= hi_a ? sa[t][e] : -INFINITY;
+                    sb[t][e] = it + 1 < n_it && pb >= lo_b && pb <= hi_b ? sb[t][e] : -INFINITY;
+                }
+            }
+            const float mx = fmaxf(fmaxf(fmaxf(sa[t][0], sa[t][1]), fmaxf(sa[t][2], sa[t][3])),
+                                   fmaxf(fmaxf(sb[t][0], sb[t][1]), fmaxf(sb[t][2], sb[t][3])));
+            if (__builtin_amdgcn_ballot_w64(mx > thr[t])) {
+                const float top = rows_max(mx); // of the slot, relative to its base
+                const bool unseen = thr[t] == -INFINITY;
+                const float d = unseen ? (top == -INFINITY ? 0.0f : top) : fmaxf(top, 0.0f);
+                const float alpha = unseen ? 1.0f : fast_exp2(-d);
+                m_base[t] += d;
+                neg_m[t] = float4_t{-m_base[t], -m_base[t], -m_base[t], -m_base[t]};
+                thr[t] = unseen && top == -INFINITY ? -INFINITY : 8.0f;
+                l_run[t] *= alpha;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    sa[t][e] -= d;
+                    sb[t][e] -= d;
+                }
+                if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
+#pragma unroll
+                    for (int u = 0; u < NT; ++u) o[t][u] *= alpha;
+                }
+            }
         }
-        if (!any) continue;
-        // S^T = K . Q^T for both pages, the K registers shared by the tiles
-        float4_t sa0[TILES], sa1[TILES], sb0[TILES], sb1[TILES];
+    };
+
+    // probabilities of the settled scores, in nine small steps per tile so that they can stand
+    // between products: step q takes the exponential of score q and splits that of score q - 1
+    float pr_[TILES];                  // exponential of the last step
+    uint32_t pbits[TILES][2], rbits[TILES][2], hi4[TILES][4], lo4[TILES][4];
+    auto prob_step = [&](int q) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
-            sa0[t] = float4_t{0.f, 0.f, 0.f, 0.f};
-            sa1[t] = float4_t{0.f, 0.f, 0.f, 0.f};
-            sb0[t] = float4_t{0.f, 0.f, 0.f, 0.f};
-            sb1[t] = float4_t{0.f, 0.f, 0.f, 0.f};
+            const float prev = pr_[t];
+            if (q < 8) pr_[t] = fast_exp2(q < 4 ? sa[t][q & 3] : sb[t][q & 3]);
+            if (q > 0) {
+                const int e = q - 1;
+                l_run[t] += prev;
+                pbits[t][e & 1] = __float_as_uint(prev);
+                // p = hi + lo with hi the upper 16 bits of p (truncated) and lo the upper 16 bits of
+                // the exact remainder: 2^-16 relative, two byte permutes per pair of values
+                rbits[t][e & 1] = __float_as_uint(prev - __uint_as_float(pbits[t][e & 1] & 0xffff0000u));
+                if (e & 1) {
+                    hi4[t][e >> 1] = __builtin_amdgcn_perm(pbits[t][1], pbits[t][0], 0x07060302u);
+                    lo4[t][e >> 1] = __builtin_amdgcn_perm(rbits[t][1], rbits[t][0], 0x07060302u);
+                }
+            }
         }
-        // The operands of a K-step are asked for DEPTH K-steps before its products are issued,
-        // and the order is pinned: left to itself the compiler keeps one read ahead, issues the
-        // product that needs the newest operand first, and every other product then waits for
-        // LDS (the two wavefronts of a SIMD cannot cover a latency each of them hits at once).
-        constexpr int DEPTH = (KK < 2 || P > 256) ? 1 : 2;
-        uint4 ra[KK], rb[KK];
+    };
+    auto probs_done = [&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int kk = 0; kk < DEPTH; ++kk) {
-            ra[kk] = kt_a[kk * 64 + lane];
-            rb[kk] = kt_b[kk * 64 + lane];
+        for (int t = 0; t < TILES; ++t) {
+            ph[t] = __builtin_bit_cast(bf16x8_t, u4{hi4[t][0], hi4[t][1], hi4[t][2], hi4[t][3]});
+            pl[t] = __builtin_bit_cast(bf16x8_t, u4{lo4[t][0], lo4[t][1], lo4[t][2], lo4[t][3]});
         }
+    };
+    u4 ra[KK], rb[KK];
+    auto ask_k = [&](const u4 *kt, int kk) __attribute__((always_inline)) {
+        ra[kk] = kt[kk * 64 + lane];
+        rb[kk] = kt[TILE_U4 + kk * 64 + lane];
+    };
+    u4 rva[KK], rvb[KK];
+    auto ask_v = [&](const u4 *vt, int kk) __attribute__((always_inline)) {
+        rva[kk] = vt[kk * 64 + lane];
+        rvb[kk] = vt[TILE_U4 + kk * 64 + lane];
+    };
+    // window 1: scores of the pair whose K tiles lie at kt (its first operands asked for already),
+    // between them the probabilities of the settled pair; the first V operands of `vt` at the end
+    auto scores = [&](const u4 *kt, const u4 *vt, auto with_probs, auto copies) __attribute__((always_inline)) {
+        constexpr bool PROBS = decltype(with_probs)::value;
+        constexpr int BEATS = 2 * KK; // (k-step, hi or lo half)
+        float4_t na[TILES], nb[TILES];
+        int q = 0;
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) {
-            if (kk + DEPTH < KK) {
-                ra[kk + DEPTH] = kt_a[(kk + DEPTH) * 64 + lane];
-                rb[kk + DEPTH] = kt_b[(kk + DEPTH) * 64 + lane];
-            }
-            __builtin_amdgcn_sched_barrier(0);
+            if (kk + DEPTH < KK) ask_k(kt, kk + DEPTH);
+            copies(kk);
+            if (PROBS && kk + DEPTH >= KK) ask_v(vt, kk + DEPTH - KK);
             const bf16x8_t ka = __builtin_bit_cast(bf16x8_t, ra[kk]);
             const bf16x8_t kb = __builtin_bit_cast(bf16x8_t, rb[kk]);
 #pragma unroll
-            for (int t = 0; t < TILES; ++t) {
-                sa0[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, qh[t][kk], sa0[t], 0, 0, 0);
-                sb0[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb, qh[t][kk], sb0[t], 0, 0, 0);
-                sa1[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, ql[t][kk], sa1[t], 0, 0, 0);
-                sb1[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb, ql[t][kk], sb1[t], 0, 0, 0);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        // the first V operands of the pair travel while the softmax runs
-        uint4 rv0[KK], rv1[KK];
+            for (int h = 0; h < 2; ++h) {
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int kk = 0; kk < DEPTH; ++kk) {
-            rv0[kk] = vt[kk * 128 + lane];
-            rv1[kk] = vt[kk * 128 + 64 + lane];
+                for (int t = 0; t < TILES; ++t) {
+                    const bf16x8_t qv = h ? ql[t][kk] : qh[t][kk];
+                    na[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, qv, kk + h == 0 ? neg_m[t] : na[t], 0, 0, 0);
+                    nb[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb, qv, kk + h == 0 ? neg_m[t] : nb[t], 0, 0, 0);
+                }
+                if (PROBS) {
+                    // steps done by the end of this beat
+                    const int until = ((kk * 2 + h + 1) * 9) / BEATS;
+#pragma unroll
+                    for (int k = 0; k < 9; ++k)
+                        if (k >= q && k < until) prob_step(k);
+                    q = until;
+                }
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
-        bf16x8_t ph[TILES], pl[TILES];
+        if (PROBS) probs_done();
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
-            float sv[8];
-            {
-                const float4_t xa = sa0[t] + sa1[t], xb = sb0[t] + sb1[t];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    sv[i] = xa[i];
-                    sv[4 + i] = xb[i];
-                }
-            }
-            const bool interior = has_b && g.ring_rows == 0 && slot_a >= t_ws_hi[t] && slot_a + 31 <= t_lim_lo[t];
-            if (!interior || !use[t]) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int slot = slot_a + (e >> 2) * 16 + j * 4 + (e & 3);
-                    int pos = slot;
-                    if (g.ring_rows > 0)
-                        pos = slot <= a.ring_t ? a.ring_base + slot : a.ring_base - g.ring_rows + slot;
-                    const bool ok = use[t] && (e < 4 || has_b) && pos >= my_ws[t] && pos <= my_limit[t];
-                    sv[e] = ok ? sv[e] : -INFINITY;
-                }
-            }
-            float m_blk = fmaxf(fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3])),
-                                fmaxf(fmaxf(sv[4], sv[5]), fmaxf(sv[6], sv[7])));
-            m_blk = rows_max(m_blk);
-            const float m_new = fmaxf(m_run[t], m_blk);
-            const float m_safe = m_new == -INFINITY ? 0.0f : m_new;
-            const float alpha = fast_exp2(m_run[t] - m_safe);
-            // p = hi + lo with hi the upper 16 bits of p (truncated) and lo the upper 16 bits of
-            // the exact remainder: 2^-16 relative, two byte permutes per pair of values
-            float psum = 0.0f;
-            uint32_t pb_[8], rb_[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float pv = fast_exp2(sv[e] - m_safe);
-                psum += pv;
-                pb_[e] = __float_as_uint(pv);
-                rb_[e] = __float_as_uint(pv - __uint_as_float(pb_[e] & 0xffff0000u));
-            }
-            ph[t] = __builtin_bit_cast(bf16x8_t, make_uint4(__builtin_amdgcn_perm(pb_[1], pb_[0], 0x07060302u),
-                                                            __builtin_amdgcn_perm(pb_[3], pb_[2], 0x07060302u),
-                                                            __builtin_amdgcn_perm(pb_[5], pb_[4], 0x07060302u),
-                                                            __builtin_amdgcn_perm(pb_[7], pb_[6], 0x07060302u)));
-            pl[t] = __builtin_bit_cast(bf16x8_t, make_uint4(__builtin_amdgcn_perm(rb_[1], rb_[0], 0x07060302u),
-                                                            __builtin_amdgcn_perm(rb_[3], rb_[2], 0x07060302u),
-                                                            __builtin_amdgcn_perm(rb_[5], rb_[4], 0x07060302u),
-                                                            __builtin_amdgcn_perm(rb_[7], rb_[6], 0x07060302u)));
-            l_run[t] = l_run[t] * alpha + psum;
-            m_run[t] = m_new;
-            if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
-#pragma unroll
-                for (int c = 0; c < NT; ++c) o[t][c] *= alpha;
-            }
+            sa[t] = na[t];
+            sb[t] = nb[t];
         }
-        // O^T += V^T . P^T over the 32 keys of the pair, the V registers shared by the tiles.
-        // Without a page B its probabilities are zero and its place holds a page the layer
-        // owns (fetch_step clamps), so the products vanish.
-        __builtin_amdgcn_sched_barrier(0);
+    };
+    // window 2: O^T += V^T . P^T over the 32 keys of the pair
+    auto accumulate = [&](const u4 *vt, auto copies) __attribute__((always_inline)) {
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) {
-            if (kk + DEPTH < KK) {
-                rv0[kk + DEPTH] = vt[(kk + DEPTH) * 128 + lane];
-                rv1[kk + DEPTH] = vt[(kk + DEPTH) * 128 + 64 + lane];
-            }
+            if (kk + DEPTH < KK) ask_v(vt, kk + DEPTH);
+            copies(kk);
             __builtin_amdgcn_sched_barrier(0);
-            const bf16x8_t v0 = __builtin_bit_cast(bf16x8_t, rv0[kk]);
-            const bf16x8_t v1 = __builtin_bit_cast(bf16x8_t, rv1[kk]);
+            // a lane's unit holds four keys of dims n and n + 16: both pages' halves side by side are the
+            // 32-key operands of the two dim tiles
+            const bf16x8_t v0 = __builtin_bit_cast(bf16x8_t, u4{rva[kk].x, rva[kk].y, rvb[kk].x, rvb[kk].y});
+            const bf16x8_t v1 = __builtin_bit_cast(bf16x8_t, u4{rva[kk].z, rva[kk].w, rvb[kk].z, rvb[kk].w});
 #pragma unroll
             for (int t = 0; t < TILES; ++t) {
                 o[t][2 * kk] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v0, ph[t], o[t][2 * kk], 0, 0, 0);
@@ -399,18 +493,73 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a) 
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-      }
-      store_step<P, PG, THREADS>(stage, kv_lds + ((step + 1) & 1) * BUF_U4, tid, a, pb0, min(step + 1, n_steps - 1),
-                                 n_it, wg_ws_lo, wg_lim_hi);
-      __syncthreads();
+    };
+
+    // ---- first pair's scores
+    const int n_steps = (n_groups + SP - 1) / SP;
+    copies_landed();
+    __syncthreads();
+    clear_v(0, kv_lds + HALF_U4);
+#pragma unroll
+    for (int kk = 0; kk < DEPTH; ++kk) ask_k(kv_lds + BUF_U4 + half * 2 * TILE_U4, kk);
+    scores(kv_lds + BUF_U4 + half * 2 * TILE_U4, nullptr, std::false_type{}, [](int) {});
+    settle(half);
+    __syncthreads(); // the second buffer is free
+
+    for (int step = 0; step < n_steps; ++step) {
+        const u4 *buf = kv_lds + (step & 1) * BUF_U4;
+#pragma unroll
+        for (int pp = 0; pp < SP; ++pp) {
+            const int group = step * SP + pp;
+            if (group >= n_groups) continue; // uniform
+            const u4 *kt = buf + (pp * HALVES + half) * 2 * TILE_U4;
+            const u4 *vt = kt + HALF_U4;
+#pragma unroll
+            for (int kk = 0; kk < DEPTH; ++kk) ask_k(kt, kk);
+            // (after the last step the copies re-read its pages into the idle buffer)
+            scores(kt, vt, std::true_type{}, [&](int kk) __attribute__((always_inline)) { copy_slot(2 * KK * pp + kk, step); });
+            accumulate(vt, [&](int kk) __attribute__((always_inline)) { copy_slot(2 * KK * pp + KK + kk, step); });
+            settle((group + 1) * HALVES + half);
+        }
+        copies_landed();
+        __syncthreads();
+        if (step + 1 < n_steps) clear_v((step + 1) * SP * GP, kv_lds + ((step + 1) & 1) * BUF_U4 + HALF_U4);
+    }
+
+    // ---- the second half's states join the first's through LDS -----------------------------
+    if constexpr (HALVES > 1) {
+        static_assert(HALVES == 2 && TW * TILES * (NT + 1) * 64 <= 2 * BUF_U4, "the second half's states fit the page buffers");
+        float4_t *xo = reinterpret_cast<float4_t *>(kv_lds) + (tw * TILES) * (NT + 1) * 64 + lane; // (the loop ends in a barrier)
+        if (half == 1) {
+#pragma unroll
+            for (int t = 0; t < TILES; ++t) {
+#pragma unroll
+                for (int u = 0; u < NT; ++u) xo[(t * (NT + 1) + u) * 64] = o[t][u];
+                xo[(t * (NT + 1) + NT) * 64] = float4_t{thr[t] == -INFINITY ? -INFINITY : m_base[t], l_run[t], 0.f, 0.f};
+            }
+        }
+        __syncthreads();
+        if (half == 1) return;
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            const float4_t ml = xo[(t * (NT + 1) + NT) * 64];
+            const float m0 = thr[t] == -INFINITY ? -INFINITY : m_base[t], m1 = ml[0];
+            const float mx = fmaxf(m0, m1);
+            const float m_safe = mx == -INFINITY ? 0.0f : mx;
+            const float w0 = fast_exp2(m0 - m_safe), w1 = fast_exp2(m1 - m_safe);
+            l_run[t] = l_run[t] * w0 + ml[1] * w1;
+#pragma unroll
+            for (int u = 0; u < NT; ++u) o[t][u] = o[t][u] * w0 + xo[(t * (NT + 1) + u) * 64] * w1;
+            m_base[t] = m_safe;
+            thr[t] = mx == -INFINITY ? -INFINITY : 8.0f;
+        }
     }
 
     // ---- every wavefront writes its own slots -------------------------------------------
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
-        float l = l_run[t];
-        l = rows_sum(l);
-        const int slot = wg_slot0 + (wave * TILES + t) * 16 + n;
+        const float l = rows_sum(l_run[t]);
+        const int slot = wg_slot0 + (tw * TILES + t) * 16 + n;
         if (!t_on[t] || slot >= n_slots) continue;
         float *dst;
         float scale = 1.0f;
@@ -421,15 +570,15 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a) 
             const long pidx = ((long)kvh * a.splits_total + a.split_base + split) * n_slots + slot;
             dst = a.part_o + pidx * g.head_dim;
             if (j == 0) {
-                a.part_m[pidx] = m_run[t];
+                a.part_m[pidx] = thr[t] == -INFINITY ? -INFINITY : m_base[t];
                 a.part_l[pidx] = l;
             }
         }
         const bool vec_ok = (g.head_dim & 3) == 0;
 #pragma unroll
-        for (int c = 0; c < NT; ++c) {
-            const int col = c * 16 + j * 4;
-            const float4_t v = o[t][c] * scale;
+        for (int u = 0; u < NT; ++u) {
+            const int col = u * 16 + j * 4;
+            const float4_t v = o[t][u] * scale;
             if (vec_ok) {
                 if (col < g.head_dim) *reinterpret_cast<float4_t *>(dst + col) = v;
             } else {
@@ -512,37 +661,48 @@ hipError_t launch_merge_rows(const DecodeArgs &a, hipStream_t s) {
 }
 
 // Query slots one workgroup of the kernel covers for a padded head_dim.
-int prefill_tile_slots(int P, bool two_tiles) {
+int prefill_tile_slots(int P, TileShape shape) {
     if (P > 256) return 64; // four wavefronts, one per SIMD (the accumulators and query halves are 256 registers)
-    return two_tiles && prefill_two_tiles_possible(P) ? 256 : 128;
+    return shape == TileShape::two_tiles && P <= 128 ? 256 : shape == TileShape::halves ? 64 : 128;
 }
-// Two query tiles per wavefront need twice the accumulator and query registers: up to
-// head_dim 128.
-bool prefill_two_tiles_possible(int P) { return P <= 128; }
 
-template <int P, int TILES, int PG, int WAVES = 8>
-static hipError_t launch_tiles(const DecodeArgs &a, dim3 grid, hipStream_t s) {
-    constexpr size_t lds = (size_t)2 * PG * 2 * (P / 32) * 64 * sizeof(uint4);
+template <int P, int TILES, int SP, int WAVES, int HALVES, bool RING>
+static hipError_t launch_tiles_of(const DecodeArgs &a, const ChunkPages &c, dim3 grid, hipStream_t s) {
+    constexpr size_t lds = (size_t)2 * 2 * SP * HALVES * 2 * (P / 32) * 64 * sizeof(uint4);
+    static_assert(lds <= 160 * 1024, "two steps of pages share the LDS of a compute unit");
     static std::atomic<uint64_t> lds_ok{0}; // per instantiation
     {
-        hipError_t e = allow_full_lds(reinterpret_cast<const void *>(&prefill_tile_kernel<P, TILES, PG, WAVES>), lds_ok);
+        hipError_t e = allow_full_lds(reinterpret_cast<const void *>(&prefill_tile_kernel<P, TILES, SP, WAVES, HALVES, RING>), lds_ok);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL((prefill_tile_kernel<P, TILES, PG, WAVES>), grid, dim3(WAVES * 64), lds, s, a);
+    hipLaunchKernelGGL((prefill_tile_kernel<P, TILES, SP, WAVES, HALVES, RING>), grid, dim3(WAVES * 64), lds, s, a, c);
     return hipGetLastError();
 }
+template <int P, int TILES, int SP, int WAVES = 8, int HALVES = 1>
+static hipError_t launch_tiles(const DecodeArgs &a, const ChunkPages &c, dim3 grid, hipStream_t s) {
+    return c.ring_pages > 0 ? launch_tiles_of<P, TILES, SP, WAVES, HALVES, true>(a, c, grid, s)
+                            : launch_tiles_of<P, TILES, SP, WAVES, HALVES, false>(a, c, grid, s);
+}
 
-hipError_t launch_prefill_tiles(const DecodeArgs &a, hipStream_t s) {
+hipError_t launch_prefill_tiles(const DecodeArgs &a, const ChunkPages &c, TileShape shape, hipStream_t s) {
     const int n_slots = a.n_queries * a.g.gqa;
-    const bool two = a.tiles2 && prefill_two_tiles_possible(a.g.P);
-    const int per_wg = prefill_tile_slots(a.g.P, two);
+    const int per_wg = prefill_tile_slots(a.g.P, shape);
+    const bool two = per_wg == 256, halves = shape == TileShape::halves;
     dim3 grid((unsigned)a.splits, (unsigned)a.g.kv_heads, (unsigned)((n_slots + per_wg - 1) / per_wg));
     switch (a.g.P) {
-    case 32: return two ? launch_tiles<32, 2, 8>(a, grid, s) : launch_tiles<32, 1, 8>(a, grid, s);
-    case 64: return two ? launch_tiles<64, 2, 8>(a, grid, s) : launch_tiles<64, 1, 8>(a, grid, s);
-    case 128: return two ? launch_tiles<128, 2, 8>(a, grid, s) : launch_tiles<128, 1, 8>(a, grid, s);
-    case 256: return launch_tiles<256, 1, 4>(a, grid, s);
-    case 512: return launch_tiles<512, 1, 2, 4>(a, grid, s);
+    case 32:
+        if (halves) return launch_tiles<32, 1, 2, 8, 2>(a, c, grid, s);
+        return two ? launch_tiles<32, 2, 4>(a, c, grid, s) : launch_tiles<32, 1, 4>(a, c, grid, s);
+    case 64:
+        if (halves) return launch_tiles<64, 1, 2, 8, 2>(a, c, grid, s);
+        return two ? launch_tiles<64, 2, 4>(a, c, grid, s) : launch_tiles<64, 1, 4>(a, c, grid, s);
+    case 128:
+        if (halves) return launch_tiles<128, 1, 2, 8, 2>(a, c, grid, s);
+        return two ? launch_tiles<128, 2, 2>(a, c, grid, s) : launch_tiles<128, 1, 4>(a, c, grid, s);
+    case 256:
+        if (halves) return launch_tiles<256, 1, 1, 8, 2>(a, c, grid, s);
+        return launch_tiles<256, 1, 2>(a, c, grid, s);
+    case 512: return launch_tiles<512, 1, 1, 4>(a, c, grid, s);
     default: return hipErrorInvalidValue;
     }
 }

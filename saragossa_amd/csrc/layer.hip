@@ -138,7 +138,8 @@ struct Tuning {
     size_t target_wgs;      // workgroups a decode launch aims for
     size_t min_pages;       // pages per split at least (0 = one per wavefront)
     size_t forced_waves;    // 4 or 8, 0 = by shape
-    bool q_vec, fused_append, prefill_tiles;
+    bool q_vec, fused_append;
+    size_t prefill_tiles;   // 0 = never, 1 = by shape, 2 = every chunk of 64 query slots and more
     size_t prefill_wgs, prefill_max_splits;
     long prefill_tiles2_min_pages; // -1 = by head_dim
 };
@@ -154,7 +155,7 @@ const Tuning &tuning() {
         t.forced_waves = env_usize("SKV_DECODE_WAVES", 0);
         t.q_vec = env_usize("SKV_Q_VEC", 1) != 0;
         t.fused_append = env_usize("SKV_FUSED_APPEND", 1) != 0;
-        t.prefill_tiles = env_usize("SKV_PREFILL_TILES", 1) != 0;
+        t.prefill_tiles = env_usize("SKV_PREFILL_TILES", 1);
         t.prefill_wgs = std::max<size_t>(env_usize("SKV_PREFILL_WGS", 256), 1);
         t.prefill_max_splits = std::max<size_t>(env_usize("SKV_PREFILL_MAX_SPLITS", 512), 1);
         t.prefill_tiles2_min_pages = std::getenv("SKV_PREFILL_TILES2_MIN_PAGES")
@@ -178,16 +179,41 @@ int choose_waves(const skv_layer *L, int n_pages_scan) {
 
 size_t decode_target_wgs() { return tuning().target_wgs; }
 
-// Two 16-slot query tiles per wavefront in the prefill tile kernel halve the LDS reads and
-// barriers per product but also the number of workgroups. Measured with 512-row chunks: at
-// head_dim 128 they win from about 256 pages of context on (+15 % at 16k-32k rows, -4..-20 %
-// under 2k rows), at head_dim 64 from about 512 pages (+10 % at 32k rows, -10..-20 % under 4k);
-// at 256 the registers do not allow them.
-bool prefill_two_tiles(const Geom &g, int n_pages_scan) {
-    if (!prefill_two_tiles_possible(g.P)) return false;
+// Shape of the prefill tile kernel's workgroups for a chunk of n_slots query slots per kv head, each
+// walking about n_pages pages. A workgroup of halves covers 64 slots instead of 128, so it fills
+// the device with fewer splits, or with none where 128-slot workgroups need two and a merge; it
+// copies each page for half as many slots. The gain is fixed, the price grows with the pages walked:
+// whole chunks over one tile / two tiles / halves on one MI355X, in us, 512 rows of q32/kv8/hd128
+// over 0, 4096, 8192, 16384 rows: 31.0/39.2/20.2, 83.8/82.7/76.9, 137/131/135, 244/226/249; 256 rows over
+// 4096, 8192, 16384: 51.4/56.0/48.6, 77.6/79.7/76.8, 132/127/135; 512 rows of q16/kv2/hd256 (no two tiles, and halves
+// still need two splits) over 512, 2048, 4096: 41.1/39.1, 58.7/57.6, 81.2/83.2; 1024 rows over 2048, 4096,
+// 8192: 101/92.5, 150/146, 246/251; 1024 rows of hd128, where no shape is split, over 512, 4096, 8192:
+// 53.0/68.8/55.2, 147/151/154, 256/247/268. Two tiles (half the LDS reads per product, half the
+// workgroups) pay from about the same walks on.
+TileShape prefill_shape(const Geom &g, size_t n_slots, size_t n_pages) {
+    if (g.P > 256) return TileShape::one_tile;
     const long knob = tuning().prefill_tiles2_min_pages;
-    const long min_pages = knob >= 0 ? knob : (g.P <= 64 ? 512 : 256);
-    return (long)n_pages_scan >= min_pages;
+    if (knob >= 0) return g.P <= 128 && (long)n_pages >= knob ? TileShape::two_tiles : TileShape::one_tile;
+    const size_t wgs = (n_slots + 63) / 64 * (size_t)g.kv_heads, walk = wgs * n_pages;
+    if (wgs <= 256 && walk < (wgs >= 192 ? 110000u : 40000u)) return TileShape::halves;
+    return g.P <= 128 && walk >= (wgs <= 256 ? 110000u : 250000u) ? TileShape::two_tiles : TileShape::one_tile;
+}
+
+// Whether a chunk of n_slots query slots per kv head over n_pages pages takes the kernel that shares each
+// page among 64 to 256 slots through LDS, or the decode kernel's multi-query mode (speculative verify rows,
+// short chunks over short contexts): one workgroup per 16 slots that streams the pages into its own
+// registers, without a prologue to speak of, but asks for every page once per 16 slots. The line is
+// the number of (16 slots, page) pairs where those requests cost what the tile kernel's start does.
+// Whole chunks, tile kernel / multi-query mode, in us on one MI355X: q32/kv8/hd128, 32 rows over 2048,
+// 8192, 32000 rows: 21.5/15.6, 32.1/25.9, 53.9/80.2; 256 rows over 1024, 2048: 28.5/24.1, 35.3/35.7; 512 rows over
+// 0, 512: 19.7/19.4, 26.8/32.5; q16/kv2/hd256, 16 rows over 8192, 32000: 37.5/19.7, 58.0/44.9; 64 rows over
+// 2048, 8192: 29.8/25.2, 41.7/40.5; 256 rows over 1024, 2048: 34.5/30.1, 39.2/44.6; q8/kv2/hd512, 64 rows over 2048,
+// 8192: 43.4/36.6, 55.6/77.5; 128 rows over 1024, 2048: 43.4/42.3, 46.1/54.7; q8/kv2/hd64, 256 rows over
+// 1024, 2048: 17.0/16.0, 19.1/19.8; 512 rows over 512, 1024: 16.6/15.1, 17.7/19.0.
+bool takes_tile_kernel(const Geom &g, size_t n_slots, size_t n_pages) {
+    if (tuning().prefill_tiles != 1 || n_slots < 64) return tuning().prefill_tiles > 1 && n_slots >= 64;
+    const size_t limit = g.P <= 64 ? 18000 : g.P == 128 ? 42000 : g.P == 256 ? 22000 : 6000;
+    return (n_slots + 15) / 16 * (size_t)g.kv_heads * n_pages >= limit;
 }
 
 int choose_splits(const skv_layer *L, int n_pages_scan, size_t rows, int waves, size_t target_wgs) {
@@ -271,11 +297,13 @@ void fill_decode_args(const skv_layer *L, const float *q_dev, float *out_dev, si
 }
 
 // Split partials of a multi-query launch live in the context's scratch, grown on demand:
-// [kv_heads][n_sets][n_queries * gqa] of (o[head_dim], m, l).
-int32_t multi_query_partials(skv_layer *L, hipStream_t s, size_t n_sets, size_t n_queries, DecodeArgs &a) {
+// [kv_heads][n_sets][n_queries * gqa] of (o[head_dim], m, l); in front of them `page_bytes` for
+// pages of the chunk's own rows (*pages, a multiple of 256).
+int32_t multi_query_partials(skv_layer *L, hipStream_t s, size_t n_sets, size_t n_queries, DecodeArgs &a,
+                             size_t page_bytes = 0, void **pages = nullptr) {
     const Geom &g = L->g;
     const size_t n_part = (size_t)g.kv_heads * n_sets * n_queries * g.gqa;
-    const size_t need = n_part * ((size_t)g.head_dim + 2) * sizeof(float);
+    const size_t need = page_bytes + n_part * ((size_t)g.head_dim + 2) * sizeof(float);
     skv_ctx *c = L->ctx;
     void *buf = nullptr;
     void *old = nullptr;     // this stream's buffer, too small: freed once the stream has drained
@@ -317,10 +345,26 @@ int32_t multi_query_partials(skv_layer *L, hipStream_t s, size_t n_sets, size_t 
         slot.used = ++c->mq_clock;
         buf = p;
     }
-    a.part_o = reinterpret_cast<float *>(buf);
+    if (pages) *pages = buf;
+    a.part_o = reinterpret_cast<float *>(static_cast<char *>(buf) + page_bytes);
     a.part_m = a.part_o + n_part * g.head_dim;
     a.part_l = a.part_m + n_part;
     return SKV_OK;
+}
+
+// The layer's pages as the queries of a chunk walk them: from position 0 on on a full layer, from
+// position `lo` to the last row before `end` on a ring.
+ChunkPages layer_pages(const skv_layer *L, size_t lo, size_t end) {
+    ChunkPages c{};
+    c.n_old = INT32_MAX;
+    c.new_pos0 = INT32_MAX;
+    if (L->g.ring_rows > 0) {
+        c.n_old = lo < end ? (int)((end - 1) / 16 - lo / 16) + 1 : 0;
+        c.first_pos = (int)(lo / 16 * 16);
+        c.ring_pages = L->g.ring_rows / 16;
+        c.start = (int)(lo / 16 % (size_t)c.ring_pages);
+    }
+    return c;
 }
 
 // k_new / v_new non-null: the row at position len-1 has not been written yet and the
@@ -446,15 +490,22 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
         a.gate = pre->gate;
         a.q_head_stride = pre->q_head_stride;
     }
-    // Chunks of at least 64 query slots take the kernel that shares each K/V page among 128
-    // or 256 slots through LDS; shorter ones (speculative verify rows) the decode kernel's
-    // multi-query mode, one workgroup per 16 slots.
-    const bool use_tiles = tuning().prefill_tiles && n_queries > 1 && n_queries * (size_t)g.gqa >= 64;
+    const bool use_tiles = n_queries > 1 && takes_tile_kernel(g, n_queries * (size_t)g.gqa, (size_t)a.n_pages);
+    TileShape shape = TileShape::one_tile;
     if (n_queries > 1) {
         // split the context only while the query tiles alone leave compute units idle, and
         // keep the partials in the context's scratch
-        a.tiles2 = use_tiles && prefill_two_tiles(g, a.n_pages) ? 1 : 0;
-        const size_t per_wg = use_tiles ? (size_t)prefill_tile_slots(g.P, a.tiles2 != 0) : 16;
+        shape = prefill_shape(g, n_queries * (size_t)g.gqa, (size_t)a.n_pages);
+        if (!use_tiles && g.P <= 256 && tuning().forced_waves == 0) {
+            // eight wavefronts, one page each before the context is split; four where the slot tiles
+            // alone are two workgroups and more for every compute unit and narrow enough that it holds
+            // several (256 rows of q32/kv8/hd128 over 0, 1024 rows: 11.7/24.1 us with four, 14.1/24.4 with
+            // eight; 256 rows of q16/kv2/hd256: 14.2/30.1 and 13.5/24.6)
+            const size_t slot_tiles = (n_queries * (size_t)g.gqa + 15) / 16 * (size_t)g.kv_heads;
+            a.waves = g.P <= 128 && slot_tiles >= 512 ? 4 : 8;
+            a.splits = choose_splits(L, a.n_pages, L->len - window_start, a.waves, 256);
+        }
+        const size_t per_wg = use_tiles ? (size_t)prefill_tile_slots(g.P, shape) : 16;
         const size_t tiles = (n_queries * (size_t)g.gqa + per_wg - 1) / per_wg * (size_t)g.kv_heads;
         size_t want = std::max<size_t>((use_tiles ? tuning().prefill_wgs : 256) / tiles, 1);
         if (use_tiles) {
@@ -473,12 +524,22 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
         if (rc2) return rc2;
     }
     if (use_tiles) {
-        SKV_HIP(launch_prefill_tiles(a, s));
+        const size_t lo = std::max(window_start, skv_window_start(L->len - n_queries, L->window));
+        SKV_HIP(launch_prefill_tiles(a, layer_pages(L, lo, L->len), shape, s));
         if (a.splits > 1) SKV_HIP(launch_merge_rows(a, s));
         return SKV_OK;
     }
     SKV_HIP(launch_decode(a, s));
     return SKV_OK;
+}
+
+// Batches: whole groups of four rows at positions that are multiples of 4 write V in 16-byte units.
+void plan_batch(AppendArgs &a) {
+    if (a.n_rows < 8) return;
+    a.by_page = 1;
+    const long lead = (4 - (a.first_pos & 3)) & 3;
+    a.v_grp_first = (int)lead;
+    a.v_grp_rows = (int)((a.n_rows - lead) & ~3L);
 }
 
 int32_t encode_append(skv_layer *L, hipStream_t s, const float *k_dev, const float *v_dev,
@@ -512,13 +573,7 @@ int32_t encode_append(skv_layer *L, hipStream_t s, const float *k_dev, const flo
             L->floor_pos = std::max(L->floor_pos, L->len - (size_t)L->g.ring_rows);
         return SKV_OK;
     }
-    // whole groups of four rows at positions that are multiples of 4 write V in 16-byte units
-    if (a.n_rows >= 8) {
-        a.by_page = 1;
-        const long lead = (4 - (a.first_pos & 3)) & 3;
-        a.v_grp_first = (int)lead;
-        a.v_grp_rows = (int)((a.n_rows - lead) & ~3L);
-    }
+    plan_batch(a);
     SKV_HIP(launch_append(a, s));
     L->len += n_rows;
     if (L->g.ring_rows > 0 && L->len > (size_t)L->g.ring_rows)
@@ -1023,22 +1078,70 @@ int32_t skv_decode_step_static_device(skv_layer *L, skv_stream stream, const voi
     return skv::fail_exception();
 }
 
-// A chunk of c > 1 rows on a ring layer. The ring holds exactly the window (rounded up to a
-// page), so the chunk's own rows overwrite rows its first queries still attend. The chunk
-// is therefore attended in two phases around the append: first every query over the rows
-// already in the ring (capped at the last old position), then, once the chunk is appended,
-// over the chunk's own rows (from its first position up to each query's own). Both phases
-// leave (o, m, l) partials; one merge produces the context. c <= ring_rows.
+// A chunk of c > 1 rows on a bf16 ring layer. The ring holds little more than the window, so the
+// chunk's own rows overwrite rows its first queries still attend. They are therefore first
+// written to pages of the context's scratch; one launch attends the ring's rows and them, in the
+// order of positions, each workgroup only the pages its slots' windows touch; then the rows go
+// into the ring. (Two launches around the append, over the old rows and over the new ones,
+// each over the whole ring and with partials of its own: 93 us for 512 rows of q16/kv8/hd256 on a
+// ring of 1056 rows, against 50 us.)
 static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const float *k, const float *v,
                           size_t c, float *out) {
     const Geom &g = L->g;
     const size_t base = L->len;
-    const bool two = !g.f32 && prefill_two_tiles(g, L->n_pages);
-    const size_t per_wg = g.f32 ? 16 : (size_t)prefill_tile_slots(g.P, two);
+    // the rows in the ring that the first query attends (it attends the most of them)
+    const size_t lo = std::max(L->floor_pos, skv_window_start(base, L->window));
+    ChunkPages pages = layer_pages(L, lo, base);
+    pages.new_pos0 = (int)base;
+    pages.new_first = (int)(base / 16 * 16);
+    const size_t n_new = (base + c - 1) / 16 - base / 16 + 1;
+    const size_t pool_bytes = n_new * (size_t)g.page_elems * sizeof(uint16_t); // of K and of V
+
+    DecodeArgs a{};
+    L->len += c; // the queries are the last c rows
+    fill_decode_args(L, q, out, L->floor_pos, nullptr, nullptr, c, tuning().prefill_wgs, a);
+    L->len -= c;
+    // pages a workgroup of one tile row walks: the window and the workgroup's own rows
+    const size_t walked = std::min<size_t>((size_t)pages.n_old + n_new, L->window / 16 + 2);
+    const TileShape shape = prefill_shape(g, c * (size_t)g.gqa, walked);
+    const size_t per_wg = (size_t)prefill_tile_slots(g.P, shape);
     const size_t tiles = (c * (size_t)g.gqa + per_wg - 1) / per_wg * (size_t)g.kv_heads;
-    auto launch_chunk = [&](const DecodeArgs &a) { return g.f32 ? launch_f32_split(a, s) : launch_prefill_tiles(a, s); };
+    size_t want = std::max<size_t>(tuning().prefill_wgs / tiles, 1);
+    want = std::min<size_t>(want, std::max<size_t>(walked / 16, 1));
+    a.splits = (int)std::min<size_t>(want, tuning().prefill_max_splits);
+    a.splits_total = a.splits;
+    void *scratch = nullptr;
+    int32_t rc = multi_query_partials(L, s, a.splits > 1 ? (size_t)a.splits : 0, c, a, 2 * pool_bytes, &scratch);
+    if (rc) return rc;
+    AppendArgs w{};
+    w.k_src = k;
+    w.v_src = v;
+    w.k_pool = static_cast<uint16_t *>(scratch);
+    w.v_pool = w.k_pool + pool_bytes / sizeof(uint16_t);
+    w.first_pos = (long)(base % 16);
+    w.n_rows = (int)c;
+    w.g = g;
+    w.g.ring_rows = 0;
+    plan_batch(w);
+    SKV_HIP(launch_append(w, s));
+    pages.k_new = w.k_pool;
+    pages.v_new = w.v_pool;
+    SKV_HIP(launch_prefill_tiles(a, pages, shape, s));
+    if (a.splits > 1) SKV_HIP(launch_merge_rows(a, s));
+    return encode_append(L, s, k, v, c);
+}
+
+// The same on an f32 ring layer, c <= ring_rows, attended in two phases around the append: first every query over the rows
+// already in the ring (capped at the last old position), then, once the chunk is appended,
+// over the chunk's own rows (from its first position up to each query's own). Both phases
+// leave (o, m, l) partials; one merge produces the context. c <= ring_rows.
+static int32_t ring_chunk_f32(skv_layer *L, hipStream_t s, const float *q, const float *k, const float *v,
+                              size_t c, float *out) {
+    const Geom &g = L->g;
+    const size_t base = L->len;
+    const size_t tiles = (c * (size_t)g.gqa + 15) / 16 * (size_t)g.kv_heads;
     auto splits_for = [&](int n_pages) {
-        size_t want = std::max<size_t>((g.f32 ? 2 : 1) * tuning().prefill_wgs / tiles, 1);
+        size_t want = std::max<size_t>(2 * tuning().prefill_wgs / tiles, 1);
         want = std::min<size_t>(want, std::max<size_t>((size_t)n_pages / 8, 1));
         return (int)std::min<size_t>(want, tuning().prefill_max_splits);
     };
@@ -1048,7 +1151,6 @@ static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const flo
         fill_decode_args(L, q, out, L->floor_pos, nullptr, nullptr, c, tuning().prefill_wgs, a1);
         a1.q_pos0 = (int)base;
         a1.limit_cap = (int)base - 1;
-        a1.tiles2 = two ? 1 : 0;
         s1 = splits_for(a1.n_pages);
     }
     const int pages_after = (int)std::min<size_t>((base + c + 15) / 16, (size_t)L->n_pages);
@@ -1060,13 +1162,12 @@ static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const flo
         a1.splits_total = total;
         int32_t rc = multi_query_partials(L, s, (size_t)total, c, a1);
         if (rc) return rc;
-        SKV_HIP(launch_chunk(a1));
+        SKV_HIP(launch_f32_split(a1, s));
     }
     int32_t rc = encode_append(L, s, k, v, c);
     if (rc) return rc;
     fill_decode_args(L, q, out, std::max(base, L->floor_pos), nullptr, nullptr, c, tuning().prefill_wgs, a3);
     a3.q_pos0 = (int)base;
-    a3.tiles2 = two ? 1 : 0;
     a3.splits = s3;
     a3.split_base = s1;
     a3.splits_total = total;
@@ -1074,7 +1175,7 @@ static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const flo
         rc = multi_query_partials(L, s, (size_t)total, c, a3);
         if (rc) return rc;
     }
-    SKV_HIP(launch_chunk(a3));
+    SKV_HIP(launch_f32_split(a3, s));
     if (total > 1) SKV_HIP(launch_merge_rows(a3, s));
     return SKV_OK;
 }
@@ -1089,16 +1190,20 @@ int32_t skv_prefill_chunk_device(skv_layer *L, skv_stream stream, const float *q
         return fail(SKV_ERR_DIMENSION, "append KV résident: capacité " +
                                            std::to_string(L->capacity) + " atteinte (overflow)");
     const size_t kv_dim = skv_kv_dim(L), q_dim = (size_t)L->g.q_heads * L->g.head_dim;
-    // Ring layers take the chunk in steps of at most the ring's rows (see ring_chunk).
+    // f32 ring layers take the chunk in steps of at most the ring's rows (see ring_chunk_f32).
     size_t step = std::min<size_t>(n_rows, 4096);
-    if (L->g.ring_rows > 0) step = std::min(step, (size_t)L->g.ring_rows);
+    if (L->g.ring_rows > 0 && L->g.f32) step = std::min(step, (size_t)L->g.ring_rows);
     const float *q = q_dev, *k = (const float *)k_dev, *v = (const float *)v_dev;
     float *out = out_dev;
     for (size_t done = 0; done < n_rows; done += step) {
         const size_t c = std::min(step, n_rows - done);
         int32_t rc;
-        if (L->g.ring_rows > 0 && c > 1) {
-            rc = ring_chunk(L, as_stream(stream), q, k, v, c, out);
+        // the first query attends window - 1 rows in front of the chunk: where none of them (no row at
+        // all before the ring is full) is overwritten by the chunk's rows, the chunk is appended first
+        // like any other
+        const size_t ring = (size_t)L->g.ring_rows;
+        if (ring > 0 && c > 1 && L->len + c > ring && c + L->window > ring + 1) {
+            rc = (L->g.f32 ? ring_chunk_f32 : ring_chunk)(L, as_stream(stream), q, k, v, c, out);
             if (rc) return rc;
             q += c * q_dim;
             k += c * kv_dim;

@@ -92,7 +92,7 @@ struct AppendArgs {
     const float *v_src;
     uint16_t *k_pool;
     uint16_t *v_pool;
-    const int32_t *table;
+    const int32_t *table; // null = page i of the pools is page i of the positions
     long first_pos; // position of the first appended row
     int n_rows;
     // rows [v_grp_first, v_grp_first + v_grp_rows) of the batch start at a position that is a
@@ -160,11 +160,32 @@ struct DecodeArgs {
     const float *gate;
     int q_head_stride;
     int q_vec;              // q is 16-byte aligned and head_dim a multiple of 8: 16-byte loads
-    int tiles2;             // prefill tile kernel: two 16-slot query tiles per wavefront
     int xchg_off;           // split kernel: byte offset in LDS of the wavefronts' exchange area (0 = it reuses the staging area); set by the launcher
     Geom g;
 };
 static_assert(sizeof(DecodeArgs) <= 256, "sixteen of them must fit the kernel argument block");
+
+// The pages a chunk's queries walk, as a list in the order of positions: n_old entries of the
+// layer's own pages, then pages outside the layer that hold the chunk's new rows (ring layers,
+// whose own pages must not be overwritten while they are still attended; none on full layers).
+// Both kinds are aligned to positions that are multiples of 16, so the page in which the new
+// rows begin is in the list twice: its old entry speaks for positions below new_pos0, its new one
+// for the others.
+struct ChunkPages {
+    int n_old;           // INT32_MAX = the layer's pages only
+    int first_pos;       // position of entry 0's first row
+    int start;           // entry e < n_old is table[start + e], less ring_pages when past the ring's end
+    int ring_pages;      // 0 = not a ring
+    int new_pos0;        // first new position (INT32_MAX = none)
+    int new_first;       // position of the first new page's first row
+    const uint16_t *k_new; // tiles of the new pages, in order
+    const uint16_t *v_new;
+};
+
+// How a workgroup of the prefill tile kernel divides its work among its wavefronts: one 16-slot
+// query tile each; two tiles each (head_dim up to 128); or two halves, each half of the
+// wavefronts holding the same tiles and walking every other page pair.
+enum class TileShape { one_tile, two_tiles, halves };
 
 // Standalone per-head RMSNorm + rotation of one row (the same arithmetic as the fused step).
 struct NormRopeArgs {
@@ -336,9 +357,8 @@ hipError_t launch_decode(const DecodeArgs &a, hipStream_t s);
 hipError_t launch_decode_batch(const DecodeBatchArgs &b, int n_seq, hipStream_t s);
 hipError_t launch_f32_split_batch(const DecodeBatchArgs &b, int n_seq, int max_splits, hipStream_t s);
 hipError_t launch_merge(const DecodeArgs &a, hipStream_t s);        // split-K partials -> context
-hipError_t launch_prefill_tiles(const DecodeArgs &a, hipStream_t s); // chunked prefill, no merge
-int prefill_tile_slots(int P, bool two_tiles);
-bool prefill_two_tiles_possible(int P);
+hipError_t launch_prefill_tiles(const DecodeArgs &a, const ChunkPages &c, TileShape shape, hipStream_t s); // chunked prefill, no merge
+int prefill_tile_slots(int P, TileShape shape);
 hipError_t launch_merge_rows(const DecodeArgs &a, hipStream_t s);    // the same merge for many query slots
 hipError_t launch_naive(const NaiveArgs &a, hipStream_t s);
 int decode_max_splits();

@@ -1,0 +1,83 @@
+"""The prefill tile kernel in each of its workgroup shapes, at the edges of its tiles: chunks that end
+inside a slot tile, a page pair and a barrier step; caches that begin the chunk inside a page; ring
+layers whose chunk starts before, at and long after the ring is full (its rows are attended
+from pages of their own and appended afterwards). Contexts within 1e-4 of the oracle (queries and
+probabilities carry 16 bits: about 1e-5 of values of order one), rows bit for bit."""
+import os
+
+import numpy as np
+import pytest
+
+import oracle
+import saragossa_amd as skv
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = {"halves": {}, "one_tile": {"SKV_PREFILL_TILES2_MIN_PAGES": "1000000"}, "two_tiles": {"SKV_PREFILL_TILES2_MIN_PAGES": "0"}}
+
+
+@pytest.fixture(params=SHAPES, ids=str)
+def shape(request):
+    env = dict(SHAPES[request.param], SKV_PREFILL_TILES="2")  # the tile kernel for every chunk of 64 slots and more
+    saved = {k: os.environ.get(k) for k in env}
+    os.environ.update(env)
+    skv.flags.reload()
+    yield request.param
+    for k, v in saved.items():
+        os.environ.pop(k) if v is None else os.environ.__setitem__(k, v)
+    skv.flags.reload()
+
+
+@pytest.mark.parametrize("dims,window,base,chunks", [
+    ((4, 2, 16), 0, 0, (33, 64)),        # the narrowest head, from an empty cache
+    ((8, 2, 64), 0, 31, (17, 130)),      # base at the end of a page pair
+    ((4, 1, 80), 0, 5, (16, 65)),        # padded head, slots in one tile row and one more
+    ((32, 8, 128), 0, 509, (66,)),       # splits of unequal length
+    ((16, 2, 256), 0, 255, (41, 8)),
+    ((6, 1, 40), 0, 1, (11, 43)),        # heads per group not a power of two, 66 and 258 slots
+    ((4, 1, 320), 0, 77, (16, 40)),      # wide heads
+    ((8, 2, 64), 40, 0, (100, 200)),     # ring: chunk longer than the ring from the start
+    ((8, 2, 64), 48, 47, (90, 17)),      # ring: window of whole pages, chunk starts inside a page
+    ((16, 8, 256), 33, 300, (130,)),
+    ((4, 2, 16), 17, 64, (64, 33)),      # ring: chunk starts at a page boundary; padded head
+])
+def test_chunks_in_every_shape(state, shape, dims, window, base, chunks):
+    q_heads, kv_heads, head_dim = dims
+    kv_dim, q_dim = kv_heads * head_dim, q_heads * head_dim
+    rng = np.random.default_rng(base + head_dim)
+    kv = state.full_attention_bf16(base + sum(chunks), q_heads, kv_heads, head_dim, window=window)
+    kv.set_block_table(rng.permutation(kv.pages()).astype(np.int32))
+    lay = oracle.layout(q_heads, kv_heads, head_dim, sliding_window=window)
+    cache = oracle.LayerKvCache("bf16r")
+    if base:
+        k0, v0 = (rng.standard_normal((base, kv_dim), dtype=np.float32) for _ in range(2))
+        kv.seed(k0, v0, base)
+        cache.append_batch(k0, v0, lay)
+    for c in chunks:
+        q = rng.standard_normal((c, q_dim), dtype=np.float32)
+        k, v = (rng.standard_normal((c, kv_dim), dtype=np.float32) for _ in range(2))
+        got = kv.prefill_rows(q, k, v)
+        want = oracle.cached_attention_prefill_rows(q, k, v, cache, lay)
+        assert np.abs(got - want).max() <= 1e-4, (shape, c)
+    first = max(0, kv.len() - window) if window else 0
+    gk, gv = kv.read_rows_f32(first, kv.len() - first)
+    assert np.array_equal(gk, cache.keys()[first:]) and np.array_equal(gv, cache.values()[first:])
+    kv.close()
+
+
+def test_scores_that_climb(state, shape):
+    """Keys that grow along the context move the softmax base again and again (it follows a slot's
+    scores only once they pass it by 2^8), and fall below it by far more."""
+    rng = np.random.default_rng(3)
+    q_heads, kv_heads, head_dim, n = 8, 2, 64, 300
+    kv = state.full_attention_bf16(n, q_heads, kv_heads, head_dim)
+    lay = oracle.layout(q_heads, kv_heads, head_dim)
+    cache = oracle.LayerKvCache("bf16r")
+    q = np.abs(rng.standard_normal((n, q_heads * head_dim), dtype=np.float32))
+    scale = np.linspace(0.0, 9.0, n, dtype=np.float32)[:, None] * np.where(np.arange(n) % 3 == 0, -1.0, 1.0).astype(np.float32)[:, None]
+    k = np.abs(rng.standard_normal((n, kv_heads * head_dim), dtype=np.float32)) * scale
+    v = rng.standard_normal((n, kv_heads * head_dim), dtype=np.float32)
+    got = kv.prefill_rows(q, k, v)
+    want = oracle.cached_attention_prefill_rows(q, k, v, cache, lay)
+    # scores reach 9 * 64 * 0.64 / 8 = 46; two 8-bit terms a query: 2^-17 of them as an error of the exponent
+    assert np.abs(got - want).max() <= 46 * 2.0 ** -16 * np.abs(v).max()
