@@ -28,9 +28,12 @@ bool f32_decode_kernel_serves(const DecodeArgs &a);
 // append: rows [n_rows, kv_dim] f32 -> tiles, verbatim. One thread per (row, kv head, four
 // dims): a 16-byte K store and four 4-byte V stores.
 // ------------------------------------------------------------------------------------
+// four-dim groups of a row: those of head_dim, in pages without a table (scratch) those of the padding too
+__host__ __device__ inline int append_f32_groups(const AppendArgs &a) { return a.table ? (a.g.head_dim + 3) >> 2 : a.g.P >> 2; }
+
 __global__ __launch_bounds__(256) void append_f32_kernel(AppendArgs a) {
     const Geom g = a.g;
-    const int groups = (g.head_dim + 3) >> 2;
+    const int groups = append_f32_groups(a);
     const long per_row = (long)g.kv_heads * groups;
     const long total = per_row * a.n_rows;
     const int kv_dim = g.kv_heads * g.head_dim;
@@ -42,7 +45,7 @@ __global__ __launch_bounds__(256) void append_f32_kernel(AppendArgs a) {
         const int kvh = rem / groups;
         const int d0 = (rem - kvh * groups) * 4;
         const long slot = slot_of(a.first_pos + row, g.ring_rows);
-        const int page = a.table[slot >> 4];
+        const int page = a.table ? a.table[slot >> 4] : (int)(slot >> 4);
         const int r = (int)(slot & 15);
         // tile_elems and page_elems count 16-bit units: two per float
         const long tile = ((long)page * g.page_elems + (long)kvh * g.tile_elems) >> 1;
@@ -59,7 +62,7 @@ __global__ __launch_bounds__(256) void append_f32_kernel(AppendArgs a) {
 }
 
 hipError_t launch_append_f32(const AppendArgs &a, hipStream_t s) {
-    const long total = (long)a.g.kv_heads * ((a.g.head_dim + 3) >> 2) * a.n_rows;
+    const long total = (long)a.g.kv_heads * append_f32_groups(a) * a.n_rows;
     long blocks = (total + 255) / 256;
     if (blocks > 65535 * 4) blocks = 65535 * 4;
     hipLaunchKernelGGL(append_f32_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a);

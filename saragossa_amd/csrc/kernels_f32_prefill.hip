@@ -1,0 +1,558 @@
+// gfx950 kernels of the KV hot path, part 5: chunked prefill over the f32 cache on the bf16 matrix
+// instruction, with every f32 factor as three bf16 terms.
+#include <type_traits>
+
+#include "chunk_pages.h"
+
+namespace skv {
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
+typedef __attribute__((ext_vector_type(4))) float float4_t;
+typedef __attribute__((ext_vector_type(4))) unsigned int u4;
+
+namespace {
+
+__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+// upper halves of two words, the first in the low half
+__device__ __forceinline__ uint32_t upper_halves(uint32_t x, uint32_t y) { return __builtin_amdgcn_perm(y, x, 0x07060302u); }
+__device__ __forceinline__ uint32_t bf16_pair(float x, float y) {
+    typedef __attribute__((ext_vector_type(2))) float f2;
+    typedef __attribute__((ext_vector_type(2))) __bf16 b2;
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{x, y}, b2));
+}
+// Two f32 values as three bf16 terms each, x = t0 + t1 + t2 exactly (24 bits in 8 + 8 + 8): the upper
+// half cut off (so that the largest finite values do not round to infinity), the remainder rounded
+// to nearest (so that what the products below leave out has no sign of its own), the rest. A
+// term can be inexact only where it is below the smallest bf16, 2^-133.
+__device__ __forceinline__ void three_terms(float x, float y, uint32_t &t0, uint32_t &t1, uint32_t &t2) {
+    const uint32_t xb = __float_as_uint(x), yb = __float_as_uint(y);
+    t0 = upper_halves(xb, yb);
+    const float x1 = x - __uint_as_float(xb & 0xffff0000u), y1 = y - __uint_as_float(yb & 0xffff0000u);
+    t1 = bf16_pair(x1, y1);
+    t2 = upper_halves(__float_as_uint(x1 - __uint_as_float(t1 << 16)), __float_as_uint(y1 - __uint_as_float(t1 & 0xffff0000u)));
+}
+
+// The products of two factors of three terms that are kept, (left term, right term); the even ones
+// go to one accumulator, the odd ones to another. The three left out are below 2^-24 of it, less than the rounding of
+// one f32 product, and of either sign.
+struct TermPair {
+    int l, r;
+};
+// steps of `n` done before beat b, spread over the beats [from, to)
+__host__ __device__ constexpr int done_before(int b, int n, int from, int to) { return b <= from ? 0 : b >= to ? n : (b - from) * n / (to - from); }
+
+constexpr TermPair TERMS[6] = {{0, 0}, {0, 1}, {1, 0}, {1, 1}, {2, 0}, {0, 2}};
+
+} // namespace
+
+// ------------------------------------------------------------------------------------
+// prefill_tile_kernel (kernels_prefill.hip) on f32 pages: the same slots, splits, page list, softmax
+// base and pipeline (scores of the next pair with this pair's exponentials between them, then this
+// pair's accumulation). Six bf16 products of three-term factors replace one f32 product: the f32
+// instruction does 4 keys' or dims' worth in the cycles in which the bf16 one does 64, so six
+// are 2.6 times as fast (157 TFLOP/s against 2.5 PFLOP/s / 6), and no less exact: the factors are
+// split without a rounding, what is left out is below 2^-24 of a product, and sums are in f32
+// in both.
+//
+// Pages come through registers, where all threads split each value once for the whole
+// workgroup, and go to LDS as three planes of bf16 operands. K and V have one buffer each: V of a
+// group of pairs is stored while the scores of the next group are computed, K of the group after
+// that while the accumulation runs, with a barrier behind each window; the loads are issued a
+// window ahead. Bound by the matrix pipes: 512 rows as one call, in us on one MI355X, against
+// f32_split_kernel (kernels_f32.hip): q32/kv8/hd128 over 512, 1536, 4700, 16384 rows 83.5 -> 62.9, 162 -> 100,
+// 400 -> 218, 1267 -> 650 (215 TFLOP/s of f32 products, 1290 of bf16 ones); q16/kv2/hd256 96.6 -> 65.5,
+// 180 -> 102, 432 -> 217, 1335 -> 636. At head_dim 256 the third terms of the queries live in LDS: in registers
+// they spill (683 us over 16384 rows).
+// ------------------------------------------------------------------------------------
+template <int P, int TILES, int WAVES, int HALVES, bool RING>
+__global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, ChunkPages c) {
+    constexpr int THREADS = WAVES * 64;
+    constexpr int KK = P / 32;
+    constexpr int NT = P / 16;
+    constexpr int PLANE = 4 * P;                 // 16-byte units of one term of a pair's K (or V)
+    constexpr int GP = 2 * HALVES;               // pages of a group: a pair for each half
+    constexpr int CU = (HALVES * PLANE + THREADS - 1) / THREADS; // bf16 units of K, and of V, a thread makes per group
+    constexpr bool FULL = HALVES * PLANE % THREADS == 0;
+    extern __shared__ __attribute__((aligned(16))) u4 kv_planes[]; // [HALVES][3][PLANE] K | [HALVES][3][PLANE] V
+    constexpr int V_AT = HALVES * 3 * PLANE;
+
+    const Geom g = a.g;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 15;
+    const int j = lane >> 4;
+    const int split = blockIdx.x;
+    const int kvh = blockIdx.y;
+    const int G = g.gqa;
+    const int n_slots = a.n_queries * G;
+    constexpr int TW = WAVES / HALVES;
+    const int half = HALVES > 1 ? wave / TW : 0;
+    const int tw = HALVES > 1 ? wave % TW : wave;
+    const int wg_slot0 = blockIdx.z * (TW * TILES * 16);
+    const int wg_slot1 = min(n_slots, wg_slot0 + TW * TILES * 16) - 1;
+
+    auto limit_of = [&](int slot) { return a.q_pos0 + slot / G; };
+    auto ws_of = [&](int slot) { return a.window > 0 ? max(a.window_start, limit_of(slot) + 1 - a.window) : a.window_start; };
+    const int wg_ws_lo = ws_of(wg_slot0);
+    const int wg_lim_hi = limit_of(wg_slot1);
+    auto entry_of = [&](int pos) {
+        if (!RING) return pos >> 4;
+        return pos < c.new_pos0 ? max((pos - c.first_pos) >> 4, 0) : c.n_old + ((pos - c.new_first) >> 4);
+    };
+    const int e_lo = entry_of(wg_ws_lo);
+    const int e_hi = entry_of(wg_lim_hi) + 1;
+    const unsigned span = (unsigned)(e_hi - e_lo);
+    const int pb0 = e_lo + (int)(((unsigned)split * span) / (unsigned)a.splits);
+    const int pb1 = e_lo + (int)(((unsigned)(split + 1) * span) / (unsigned)a.splits);
+    const int n_it = pb1 - pb0;
+    const int n_groups = (n_it + GP - 1) / GP;
+
+    // ---- pages: memory -> registers. Places of the tiles one per lane, asked for a group ahead and
+    // read with v_readlane (a scalar read of the table would stall every LDS read in flight).
+    auto entry = [&](int it) { return min(pb0 + it, e_hi - 1); }; // past the end: a page again, unused
+    uint32_t ids;
+    auto ask_ids = [&](int it) __attribute__((always_inline)) { ids = entry_tile<RING>(a, c, entry(it + lane), kvh); };
+    auto tile_of = [&](int it0, int d, bool v) __attribute__((always_inline)) {
+        const uint16_t *pool = v ? a.v_pool : a.k_pool;
+        if (RING && entry(it0 + d) >= c.n_old) pool = v ? c.v_new : c.k_new;
+        return reinterpret_cast<const float4_t *>(pool) + (uint32_t)__builtin_amdgcn_readlane(ids, d);
+    };
+    // unit u of a thread, of the PLANE * HALVES bf16 units of a group: eight dims of a row of K (two
+    // f32 units 16 apart), or four keys of a dim from both pages of V
+    // At head_dim 256 K and V take turns in the same registers: loads go out at the end of a window and
+    // are split in the second half of the next.
+    constexpr bool SHARE = P > 128;
+    float4_t kx[CU][2], vx_own[SHARE ? 1 : CU][2];
+    float4_t(&vx)[CU][2] = [&]() -> float4_t(&)[CU][2] {
+        if constexpr (SHARE) return kx;
+        else return vx_own;
+    }();
+    auto load_k = [&](int it0, int d) __attribute__((always_inline)) { // pages it0 + d ..
+#pragma unroll
+        for (int u = 0; u < CU; ++u) {
+            const int i = tid + u * THREADS;
+            const int pg = min(__builtin_amdgcn_readfirstlane(i / (PLANE / 2)), GP - 1);
+            const int du = i & (PLANE / 2 - 1);
+            const float4_t *t = tile_of(it0, d + pg, false) + (du >> 5) * 64 + ((du >> 4) & 1) * 32 + (du & 15);
+            kx[u][0] = t[0];
+            kx[u][1] = t[16];
+        }
+    };
+    auto load_v = [&](int it0, int d) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < CU; ++u) {
+            const int i = tid + u * THREADS;
+            const int pr = min(__builtin_amdgcn_readfirstlane(i / PLANE), HALVES - 1);
+            vx[u][0] = tile_of(it0, d + 2 * pr, true)[i & (PLANE - 1)];
+            vx[u][1] = tile_of(it0, d + 2 * pr + 1, true)[i & (PLANE - 1)];
+        }
+    };
+    // Keys that no slot of the workgroup attends: zero probability, but 0 x NaN is NaN, so on the
+    // pages at the edges of the attended range their V values become zero in the registers (the
+    // reference never reads those rows, src/decode_resident/kernels.rs:11-88).
+    const Inner wg_in = inner_entries<RING>(c, pb0, pb1, wg_ws_lo, wg_lim_hi);
+    auto mask_v = [&](int first_page) __attribute__((always_inline)) {
+        const int e0 = pb0 + first_page, e1 = e0 + GP;
+        if ((e0 >= wg_in.o0 && e1 <= wg_in.o1) || (RING && e0 >= wg_in.n0 && e1 <= wg_in.n1)) return; // uniform
+#pragma unroll
+        for (int u = 0; u < CU; ++u) {
+            const int i = tid + u * THREADS;
+            const int pr = __builtin_amdgcn_readfirstlane(i / PLANE);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int it = first_page + 2 * pr + h;
+                const int e = entry(it);
+                const int pos0 = entry_pos<RING>(c, e) + ((i >> 4) & 3) * 4;
+                const int lo = max(wg_ws_lo, entry_lo<RING>(c, e)), hi = min(wg_lim_hi, entry_hi<RING>(c, e));
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    vx[u][h][r] = it < n_it && pos0 + r >= lo && pos0 + r <= hi ? vx[u][h][r] : 0.0f;
+            }
+        }
+    };
+    // Splitting in small steps that can stand between products: step s splits two values of unit s / 4;
+    // the unit's last step stores its three terms.
+    constexpr int SPLIT_STEPS = CU * 4;
+    uint32_t t0[4], t1[4], t2[4];
+    auto split_step = [&](int s, bool v) __attribute__((always_inline)) {
+        const int u = s >> 2, k = s & 3;
+        const float4_t x = v ? vx[u][k >> 1] : kx[u][k >> 1];
+        three_terms((k & 1) ? x[2] : x[0], (k & 1) ? x[3] : x[1], t0[k], t1[k], t2[k]);
+        if (k == 3) {
+            const int i = tid + u * THREADS;
+            // K: [half][term][page of the pair][P/2 * 4 units]; V: [half][term][PLANE]
+            const int h = i / PLANE;
+            if (FULL || h < HALVES) {
+                u4 *dst = kv_planes + (v ? V_AT : 0) + h * 3 * PLANE + (i & (PLANE - 1));
+                dst[0] = u4{t0[0], t0[1], t0[2], t0[3]};
+                dst[PLANE] = u4{t1[0], t1[1], t1[2], t1[3]};
+                dst[2 * PLANE] = u4{t2[0], t2[1], t2[2], t2[3]};
+            }
+        }
+    };
+
+    ask_ids(0);
+    load_k(0, 0);
+    // ---- this wavefront's query tiles ------------------------------------------------
+    int my_limit[TILES], my_ws[TILES];
+    int t_ws_hi[TILES], t_lim_lo[TILES];
+    bool t_on[TILES];
+    // (at head_dim 256 the third terms, used once per K-step and page, live in LDS behind the planes)
+    constexpr int QT = P > 128 ? 2 : 3;
+    bf16x8_t q[TILES][KK][QT];
+    u4 *q_third = kv_planes + 2 * V_AT + wave * TILES * KK * 64 + lane; // the wavefront's own
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+        const int s0 = wg_slot0 + (tw * TILES + t) * 16;
+        t_on[t] = s0 < n_slots;
+        const int s_last = min(s0 + 15, n_slots - 1);
+        const int my_slot = min(s0 + n, n_slots - 1);
+        my_limit[t] = limit_of(my_slot);
+        my_ws[t] = ws_of(my_slot);
+        t_lim_lo[t] = limit_of(min(s0, n_slots - 1));
+        t_ws_hi[t] = ws_of(s_last);
+        const float *qrow = a.q + ((long)(my_slot / G) * g.q_heads + kvh * G + my_slot % G) * g.head_dim;
+        float qv[KK][8];
+        if (a.q_vec) {
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) {
+                const float4_t *qp = reinterpret_cast<const float4_t *>(qrow + min(kk * 32 + j * 8, g.head_dim - 8));
+                const float4_t x0 = qp[0], x1 = qp[1];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    qv[kk][e] = x0[e];
+                    qv[kk][4 + e] = x1[e];
+                }
+            }
+        } else {
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) qv[kk][e] = qrow[min(kk * 32 + j * 8 + e, g.head_dim - 1)];
+            }
+        }
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) {
+            uint32_t w[3][4];
+#pragma unroll
+            for (int e2 = 0; e2 < 4; ++e2) {
+                const int d = kk * 32 + j * 8 + e2 * 2;
+                const float x = d < g.head_dim ? qv[kk][e2 * 2] * a.qscale : 0.0f;
+                const float y = d + 1 < g.head_dim ? qv[kk][e2 * 2 + 1] * a.qscale : 0.0f;
+                three_terms(x, y, w[0][e2], w[1][e2], w[2][e2]);
+            }
+#pragma unroll
+            for (int k = 0; k < QT; ++k) q[t][kk][k] = __builtin_bit_cast(bf16x8_t, u4{w[k][0], w[k][1], w[k][2], w[k][3]});
+            if constexpr (QT == 2) q_third[(t * KK + kk) * 64] = u4{w[2][0], w[2][1], w[2][2], w[2][3]};
+        }
+    }
+
+    float4_t o[TILES][NT];
+    float4_t neg_m[TILES];
+    float m_base[TILES], thr[TILES], l_run[TILES];
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+#pragma unroll
+        for (int u = 0; u < NT; ++u) o[t][u] = float4_t{0.f, 0.f, 0.f, 0.f};
+        m_base[t] = 0.0f;
+        neg_m[t] = float4_t{0.f, 0.f, 0.f, 0.f};
+        thr[t] = -INFINITY;
+        l_run[t] = 0.0f;
+    }
+    float4_t sa[TILES], sb[TILES];
+    bf16x8_t p[TILES][3];
+
+    int in0, in1, in2, in3; // pairs whose keys every slot of the wavefront attends
+    {
+        int lo = t_ws_hi[0], hi = t_lim_lo[0];
+#pragma unroll
+        for (int t = 1; t < TILES; ++t) {
+            lo = max(lo, t_ws_hi[t]);
+            hi = min(hi, t_lim_lo[t]);
+        }
+        const Inner r = inner_entries<RING>(c, pb0, pb1, lo, hi);
+        in0 = (r.o0 - pb0 + 1) >> 1;
+        in1 = (r.o1 - pb0) >> 1;
+        in2 = (r.n0 - pb0 + 1) >> 1;
+        in3 = (r.n1 - pb0) >> 1;
+    }
+    auto settle = [&](int pair) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            if (!((pair >= in0 && pair < in1) || (RING && pair >= in2 && pair < in3))) { // uniform
+                const int it = 2 * pair;
+                const int ea = entry(it), eb = entry(it + 1);
+                const int pos_a = entry_pos<RING>(c, ea), pos_b = entry_pos<RING>(c, eb);
+                const int lo_a = max(my_ws[t], entry_lo<RING>(c, ea)), hi_a = min(my_limit[t], entry_hi<RING>(c, ea));
+                const int lo_b = max(my_ws[t], entry_lo<RING>(c, eb)), hi_b = min(my_limit[t], entry_hi<RING>(c, eb));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int pa = pos_a + j * 4 + e, pb = pos_b + j * 4 + e;
+                    sa[t][e] = it < n_it && pa >= lo_a && pa <= hi_a ? sa[t][e] : -INFINITY;
+                    sb[t][e] = it + 1 < n_it && pb >= lo_b && pb <= hi_b ? sb[t][e] : -INFINITY;
+                }
+            }
+            const float mx = fmaxf(fmaxf(fmaxf(sa[t][0], sa[t][1]), fmaxf(sa[t][2], sa[t][3])),
+                                   fmaxf(fmaxf(sb[t][0], sb[t][1]), fmaxf(sb[t][2], sb[t][3])));
+            if (__builtin_amdgcn_ballot_w64(mx > thr[t])) {
+                const float top = rows_max(mx);
+                const bool unseen = thr[t] == -INFINITY;
+                const float d = unseen ? (top == -INFINITY ? 0.0f : top) : fmaxf(top, 0.0f);
+                const float alpha = unseen ? 1.0f : fast_exp2(-d);
+                m_base[t] += d;
+                neg_m[t] = float4_t{-m_base[t], -m_base[t], -m_base[t], -m_base[t]};
+                thr[t] = unseen && top == -INFINITY ? -INFINITY : 8.0f;
+                l_run[t] *= alpha;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    sa[t][e] -= d;
+                    sb[t][e] -= d;
+                }
+                if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
+#pragma unroll
+                    for (int u = 0; u < NT; ++u) o[t][u] *= alpha;
+                }
+            }
+        }
+    };
+
+    // probabilities of the settled scores in nine steps: exponential of score s, every other one the
+    // three terms of the two before it
+    float pe[TILES][2];
+    uint32_t pw[TILES][3][4];
+    auto prob_step = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            if (s >= 2 && (s & 1) == 0) {
+                l_run[t] += pe[t][0];
+                l_run[t] += pe[t][1];
+                const int k = (s >> 1) - 1;
+                three_terms(pe[t][0], pe[t][1], pw[t][0][k], pw[t][1][k], pw[t][2][k]);
+            }
+            if (s < 8) pe[t][s & 1] = fast_exp2(s < 4 ? sa[t][s & 3] : sb[t][s & 3]);
+        }
+    };
+
+    const u4 *k_half = kv_planes + half * 3 * PLANE + lane;
+    const u4 *v_half = kv_planes + V_AT + half * 3 * PLANE + lane;
+    constexpr int BEATS = 2 * KK * 6;
+    static_assert(BEATS >= 9 && BEATS >= SPLIT_STEPS * (SHARE ? 2 : 1), "at most one step of each kind between two products");
+    // operand set `at` of a window, K-step at / 2 of page A or B, dim tile `at` of V: three terms
+    u4 op[2 * KK][3];
+    u4 q2[KK][TILES]; // QT == 2: the third terms of K-step at / 2
+    auto ask_k = [&](int at) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) op[at][k] = k_half[k * PLANE + (at & 1) * (PLANE / 2) + (at >> 1) * 64];
+        if constexpr (QT == 2) {
+#pragma unroll
+            for (int t = 0; t < TILES; ++t)
+                if ((at & 1) == 0) q2[at >> 1][t] = q_third[(t * KK + (at >> 1)) * 64];
+        }
+    };
+    auto ask_v = [&](int at) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) op[at][k] = v_half[k * PLANE + at * 64];
+    };
+    // window 1: scores of the next group, between them the probabilities of this one and the splitting of
+    // this group's V
+    auto scores = [&](auto first) __attribute__((always_inline)) {
+        constexpr bool FIRST = decltype(first)::value;
+        // two accumulators a page, the leading products in the one that starts from -m
+        float4_t na[TILES][2], ma[TILES][2];
+        ask_k(0);
+#pragma unroll
+        for (int at = 0; at < 2 * KK; ++at) {
+            if (at + 1 < 2 * KK) ask_k(at + 1);
+            const int pg = at & 1;
+#pragma unroll
+            for (int b = 0; b < 6; ++b) {
+                __builtin_amdgcn_sched_barrier(0);
+                const bf16x8_t kv = __builtin_bit_cast(bf16x8_t, op[at][TERMS[b].l]);
+#pragma unroll
+                for (int t = 0; t < TILES; ++t) {
+                    const bf16x8_t qv = QT == 2 && TERMS[b].r == 2 ? __builtin_bit_cast(bf16x8_t, q2[at >> 1][t])
+                                                                   : q[t][at >> 1][TERMS[b].r < QT ? TERMS[b].r : 0];
+                    if ((b & 1) == 0) {
+                        na[t][pg] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kv, qv, at < 2 && b == 0 ? neg_m[t] : na[t][pg], 0, 0, 0);
+                    } else {
+                        const float4_t zero = float4_t{0.f, 0.f, 0.f, 0.f};
+                        ma[t][pg] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kv, qv, at < 2 && b == 1 ? zero : ma[t][pg], 0, 0, 0);
+                    }
+                }
+                if (!FIRST) {
+                    constexpr int P_TO = SHARE ? BEATS / 2 : BEATS, S_FROM = SHARE ? BEATS / 2 : 0;
+                    const int beat = at * 6 + b; // at most one step of each kind a beat
+                    const int ps = done_before(beat, 9, 0, P_TO), ss = done_before(beat, SPLIT_STEPS, S_FROM, BEATS);
+                    if (done_before(beat + 1, 9, 0, P_TO) > ps) prob_step(ps);
+                    if (done_before(beat + 1, SPLIT_STEPS, S_FROM, BEATS) > ss) split_step(ss, true);
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            if (!FIRST) {
+#pragma unroll
+                for (int k = 0; k < 3; ++k) p[t][k] = __builtin_bit_cast(bf16x8_t, u4{pw[t][k][0], pw[t][k][1], pw[t][k][2], pw[t][k][3]});
+            }
+            sa[t] = na[t][0] + ma[t][0];
+            sb[t] = na[t][1] + ma[t][1];
+        }
+    };
+    // window 2: accumulation of this group, between its products the splitting of K two groups on
+    auto accumulate = [&]() __attribute__((always_inline)) {
+        ask_v(0);
+#pragma unroll
+        for (int at = 0; at < NT; ++at) {
+            if (at + 1 < NT) ask_v(at + 1);
+#pragma unroll
+            for (int b = 0; b < 6; ++b) {
+                __builtin_amdgcn_sched_barrier(0);
+                const bf16x8_t vv = __builtin_bit_cast(bf16x8_t, op[at][TERMS[b].l]);
+#pragma unroll
+                for (int t = 0; t < TILES; ++t)
+                    o[t][at] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv, p[t][TERMS[b].r], o[t][at], 0, 0, 0);
+                constexpr int S_FROM = SHARE ? BEATS / 2 : 0;
+                const int beat = at * 6 + b, ss = done_before(beat, SPLIT_STEPS, S_FROM, BEATS);
+                if (done_before(beat + 1, SPLIT_STEPS, S_FROM, BEATS) > ss) split_step(ss, false);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    // ---- first group's scores, the second's K on its way
+#pragma unroll
+    for (int s = 0; s < SPLIT_STEPS; ++s) split_step(s, false);
+    load_k(0, GP);
+    if constexpr (!SHARE) load_v(0, 0);
+    __syncthreads();
+    scores(std::true_type{});
+    settle(half);
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < SPLIT_STEPS; ++s) split_step(s, false);
+    if constexpr (SHARE) load_v(0, 0);
+    ask_ids(GP);
+    __syncthreads();
+
+    // Group by group: K of the next group is in LDS, V of this one in registers.
+    for (int group = 0; group < n_groups; ++group) {
+        const int it0 = (group + 1) * GP; // lane 0's entry of ids: the first page of the next group
+        mask_v(group * GP);
+        if constexpr (!SHARE) load_k(it0, GP);
+        scores(std::false_type{});
+        if constexpr (SHARE) load_k(it0, GP);
+        __syncthreads();
+        if constexpr (!SHARE) load_v(it0, 0);
+        if constexpr (!SHARE) ask_ids(it0 + GP);
+        accumulate();
+        if constexpr (SHARE) {
+            load_v(it0, 0);
+            ask_ids(it0 + GP);
+        }
+        settle((group + 1) * HALVES + half);
+        __syncthreads();
+    }
+
+    // ---- the second half's states join the first's through LDS -----------------------------
+    if constexpr (HALVES > 1) {
+        static_assert(HALVES == 2 && TW * TILES * (NT + 1) * 64 <= 2 * V_AT, "the second half's states fit the page buffers");
+        float4_t *xo = reinterpret_cast<float4_t *>(kv_planes) + (tw * TILES) * (NT + 1) * 64 + lane;
+        if (half == 1) {
+#pragma unroll
+            for (int t = 0; t < TILES; ++t) {
+#pragma unroll
+                for (int u = 0; u < NT; ++u) xo[(t * (NT + 1) + u) * 64] = o[t][u];
+                xo[(t * (NT + 1) + NT) * 64] = float4_t{thr[t] == -INFINITY ? -INFINITY : m_base[t], l_run[t], 0.f, 0.f};
+            }
+        }
+        __syncthreads();
+        if (half == 1) return;
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            const float4_t ml = xo[(t * (NT + 1) + NT) * 64];
+            const float m0 = thr[t] == -INFINITY ? -INFINITY : m_base[t], m1 = ml[0];
+            const float mx = fmaxf(m0, m1);
+            const float m_safe = mx == -INFINITY ? 0.0f : mx;
+            const float w0 = fast_exp2(m0 - m_safe), w1 = fast_exp2(m1 - m_safe);
+            l_run[t] = l_run[t] * w0 + ml[1] * w1;
+#pragma unroll
+            for (int u = 0; u < NT; ++u) o[t][u] = o[t][u] * w0 + xo[(t * (NT + 1) + u) * 64] * w1;
+            m_base[t] = m_safe;
+            thr[t] = mx == -INFINITY ? -INFINITY : 8.0f;
+        }
+    }
+
+    // ---- every wavefront writes its own slots -------------------------------------------
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+        const float l = rows_sum(l_run[t]);
+        const int slot = wg_slot0 + (tw * TILES + t) * 16 + n;
+        if (!t_on[t] || slot >= n_slots) continue;
+        float *dst;
+        float scale = 1.0f;
+        if (a.splits_total == 1) {
+            scale = 1.0f / l;
+            dst = a.out + ((long)(slot / G) * g.q_heads + kvh * G + slot % G) * g.head_dim;
+        } else {
+            const long pidx = ((long)kvh * a.splits_total + a.split_base + split) * n_slots + slot;
+            dst = a.part_o + pidx * g.head_dim;
+            if (j == 0) {
+                a.part_m[pidx] = thr[t] == -INFINITY ? -INFINITY : m_base[t];
+                a.part_l[pidx] = l;
+            }
+        }
+        const bool vec_ok = (g.head_dim & 3) == 0;
+#pragma unroll
+        for (int u = 0; u < NT; ++u) {
+            const int col = u * 16 + j * 4;
+            const float4_t v = o[t][u] * scale;
+            if (vec_ok) {
+                if (col < g.head_dim) *reinterpret_cast<float4_t *>(dst + col) = v;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (col + i < g.head_dim) dst[col + i] = v[i];
+            }
+        }
+    }
+}
+
+// Query slots of a workgroup; 0 = the kernel does not serve the head_dim.
+int f32_prefill_slots(int P, bool halves) { return P > 256 ? 0 : halves && P <= 128 ? 64 : 128; }
+
+template <int P, int TILES, int WAVES, int HALVES, bool RING>
+static hipError_t launch_f32_prefill_of(const DecodeArgs &a, const ChunkPages &c, dim3 grid, hipStream_t s) {
+    constexpr size_t lds = ((size_t)2 * HALVES * 3 * 4 * P + (P > 128 ? WAVES * TILES * (P / 32) * 64 : 0)) * sizeof(u4);
+    static_assert(lds <= 160 * 1024, "a group's K and V (and the queries' third terms) share the LDS of a compute unit");
+    static std::atomic<uint64_t> lds_ok{0}; // per instantiation
+    {
+        hipError_t e = allow_full_lds(reinterpret_cast<const void *>(&f32_prefill_kernel<P, TILES, WAVES, HALVES, RING>), lds_ok);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL((f32_prefill_kernel<P, TILES, WAVES, HALVES, RING>), grid, dim3(WAVES * 64), lds, s, a, c);
+    return hipGetLastError();
+}
+template <int P, int TILES, int WAVES, int HALVES>
+static hipError_t launch_f32_prefill_p(const DecodeArgs &a, const ChunkPages &c, dim3 grid, hipStream_t s) {
+    return c.ring_pages > 0 ? launch_f32_prefill_of<P, TILES, WAVES, HALVES, true>(a, c, grid, s)
+                            : launch_f32_prefill_of<P, TILES, WAVES, HALVES, false>(a, c, grid, s);
+}
+
+hipError_t launch_f32_prefill(const DecodeArgs &a, const ChunkPages &c, bool halves, hipStream_t s) {
+    const int n_slots = a.n_queries * a.g.gqa;
+    const int per_wg = f32_prefill_slots(a.g.P, halves);
+    if (per_wg == 0) return hipErrorInvalidValue;
+    halves = per_wg == 64;
+    dim3 grid((unsigned)a.splits, (unsigned)a.g.kv_heads, (unsigned)((n_slots + per_wg - 1) / per_wg));
+    switch (a.g.P) {
+    case 32: return halves ? launch_f32_prefill_p<32, 1, 8, 2>(a, c, grid, s) : launch_f32_prefill_p<32, 1, 8, 1>(a, c, grid, s);
+    case 64: return halves ? launch_f32_prefill_p<64, 1, 8, 2>(a, c, grid, s) : launch_f32_prefill_p<64, 1, 8, 1>(a, c, grid, s);
+    case 128: return halves ? launch_f32_prefill_p<128, 1, 8, 2>(a, c, grid, s) : launch_f32_prefill_p<128, 1, 8, 1>(a, c, grid, s);
+    case 256: return launch_f32_prefill_p<256, 1, 8, 1>(a, c, grid, s);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+} // namespace skv

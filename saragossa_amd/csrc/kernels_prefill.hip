@@ -2,7 +2,7 @@
 // matrix-core-bound kernel of the path.
 #include <type_traits>
 
-#include "skv_internal.h"
+#include "chunk_pages.h"
 
 namespace skv {
 
@@ -57,55 +57,6 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // 57.2 -> 41.1, 106 -> 86.5, 256 -> 225; q16/kv2/hd256 40.0 -> 24.3, 55.7 -> 50.5, 97.9 -> 89.0, 247 -> 225 (where
 // the matrix pipes alone need 130).
 // ------------------------------------------------------------------------------------
-
-// Entry e of the launch's page list: where its tiles lie (of the workgroup's kv head, in 16-byte
-// units from its pool's start), which position its first row has, and the first and last
-// position whose rows it may speak for. On full layers entry e is logical page e.
-template <bool RING>
-__device__ __forceinline__ uint32_t entry_tile(const DecodeArgs &a, const ChunkPages &c, int e, int kvh) {
-    int page;
-    if constexpr (RING) {
-        int at = c.start + min(e, c.n_old - 1);
-        if (at >= c.ring_pages) at -= c.ring_pages;
-        page = e < c.n_old ? a.table[max(at, 0)] : e - c.n_old;
-    } else {
-        page = a.table[e];
-    }
-    return (uint32_t)page * (uint32_t)(a.g.page_elems >> 3) + (uint32_t)kvh * (uint32_t)(a.g.tile_elems >> 3);
-}
-template <bool RING>
-__device__ __forceinline__ int entry_pos(const ChunkPages &c, int e) {
-    if constexpr (!RING) return e * 16;
-    return e < c.n_old ? c.first_pos + e * 16 : c.new_first + (e - c.n_old) * 16;
-}
-template <bool RING>
-__device__ __forceinline__ int entry_lo(const ChunkPages &c, int e) {
-    return !RING || e < c.n_old ? INT32_MIN : c.new_pos0;
-}
-template <bool RING>
-__device__ __forceinline__ int entry_hi(const ChunkPages &c, int e) {
-    return !RING || e >= c.n_old ? INT32_MAX : c.new_pos0 - 1;
-}
-// The entries [e0, e1) of [first, last) all of whose rows lie in [lo, hi] and are the entry's to
-// speak for, as two ranges: old entries, new ones.
-struct Inner {
-    int o0, o1, n0, n1;
-};
-template <bool RING>
-__device__ __forceinline__ Inner inner_entries(const ChunkPages &c, int first, int last, int lo, int hi) {
-    Inner r;
-    if constexpr (!RING) {
-        r.o0 = max(first, (lo + 15) >> 4);
-        r.o1 = min(last, (hi - 15 >= 0 ? (hi - 15) >> 4 : -1) + 1);
-        r.n0 = r.n1 = 0;
-    } else {
-        r.o0 = max(first, (lo - c.first_pos + 15) >> 4);
-        r.o1 = min(min(last, c.n_old), ((min(hi, c.new_pos0 - 1) - 15 - c.first_pos) >> 4) + 1);
-        r.n0 = max(max(first, c.n_old), c.n_old + ((max(lo, c.new_pos0) - c.new_first + 15) >> 4));
-        r.n1 = min(last, c.n_old + ((hi - 15 - c.new_first) >> 4) + 1);
-    }
-    return r;
-}
 
 // 64 x 16 bytes straight from memory to LDS, lane l's to lds + 16 l (`lds` the same in every lane), no
 // register in between. In assembly because the compiler, which cannot tell the two halves of the

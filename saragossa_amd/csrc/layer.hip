@@ -216,6 +216,36 @@ bool takes_tile_kernel(const Geom &g, size_t n_slots, size_t n_pages) {
     return (n_slots + 15) / 16 * (size_t)g.kv_heads * n_pages >= limit;
 }
 
+// The same questions for f32 layers: the kernel that splits its factors into bf16 terms (head_dim up to
+// 256) or the one that streams pages into the f32 instruction, 16 slots a workgroup. Whole chunks, streaming /
+// one tile / halves, in us: q32/kv8/hd128, 32 rows over 2048, 8192 rows 28.9/37.5/32.6, 59.7/50.3/49.3; 128 rows
+// over 512, 2048: 28.7/39.0/31.9, 60.7/45.6/45.1; 512 rows over 0, 512, 2048, 8192: 44.0/45.5/39.4, 82.5/63.7/62.2,
+// 197/122/131, 656/354/405; q16/kv2/hd256, 64 rows over 2048, 8192: 54.2/60.7, 119/76.6; 256 rows over 0, 512, 2048:
+// 34.1/49.8, 58.7/57.9, 119/71.9; q8/kv2/hd64, 256 rows over 2048, 8192: 24.1/28.0/26.6, 54.6/45.3/45.3; 512 rows over
+// 512, 2048: 22.1/25.1/21.8, 37.5/32.8/31.2.
+bool takes_f32_chunk_kernel(const Geom &g, size_t n_slots, size_t n_pages) {
+    if (f32_prefill_slots(g.P, false) == 0 || n_slots < 64 || tuning().prefill_tiles == 0) return false;
+    if (tuning().prefill_tiles > 1) return true;
+    const size_t limit = g.P <= 64 ? 25000 : g.P == 128 ? 16000 : 11500;
+    return (n_slots + 15) / 16 * (size_t)g.kv_heads * n_pages >= limit;
+}
+bool f32_halves(const Geom &g, size_t n_slots, size_t n_pages) {
+    if (tuning().prefill_tiles2_min_pages >= 0) return false;
+    const size_t wgs = (n_slots + 63) / 64 * (size_t)g.kv_heads, walk = wgs * n_pages;
+    if (n_slots <= 64) return true; // a workgroup of 128 slots would be half empty
+    return wgs <= 256 && walk < (g.P <= 64 ? 17000u : wgs >= 192 ? 25000u : 8500u);
+}
+
+// Splits of the context for a chunk whose workgroups cover per_wg slots: while the slot tiles alone
+// leave compute units idle, and at least 16 pages each.
+int chunk_splits(const Geom &g, size_t n_queries, size_t per_wg, size_t n_pages) {
+    if (!skv_flag_sdpa_2pass_enabled()) return 1;
+    const size_t tiles = (n_queries * (size_t)g.gqa + per_wg - 1) / per_wg * (size_t)g.kv_heads;
+    size_t want = std::max<size_t>(tuning().prefill_wgs / tiles, 1);
+    want = std::min<size_t>(want, std::max<size_t>(n_pages / 16, 1));
+    return (int)std::min<size_t>(want, tuning().prefill_max_splits);
+}
+
 int choose_splits(const skv_layer *L, int n_pages_scan, size_t rows, int waves, size_t target_wgs) {
     const Tuning &t = tuning();
     if (!skv_flag_sdpa_2pass_enabled() || rows < t.split_min_len) return 1;
@@ -431,6 +461,19 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
             a.q_head_stride = pre->q_head_stride;
         }
         if (attn_scalar > 0.0f) a.qscale = (1.0f / std::sqrt(attn_scalar)) * 1.4426950408889634f;
+        if (n_queries > 1 && takes_f32_chunk_kernel(g, n_queries * (size_t)g.gqa, (size_t)a.n_pages)) {
+            const bool halves = f32_halves(g, n_queries * (size_t)g.gqa, (size_t)a.n_pages);
+            a.splits = chunk_splits(g, n_queries, (size_t)f32_prefill_slots(g.P, halves), (size_t)a.n_pages);
+            a.splits_total = a.splits;
+            if (a.splits > 1) {
+                int32_t rc2 = multi_query_partials(L, s, (size_t)a.splits, n_queries, a);
+                if (rc2) return rc2;
+            }
+            const size_t lo = std::max(window_start, skv_window_start(L->len - n_queries, L->window));
+            SKV_HIP(launch_f32_prefill(a, layer_pages(L, lo, L->len), halves, s));
+            if (a.splits > 1) SKV_HIP(launch_merge_rows(a, s));
+            return SKV_OK;
+        }
         if (n_queries > 1) {
             const size_t tiles = (n_queries * (size_t)g.gqa + 15) / 16 * (size_t)g.kv_heads;
             const size_t want = std::max<size_t>(2 * decode_target_wgs() / tiles, 1);
@@ -1078,7 +1121,7 @@ int32_t skv_decode_step_static_device(skv_layer *L, skv_stream stream, const voi
     return skv::fail_exception();
 }
 
-// A chunk of c > 1 rows on a bf16 ring layer. The ring holds little more than the window, so the
+// A chunk of c > 1 rows on a ring layer (bf16, or f32 where the f32 chunk kernel serves the head_dim). The ring holds little more than the window, so the
 // chunk's own rows overwrite rows its first queries still attend. They are therefore first
 // written to pages of the context's scratch; one launch attends the ring's rows and them, in the
 // order of positions, each workgroup only the pages its slots' windows touch; then the rows go
@@ -1104,11 +1147,8 @@ static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const flo
     // pages a workgroup of one tile row walks: the window and the workgroup's own rows
     const size_t walked = std::min<size_t>((size_t)pages.n_old + n_new, L->window / 16 + 2);
     const TileShape shape = prefill_shape(g, c * (size_t)g.gqa, walked);
-    const size_t per_wg = (size_t)prefill_tile_slots(g.P, shape);
-    const size_t tiles = (c * (size_t)g.gqa + per_wg - 1) / per_wg * (size_t)g.kv_heads;
-    size_t want = std::max<size_t>(tuning().prefill_wgs / tiles, 1);
-    want = std::min<size_t>(want, std::max<size_t>(walked / 16, 1));
-    a.splits = (int)std::min<size_t>(want, tuning().prefill_max_splits);
+    const bool halves = g.f32 && f32_halves(g, c * (size_t)g.gqa, walked);
+    a.splits = chunk_splits(g, c, (size_t)(g.f32 ? f32_prefill_slots(g.P, halves) : prefill_tile_slots(g.P, shape)), walked);
     a.splits_total = a.splits;
     void *scratch = nullptr;
     int32_t rc = multi_query_partials(L, s, a.splits > 1 ? (size_t)a.splits : 0, c, a, 2 * pool_bytes, &scratch);
@@ -1122,16 +1162,16 @@ static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const flo
     w.n_rows = (int)c;
     w.g = g;
     w.g.ring_rows = 0;
-    plan_batch(w);
-    SKV_HIP(launch_append(w, s));
+    if (!g.f32) plan_batch(w);
+    SKV_HIP(g.f32 ? launch_append_f32(w, s) : launch_append(w, s));
     pages.k_new = w.k_pool;
     pages.v_new = w.v_pool;
-    SKV_HIP(launch_prefill_tiles(a, pages, shape, s));
+    SKV_HIP(g.f32 ? launch_f32_prefill(a, pages, halves, s) : launch_prefill_tiles(a, pages, shape, s));
     if (a.splits > 1) SKV_HIP(launch_merge_rows(a, s));
     return encode_append(L, s, k, v, c);
 }
 
-// The same on an f32 ring layer, c <= ring_rows, attended in two phases around the append: first every query over the rows
+// The same on an f32 ring layer of wider heads, c <= ring_rows, attended in two phases around the append: first every query over the rows
 // already in the ring (capped at the last old position), then, once the chunk is appended,
 // over the chunk's own rows (from its first position up to each query's own). Both phases
 // leave (o, m, l) partials; one merge produces the context. c <= ring_rows.
@@ -1190,9 +1230,10 @@ int32_t skv_prefill_chunk_device(skv_layer *L, skv_stream stream, const float *q
         return fail(SKV_ERR_DIMENSION, "append KV résident: capacité " +
                                            std::to_string(L->capacity) + " atteinte (overflow)");
     const size_t kv_dim = skv_kv_dim(L), q_dim = (size_t)L->g.q_heads * L->g.head_dim;
-    // f32 ring layers take the chunk in steps of at most the ring's rows (see ring_chunk_f32).
+    // f32 ring layers of wide heads take the chunk in steps of at most the ring's rows (see ring_chunk_f32).
+    const bool two_phase = L->g.f32 && f32_prefill_slots(L->g.P, false) == 0;
     size_t step = std::min<size_t>(n_rows, 4096);
-    if (L->g.ring_rows > 0 && L->g.f32) step = std::min(step, (size_t)L->g.ring_rows);
+    if (L->g.ring_rows > 0 && two_phase) step = std::min(step, (size_t)L->g.ring_rows);
     const float *q = q_dev, *k = (const float *)k_dev, *v = (const float *)v_dev;
     float *out = out_dev;
     for (size_t done = 0; done < n_rows; done += step) {
@@ -1203,7 +1244,7 @@ int32_t skv_prefill_chunk_device(skv_layer *L, skv_stream stream, const float *q
         // like any other
         const size_t ring = (size_t)L->g.ring_rows;
         if (ring > 0 && c > 1 && L->len + c > ring && c + L->window > ring + 1) {
-            rc = (L->g.f32 ? ring_chunk_f32 : ring_chunk)(L, as_stream(stream), q, k, v, c, out);
+            rc = (two_phase ? ring_chunk_f32 : ring_chunk)(L, as_stream(stream), q, k, v, c, out);
             if (rc) return rc;
             q += c * q_dim;
             k += c * kv_dim;

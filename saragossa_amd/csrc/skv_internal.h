@@ -359,6 +359,8 @@ hipError_t launch_f32_split_batch(const DecodeBatchArgs &b, int n_seq, int max_s
 hipError_t launch_merge(const DecodeArgs &a, hipStream_t s);        // split-K partials -> context
 hipError_t launch_prefill_tiles(const DecodeArgs &a, const ChunkPages &c, TileShape shape, hipStream_t s); // chunked prefill, no merge
 int prefill_tile_slots(int P, TileShape shape);
+hipError_t launch_f32_prefill(const DecodeArgs &a, const ChunkPages &c, bool halves, hipStream_t s); // the same on f32 pages
+int f32_prefill_slots(int P, bool halves); // query slots of a workgroup, 0 = head_dim not served
 hipError_t launch_merge_rows(const DecodeArgs &a, hipStream_t s);    // the same merge for many query slots
 hipError_t launch_naive(const NaiveArgs &a, hipStream_t s);
 int decode_max_splits();

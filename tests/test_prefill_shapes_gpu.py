@@ -1,8 +1,9 @@
-"""The prefill tile kernel in each of its workgroup shapes, at the edges of its tiles: chunks that end
+"""The prefill kernels of both elements in each of its workgroup shapes, at the edges of its tiles: chunks that end
 inside a slot tile, a page pair and a barrier step; caches that begin the chunk inside a page; ring
 layers whose chunk starts before, at and long after the ring is full (its rows are attended
-from pages of their own and appended afterwards). Contexts within 1e-4 of the oracle (queries and
-probabilities carry 16 bits: about 1e-5 of values of order one), rows bit for bit."""
+from pages of their own and appended afterwards). Contexts within 1e-4 of the oracle on bf16 layers
+(queries and probabilities carry 16 bits: about 1e-5 of values of order one), within 2e-5 on f32 ones
+(two f32 sums of up to 600 products in different orders), rows bit for bit."""
 import os
 
 import numpy as np
@@ -41,14 +42,16 @@ def shape(request):
     ((16, 8, 256), 33, 300, (130,)),
     ((4, 2, 16), 17, 64, (64, 33)),      # ring: chunk starts at a page boundary; padded head
 ])
-def test_chunks_in_every_shape(state, shape, dims, window, base, chunks):
+@pytest.mark.parametrize("element,tol", [("bf16", 1e-4), ("f32", 2e-5)])
+def test_chunks_in_every_shape(state, shape, element, tol, dims, window, base, chunks):
     q_heads, kv_heads, head_dim = dims
     kv_dim, q_dim = kv_heads * head_dim, q_heads * head_dim
     rng = np.random.default_rng(base + head_dim)
-    kv = state.full_attention_bf16(base + sum(chunks), q_heads, kv_heads, head_dim, window=window)
+    make = state.full_attention_f32 if element == "f32" else state.full_attention_bf16
+    kv = make(base + sum(chunks), q_heads, kv_heads, head_dim, window=window)
     kv.set_block_table(rng.permutation(kv.pages()).astype(np.int32))
     lay = oracle.layout(q_heads, kv_heads, head_dim, sliding_window=window)
-    cache = oracle.LayerKvCache("bf16r")
+    cache = oracle.LayerKvCache("f32" if element == "f32" else "bf16r")
     if base:
         k0, v0 = (rng.standard_normal((base, kv_dim), dtype=np.float32) for _ in range(2))
         kv.seed(k0, v0, base)
@@ -58,26 +61,55 @@ def test_chunks_in_every_shape(state, shape, dims, window, base, chunks):
         k, v = (rng.standard_normal((c, kv_dim), dtype=np.float32) for _ in range(2))
         got = kv.prefill_rows(q, k, v)
         want = oracle.cached_attention_prefill_rows(q, k, v, cache, lay)
-        assert np.abs(got - want).max() <= 1e-4, (shape, c)
+        assert np.abs(got - want).max() <= tol, (shape, c)
     first = max(0, kv.len() - window) if window else 0
     gk, gv = kv.read_rows_f32(first, kv.len() - first)
     assert np.array_equal(gk, cache.keys()[first:]) and np.array_equal(gv, cache.values()[first:])
     kv.close()
 
 
-def test_scores_that_climb(state, shape):
+@pytest.mark.parametrize("element", ["bf16", "f32"])
+def test_scores_that_climb(state, shape, element):
     """Keys that grow along the context move the softmax base again and again (it follows a slot's
     scores only once they pass it by 2^8), and fall below it by far more."""
     rng = np.random.default_rng(3)
     q_heads, kv_heads, head_dim, n = 8, 2, 64, 300
-    kv = state.full_attention_bf16(n, q_heads, kv_heads, head_dim)
+    make = state.full_attention_f32 if element == "f32" else state.full_attention_bf16
+    kv = make(n, q_heads, kv_heads, head_dim)
     lay = oracle.layout(q_heads, kv_heads, head_dim)
-    cache = oracle.LayerKvCache("bf16r")
+    cache = oracle.LayerKvCache("f32" if element == "f32" else "bf16r")
     q = np.abs(rng.standard_normal((n, q_heads * head_dim), dtype=np.float32))
     scale = np.linspace(0.0, 9.0, n, dtype=np.float32)[:, None] * np.where(np.arange(n) % 3 == 0, -1.0, 1.0).astype(np.float32)[:, None]
     k = np.abs(rng.standard_normal((n, kv_heads * head_dim), dtype=np.float32)) * scale
     v = rng.standard_normal((n, kv_heads * head_dim), dtype=np.float32)
     got = kv.prefill_rows(q, k, v)
     want = oracle.cached_attention_prefill_rows(q, k, v, cache, lay)
-    # scores reach 9 * 64 * 0.64 / 8 = 46; two 8-bit terms a query: 2^-17 of them as an error of the exponent
-    assert np.abs(got - want).max() <= 46 * 2.0 ** -16 * np.abs(v).max()
+    # scores reach 9 * 64 * 0.64 / 8 = 46: on bf16 layers two 8-bit terms a query, 2^-17 of the score as an
+    # error of the exponent; on f32 ones a rounding of 2^-24 of the score at each of 64 sums
+    assert np.abs(got - want).max() <= 46 * np.abs(v).max() * (2.0 ** -16 if element == "bf16" else 64 * 2.0 ** -24)
+
+
+def test_f32_chunk_is_no_less_exact_than_f32_sums(state, shape):
+    """Three bf16 terms a factor, against 64 bits: no further off than torch's own f32 attention over
+    the same rows, whose sums are f32 products (a margin of 1.5 for the order of the sums)."""
+    import torch
+    q_heads, kv_heads, head_dim, base, n = 8, 2, 128, 700, 96
+    gen = torch.Generator().manual_seed(5)
+    k, v = (torch.randn(base + n, kv_heads * head_dim, generator=gen) * torch.exp(torch.randn(base + n, 1, generator=gen)) for _ in range(2))
+    q = torch.randn(n, q_heads * head_dim, generator=gen)
+    kv = state.full_attention_f32(base + n, q_heads, kv_heads, head_dim)
+    kv.seed(k[:base].numpy(), v[:base].numpy(), base)
+    got = torch.from_numpy(kv.prefill_rows(q.numpy(), k[base:].numpy(), v[base:].numpy()))
+
+    def attend(dt):
+        out = torch.empty(n, q_heads * head_dim, dtype=dt)
+        hidden = torch.arange(base + n)[None] > base + torch.arange(n)[:, None]
+        for h in range(q_heads):
+            g = h // (q_heads // kv_heads)
+            cols, own = slice(h * head_dim, (h + 1) * head_dim), slice(g * head_dim, (g + 1) * head_dim)
+            s = q[:, cols].to(dt) @ k[:, own].to(dt).T.contiguous() / head_dim ** 0.5
+            out[:, cols] = torch.softmax(s.masked_fill(hidden, -float("inf")), -1) @ v[:, own].to(dt)
+        return out
+
+    want, f32 = attend(torch.float64), attend(torch.float32)
+    assert (got.double() - want).norm() <= 1.5 * (f32.double() - want).norm()
