@@ -17,106 +17,137 @@ __device__ __forceinline__ float bf16_to_f32(uint16_t b) {
 }
 
 // ------------------------------------------------------------------------------------
-// append: f32 rows -> bf16 tiles. One thread per (row, kv head, 8-dim group): a 16-byte
-// store into the K tile, eight 2-byte stores into the transposed V tile. In a batch, the
-// rows that form whole position-aligned groups of four take a second kind of work item for
-// V instead: one thread per (row group, kv head, 32-dim block, column) gathers 4 rows x 2
-// dims and writes the 16 contiguous bytes they occupy in the tile.
+// append: f32 rows -> tiles, bf16 (rounded as above) or f32 (verbatim). One workgroup per page of
+// positions and kv head; its threads take the tile's 16-byte units as they lie in memory, K units
+// (8 or 4 dims of one row) and V units (4 rows of two dims or one), so stores are whole units
+// side by side and loads are runs of 64 bytes and more; rows outside the batch leave their K units
+// alone, and the V units they share with rows inside are written element by element.
 // Stands in for copy_at_f32_to_bf16 (src/decode_resident/kernels.rs:1036-1044).
+// Bound by the launch and one round trip up to about a thousand rows, then by memory. Kernel times
+// on one MI355X in us, against one thread per (row, 8 or 4 dims) with 64-bit divisions and V stores of an
+// element or, in whole groups, one unit: 1 row of 8 x 128 4.1 -> 3.0, 512 rows of 8 x 128 5.0 -> 3.4 (f32 7.6 -> 3.6),
+// of 8 x 256 6.3 -> 4.5 (f32 16.0 -> 5.0), 32768 rows of 8 x 128 142 -> 92 = 4.4 TB/s (f32 463 -> 121).
 // ------------------------------------------------------------------------------------
-// 8-dim groups of a row: those of head_dim (a layer's pools are zero in the padding from the start),
-// in pages without a table, which are scratch, those of the padding too.
-__host__ __device__ inline int append_groups(const AppendArgs &a) { return a.table ? (a.g.head_dim + 7) >> 3 : a.g.P >> 3; }
-
+template <bool F32, int UNITS> // UNITS: units of K, and of V, a thread takes
 __global__ __launch_bounds__(256) void append_kernel(AppendArgs a) {
+    typedef __attribute__((ext_vector_type(4))) float f4;
+    typedef __attribute__((ext_vector_type(4))) uint32_t w4;
     const Geom g = a.g;
-    const int groups = append_groups(a);
-    const long per_row = (long)g.kv_heads * groups;
-    const long page0 = a.first_pos >> 4; // first page of positions the batch touches
-    const long n_blk = ((a.first_pos + a.n_rows + 15) >> 4) - page0;
-    const long total_rows = a.by_page ? n_blk * per_row * 16 : per_row * a.n_rows;
+    const int kvh = blockIdx.y;
+    const long pos0 = (a.first_pos / 16 + blockIdx.x) * 16; // position of the page's first row
+    const long slot = slot_of(pos0, g.ring_rows);
+    const int page = a.table ? a.table[slot >> 4] : (int)(slot >> 4);
+    const long row0 = pos0 - a.first_pos; // batch row of the page's first row
+    const int r_lo = row0 < 0 ? (int)-row0 : 0, r_hi = (int)min(16l, a.n_rows - row0); // rows of the page in the batch
     const int kv_dim = g.kv_heads * g.head_dim;
-    const int per_grp = g.kv_heads * (g.P >> 5) * 16;
-    const long total = total_rows + (long)(a.v_grp_rows >> 2) * per_grp;
-    for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < total;
-         t += (long)gridDim.x * blockDim.x) {
-        if (t >= total_rows) {
-            // V of one aligned group of four rows: columns c and c + 16 of a 32-dim block
-            const long u = t - total_rows;
-            const int grp4 = (int)(u / per_grp);
-            int rem = (int)(u - (long)grp4 * per_grp);
-            const int kvh = rem / ((g.P >> 5) * 16);
-            rem -= kvh * ((g.P >> 5) * 16);
-            const int db = rem >> 4, c = rem & 15;
-            const int row0 = a.v_grp_first + grp4 * 4;
-            const long slot = slot_of(a.first_pos + row0, g.ring_rows); // a multiple of 4
-            const int page = a.table ? a.table[slot >> 4] : (int)(slot >> 4);
-            const long tile = (long)page * g.page_elems + (long)kvh * g.tile_elems;
-            const int d0 = db * 32 + c, d1 = d0 + 16;
-            const float *vs = a.v_src + (long)row0 * kv_dim + kvh * g.head_dim;
-            uint16_t lo[4], hi[4];
+    const float *ks = a.k_src + row0 * kv_dim + kvh * g.head_dim;
+    const float *vs = a.v_src + row0 * kv_dim + kvh * g.head_dim;
+    const long tile = (long)page * g.page_elems + (long)kvh * g.tile_elems;
+    w4 *kt = reinterpret_cast<w4 *>(a.k_pool + tile), *vt = reinterpret_cast<w4 *>(a.v_pool + tile);
+    const int units = g.tile_elems >> 3;
+    // K units past head_dim: a layer's pools are zero there from the start, scratch pages are not
+    const int k_units = a.table ? ((g.head_dim + (F32 ? 3 : 7)) / (F32 ? 4 : 8)) * 16 : units;
+    constexpr int KE = F32 ? 4 : 8; // dims of a K unit
+    constexpr int VD = F32 ? 1 : 2; // dims of a V unit
+
+    float kx[UNITS][KE], vx[UNITS][4][VD];
+    int kr[UNITS], kd[UNITS], vr[UNITS], vd[UNITS];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                lo[r] = d0 < g.head_dim ? bf16_bits(vs[(long)r * kv_dim + d0]) : (uint16_t)0;
-                hi[r] = d1 < g.head_dim ? bf16_bits(vs[(long)r * kv_dim + d1]) : (uint16_t)0;
+    for (int i = 0; i < UNITS; ++i) {
+        const int u = threadIdx.x + i * blockDim.x;
+        // unit u of a K tile: row u % 16; dims 8 (u / 16) .., or 16 (u / 64) + 4 (u / 16 % 4) ..
+        kr[i] = u & 15;
+        kd[i] = (u >> 4) * KE;
+        // unit u of a V tile: rows 4 (u / 16 % 4) ..; dims 32 (u / 64) + u % 16 and the one 16 further, or 16 (u / 64) + u % 16
+        vr[i] = ((u >> 4) & 3) * 4;
+        vd[i] = (u >> 6) * 16 * VD + (u & 15);
+        const int row = min(max(kr[i], r_lo), r_hi - 1); // clamped: loads are unconditional, one round trip
+        if (a.vec && kd[i] + KE <= g.head_dim) {
+#pragma unroll
+            for (int e = 0; e < KE; e += 4) {
+                const f4 x = *reinterpret_cast<const f4 *>(ks + (long)row * kv_dim + kd[i] + e);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) kx[i][e + t] = x[t];
             }
-            uint4 pk;
-            pk.x = lo[0] | ((uint32_t)lo[1] << 16);
-            pk.y = lo[2] | ((uint32_t)lo[3] << 16);
-            pk.z = hi[0] | ((uint32_t)hi[1] << 16);
-            pk.w = hi[2] | ((uint32_t)hi[3] << 16);
-            *reinterpret_cast<uint4 *>(a.v_pool + tile + v_index(g.P, (int)(slot & 15), d0)) = pk;
-            continue;
-        }
-        int row, kvh, grp;
-        if (a.by_page) {
-            const long blk = t / (per_row * 16);
-            const int rem = (int)(t - blk * per_row * 16);
-            const long pos = (page0 + blk) * 16 + (rem & 15);
-            if (pos < a.first_pos || pos >= a.first_pos + a.n_rows) continue;
-            row = (int)(pos - a.first_pos);
-            grp = (rem >> 4) % groups;
-            kvh = (rem >> 4) / groups;
         } else {
-            row = (int)(t / per_row);
-            const int rem = (int)(t - (long)row * per_row);
-            kvh = rem / groups;
-            grp = rem - kvh * groups;
+#pragma unroll
+            for (int e = 0; e < KE; ++e) kx[i][e] = ks[(long)row * kv_dim + min(kd[i] + e, g.head_dim - 1)];
         }
-        const long slot = slot_of(a.first_pos + row, g.ring_rows);
-        const int page = a.table ? a.table[slot >> 4] : (int)(slot >> 4);
-        const int r = (int)(slot & 15);
-        const long tile = (long)page * g.page_elems + (long)kvh * g.tile_elems;
-        const float *ks = a.k_src + (long)row * kv_dim + kvh * g.head_dim + grp * 8;
-        const float *vs = a.v_src + (long)row * kv_dim + kvh * g.head_dim + grp * 8;
-        const int d0 = grp * 8;
-        const int nd = min(8, g.head_dim - d0);
-        uint16_t kb[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) kb[e] = e < nd ? bf16_bits(ks[e]) : (uint16_t)0;
-        uint4 pk;
-        pk.x = kb[0] | ((uint32_t)kb[1] << 16);
-        pk.y = kb[2] | ((uint32_t)kb[3] << 16);
-        pk.z = kb[4] | ((uint32_t)kb[5] << 16);
-        pk.w = kb[6] | ((uint32_t)kb[7] << 16);
-        *reinterpret_cast<uint4 *>(a.k_pool + tile + k_index(g.P, r, d0)) = pk;
-        if (row >= a.v_grp_first && row < a.v_grp_first + a.v_grp_rows) continue; // V by groups
+        for (int r = 0; r < 4; ++r) {
+            const int vrow = min(max(vr[i] + r, r_lo), r_hi - 1);
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-            if (e < nd) a.v_pool[tile + v_index(g.P, r, d0 + e)] = bf16_bits(vs[e]);
+            for (int d = 0; d < VD; ++d) vx[i][r][d] = vs[(long)vrow * kv_dim + min(vd[i] + 16 * d, g.head_dim - 1)];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < UNITS; ++i) {
+        const int u = threadIdx.x + i * blockDim.x;
+        if (u < k_units && kr[i] >= r_lo && kr[i] < r_hi) {
+            w4 w;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                if constexpr (F32) {
+                    w[t] = kd[i] + t < g.head_dim ? __float_as_uint(kx[i][t]) : 0u;
+                } else {
+                    const uint32_t lo = kd[i] + 2 * t < g.head_dim ? bf16_bits(kx[i][2 * t]) : 0u;
+                    const uint32_t hi = kd[i] + 2 * t + 1 < g.head_dim ? bf16_bits(kx[i][2 * t + 1]) : 0u;
+                    w[t] = lo | (hi << 16);
+                }
+            }
+            kt[u] = w;
+        }
+        if (u < units && vd[i] < g.head_dim && vr[i] + 3 >= r_lo && vr[i] < r_hi) {
+            w4 w;
+            if constexpr (F32) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) w[r] = __float_as_uint(vx[i][r][0]);
+            } else {
+#pragma unroll
+                for (int d = 0; d < 2; ++d) {
+                    const bool in = vd[i] + 16 * d < g.head_dim;
+#pragma unroll
+                    for (int r = 0; r < 4; r += 2)
+                        w[d * 2 + (r >> 1)] = in ? bf16_bits(vx[i][r][d]) | ((uint32_t)bf16_bits(vx[i][r + 1][d]) << 16) : 0u;
+                }
+            }
+            if (vr[i] >= r_lo && vr[i] + 4 <= r_hi) {
+                vt[u] = w;
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if (vr[i] + r < r_lo || vr[i] + r >= r_hi) continue;
+                    if constexpr (F32) {
+                        reinterpret_cast<uint32_t *>(vt + u)[r] = w[r];
+                    } else {
+                        uint16_t *dst = reinterpret_cast<uint16_t *>(vt + u);
+                        dst[r] = (uint16_t)(w[r >> 1] >> ((r & 1) * 16));
+                        dst[4 + r] = (uint16_t)(w[2 + (r >> 1)] >> ((r & 1) * 16));
+                    }
+                }
+            }
+        }
     }
 }
 
 hipError_t launch_append(const AppendArgs &a, hipStream_t s) {
-    const int groups = append_groups(a);
-    const long n_blk = ((a.first_pos + a.n_rows + 15) >> 4) - (a.first_pos >> 4);
-    const long row_items = a.by_page ? n_blk * 16 : (long)a.n_rows;
-    const long total = (long)a.g.kv_heads * groups * row_items +
-                       (long)(a.v_grp_rows >> 2) * a.g.kv_heads * (a.g.P >> 5) * 16;
-    if (total <= 0) return hipSuccess;
-    long blocks = (total + 255) / 256;
-    if (blocks > 65535 * 4) blocks = 65535 * 4;
-    hipLaunchKernelGGL(append_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a);
+    if (a.n_rows <= 0) return hipSuccess;
+    AppendArgs b = a;
+    b.vec = ((uintptr_t)a.k_src & 15) == 0 && (a.g.head_dim & 3) == 0; // 16-byte loads of K
+    const int units = a.g.tile_elems >> 3;
+    const long pages = (a.first_pos + a.n_rows + 15) / 16 - a.first_pos / 16;
+    const dim3 grid((unsigned)pages, (unsigned)a.g.kv_heads), block((unsigned)(units < 256 ? units : 256));
+    const int per = (units + 255) / 256;
+    if (a.g.f32) {
+        if (per <= 1) hipLaunchKernelGGL((append_kernel<true, 1>), grid, block, 0, s, b);
+        else if (per <= 2) hipLaunchKernelGGL((append_kernel<true, 2>), grid, block, 0, s, b);
+        else if (per <= 4) hipLaunchKernelGGL((append_kernel<true, 4>), grid, block, 0, s, b);
+        else hipLaunchKernelGGL((append_kernel<true, 8>), grid, block, 0, s, b);
+    } else {
+        if (per <= 1) hipLaunchKernelGGL((append_kernel<false, 1>), grid, block, 0, s, b);
+        else if (per <= 2) hipLaunchKernelGGL((append_kernel<false, 2>), grid, block, 0, s, b);
+        else hipLaunchKernelGGL((append_kernel<false, 4>), grid, block, 0, s, b);
+    }
     return hipGetLastError();
 }
 

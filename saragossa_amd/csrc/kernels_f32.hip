@@ -24,51 +24,6 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 
 bool f32_decode_kernel_serves(const DecodeArgs &a);
 
-// ------------------------------------------------------------------------------------
-// append: rows [n_rows, kv_dim] f32 -> tiles, verbatim. One thread per (row, kv head, four
-// dims): a 16-byte K store and four 4-byte V stores.
-// ------------------------------------------------------------------------------------
-// four-dim groups of a row: those of head_dim, in pages without a table (scratch) those of the padding too
-__host__ __device__ inline int append_f32_groups(const AppendArgs &a) { return a.table ? (a.g.head_dim + 3) >> 2 : a.g.P >> 2; }
-
-__global__ __launch_bounds__(256) void append_f32_kernel(AppendArgs a) {
-    const Geom g = a.g;
-    const int groups = append_f32_groups(a);
-    const long per_row = (long)g.kv_heads * groups;
-    const long total = per_row * a.n_rows;
-    const int kv_dim = g.kv_heads * g.head_dim;
-    float *k_pool = reinterpret_cast<float *>(a.k_pool);
-    float *v_pool = reinterpret_cast<float *>(a.v_pool);
-    for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += (long)gridDim.x * blockDim.x) {
-        const int row = (int)(t / per_row);
-        const int rem = (int)(t - (long)row * per_row);
-        const int kvh = rem / groups;
-        const int d0 = (rem - kvh * groups) * 4;
-        const long slot = slot_of(a.first_pos + row, g.ring_rows);
-        const int page = a.table ? a.table[slot >> 4] : (int)(slot >> 4);
-        const int r = (int)(slot & 15);
-        // tile_elems and page_elems count 16-bit units: two per float
-        const long tile = ((long)page * g.page_elems + (long)kvh * g.tile_elems) >> 1;
-        const float *ks = a.k_src + (long)row * kv_dim + kvh * g.head_dim + d0;
-        const float *vs = a.v_src + (long)row * kv_dim + kvh * g.head_dim + d0;
-        float4_t kq;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) kq[e] = d0 + e < g.head_dim ? ks[e] : 0.0f;
-        *reinterpret_cast<float4_t *>(k_pool + tile + k_index_f32(r, d0)) = kq;
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (d0 + e < g.head_dim) v_pool[tile + v_index_f32(r, d0 + e)] = vs[e];
-    }
-}
-
-hipError_t launch_append_f32(const AppendArgs &a, hipStream_t s) {
-    const long total = (long)a.g.kv_heads * append_f32_groups(a) * a.n_rows;
-    long blocks = (total + 255) / 256;
-    if (blocks > 65535 * 4) blocks = 65535 * 4;
-    hipLaunchKernelGGL(append_f32_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a);
-    return hipGetLastError();
-}
-
 // gather: tiles -> row-major f32 rows [n_rows, kv_dim], through the block table.
 __global__ __launch_bounds__(256) void gather_f32_kernel(GatherArgs a) {
     const Geom g = a.g;

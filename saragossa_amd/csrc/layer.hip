@@ -576,15 +576,6 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
     return SKV_OK;
 }
 
-// Batches: whole groups of four rows at positions that are multiples of 4 write V in 16-byte units.
-void plan_batch(AppendArgs &a) {
-    if (a.n_rows < 8) return;
-    a.by_page = 1;
-    const long lead = (4 - (a.first_pos & 3)) & 3;
-    a.v_grp_first = (int)lead;
-    a.v_grp_rows = (int)((a.n_rows - lead) & ~3L);
-}
-
 int32_t encode_append(skv_layer *L, hipStream_t s, const float *k_dev, const float *v_dev,
                       size_t n_rows) {
     if (n_rows == 0) return SKV_OK;
@@ -609,14 +600,6 @@ int32_t encode_append(skv_layer *L, hipStream_t s, const float *k_dev, const flo
         a.first_pos += (long)skip;
         a.n_rows = L->g.ring_rows;
     }
-    if (L->g.f32) {
-        SKV_HIP(launch_append_f32(a, s));
-        L->len += n_rows;
-        if (L->g.ring_rows > 0 && L->len > (size_t)L->g.ring_rows)
-            L->floor_pos = std::max(L->floor_pos, L->len - (size_t)L->g.ring_rows);
-        return SKV_OK;
-    }
-    plan_batch(a);
     SKV_HIP(launch_append(a, s));
     L->len += n_rows;
     if (L->g.ring_rows > 0 && L->len > (size_t)L->g.ring_rows)
@@ -1162,8 +1145,7 @@ static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const flo
     w.n_rows = (int)c;
     w.g = g;
     w.g.ring_rows = 0;
-    if (!g.f32) plan_batch(w);
-    SKV_HIP(g.f32 ? launch_append_f32(w, s) : launch_append(w, s));
+    SKV_HIP(launch_append(w, s));
     pages.k_new = w.k_pool;
     pages.v_new = w.v_pool;
     SKV_HIP(g.f32 ? launch_f32_prefill(a, pages, halves, s) : launch_prefill_tiles(a, pages, shape, s));

@@ -95,14 +95,7 @@ struct AppendArgs {
     const int32_t *table; // null = page i of the pools is page i of the positions
     long first_pos; // position of the first appended row
     int n_rows;
-    // rows [v_grp_first, v_grp_first + v_grp_rows) of the batch start at a position that is a
-    // multiple of 4 and come in whole groups of 4: their V elements are written as 16-byte
-    // units of the transposed tile (4 rows x 2 dims) instead of 2-byte stores
-    int v_grp_first;
-    int v_grp_rows;
-    // batches: row items are numbered page by page with the row inside the page fastest, so
-    // that sixteen neighbouring threads write 256 contiguous bytes of a K tile
-    int by_page;
+    int vec;        // K rows may be read 16 bytes at a time (set by the launcher)
     Geom g;
 };
 
@@ -349,7 +342,6 @@ hipError_t launch_append(const AppendArgs &a, hipStream_t s);
 hipError_t launch_gather(const GatherArgs &a, hipStream_t s);
 // f32 storage mode: rows in and out (k_dst / v_dst of GatherArgs then point at f32 rows), and
 // the split launch for one query row or a chunk (the caller merges as for bf16)
-hipError_t launch_append_f32(const AppendArgs &a, hipStream_t s);
 hipError_t launch_gather_f32(const GatherArgs &a, hipStream_t s);
 hipError_t launch_f32_split(const DecodeArgs &a, hipStream_t s);
 bool f32_decode_kernel_serves(const DecodeArgs &a); // the launch takes the kernel that can also append the row

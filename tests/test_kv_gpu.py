@@ -309,3 +309,38 @@ def test_layer_bytes_is_what_a_created_layer_takes(dtype, window):
         kv.close()
     finally:
         st.close()
+
+
+@pytest.mark.parametrize("element", ["bf16", "f32"])
+@pytest.mark.parametrize("dims,window,first,counts,pad", [
+    ((4, 2, 16), 0, 3, (1, 2, 9, 30), 0),      # rows inside one page, across an edge, groups of four cut at both ends
+    ((6, 1, 40), 0, 15, (1, 16, 17), 0),       # head_dim not a multiple of 16
+    ((3, 3, 7), 0, 0, (5, 12), 0),             # nor of four
+    ((8, 2, 64), 0, 2, (21,), 1),              # rows at an address that is not a multiple of 16
+    ((4, 1, 320), 0, 30, (4, 33), 0),          # several units a thread, padded head
+    ((2, 2, 512), 0, 7, (10,), 0),
+    ((8, 2, 64), 33, 40, (3, 50, 200), 0),     # ring: wraps inside a page, more rows than the ring holds
+])
+def test_append_batches_at_page_edges(state, element, dims, window, first, counts, pad):
+    """Batches of rows land bit for bit, and leave their neighbours in shared pages alone."""
+    import torch
+    q_heads, kv_heads, head_dim = dims
+    kv_dim = kv_heads * head_dim
+    rng = np.random.default_rng(head_dim + first)
+    make = state.full_attention_f32 if element == "f32" else state.full_attention_bf16
+    kv = make(first + sum(counts) + 1, q_heads, kv_heads, head_dim, window=window)
+    kv.set_block_table(rng.permutation(kv.pages()).astype(np.int32))
+    want = [np.zeros((0, kv_dim), np.float32)] * 2
+    for n in ((first,) if first else ()) + counts:
+        rows = [rng.standard_normal((n, kv_dim), dtype=np.float32) for _ in range(2)]
+        bufs = [torch.zeros(n * kv_dim + pad, device="cuda") for _ in range(2)]
+        for b, r in zip(bufs, rows):
+            b[pad:].copy_(torch.from_numpy(r.reshape(-1)))
+        kv.encode_append_batch(torch.cuda.current_stream().cuda_stream, bufs[0].data_ptr() + 4 * pad,
+                               bufs[1].data_ptr() + 4 * pad, n)
+        torch.cuda.synchronize()
+        rows = rows if element == "f32" else [oracle.bf16_round(r.reshape(-1)).reshape(r.shape) for r in rows]
+        want = [np.concatenate([w, r]) for w, r in zip(want, rows)]
+        lo = max(0, kv.len() - window) if window else 0
+        for got, w in zip(kv.read_rows_f32(lo, kv.len() - lo), want):
+            assert np.array_equal(got, w[lo:]), n
