@@ -17,8 +17,8 @@ __device__ __forceinline__ float bf16_to_f32(uint16_t b) {
 }
 
 // ------------------------------------------------------------------------------------
-// append: f32 rows -> tiles, bf16 (rounded as above) or f32 (verbatim). One workgroup per page of
-// positions and kv head; its threads take the tile's 16-byte units as they lie in memory, K units
+// append: f32 rows -> tiles, bf16 (rounded as above) or f32 (verbatim). One or more workgroups per page of
+// positions and kv head; their threads take the tile's 16-byte units as they lie in memory, K units
 // (8 or 4 dims of one row) and V units (4 rows of two dims or one), so stores are whole units
 // side by side and loads are runs of 64 bytes and more; rows outside the batch leave their K units
 // alone, and the V units they share with rows inside are written element by element.
@@ -26,7 +26,8 @@ __device__ __forceinline__ float bf16_to_f32(uint16_t b) {
 // Bound by the launch and one round trip up to about a thousand rows, then by memory. Kernel times
 // on one MI355X in us, against one thread per (row, 8 or 4 dims) with 64-bit divisions and V stores of an
 // element or, in whole groups, one unit: 1 row of 8 x 128 4.1 -> 3.0, 512 rows of 8 x 128 5.0 -> 3.4 (f32 7.6 -> 3.6),
-// of 8 x 256 6.3 -> 4.5 (f32 16.0 -> 5.0), 32768 rows of 8 x 128 142 -> 92 = 4.4 TB/s (f32 463 -> 121).
+// 32768 rows of 8 x 128 142 -> 92 = 4.4 TB/s (f32 463 -> 121); as calls in a row, 1 row of 2 x 512 f32 2.9 -> 1.9,
+// 6 rows of 2 x 256 bf16 4.4 -> 2.2, 130 rows of 8 x 256 f32 5.4 -> 2.4.
 // ------------------------------------------------------------------------------------
 template <bool F32, int UNITS> // UNITS: units of K, and of V, a thread takes
 __global__ __launch_bounds__(256) void append_kernel(AppendArgs a) {
@@ -54,7 +55,7 @@ __global__ __launch_bounds__(256) void append_kernel(AppendArgs a) {
     int kr[UNITS], kd[UNITS], vr[UNITS], vd[UNITS];
 #pragma unroll
     for (int i = 0; i < UNITS; ++i) {
-        const int u = threadIdx.x + i * blockDim.x;
+        const int u = threadIdx.x + (blockIdx.z * UNITS + i) * blockDim.x;
         // unit u of a K tile: row u % 16; dims 8 (u / 16) .., or 16 (u / 64) + 4 (u / 16 % 4) ..
         kr[i] = u & 15;
         kd[i] = (u >> 4) * KE;
@@ -82,7 +83,7 @@ __global__ __launch_bounds__(256) void append_kernel(AppendArgs a) {
     }
 #pragma unroll
     for (int i = 0; i < UNITS; ++i) {
-        const int u = threadIdx.x + i * blockDim.x;
+        const int u = threadIdx.x + (blockIdx.z * UNITS + i) * blockDim.x;
         if (u < k_units && kr[i] >= r_lo && kr[i] < r_hi) {
             w4 w;
 #pragma unroll
@@ -136,8 +137,15 @@ hipError_t launch_append(const AppendArgs &a, hipStream_t s) {
     b.vec = ((uintptr_t)a.k_src & 15) == 0 && (a.g.head_dim & 3) == 0; // 16-byte loads of K
     const int units = a.g.tile_elems >> 3;
     const long pages = (a.first_pos + a.n_rows + 15) / 16 - a.first_pos / 16;
-    const dim3 grid((unsigned)pages, (unsigned)a.g.kv_heads), block((unsigned)(units < 256 ? units : 256));
-    const int per = (units + 255) / 256;
+    // A tile of more than 256 units is shared by workgroups of 256 units each while those are at most
+    // 4096, else one workgroup takes it whole, several units a thread: shared / whole in us, 1 row of 2 x 512
+    // f32 1.9/4.2, 512 rows of 2 x 256 bf16 2.4/3.0, of 2 x 512 2.8/4.4, of 8 x 256 3.4/3.9 (f32 3.7/4.3), 2048 rows of
+    // 8 x 256 7.4/7.7 (f32, 4128 workgroups, 10.2/9.4).
+    const int rounds = (units + 255) / 256;
+    const bool spread = pages * a.g.kv_heads * rounds <= 4096;
+    const int per = spread ? 1 : rounds;
+    const dim3 grid((unsigned)pages, (unsigned)a.g.kv_heads, (unsigned)(spread ? rounds : 1));
+    const dim3 block((unsigned)(units < 256 ? units : 256));
     if (a.g.f32) {
         if (per <= 1) hipLaunchKernelGGL((append_kernel<true, 1>), grid, block, 0, s, b);
         else if (per <= 2) hipLaunchKernelGGL((append_kernel<true, 2>), grid, block, 0, s, b);

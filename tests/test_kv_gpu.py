@@ -317,8 +317,9 @@ def test_layer_bytes_is_what_a_created_layer_takes(dtype, window):
     ((6, 1, 40), 0, 15, (1, 16, 17), 0),       # head_dim not a multiple of 16
     ((3, 3, 7), 0, 0, (5, 12), 0),             # nor of four
     ((8, 2, 64), 0, 2, (21,), 1),              # rows at an address that is not a multiple of 16
-    ((4, 1, 320), 0, 30, (4, 33), 0),          # several units a thread, padded head
+    ((4, 1, 320), 0, 30, (4, 33), 0),          # several workgroups a tile, padded head
     ((2, 2, 512), 0, 7, (10,), 0),
+    ((2, 2, 512), 0, 5, (8230,), 0),           # more tiles than get several workgroups each
     ((8, 2, 64), 33, 40, (3, 50, 200), 0),     # ring: wraps inside a page, more rows than the ring holds
 ])
 def test_append_batches_at_page_edges(state, element, dims, window, first, counts, pad):
