@@ -597,26 +597,14 @@ __global__ __launch_bounds__(64) void norm_rope_wave_kernel(NormRopeArgs a) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const float iv = __shfl(inv, pr[u], 64);
-        f4 n = x[u] * iv;
-        n = n * w[u];
+        f4 n;
         if (a.rope && c4[u] < rope4) {
-            if (a.rope_style == 1) {
-                const float a0 = n[0] * r0[u][0], b0 = n[1] * r0[u][1], c0 = n[0] * r0[u][1], d0 = n[1] * r0[u][0];
-                const float a1 = n[2] * r0[u][2], b1 = n[3] * r0[u][3], c1 = n[2] * r0[u][3], d1 = n[3] * r0[u][2];
-                n = f4{a0 - b0, c0 + d0, a1 - b1, c1 + d1};
-            } else {
-                const bool is_first = c4[u] < half4;
-                const int oc4 = is_first ? c4[u] + half4 : c4[u] - half4;
-                f4 o = raw[pr[u] * (HD4 + 1) + oc4] * iv;
-                o = o * ow[u];
-                const float cs[4] = {r0[u][0], r0[u][2], r1[u][0], r1[u][2]};
-                const float sn[4] = {r0[u][1], r0[u][3], r1[u][1], r1[u][3]};
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float nc = n[e] * cs[e], os = o[e] * sn[e];
-                    n[e] = is_first ? nc - os : os + nc;
-                }
-            }
+            const bool is_first = c4[u] < half4;
+            const int oc4 = a.rope_style == 1 ? c4[u] : is_first ? c4[u] + half4 : c4[u] - half4;
+            n = norm_rope_unit(x[u], raw[pr[u] * (HD4 + 1) + oc4], w[u], ow[u], r0[u], r1[u], iv, a.rope_style, is_first);
+        } else {
+            n = x[u] * iv;
+            n = n * w[u];
         }
         if (mine[u])
             *reinterpret_cast<f4 *>(a.out + ((long)(pair0 + pr[u]) * hd4 + c4[u]) * 4) = n;

@@ -1,6 +1,6 @@
 // gfx950 kernels of the KV hot path, part 2: split-K GQA decode attention over the
 // paged bf16 cache on the matrix cores, and the merge of its partials.
-#include "skv_internal.h"
+#include "pre_kv.h"
 
 namespace skv {
 
@@ -112,17 +112,8 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
     uint4 *q_lo = smem + KK * 64;
     uint16_t *new_k = reinterpret_cast<uint16_t *>(smem + 2 * KK * 64); // [P] appended row
     uint16_t *new_v = new_k + P;
-    // PRE: raw and finished rows of the group's queries plus the new k row, weights, rotation
-    constexpr int PS = P + 1;      // row stride: lanes walking different rows hit different banks
-    constexpr int PRE_ROWS = 17;   // 16 query slots + the k row
-    float *pre_raw = reinterpret_cast<float *>(new_v + P); // [PRE_ROWS][PS]
-    float *pre_out = pre_raw + PRE_ROWS * PS;              // [PRE_ROWS][PS]
-    float *pre_wq = pre_out + PRE_ROWS * PS;               // [P]
-    float *pre_wk = pre_wq + P;                            // [P]
-    float *pre_rope = pre_wk + P;                          // [P]: (cos, sin) pairs
-    float *pre_inv = pre_rope + P;                         // [PRE_ROWS] (+5 keeps pre_sq 16-byte aligned)
-    constexpr int SQS = P + 4;                             // 16-byte aligned rows, conflict-free
-    float *pre_sq = pre_inv + PRE_ROWS + 5;                // [PRE_ROWS][SQS]: squares, zero padded
+    using Pre = PreKvStage<P, THREADS>;
+    float *pre_lds = reinterpret_cast<float *>(new_v + P); // PRE: the pre-KV step's staging area
 
     // pages this workgroup's slots can see, divided among the splits
     const int page_lo = g.ring_rows > 0 ? 0 : ws_lo >> 4;
@@ -171,25 +162,8 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
             v_rows[u] = a.v_new[kvh * g.head_dim + tid + u * THREADS];
         }
     }
-    // PRE: raw query rows of the group (and the raw k row, already in k_row)
-    constexpr int PRE_U = PRE ? (16 * P + THREADS - 1) / THREADS : 1;
-    float pre_q[PRE_U];
-    float pre_w0[NE], pre_w1[NE], pre_r[NE];
-    if (PRE) {
-#pragma unroll
-        for (int u = 0; u < PRE_U; ++u) {
-            const int e = tid + u * THREADS;
-            const int r = e / P, c = e % P;
-            pre_q[u] = (r < rows && c < g.head_dim) ? a.q[(long)(kvh * G + r) * q_stride + c] : 0.0f;
-        }
-#pragma unroll
-        for (int u = 0; u < NE; ++u) {
-            const int d = tid + u * THREADS;
-            pre_w0[u] = (a.q_norm_w && d < g.head_dim) ? a.q_norm_w[d] : 1.0f;
-            pre_w1[u] = (a.k_norm_w && d < g.head_dim) ? a.k_norm_w[d] : 1.0f;
-            pre_r[u] = (a.rope && d < a.rope_dims) ? a.rope[d] : 0.0f;
-        }
-    }
+    Pre pre; // PRE: the raw query rows of the group (the raw k row is in k_rows), weights, rotation
+    if constexpr (PRE) pre.load(a, kvh, rows, q_stride, tid);
 
     // Block-table entries of the next 64 iterations, one per lane.
     int ids = 0;
@@ -230,70 +204,62 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
     }
     // Unconditional (a wavefront without pages reads physical page 0 and ignores it): a
     // conditional load here makes the compiler wait for these pages before the queries.
-    // The first page's table entry comes through the scalar unit (the address is the same in
-    // every lane): that read is counted apart from the vector loads above, so the first K/V
-    // request waits for it alone and not for the queries, nor, in the workgroup that
-    // appends, for the new row, which no other workgroup has pulled into a cache.
+    // The first page's table entry comes through the scalar unit: that read is counted apart from
+    // the vector loads above, so the first K request waits for it alone and not for the queries, nor,
+    // in the workgroup that appends, for the new row, which no other workgroup has pulled into a
+    // cache. V, which is needed later, is asked for behind the barriers: a compute unit accepts
+    // requests only as fast as memory answers, and a wavefront does not reach a barrier before its
+    // own are accepted. Decode steps, V behind the staging barrier / with K, in us: q32/kv8/hd128 over
+    // 1024, 16384 rows 6.9/7.1, 15.3/15.1; q16/kv2/hd256 over 8192, 32768 rows 9.8/10.4, 17.6/17.8. With the pre-KV
+    // step behind the ordered sums (two tokens through ten gated layers of q16/kv2/hd256 over 32768 rows:
+    // 365 us; with K 380; behind the last barrier 376). A chunk's few rows have V with K (six rows over
+    // 8192 of q16/kv2/hd256, whole pass over 10 layers 258/262).
     uint4 kr[KK], vr[KK];
-    {
-        typedef const __attribute__((address_space(4))) int32_t *const_i32_ptr;
-        const int pg = reinterpret_cast<const_i32_ptr>(reinterpret_cast<uintptr_t>(a.table))[min(pb0 + wave + rot * WAVES, max(page_hi - 1, 0))];
-        load_k<KK>(kr, a, pg, kvh, lane);
-        load_v<KK>(vr, a, pg, kvh, lane);
-    }
-    if (PRE) {
-        auto sq_of = [](float x) {
-#pragma clang fp contract(off)
-            return x * x;
-        };
-        // rows 0..rows-1: the group's queries; row `rows`: the new k row (appending workgroup)
-#pragma unroll
-        for (int u = 0; u < PRE_U; ++u) {
-            const int e = tid + u * THREADS;
-            const int r = e / P, c = e % P;
-            if (r < rows) {
-                pre_raw[r * PS + c] = pre_q[u];
-                pre_sq[r * SQS + c] = sq_of(pre_q[u]);
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < NE; ++u) {
-            const int d = tid + u * THREADS;
-            if (d < P) {
-                pre_raw[rows * PS + d] = k_rows[u];
-                pre_sq[rows * SQS + d] = sq_of(k_rows[u]);
-                pre_wq[d] = pre_w0[u];
-                pre_wk[d] = pre_w1[u];
-                pre_rope[d] = pre_r[u];
-            }
-        }
-        __syncthreads();
+    const int pg = table_entry<PRE>(a.table, min(pb0 + wave + rot * WAVES, max(page_hi - 1, 0)));
+    load_k<KK>(kr, a, pg, kvh, lane);
+    if constexpr (MQ) load_v<KK>(vr, a, pg, kvh, lane);
+    // the appended row's tile; its page's physical id comes with the arguments: a table lookup would wait for
+    // every load issued before it, the first K page included
+    auto new_tile = [&]() __attribute__((always_inline)) { return (long)a.new_page * g.page_elems + (long)kvh * g.tile_elems; };
+    if constexpr (PRE) {
+        pre.stage(pre_lds, a, rows, k_rows, tid);
+        // query slots that the group does not fill
+        for (int idx = tid; idx < KK * 64; idx += THREADS)
+            if ((idx & 15) >= rows) q_hi[idx] = q_lo[idx] = make_uint4(0, 0, 0, 0);
         const int n_rows = rows + (appends ? 1 : 0);
-        if (tid < n_rows) {
-            const bool is_k = tid == rows;
-            const bool has_norm = is_k ? a.k_norm_w != nullptr : a.q_norm_w != nullptr;
-            pre_inv[tid] = has_norm ? head_inv_rms_sq(pre_sq + tid * SQS, P, g.head_dim, a.eps) : 1.0f;
-        }
         __syncthreads();
-        const float *rope = a.rope ? pre_rope : nullptr;
-        for (int e = tid; e < n_rows * P; e += THREADS) {
-            const int r = e / P, c = e % P;
-            if (c < g.head_dim) {
-                const bool is_k = r == rows;
-                const float *w = is_k ? (a.k_norm_w ? pre_wk : nullptr) : (a.q_norm_w ? pre_wq : nullptr);
-                pre_out[r * PS + c] = norm_rope_elem(pre_raw + r * PS, c, pre_inv[r], w, rope,
-                                                     a.rope_dims, a.rope_style);
-            }
-        }
+        Pre::scales(pre_lds, a, rows, n_rows, tid);
         __syncthreads();
+        load_v<KK>(vr, a, pg, kvh, lane);
+        // finished queries go straight to their operand layout (hi and lo halves), the finished k row to the
+        // pool and to LDS
+        Pre::each(pre_lds, a, rows, n_rows, tid, [&](int r, int c4, float4_t v) __attribute__((always_inline)) {
+#pragma clang fp contract(off)
+            if (r < rows) {
+                uint32_t hi[2] = {0, 0}, lo[2] = {0, 0};
 #pragma unroll
-        for (int u = 0; u < NE; ++u)
-            if (appends && tid + u * THREADS < g.head_dim) k_rows[u] = pre_out[rows * PS + tid + u * THREADS];
+                for (int i = 0; i < 4; ++i) {
+                    const float x = v[i] * a.qscale;
+                    const uint16_t hb = bf16_bits(x);
+                    hi[i >> 1] |= (uint32_t)hb << (16 * (i & 1));
+                    lo[i >> 1] |= (uint32_t)bf16_bits(x - bf16_to_f32(hb)) << (16 * (i & 1));
+                }
+                const int at = ((c4 >> 1) * 16 + r) * 2 + (c4 & 1); // 8-byte units: [P/8][16 slots][2]
+                reinterpret_cast<uint2 *>(q_hi)[at] = make_uint2(hi[0], hi[1]);
+                reinterpret_cast<uint2 *>(q_lo)[at] = make_uint2(lo[0], lo[1]);
+            } else {
+                uint2 kb;
+                kb.x = bf16_bits(v[0]) | (uint32_t)bf16_bits(v[1]) << 16;
+                kb.y = bf16_bits(v[2]) | (uint32_t)bf16_bits(v[3]) << 16;
+                // (a unit past head_dim is padding, zero already; one across it stores its zeros again)
+                if (c4 * 4 < g.head_dim)
+                    *reinterpret_cast<uint2 *>(const_cast<uint16_t *>(a.k_pool) + new_tile() + k_index(P, r_new, c4 * 4)) = kb;
+                *reinterpret_cast<uint2 *>(new_k + c4 * 4) = kb;
+            }
+        });
     }
     if (appends) {
-        // the page's physical id comes with the arguments: a table lookup here would wait for
-        // every load issued before it, the first K/V page included
-        const long tile_at = (long)a.new_page * g.page_elems + (long)kvh * g.tile_elems;
+        const long tile_at = new_tile();
 #pragma unroll
         for (int u = 0; u < NE; ++u) {
             const int d = tid + u * THREADS;
@@ -302,28 +268,16 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
                 if (d < g.head_dim) {
                     kb = bf16_bits(k_rows[u]);
                     vb = bf16_bits(v_rows[u]);
-                    const_cast<uint16_t *>(a.k_pool)[tile_at + k_index(P, r_new, d)] = kb;
+                    if (!PRE) const_cast<uint16_t *>(a.k_pool)[tile_at + k_index(P, r_new, d)] = kb;
                     const_cast<uint16_t *>(a.v_pool)[tile_at + v_index(P, r_new, d)] = vb;
                 }
-                new_k[d] = kb;
+                if (!PRE) new_k[d] = kb;
                 new_v[d] = vb;
             }
         }
     }
-    if (PRE) {
 #pragma unroll
-        for (int u = 0; u < QI; ++u) {
-            const int idx = min(tid + u * THREADS, KK * 64 - 1);
-            const int kk = idx >> 6;
-            const int jj = (idx >> 4) & 3;
-            const int qs = min(idx & 15, rows - 1);
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-                qv[u][e] = pre_out[qs * PS + min(kk * 32 + jj * 8 + e, g.head_dim - 1)];
-        }
-    }
-#pragma unroll
-    for (int u = 0; u < QI; ++u) {
+    for (int u = 0; u < (PRE ? 0 : QI); ++u) {
         const int idx = tid + u * THREADS;
         if (idx < KK * 64) {
             const int kk = idx >> 6;
@@ -350,6 +304,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
         }
     }
     __syncthreads();
+    if constexpr (!MQ && !PRE) load_v<KK>(vr, a, pg, kvh, lane);
 
     float4_t o[NT];
 #pragma unroll
@@ -850,7 +805,7 @@ template <int P, int WAVES, bool MQ, bool PRE>
 static hipError_t launch_split_mq(const DecodeArgs &a, hipStream_t s) {
     constexpr int KK = P / 32;
     size_t stage = (size_t)2 * KK * 64 * sizeof(uint4) + 2 * P * sizeof(uint16_t);
-    if (PRE) stage += ((size_t)2 * 17 * (P + 1) + 3 * P + 22 + 17 * (P + 4)) * sizeof(float);
+    if (PRE) stage += PreKvStage<P, WAVES * 64>::LDS_FLOATS * sizeof(float);
     const int n_slots = a.n_queries * a.g.gqa;
     const int rows = n_slots < 16 ? n_slots : 16;
     const size_t xchg = ((size_t)WAVES * rows * (P + 4) + 2 * WAVES * rows) * sizeof(float);

@@ -12,7 +12,7 @@
 //   V: float4 unit (c, jj, dd) = rows 4jj .. 4jj+3 of dim 16c + dd, at unit index c * 64 + jj * 16 + dd
 #include <type_traits>
 
-#include "skv_internal.h"
+#include "pre_kv.h"
 
 namespace skv {
 
@@ -484,68 +484,79 @@ __device__ __forceinline__ void f32_decode_body(const DecodeArgs &a, const int s
     const int r_new = a.new_slot & 15;
     const bool appends = a.k_new != nullptr && pb_new >= pb0 && pb_new < pb1;
 
-    // ---- PRE: q and the new k row arrive raw; the per-head RMSNorm and the rotation of the
-    // position are applied here, in LDS (the area the wavefronts' states use at the end), with
-    // the arithmetic and the order of rms_norm_rope_heads_at (src/decoder/attention_ops.rs:682-777),
-    // so that the finished rows, and the k row this launch stores, equal the CPU path's.
-    constexpr int PS = P + 1;      // row stride: lanes walking different rows hit different banks
-    constexpr int SQS = P + 4;     // squares: 16-byte aligned rows
-    constexpr int PRE_ROWS = 17;   // 16 query slots + the k row
-    float *pre_raw = reinterpret_cast<float *>(xch);   // [PRE_ROWS][PS]
-    float *pre_out = pre_raw + PRE_ROWS * PS;          // [PRE_ROWS][PS]
-    float *pre_wq = pre_out + PRE_ROWS * PS;           // [P]
-    float *pre_wk = pre_wq + P;                        // [P]
-    float *pre_rope = pre_wk + P;                      // [P]: (cos, sin) pairs
-    float *pre_inv = pre_rope + P;                     // [PRE_ROWS] (+5 keeps pre_sq 16-byte aligned)
-    float *pre_sq = pre_inv + PRE_ROWS + 5;            // [PRE_ROWS][SQS]
-    static_assert(!PRE || ((size_t)(2 * PRE_ROWS * PS + 3 * P + PRE_ROWS + 5 + PRE_ROWS * SQS) * sizeof(float) <=
-                           (size_t)WAVES * NT * 64 * sizeof(float4_t)),
+    float4_t k_first[NT], v_first[NT]; // PRE: the first page
+    auto tile_in = [&](int page, const float *pool) __attribute__((always_inline)) {
+        return reinterpret_cast<const float4_t *>(pool + (((long)page * g.page_elems + (long)kvh * g.tile_elems) >> 1)) + lane;
+    };
+    auto tile_of = [&](int idx, const float *pool) __attribute__((always_inline)) {
+        return tile_in(__builtin_amdgcn_readlane(ids, idx), pool);
+    };
+    auto load_tile = [&](const float4_t *t, float4_t (&dst)[NT]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int m = 0; m < NT; ++m) dst[m] = __builtin_nontemporal_load(t + m * 64);
+    };
+
+    // ---- PRE: q and the new k row arrive raw and are finished here, in the area the wavefronts'
+    // states use at the end
+    using Pre = PreKvStage<P, THREADS>;
+    float *pre_lds = reinterpret_cast<float *>(xch);
+    static_assert(!PRE || Pre::LDS_FLOATS * sizeof(float) <= (size_t)WAVES * NT * 64 * sizeof(float4_t),
                   "the pre-KV scratch fits the exchange area it borrows");
     const int rows = min(16, n_slots - slot0);
+    auto new_tile = [&]() __attribute__((always_inline)) { // of the appended row
+        return ((long)a.new_page * g.page_elems + (long)kvh * g.tile_elems) >> 1;
+    };
     if constexpr (PRE) {
-        auto sq_of = [](float x) {
-#pragma clang fp contract(off)
-            return x * x;
-        };
-        for (int e = tid; e < rows * P; e += THREADS) {
-            const int r = e / P, c = e % P;
-            const float x = c < g.head_dim ? a.q[(long)(kvh * G + slot0 + r) * q_stride + c] : 0.0f;
-            pre_raw[r * PS + c] = x;
-            pre_sq[r * SQS + c] = sq_of(x);
+        // elements tid, tid + THREADS of the new row, ahead of the page
+        float k_rows[Pre::NE], v_rows[Pre::NE];
+#pragma unroll
+        for (int u = 0; u < Pre::NE; ++u) {
+            const int d = tid + u * THREADS;
+            const bool has = appends && d < g.head_dim;
+            k_rows[u] = has ? a.k_new[kvh * g.head_dim + d] : 0.0f;
+            v_rows[u] = has ? a.v_new[kvh * g.head_dim + d] : 0.0f;
         }
-        for (int c = tid; c < P; c += THREADS) {
-            const float x = (appends && c < g.head_dim) ? a.k_new[kvh * g.head_dim + c] : 0.0f;
-            pre_raw[rows * PS + c] = x;
-            pre_sq[rows * SQS + c] = sq_of(x);
-            pre_wq[c] = (a.q_norm_w && c < g.head_dim) ? a.q_norm_w[c] : 1.0f;
-            pre_wk[c] = (a.k_norm_w && c < g.head_dim) ? a.k_norm_w[c] : 1.0f;
-            pre_rope[c] = (a.rope && c < a.rope_dims) ? a.rope[c] : 0.0f;
-        }
-        __syncthreads();
+        Pre pre;
+        pre.load(a, kvh, rows, q_stride, tid);
+        // The first K tile on its way meanwhile, V behind the ordered sums: one token through 36 layers of
+        // q32/kv8/hd128 over 5003 rows 526 us, with both tiles asked for here 586, K here and V behind the
+        // last barrier 534, both there 554.
+        const int pg = table_entry<true>(a.table, min(pb, last_page));
+        load_tile(tile_in(pg, k_pool), k_first);
+        pre.stage(pre_lds, a, rows, k_rows, tid);
+        // query slots that the group does not fill
+        for (int idx = tid; idx < NT * 64; idx += THREADS)
+            if ((idx & 15) >= rows) q_lds[idx] = float4_t{0.f, 0.f, 0.f, 0.f};
         const int n_rows = rows + (appends ? 1 : 0);
-        if (tid < n_rows) {
-            const bool is_k = tid == rows;
-            const bool has_norm = is_k ? a.k_norm_w != nullptr : a.q_norm_w != nullptr;
-            pre_inv[tid] = has_norm ? head_inv_rms_sq(pre_sq + tid * SQS, P, g.head_dim, a.eps) : 1.0f;
-        }
         __syncthreads();
-        const float *rope = a.rope ? pre_rope : nullptr;
-        for (int e = tid; e < n_rows * P; e += THREADS) {
-            const int r = e / P, c = e % P;
-            if (c < g.head_dim) {
-                const bool is_k = r == rows;
-                const float *w = is_k ? (a.k_norm_w ? pre_wk : nullptr) : (a.q_norm_w ? pre_wq : nullptr);
-                pre_out[r * PS + c] = norm_rope_elem(pre_raw + r * PS, c, pre_inv[r], w, rope, a.rope_dims, a.rope_style);
+        Pre::scales(pre_lds, a, rows, n_rows, tid);
+        __syncthreads();
+        load_tile(tile_in(pg, v_pool), v_first);
+        Pre::each(pre_lds, a, rows, n_rows, tid, [&](int r, int c4, float4_t v) __attribute__((always_inline)) {
+            if (r < rows) {
+                q_lds[(c4 >> 2) * 64 + (c4 & 3) * 16 + r] = v * a.qscale;
+            } else {
+                // (a unit past head_dim is padding, zero already; one across it stores its zeros again)
+                if (c4 * 4 < g.head_dim)
+                    *reinterpret_cast<float4_t *>(const_cast<float *>(k_pool) + new_tile() + k_index_f32(r_new, c4 * 4)) = v;
+                *reinterpret_cast<float4_t *>(new_k + c4 * 4) = v;
+            }
+        });
+        if (appends) {
+#pragma unroll
+            for (int u = 0; u < Pre::NE; ++u) {
+                const int d = tid + u * THREADS;
+                if (d < g.head_dim) const_cast<float *>(v_pool)[new_tile() + v_index_f32(r_new, d)] = v_rows[u];
+                if (d < P) new_v[d] = v_rows[u];
             }
         }
-        __syncthreads();
     }
-    if (appends) {
-        const long tile_at = ((long)a.new_page * g.page_elems + (long)kvh * g.tile_elems) >> 1;
+    if (!PRE && appends) {
+        const long tile_at = new_tile();
         for (int d = tid; d < P; d += THREADS) {
             float kf = 0.0f, vf = 0.0f;
             if (d < g.head_dim) {
-                kf = PRE ? pre_out[rows * PS + d] : a.k_new[kvh * g.head_dim + d];
+                kf = a.k_new[kvh * g.head_dim + d];
                 vf = a.v_new[kvh * g.head_dim + d];
                 const_cast<float *>(k_pool)[tile_at + k_index_f32(r_new, d)] = kf;
                 const_cast<float *>(v_pool)[tile_at + v_index_f32(r_new, d)] = vf;
@@ -556,7 +567,7 @@ __device__ __forceinline__ void f32_decode_body(const DecodeArgs &a, const int s
     }
 
     // ---- queries of the group to LDS, scaled; dims past head_dim are zero
-    {
+    if constexpr (!PRE) {
         constexpr int QU = (NT * 64 + THREADS - 1) / THREADS;
         float4_t qv[QU];
 #pragma unroll
@@ -564,18 +575,12 @@ __device__ __forceinline__ void f32_decode_body(const DecodeArgs &a, const int s
             const int idx = min(tid + u * THREADS, NT * 64 - 1);
             const int m = idx >> 6, nn = idx & 15, jj = (idx >> 4) & 3;
             const int slot = min(slot0 + nn, n_slots - 1);
-            if constexpr (PRE) {
-                const float *qrow = pre_out + (slot - slot0) * PS;
+            const float *qrow = a.q + (long)(kvh * G + slot) * q_stride;
+            if (a.q_vec) {
+                qv[u] = *reinterpret_cast<const float4_t *>(qrow + min(m * 16 + jj * 4, g.head_dim - 4));
+            } else {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) qv[u][e] = qrow[min(m * 16 + jj * 4 + e, g.head_dim - 1)];
-            } else {
-                const float *qrow = a.q + (long)(kvh * G + slot) * q_stride;
-                if (a.q_vec) {
-                    qv[u] = *reinterpret_cast<const float4_t *>(qrow + min(m * 16 + jj * 4, g.head_dim - 4));
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) qv[u][e] = qrow[min(m * 16 + jj * 4 + e, g.head_dim - 1)];
-                }
             }
         }
 #pragma unroll
@@ -590,22 +595,36 @@ __device__ __forceinline__ void f32_decode_body(const DecodeArgs &a, const int s
             }
         }
     }
-    float4_t kq[NT], vq[NT];
-    auto tile_of = [&](int idx, const float *pool) __attribute__((always_inline)) {
-        const int page = __builtin_amdgcn_readlane(ids, idx);
-        return reinterpret_cast<const float4_t *>(pool + (((long)page * g.page_elems + (long)kvh * g.tile_elems) >> 1)) + lane;
-    };
-    auto load_tile = [&](const float4_t *t, float4_t (&dst)[NT]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int m = 0; m < NT; ++m) dst[m] = __builtin_nontemporal_load(t + m * 64);
-    };
-    // The queries are staged before the first page is asked for: a compute unit accepts
+    // Without the pre-KV step the queries are staged before the first page is asked for: a compute unit accepts
     // requests only as fast as memory answers them, and a barrier behind a page's loads would
     // hold every wavefront until the last one's were accepted. The first page comes without a
     // condition (a wavefront without pages reads a page it ignores).
     __syncthreads();
-    load_tile(tile_of(0, k_pool), kq);
-    load_tile(tile_of(0, v_pool), vq);
+    float4_t kq[NT], vq[NT];
+    if constexpr (PRE) {
+#pragma unroll
+        for (int m = 0; m < NT; ++m) {
+            kq[m] = k_first[m];
+            vq[m] = v_first[m];
+        }
+    } else {
+        // In order: asked for last, the block that the first product needs would hold it up for the whole
+        // tile (a decode step of q24/kv8/hd128, ring of 1024 rows, two sequences, 11.6 -> 11.3 us). With eight
+        // wavefronts, the short contexts' shape, those without a page ask for none.
+        const float4_t *k0 = tile_of(0, k_pool), *v0 = tile_of(0, v_pool);
+        if constexpr (WAVES == 4) {
+#pragma unroll
+            for (int m = 0; m < NT; ++m) {
+                kq[m] = __builtin_nontemporal_load(k0 + m * 64);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            load_tile(v0, vq);
+        } else if (n_it > 0) {
+            load_tile(k0, kq);
+            __builtin_amdgcn_sched_barrier(0);
+            load_tile(v0, vq);
+        }
+    }
 
     float4_t o[NT];
 #pragma unroll

@@ -110,7 +110,8 @@ struct GatherArgs {
     Geom g;
 };
 
-struct DecodeArgs {
+// (aligned: in a batch's array no member straddles the scalar unit's 64-byte lines more than in one)
+struct alignas(64) DecodeArgs {
     const float *q;  // [n_queries][q_heads*head_dim] f32
     float *out;      // [n_queries][q_heads*head_dim] f32
     const uint16_t *k_pool;
@@ -268,20 +269,39 @@ __device__ __forceinline__ float head_inv_rms(const float *row, int head_dim, fl
     const float mean_square = sum / (float)head_dim;
     return 1.0f / sqrtf(mean_square + eps);
 }
-// The same from the squares, already taken (x * x, rounded) and padded with zeros to a
-// multiple of 16 entries at a 16-byte aligned address: the adds stay in index order, the
-// loads come sixteen values at a time.
-__device__ __forceinline__ float head_inv_rms_sq(const float *sq, int padded, int head_dim, float eps) {
+// The same from the squares, already taken (x * x, rounded) and padded with zeros to PADDED entries
+// (32, 64 or a multiple of 128) at a 16-byte aligned address: the adds stay in index order, the
+// 16-byte loads of a round are asked for before the adds of the round before (asked for four at a time and
+// waited for, the LDS's latency was as long again as the adds). The loop stays a loop: unrolled, every
+// load moves to its top and the page registers of the caller spill.
+template <int PADDED>
+__device__ __forceinline__ float head_inv_rms_sq(const float *sq, int head_dim, float eps) {
 #pragma clang fp contract(off)
     typedef __attribute__((ext_vector_type(4))) float f4;
+    constexpr int R = PADDED <= 64 ? PADDED / 8 : PADDED <= 128 ? 8 : 4; // units of a round
+    constexpr int N = PADDED / (8 * R);                                  // pairs of rounds
     const f4 *p = reinterpret_cast<const f4 *>(sq);
     float sum = 0.0f;
-    for (int c = 0; c < padded / 4; c += 4) {
-        const f4 v0 = p[c], v1 = p[c + 1], v2 = p[c + 2], v3 = p[c + 3];
-        sum = sum + v0.x; sum = sum + v0.y; sum = sum + v0.z; sum = sum + v0.w;
-        sum = sum + v1.x; sum = sum + v1.y; sum = sum + v1.z; sum = sum + v1.w;
-        sum = sum + v2.x; sum = sum + v2.y; sum = sum + v2.z; sum = sum + v2.w;
-        sum = sum + v3.x; sum = sum + v3.y; sum = sum + v3.z; sum = sum + v3.w;
+    f4 x[R], y[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) x[i] = p[i];
+#pragma unroll 1
+    for (int k = 0; k < N; ++k) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) y[i] = p[(2 * k + 1) * R + i];
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum = sum + x[i][e];
+        }
+        const f4 *next = p + (k + 1 < N ? 2 * (k + 1) * R : 0); // (the last round reads a unit it ignores)
+#pragma unroll
+        for (int i = 0; i < R; ++i) x[i] = next[i];
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum = sum + y[i][e];
+        }
     }
     const float mean_square = sum / (float)head_dim;
     return 1.0f / sqrtf(mean_square + eps);
@@ -314,6 +334,34 @@ __device__ __forceinline__ float norm_rope_elem(const float *row, int c, float i
     const float first = normed(i0), second = normed(i1);
     const float fc = first * cs, ss = second * sn, fs = first * sn, sc = second * cs;
     return is_first ? fc - ss : fs + sc;
+}
+// Four dims of a head, x, after norm and rotation. Interleaved pairs (style 1): r0 holds the unit's two
+// (cos, sin). Halves: `other` and `ow` are the partner unit and its weights, r0 and r1 the (cos, sin) of the
+// pairs, and the unit lies in the first half or not.
+__device__ __forceinline__ __attribute__((ext_vector_type(4))) float
+norm_rope_unit(__attribute__((ext_vector_type(4))) float x, __attribute__((ext_vector_type(4))) float other,
+               __attribute__((ext_vector_type(4))) float w, __attribute__((ext_vector_type(4))) float ow,
+               __attribute__((ext_vector_type(4))) float r0, __attribute__((ext_vector_type(4))) float r1, float inv,
+               int style, bool is_first) {
+#pragma clang fp contract(off)
+    typedef __attribute__((ext_vector_type(4))) float f4;
+    f4 n = x * inv;
+    n = n * w;
+    if (style == 1) {
+        const float a0 = n[0] * r0[0], b0 = n[1] * r0[1], c0 = n[0] * r0[1], d0 = n[1] * r0[0];
+        const float a1 = n[2] * r0[2], b1 = n[3] * r0[3], c1 = n[2] * r0[3], d1 = n[3] * r0[2];
+        return f4{a0 - b0, c0 + d0, a1 - b1, c1 + d1};
+    }
+    f4 o = other * inv;
+    o = o * ow;
+    const float cs[4] = {r0[0], r0[2], r1[0], r1[2]};
+    const float sn[4] = {r0[1], r0[3], r1[1], r1[3]};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float nc = n[e] * cs[e], os = o[e] * sn[e];
+        n[e] = is_first ? nc - os : os + nc;
+    }
+    return n;
 }
 #endif
 

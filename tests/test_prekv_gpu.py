@@ -177,7 +177,7 @@ CASES = [
 ]
 
 
-def run_prekv(state, dims, window, start, steps, rope_dims, theta, attn_scalar, norms, element="bf16"):
+def run_prekv(state, dims, window, start, steps, rope_dims, theta, attn_scalar, norms, element="bf16", style=0):
     q_heads, kv_heads, head_dim = dims
     kv_dim, q_dim = kv_heads * head_dim, q_heads * head_dim
     eps = 1.0e-6
@@ -194,7 +194,7 @@ def run_prekv(state, dims, window, start, steps, rope_dims, theta, attn_scalar, 
     def cpu_pre(x, heads, w, position):
         if w is None:
             return oracle.apply_rope_heads_at(x, heads, head_dim, rope_dims, theta, position)[0]
-        return oracle.rms_norm_rope_heads_at(x, heads, head_dim, rope_dims, w, eps, theta, position)[0]
+        return oracle.rms_norm_rope_heads_at(x, heads, head_dim, rope_dims, w, eps, theta, position, style=style)[0]
 
     qw, kw = (q_norm if norms[0] else None), (k_norm if norms[1] else None)
     if start:
@@ -203,7 +203,7 @@ def run_prekv(state, dims, window, start, steps, rope_dims, theta, attn_scalar, 
         k0 = np.stack([cpu_pre(k0[r], kv_heads, kw, r) for r in range(start)])
         kv.seed(k0, v0, start)
         cache.append_batch(k0, v0, lay)
-    rope = state.rope_table(cap, rope_dims, theta)
+    rope = state.rope_table(cap, rope_dims, theta, style=style)
     # raw q | k | v of a token sit in one buffer, like the fused QKV projection's output
     # Without norms and with attn_scalar 1 the scores are raw dot products: keep them at a
     # magnitude a model produces (the device splits q into two bf16 terms, 2^-17 relative, so
@@ -245,6 +245,20 @@ def run_prekv(state, dims, window, start, steps, rope_dims, theta, attn_scalar, 
 def test_fused_prekv_steps_match_oracle(state, dims, window, start, steps, rope_dims, theta,
                                         attn_scalar, norms):
     run_prekv(state, dims, window, start, steps, rope_dims, theta, attn_scalar, norms)
+
+
+@pytest.mark.parametrize("element", ["bf16", "f32"])
+@pytest.mark.parametrize("dims,rope_dims,style,start", [
+    ((16, 1, 128), 128, 0, 40),   # sixteen heads a group: every query slot, k row behind them
+    ((16, 1, 256), 64, 1, 2100),  # interleaved pairs in whole units, two units and more per thread
+    ((8, 2, 64), 36, 0, 17),      # halves that are no whole units: element by element
+    ((6, 2, 40), 22, 1, 15),      # interleaved, not in whole units
+    ((4, 2, 18), 8, 0, 3),        # heads of half a unit more than four: no 16-byte loads
+    ((6, 2, 20), 16, 0, 31),      # whole units, no 16-byte loads of q
+    ((3, 1, 12), 12, 1, 0),       # a quarter of the padded head, from an empty cache
+])
+def test_fused_prekv_unit_edges(state, dims, rope_dims, style, start, element):
+    run_prekv(state, dims, 0, start, 6, rope_dims, 1.0e6, None, (True, True), element=element, style=style)
 
 
 @pytest.mark.parametrize("dims,window,start,steps,rope_dims,theta,attn_scalar,norms",
