@@ -208,6 +208,23 @@ def lib():
     return _lib
 
 
+def calls():
+    """The module of csrc/calls.c: the per-token calls without ctypes, on the same library."""
+    lib()
+    try:
+        from . import _calls
+    except ImportError as e:
+        raise DeviceError(f"saragossa_amd/_calls.so cannot be loaded ({e}): build it with `python -c "
+                          "'import __graft_entry__ as g; g.build()'`") from e
+    return _calls
+
+
+def settle(rc: int, fn, *args) -> None:
+    """The end of a call of `calls()` that did not return 0: its status, or the ctypes call it stands for where it
+    did not take the arguments."""
+    check(fn(*args) if rc < 0 else rc)
+
+
 def check(rc: int) -> None:
     if rc != OK:
         msg = lib().skv_last_error().decode("utf-8", "replace")

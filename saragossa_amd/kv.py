@@ -11,7 +11,7 @@ import ctypes as C
 
 import numpy as np
 
-from ._lib import DTYPE_BF16, DTYPE_F32, check, lib
+from ._lib import DTYPE_BF16, DTYPE_F32, calls, check, lib, settle
 
 
 def _f32(a) -> np.ndarray:
@@ -26,15 +26,15 @@ class DecodeResidentState:
     """DecodeResidentState::new (src/decoder/resident/setup.rs:237, 675)."""
 
     def __init__(self, device: int = 0):
-        self._l = lib()
+        self._l, self._c = lib(), calls()
         h = C.c_void_p()
         check(self._l.skv_ctx_create(device, C.byref(h)))
-        self._h = h
+        self._h, self._p = h, h.value  # the handle, for ctypes and for calls()
 
     def close(self) -> None:
         if getattr(self, "_h", None):
             self._l.skv_ctx_destroy(self._h)
-            self._h = None
+            self._h = self._p = None
 
     def __del__(self):
         self.close()
@@ -81,9 +81,11 @@ class DecodeResidentState:
     def encode_rms_norm_rope_rows(self, stream, rope, position_offset, x_ptr, weight_ptr, n_rows, heads,
                                   head_dim, eps, out_ptr) -> None:
         """rms_norm_rope_heads_at for n_rows rows at positions position_offset.. (device in/out)."""
-        check(self._l.skv_rms_norm_rope_rows_device(
-            self._h, stream, None if rope is None else rope._h, position_offset, x_ptr, weight_ptr,
-            n_rows, heads, head_dim, eps, out_ptr))
+        rc = self._c.rms_norm_rope_rows(self._p, stream, None if rope is None else rope._p, position_offset, x_ptr,
+                                        weight_ptr, n_rows, heads, head_dim, eps, out_ptr)
+        if rc:
+            settle(rc, self._l.skv_rms_norm_rope_rows_device, self._h, stream, None if rope is None else rope._h,
+                   position_offset, x_ptr, weight_ptr, n_rows, heads, head_dim, eps, out_ptr)
 
     def encode_attn_gate(self, stream, ctx_ptr, gate_ptr, gate_head_stride, heads, head_dim,
                          out_ptr) -> None:
@@ -139,12 +141,12 @@ class RopeTable:
         h = C.c_void_p()
         check(self._l.skv_rope_create(ctx._h, max_positions, rope_dims, frequency_dim, theta,
                                       position_scale, style, C.byref(h)))
-        self._h = h
+        self._h, self._p = h, h.value
 
     def close(self) -> None:
         if getattr(self, "_h", None):
             self._l.skv_rope_destroy(self._h)
-            self._h = None
+            self._h = self._p = None
 
     def __del__(self):
         self.close()
@@ -155,13 +157,13 @@ class FullAttentionState:
 
     def __init__(self, ctx: DecodeResidentState, handle):
         self._ctx = ctx  # keeps the context alive
-        self._l = ctx._l
-        self._h = handle
+        self._l, self._c = ctx._l, ctx._c
+        self._h, self._p = handle, handle.value
 
     def close(self) -> None:
         if getattr(self, "_h", None):
             self._l.skv_layer_destroy(self._h)
-            self._h = None
+            self._h = self._p = None
 
     def __del__(self):
         self.close()
@@ -188,7 +190,9 @@ class FullAttentionState:
         check(self._l.skv_layer_set_block_table(self._h, _p(t), t.size))
 
     def truncate(self, n: int) -> None:
-        check(self._l.skv_truncate(self._h, n))
+        rc = self._c.truncate_rows(self._p, n)
+        if rc:
+            settle(rc, self._l.skv_truncate, self._h, n)
 
     # ---- host entry points
     def seed(self, keys_rows, values_rows, n_rows: int) -> None:
@@ -225,7 +229,9 @@ class FullAttentionState:
         return out
 
     def encode_prefill_rows(self, stream, q_ptr, k_ptr, v_ptr, n_rows, out_ptr) -> None:
-        check(self._l.skv_prefill_chunk_device(self._h, stream, q_ptr, k_ptr, v_ptr, n_rows, out_ptr))
+        rc = self._c.prefill_chunk(self._p, stream, q_ptr, k_ptr, v_ptr, n_rows, out_ptr)
+        if rc:
+            settle(rc, self._l.skv_prefill_chunk_device, self._h, stream, q_ptr, k_ptr, v_ptr, n_rows, out_ptr)
 
     def read_rows(self, first: int = 0, n: int | None = None):
         """Logical rows as bf16 bit patterns, ([n, kv_dim] uint16, same)."""
@@ -251,13 +257,17 @@ class FullAttentionState:
         check(self._l.skv_append_device(self._h, stream, k_ptr, k_off, v_ptr, v_off))
 
     def encode_append_batch(self, stream, k_ptr, v_ptr, n_rows) -> None:
-        check(self._l.skv_append_batch_device(self._h, stream, k_ptr, v_ptr, n_rows))
+        rc = self._c.append_batch(self._p, stream, k_ptr, v_ptr, n_rows)
+        if rc:
+            settle(rc, self._l.skv_append_batch_device, self._h, stream, k_ptr, v_ptr, n_rows)
 
     def encode_attention_decode(self, stream, q_ptr, out_ptr) -> None:
         self.encode_attention_decode_windowed(stream, q_ptr, out_ptr, 0)
 
     def encode_attention_decode_windowed(self, stream, q_ptr, out_ptr, window_start) -> None:
-        check(self._l.skv_attention_device(self._h, stream, q_ptr, out_ptr, window_start))
+        rc = self._c.attention(self._p, stream, q_ptr, out_ptr, window_start)
+        if rc:
+            settle(rc, self._l.skv_attention_device, self._h, stream, q_ptr, out_ptr, window_start)
 
     def encode_probe_read_pages(self, stream) -> None:
         """Measurement aid: a launch that only fetches the cached K and V pages, with the
@@ -275,8 +285,9 @@ class FullAttentionState:
         check(self._l.skv_probe_merge_device(self._h, stream, out_ptr))
 
     def encode_decode_step(self, stream, k_ptr, k_off, v_ptr, v_off, q_ptr, out_ptr) -> None:
-        check(self._l.skv_decode_step_device(self._h, stream, k_ptr, k_off, v_ptr, v_off, q_ptr,
-                                             out_ptr))
+        rc = self._c.decode_step(self._p, stream, k_ptr, k_off, v_ptr, v_off, q_ptr, out_ptr)
+        if rc:
+            settle(rc, self._l.skv_decode_step_device, self._h, stream, k_ptr, k_off, v_ptr, v_off, q_ptr, out_ptr)
 
     def encode_decode_step_static(self, stream, k_ptr, k_off, v_ptr, v_off, q_ptr, out_ptr) -> None:
         """encode_decode_step for callers that cannot allocate: the split partials live in the
@@ -288,17 +299,21 @@ class FullAttentionState:
                                  v_off, q_norm_ptr, k_norm_ptr, eps, attn_scalar, out_ptr) -> None:
         """The q/k norms, rotation, query scale, append and attention of
         encode_resident_full_layer (src/decode_resident/layers.rs:214-288) in one call."""
-        check(self._l.skv_decode_step_prekv_device(
-            self._h, stream, None if rope is None else rope._h, position, q_ptr, q_off, k_ptr,
-            k_off, v_ptr, v_off, q_norm_ptr, k_norm_ptr, eps, attn_scalar, out_ptr))
+        rc = self._c.decode_step_prekv(self._p, stream, None if rope is None else rope._p, position, q_ptr, q_off,
+                                       k_ptr, k_off, v_ptr, v_off, q_norm_ptr, k_norm_ptr, eps, attn_scalar, out_ptr)
+        if rc:
+            settle(rc, self._l.skv_decode_step_prekv_device, self._h, stream, None if rope is None else rope._h, position,
+                   q_ptr, q_off, k_ptr, k_off, v_ptr, v_off, q_norm_ptr, k_norm_ptr, eps, attn_scalar, out_ptr)
 
     def encode_decode_step_gated(self, stream, rope, position, qg_ptr, qg_off, k_ptr, k_off, v_ptr,
                                  v_off, q_norm_ptr, k_norm_ptr, eps, attn_scalar, out_ptr) -> None:
         """encode_decode_step_prekv for a layer with an output gate: qg is the gated q
         projection (per head: q then gate) and the context comes out times sigmoid(gate)."""
-        check(self._l.skv_decode_step_gated_device(
-            self._h, stream, None if rope is None else rope._h, position, qg_ptr, qg_off, k_ptr,
-            k_off, v_ptr, v_off, q_norm_ptr, k_norm_ptr, eps, attn_scalar, out_ptr))
+        rc = self._c.decode_step_gated(self._p, stream, None if rope is None else rope._p, position, qg_ptr, qg_off,
+                                       k_ptr, k_off, v_ptr, v_off, q_norm_ptr, k_norm_ptr, eps, attn_scalar, out_ptr)
+        if rc:
+            settle(rc, self._l.skv_decode_step_gated_device, self._h, stream, None if rope is None else rope._h, position,
+                   qg_ptr, qg_off, k_ptr, k_off, v_ptr, v_off, q_norm_ptr, k_norm_ptr, eps, attn_scalar, out_ptr)
 
     def encode_gather(self, stream, first, n, k_dst_ptr, v_dst_ptr) -> None:
         check(self._l.skv_gather_device(self._h, stream, first, n, k_dst_ptr, v_dst_ptr))

@@ -7,6 +7,7 @@ import re
 import subprocess
 import sys
 
+import numpy as np
 import pytest
 
 import saragossa_amd as skv
@@ -210,3 +211,22 @@ def test_memory_guard_flags_follow_the_reference():
     d = _flags_in_subprocess({"RETI_MEMORY_CAP_BYTES": "-5", "RETI_SERVE_MEMORY_CAP_BYTES": "68719476736",
                               "RETI_SERVE_MEMORY_HEADROOM_BYTES": " 1073741824"})
     assert (d["mcap"], d["scap"], d["shead"]) == (None, 1 << 36, 1 << 30)
+
+
+@pytest.mark.parametrize("name,symbol", [
+    ("truncate_rows", "skv_truncate"), ("append_batch", "skv_append_batch_device"),
+    ("attention", "skv_attention_device"), ("decode_step", "skv_decode_step_device"),
+    ("decode_step_prekv", "skv_decode_step_prekv_device"), ("decode_step_gated", "skv_decode_step_gated_device"),
+    ("prefill_chunk", "skv_prefill_chunk_device"), ("rms_norm_rope_rows", "skv_rms_norm_rope_rows_device")])
+def test_calls_module_stands_for_ctypes(name, symbol):
+    """The functions of csrc/calls.c take what their ctypes counterparts take, in the same order, and leave
+    arguments of other types to them."""
+    _, kinds = _lib.SIGNATURES[symbol]
+    fast, slow = getattr(_lib.calls(), name), getattr(skv.lib(), symbol)
+    null = [None if k is ctypes.c_void_p else 0.5 if k is ctypes.c_float else 1 for k in kinds]
+    assert fast(*null) == slow(*null) == _lib.ERR_DEVICE      # a null handle, reported by the library
+    assert fast(*null[:-1]) == fast(*null, 1) == -1            # another number of arguments
+    for i, k in enumerate(kinds):
+        odd = [True, "1", 2.0, np.int64(3)] if k is not ctypes.c_float else [1, None, "1"]
+        for x in odd + ([None] if k is ctypes.c_size_t else []):
+            assert fast(*null[:i], x, *null[i + 1:]) == -1, (i, x)
