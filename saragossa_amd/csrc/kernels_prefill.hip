@@ -48,8 +48,8 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // exponential needs no subtraction, and only a score above m + 8 makes the wavefront move the
 // bases and rescale its sums. Probabilities stay below 2^8 and are split relatively, so
 // nothing is lost; partials carry (o, base, l) and any base serves the merge.
-// With HALVES = 2 the wavefronts are two halves that hold the same slots and take the page pairs in
-// turn; the second half's (o, m, l) join the first's through LDS at the end. Otherwise there is
+// With HALVES = 2 (or 4) the wavefronts are two halves (four quarters) that hold the same slots and take
+// the page pairs in turn; the others' (o, m, l) join the first's through LDS at the end. Otherwise there is
 // no merge inside the workgroup; with several splits the partials go to merge_rows_kernel.
 // The copies go straight from memory to LDS. 512 rows as one call (append, attention, merge), in us
 // on one MI355X, against the kernel that ran scores, softmax and accumulation of a pair one after
@@ -477,32 +477,38 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
         if (step + 1 < n_steps) clear_v((step + 1) * SP * GP, kv_lds + ((step + 1) & 1) * BUF_U4 + HALF_U4);
     }
 
-    // ---- the second half's states join the first's through LDS -----------------------------
+    // ---- the other parts' states join the first's through LDS -------------------------------
     if constexpr (HALVES > 1) {
-        static_assert(HALVES == 2 && TW * TILES * (NT + 1) * 64 <= 2 * BUF_U4, "the second half's states fit the page buffers");
+        constexpr int STATES = TW * TILES * (NT + 1) * 64; // of a part
+        static_assert((HALVES - 1) * STATES <= 2 * BUF_U4, "the other parts' states fit the page buffers");
         float4_t *xo = reinterpret_cast<float4_t *>(kv_lds) + (tw * TILES) * (NT + 1) * 64 + lane; // (the loop ends in a barrier)
-        if (half == 1) {
+        if (half > 0) {
 #pragma unroll
             for (int t = 0; t < TILES; ++t) {
+                float4_t *dst = xo + (half - 1) * STATES + t * (NT + 1) * 64;
 #pragma unroll
-                for (int u = 0; u < NT; ++u) xo[(t * (NT + 1) + u) * 64] = o[t][u];
-                xo[(t * (NT + 1) + NT) * 64] = float4_t{thr[t] == -INFINITY ? -INFINITY : m_base[t], l_run[t], 0.f, 0.f};
+                for (int u = 0; u < NT; ++u) dst[u * 64] = o[t][u];
+                dst[NT * 64] = float4_t{thr[t] == -INFINITY ? -INFINITY : m_base[t], l_run[t], 0.f, 0.f};
             }
         }
         __syncthreads();
-        if (half == 1) return;
+        if (half > 0) return;
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
-            const float4_t ml = xo[(t * (NT + 1) + NT) * 64];
-            const float m0 = thr[t] == -INFINITY ? -INFINITY : m_base[t], m1 = ml[0];
-            const float mx = fmaxf(m0, m1);
-            const float m_safe = mx == -INFINITY ? 0.0f : mx;
-            const float w0 = fast_exp2(m0 - m_safe), w1 = fast_exp2(m1 - m_safe);
-            l_run[t] = l_run[t] * w0 + ml[1] * w1;
+#pragma unroll 1
+            for (int h = 0; h < HALVES - 1; ++h) {
+                const float4_t *src = xo + h * STATES + t * (NT + 1) * 64;
+                const float4_t ml = src[NT * 64];
+                const float m0 = thr[t] == -INFINITY ? -INFINITY : m_base[t], m1 = ml[0];
+                const float mx = fmaxf(m0, m1);
+                const float m_safe = mx == -INFINITY ? 0.0f : mx;
+                const float w0 = fast_exp2(m0 - m_safe), w1 = fast_exp2(m1 - m_safe);
+                l_run[t] = l_run[t] * w0 + ml[1] * w1;
 #pragma unroll
-            for (int u = 0; u < NT; ++u) o[t][u] = o[t][u] * w0 + xo[(t * (NT + 1) + u) * 64] * w1;
-            m_base[t] = m_safe;
-            thr[t] = mx == -INFINITY ? -INFINITY : 8.0f;
+                for (int u = 0; u < NT; ++u) o[t][u] = o[t][u] * w0 + src[u * 64] * w1;
+                m_base[t] = m_safe;
+                thr[t] = mx == -INFINITY ? -INFINITY : 8.0f;
+            }
         }
     }
 
@@ -614,7 +620,7 @@ hipError_t launch_merge_rows(const DecodeArgs &a, hipStream_t s) {
 // Query slots one workgroup of the kernel covers for a padded head_dim.
 int prefill_tile_slots(int P, TileShape shape) {
     if (P > 256) return 64; // four wavefronts, one per SIMD (the accumulators and query halves are 256 registers)
-    return shape == TileShape::two_tiles && P <= 128 ? 256 : shape == TileShape::halves ? 64 : 128;
+    return shape == TileShape::two_tiles && P <= 128 ? 256 : shape == TileShape::halves || shape == TileShape::quarters ? 64 : 128;
 }
 
 template <int P, int TILES, int SP, int WAVES, int HALVES, bool RING>
@@ -648,6 +654,7 @@ hipError_t launch_prefill_tiles(const DecodeArgs &a, const ChunkPages &c, TileSh
         if (halves) return launch_tiles<64, 1, 2, 8, 2>(a, c, grid, s);
         return two ? launch_tiles<64, 2, 4>(a, c, grid, s) : launch_tiles<64, 1, 4>(a, c, grid, s);
     case 128:
+        if (shape == TileShape::quarters) return launch_tiles<128, 2, 1, 8, 4>(a, c, grid, s);
         if (halves) return launch_tiles<128, 1, 2, 8, 2>(a, c, grid, s);
         return two ? launch_tiles<128, 2, 2>(a, c, grid, s) : launch_tiles<128, 1, 4>(a, c, grid, s);
     case 256:

@@ -180,21 +180,29 @@ int choose_waves(const skv_layer *L, int n_pages_scan) {
 size_t decode_target_wgs() { return tuning().target_wgs; }
 
 // Shape of the prefill tile kernel's workgroups for a chunk of n_slots query slots per kv head, each
-// walking about n_pages pages. A workgroup of halves covers 64 slots instead of 128, so it fills
-// the device with fewer splits, or with none where 128-slot workgroups need two and a merge; it
-// copies each page for half as many slots. The gain is fixed, the price grows with the pages walked:
-// whole chunks over one tile / two tiles / halves on one MI355X, in us, 512 rows of q32/kv8/hd128
-// over 0, 4096, 8192, 16384 rows: 31.0/39.2/20.2, 83.8/82.7/76.9, 137/131/135, 244/226/249; 256 rows over
-// 4096, 8192, 16384: 51.4/56.0/48.6, 77.6/79.7/76.8, 132/127/135; 512 rows of q16/kv2/hd256 (no two tiles, and halves
-// still need two splits) over 512, 2048, 4096: 41.1/39.1, 58.7/57.6, 81.2/83.2; 1024 rows over 2048, 4096,
-// 8192: 101/92.5, 150/146, 246/251; 1024 rows of hd128, where no shape is split, over 512, 4096, 8192:
-// 53.0/68.8/55.2, 147/151/154, 256/247/268. Two tiles (half the LDS reads per product, half the
-// workgroups) pay from about the same walks on.
+// walking about n_pages pages. Workgroups of halves or quarters cover 64 slots instead of 128, so they fill
+// the device with fewer splits, or with none where 128-slot workgroups need two and a merge; they
+// copy each page for half as many slots. Quarters (head_dim 65 to 128) read LDS half as often per product as
+// halves but walk eight pages at a time and join four states. Two tiles read LDS half as often too, and need
+// the most splits: they pay on long walks. Whole chunks over layers that are not in any cache, one tile / two
+// tiles / halves / quarters, in us on one MI355X: 512 rows of q32/kv8/hd128 over 512, 2048, 4096, 8192 rows
+// 34.7/40.1/25.8/30.3, 54.9/58.2/51.7/51.5, 81.7/82.2/84.5/78.5, 135/129/149/133; 256 rows over 2048, 4096, 16384
+// 36.9/43.9/35.9/39.1, 50.3/55.5/52.1/52.2, 131/127/151/132; 1024 rows over 4096, 8192 145/149/161/157,
+// 252/244/282/266; q12/kv4/hd96, 512 rows over 4096 43.1/49.1/51.7/51.1, 1024 rows over 2048, 4096
+// 56.8/55.2/53.8/55.3, 81.5/72.6/90.5/81.5; q8/kv2/hd64, 256 rows over 4096, 16384 24.9/29.5/21.6/24.9,
+// 37.6/45.0/38.9/38.5, 1024 rows over 4096, 16384 36.3/41.9/37.2/37.4, 85.9/82.7/109/92.6; q16/kv2/hd256 (one tile /
+// halves), 512 rows over 512, 2048, 4096, 8192 38.6/37.5, 57.1/56.7, 82.0/82.4, 131/134, 1024 rows over 2048, 8192
+// 101/91.0, 245/246.
 TileShape prefill_shape(const Geom &g, size_t n_slots, size_t n_pages) {
     if (g.P > 256) return TileShape::one_tile;
     const long knob = tuning().prefill_tiles2_min_pages;
     if (knob >= 0) return g.P <= 128 && (long)n_pages >= knob ? TileShape::two_tiles : TileShape::one_tile;
     const size_t wgs = (n_slots + 63) / 64 * (size_t)g.kv_heads, walk = wgs * n_pages;
+    if (g.P == 128 && wgs <= 256) {
+        if (wgs < 192) return walk < 20000 ? TileShape::halves : walk < 95000 ? TileShape::one_tile : TileShape::two_tiles;
+        if (walk < 41000) return TileShape::halves;
+        return wgs >= 208 && walk < 100000 ? TileShape::quarters : TileShape::two_tiles;
+    }
     if (wgs <= 256 && walk < (wgs >= 192 ? 110000u : 40000u)) return TileShape::halves;
     return g.P <= 128 && walk >= (wgs <= 256 ? 110000u : 250000u) ? TileShape::two_tiles : TileShape::one_tile;
 }

@@ -177,9 +177,10 @@ struct ChunkPages {
 };
 
 // How a workgroup of the prefill tile kernel divides its work among its wavefronts: one 16-slot
-// query tile each; two tiles each (head_dim up to 128); or two halves, each half of the
-// wavefronts holding the same tiles and walking every other page pair.
-enum class TileShape { one_tile, two_tiles, halves };
+// query tile each; two tiles each (head_dim up to 128); two halves, each half of the
+// wavefronts holding the same tiles and walking every other page pair; or four quarters of two
+// wavefronts with two tiles each, walking every fourth pair (head_dim 65 to 128).
+enum class TileShape { one_tile, two_tiles, halves, quarters };
 
 // Standalone per-head RMSNorm + rotation of one row (the same arithmetic as the fused step).
 struct NormRopeArgs {

@@ -113,3 +113,31 @@ def test_f32_chunk_is_no_less_exact_than_f32_sums(state, shape):
 
     want, f32 = attend(torch.float64), attend(torch.float32)
     assert (got.double() - want).norm() <= 1.5 * (f32.double() - want).norm()
+
+
+@pytest.mark.parametrize("head_dim,window,base,rows", [
+    (72, 0, 2661, 509),     # padded head, a page that the cache and the chunk share, slots that do not fill a workgroup
+    (128, 0, 2673, 512),    # the last group of eight pages cut after one
+    (128, 3200, 3507, 500), # a ring: old pages, then pages of the chunk's own rows
+])
+def test_chunks_that_quarters_take(state, head_dim, window, base, rows):
+    """208 workgroups of 64 slots over about 200 pages: four parts of two wavefronts with two tiles each."""
+    import torch
+    heads, n = 26, base + rows
+    gen = torch.Generator().manual_seed(base)
+    k, v = (torch.randn(n, heads * head_dim, generator=gen) for _ in range(2))
+    q = torch.randn(rows, heads * head_dim, generator=gen)
+    kv = state.full_attention_bf16(n, heads, heads, head_dim, window=window)
+    kv.set_block_table(np.random.default_rng(base).permutation(kv.pages()).astype(np.int32))
+    kv.seed(k[:base].numpy(), v[:base].numpy(), base)
+    got = torch.from_numpy(kv.prefill_rows(q.numpy(), k[base:].numpy(), v[base:].numpy()))
+    at, row = torch.arange(n)[None], base + torch.arange(rows)[:, None]
+    hidden = (at > row) | (at <= row - window if window else at < 0)
+    k, v = (x.bfloat16().double() for x in (k, v))
+    want = torch.empty(rows, heads * head_dim, dtype=torch.float64)
+    for h in range(heads):
+        cols = slice(h * head_dim, (h + 1) * head_dim)
+        s = q[:, cols].double() @ k[:, cols].T.contiguous() / head_dim ** 0.5
+        want[:, cols] = torch.softmax(s.masked_fill(hidden, -float("inf")), -1) @ v[:, cols]
+    # queries and probabilities in two 8-bit terms: 2^-16 of scores up to 6, and of the probabilities
+    assert (got.double() - want).abs().max() <= 7 * 2.0 ** -16 * want.abs().max()
