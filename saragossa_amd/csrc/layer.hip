@@ -584,12 +584,8 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
     return SKV_OK;
 }
 
-int32_t encode_append(skv_layer *L, hipStream_t s, const float *k_dev, const float *v_dev,
-                      size_t n_rows) {
-    if (n_rows == 0) return SKV_OK;
-    if (L->len + n_rows > L->capacity)
-        return fail(SKV_ERR_DIMENSION, "append KV résident: capacité " +
-                                           std::to_string(L->capacity) + " atteinte (overflow)");
+// The launch arguments that append n_rows rows at the layer's length.
+AppendArgs append_args(const skv_layer *L, const float *k_dev, const float *v_dev, size_t n_rows) {
     AppendArgs a{};
     a.k_src = k_dev;
     a.v_src = v_dev;
@@ -608,10 +604,22 @@ int32_t encode_append(skv_layer *L, hipStream_t s, const float *k_dev, const flo
         a.first_pos += (long)skip;
         a.n_rows = L->g.ring_rows;
     }
-    SKV_HIP(launch_append(a, s));
+    return a;
+}
+void appended(skv_layer *L, size_t n_rows) {
     L->len += n_rows;
     if (L->g.ring_rows > 0 && L->len > (size_t)L->g.ring_rows)
         L->floor_pos = std::max(L->floor_pos, L->len - (size_t)L->g.ring_rows);
+}
+
+int32_t encode_append(skv_layer *L, hipStream_t s, const float *k_dev, const float *v_dev,
+                      size_t n_rows) {
+    if (n_rows == 0) return SKV_OK;
+    if (L->len + n_rows > L->capacity)
+        return fail(SKV_ERR_DIMENSION, "append KV résident: capacité " +
+                                           std::to_string(L->capacity) + " atteinte (overflow)");
+    SKV_HIP(launch_append(append_args(L, k_dev, v_dev, n_rows), s));
+    appended(L, n_rows);
     return SKV_OK;
 }
 
@@ -1157,8 +1165,10 @@ static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const flo
     pages.k_new = w.k_pool;
     pages.v_new = w.v_pool;
     SKV_HIP(g.f32 ? launch_f32_prefill(a, pages, halves, s) : launch_prefill_tiles(a, pages, shape, s));
-    if (a.splits > 1) SKV_HIP(launch_merge_rows(a, s));
-    return encode_append(L, s, k, v, c);
+    if (a.splits == 1) return encode_append(L, s, k, v, c);
+    SKV_HIP(launch_merge_append(a, append_args(L, k, v, c), s)); // (the caller has checked the capacity)
+    appended(L, c);
+    return SKV_OK;
 }
 
 // The same on an f32 ring layer of wider heads, c <= ring_rows, attended in two phases around the append: first every query over the rows

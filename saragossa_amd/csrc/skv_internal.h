@@ -403,6 +403,7 @@ int prefill_tile_slots(int P, TileShape shape);
 hipError_t launch_f32_prefill(const DecodeArgs &a, const ChunkPages &c, bool halves, hipStream_t s); // the same on f32 pages
 int f32_prefill_slots(int P, bool halves); // query slots of a workgroup, 0 = head_dim not served
 hipError_t launch_merge_rows(const DecodeArgs &a, hipStream_t s);    // the same merge for many query slots
+hipError_t launch_merge_append(const DecodeArgs &a, const AppendArgs &w, hipStream_t s); // that and an append nobody waits for in it
 hipError_t launch_naive(const NaiveArgs &a, hipStream_t s);
 int decode_max_splits();
 
