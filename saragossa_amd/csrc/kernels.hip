@@ -385,8 +385,12 @@ __global__ __launch_bounds__(256) void norm_rope_rows_kernel(NormRopeArgs a) {
 // 512 rows of 32 x 128 11.6 -> 6.4, of 8 x 128 8.3 -> 4.6, of 16 x 256 12.3 -> 7.0, of 2 x 256
 // 9.4 -> 4.8; 6 rows of 16 x 256 8.7 -> 4.2; 2048 rows of 32 x 128 28.4 -> 18.0; 1 row of 32 x 128
 // (one workgroup per pair) 4.2 -> 3.8.
+// ONE_ROW: the wavefront's pairs are heads of one row, so that a lane's units share their dims'
+// weights and rotations: one load of each instead of U, the loads through the cache having been as many as
+// five for every one of a row. Input rows not in a cache: 512 rows of 32 x 128 7.2 -> 6.4, of 8 x 128
+// 4.3 -> 3.9, of 16 x 256 8.3 -> 6.9, 2048 rows of 32 x 128 21.7 -> 15.6, 4096 rows of 16 x 256 41.7 -> 28.4.
 // U: 16-byte units a lane holds. HD4: units of the widest head served; EXACT: head_dim is it.
-template <int HD4, int U, bool EXACT>
+template <int HD4, int U, bool EXACT, bool ONE_ROW>
 __global__ __launch_bounds__(64) void norm_rope_wave_kernel(NormRopeArgs a) {
 #pragma clang fp contract(off)
     typedef __attribute__((ext_vector_type(4))) float f4;
@@ -418,9 +422,13 @@ __global__ __launch_bounds__(64) void norm_rope_wave_kernel(NormRopeArgs a) {
         mine[u] = pr[u] < here;
         pr[u] = min(pr[u], here - 1);
         const int at = head0 + pr[u];
-        const int r = a.heads > 1 ? (int)__umulhi((unsigned)at, a.heads_magic) : at;
+        const int r = ONE_ROW ? 0 : a.heads > 1 ? (int)__umulhi((unsigned)at, a.heads_magic) : at;
         const int row = row0 + r, h = at - r * a.heads;
         x[u] = *reinterpret_cast<const f4 *>(a.x + row * row_elems + (long)h * hstride + c4[u] * 4);
+        if (ONE_ROW && u > 0) { // the same dims of another head
+            w[u] = w[0], ow[u] = ow[0], r0[u] = r0[0], r1[u] = r1[0];
+            continue;
+        }
         const bool rotated = a.rope && c4[u] < rope4;
         // the rotation's partner unit (halves) and the first of the unit's pairs
         const int oc4 = c4[u] < half4 ? c4[u] + half4 : c4[u] - half4;
@@ -509,18 +517,25 @@ static void launch_norm_rope_wave_u(const NormRopeArgs &a, hipStream_t s) {
     constexpr int PAIRS = U * 64 / HD4;
     const long n_pairs = (long)a.n_rows * a.heads;
     const dim3 grid((unsigned)((n_pairs + PAIRS - 1) / PAIRS));
-    if (a.head_dim == HD4 * 4) hipLaunchKernelGGL((norm_rope_wave_kernel<HD4, U, true>), grid, dim3(64), 0, s, a);
-    else hipLaunchKernelGGL((norm_rope_wave_kernel<HD4, U, false>), grid, dim3(64), 0, s, a);
+    if constexpr (HD4 <= 64)
+        if (a.head_dim == HD4 * 4 && a.heads % PAIRS == 0) {
+            hipLaunchKernelGGL((norm_rope_wave_kernel<HD4, U, true, true>), grid, dim3(64), 0, s, a);
+            return;
+        }
+    if (a.head_dim == HD4 * 4) hipLaunchKernelGGL((norm_rope_wave_kernel<HD4, U, true, false>), grid, dim3(64), 0, s, a);
+    else hipLaunchKernelGGL((norm_rope_wave_kernel<HD4, U, false, false>), grid, dim3(64), 0, s, a);
 }
 
 // Two units a lane: short chains of loads and stores, and more wavefronts to overlap them. Four on
 // heads above 128 once two would make 4096 wavefronts and more, whose ordered sums then use one or
-// two lanes each (512 rows of 8 x 512 9.2 -> 7.9 us, 4096 rows of 16 x 256 33.8 -> 31.1; 32 x 128 is better
-// with two at any number of rows: 18.0 against 18.9 for 2048). Eight: 22.2 for those 2048 rows.
+// two lanes each, and on heads of 65 to 128 once they would make 8192 and all four units are of one row
+// (two / four / eight units, input rows not in a cache: 512 rows of 16 x 256 7.2/6.9/7.9 us, 4096 rows 35.3/28.4/29.8;
+// 512 rows of 32 x 128 6.3/6.5/7.4, 1024 rows 10.6/9.1/9.7, 2048 rows 18.2/15.6/16.7).
 template <int HD4> // widest head_dim / 4 served
 static hipError_t launch_norm_rope_wave(const NormRopeArgs &a, hipStream_t s) {
     constexpr int PAIRS2 = 2 * 64 / HD4;
-    if (HD4 >= 64 && (long)a.n_rows * a.heads >= 4096l * PAIRS2) launch_norm_rope_wave_u<HD4, 4>(a, s);
+    const long waves = (long)a.n_rows * a.heads / PAIRS2;
+    if (HD4 >= 64 ? waves >= 4096 : HD4 == 32 && waves >= 8192 && a.heads % 8 == 0) launch_norm_rope_wave_u<HD4, 4>(a, s);
     else launch_norm_rope_wave_u<HD4, 2>(a, s);
     return hipGetLastError();
 }

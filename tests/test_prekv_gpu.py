@@ -101,6 +101,10 @@ def test_rms_norm_rope_rows_is_bit_exact(state, heads, head_dim, rope_dims, thet
     (8, 512, 512, 513, 0, True, 0),   # four units a lane, an odd row at the end
     (16, 256, 64, 515, 0, False, 0),  # four units a lane, rotation only
     (7, 128, 0, 11, 0, True, 0),      # norm only
+    (4, 128, 128, 5, 1, True, 0),     # a wavefront's heads of one row, interleaved
+    (6, 256, 64, 3, 0, True, 0),      # the same, two heads, partial rotation
+    (32, 128, 64, 1027, 0, True, 0),  # the same, four units a lane
+    (12, 128, 128, 2731, 0, True, 0), # as many wavefronts, but eight heads would be of two rows
     (4, 64, 12, 6, 1, True, 0),       # interleaved, rotated dims of three units
     (4, 64, 12, 6, 0, True, 0),       # halves of one and a half units: the general kernel
     (8, 128, 128, 6, 0, True, 1),     # rows at an odd address: the general kernel
