@@ -1,7 +1,7 @@
 """MI355X-native KV-cache hot path of saragossa: thin Python host mirror over the C ABI.
 
 The product is ``libsaragossa_kv.so`` (hand-written gfx950 kernels behind
-``include/saragossa_kv.h``). This package only binds it with ctypes and mirrors
+``include/saragossa_kv.h``). This package only binds it (ctypes, and a small extension module for the per-token calls) and mirrors
 the reference's Rust method names so the parity tests read like the reference's
 own tests. There is no CPU fallback: without the library, or without a GPU,
 every compute call raises.
