@@ -74,7 +74,9 @@ __device__ __forceinline__ void load_v(uint4 (&v)[KK], const DecodeArgs &a, int 
 // PRE = true fuses the step before the cache (decode only): q and the appended k row arrive
 // raw, and every workgroup applies the per-head RMSNorm and the rotation of the position to
 // the rows it uses, in LDS, while its first page is in flight.
-template <int P, int WAVES, bool MQ, bool PRE>
+// ROWS: a chunk's few rows, which the launch appends (compiled apart: the larger chunks of the multi-query mode,
+// 512 rows of q32/kv8/hd128 over none, lose 2 us of 18 with it).
+template <int P, int WAVES, bool MQ, bool PRE, bool ROWS = false>
 __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int split, const int kvh,
                                                   const int tile_z) {
     constexpr int THREADS = WAVES * 64;
@@ -110,8 +112,8 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
     extern __shared__ __attribute__((aligned(16))) uint4 smem[];
     uint4 *q_hi = smem;
     uint4 *q_lo = smem + KK * 64;
-    uint16_t *new_k = reinterpret_cast<uint16_t *>(smem + 2 * KK * 64); // [P] appended row
-    uint16_t *new_v = new_k + P;
+    uint16_t *new_k = reinterpret_cast<uint16_t *>(smem + 2 * KK * 64); // [appended rows][P]
+    uint16_t *new_v = new_k + (ROWS ? C * P : P);
     using Pre = PreKvStage<P, THREADS>;
     float *pre_lds = reinterpret_cast<float *>(new_v + P); // PRE: the pre-KV step's staging area
 
@@ -146,20 +148,45 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
     // row to bf16, stores it into the pools for later steps and keeps it in LDS; the
     // wavefront that walks the page patches its registers from there, so nothing is read
     // back from memory in this launch. The row is fetched here, ahead of the pages.
-    const int pb_new = a.new_slot >> 4;
-    const int r_new = a.new_slot & 15;
-    const bool appends = a.k_new != nullptr && C == 1 && pb_new >= pb0 && pb_new < pb1;
+    // A chunk of C > 1 rows (at most MQ_APPEND_ROWS, full layers only): the same for the pages of its rows,
+    // one or two. Every workgroup whose range holds one of them keeps the rows in LDS for its wavefronts; the
+    // last tile of query slots, which sees all of them, stores them into the pools.
+    const int s_new = ROWS ? a.new_slot - (C - 1) : a.new_slot; // slot of the first appended row
+    const int pb_new = s_new >> 4, pb_last = ROWS ? a.new_slot >> 4 : pb_new;
+    const int r_new = s_new & 15;
+    const bool appends = a.k_new != nullptr && (ROWS || C == 1) && pb_last >= pb0 && pb_new < pb1;
+    const bool stores = tile == (n_slots - 1) / 16;
     // elements tid (and tid + THREADS where the head is wider than the workgroup) of the new
-    // row of this kv head
+    // row of this kv head; of a chunk, four dims at a time, row after row
     constexpr int NE = (P + THREADS - 1) / THREADS;
+    constexpr int MU = ROWS ? (MQ_APPEND_ROWS * P / 4 + THREADS - 1) / THREADS : 1;
     float k_rows[NE], v_rows[NE];
+    float4_t k_unit[MU], v_unit[MU];
+    if constexpr (ROWS) {
 #pragma unroll
-    for (int u = 0; u < NE; ++u) {
-        k_rows[u] = 0.0f;
-        v_rows[u] = 0.0f;
-        if (appends && tid + u * THREADS < g.head_dim) {
-            k_rows[u] = a.k_new[kvh * g.head_dim + tid + u * THREADS];
-            v_rows[u] = a.v_new[kvh * g.head_dim + tid + u * THREADS];
+        for (int u = 0; u < MU; ++u) {
+            const int e = tid + u * THREADS, r = e / (P / 4), d = e % (P / 4) * 4;
+            k_unit[u] = v_unit[u] = float4_t{0.f, 0.f, 0.f, 0.f};
+            if (appends && r < C) {
+                const long at = ((long)r * g.kv_heads + kvh) * g.head_dim;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (d + i < g.head_dim) {
+                        k_unit[u][i] = a.k_new[at + d + i];
+                        v_unit[u][i] = a.v_new[at + d + i];
+                    }
+                }
+            }
+        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < NE; ++u) {
+            k_rows[u] = 0.0f;
+            v_rows[u] = 0.0f;
+            if (appends && tid + u * THREADS < g.head_dim) {
+                k_rows[u] = a.k_new[kvh * g.head_dim + tid + u * THREADS];
+                v_rows[u] = a.v_new[kvh * g.head_dim + tid + u * THREADS];
+            }
         }
     }
     Pre pre; // PRE: the raw query rows of the group (the raw k row is in k_rows), weights, rotation
@@ -215,6 +242,9 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
     // 365 us; with K 380; behind the last barrier 376). A chunk's few rows have V with K (six rows over
     // 8192 of q16/kv2/hd256, whole pass over 10 layers 258/262).
     uint4 kr[KK], vr[KK];
+    // (a chunk's rows: the physical pages of the first and the last)
+    const int page_a = ROWS ? table_entry<false>(a.table, min(pb_new, max(page_hi - 1, 0))) : 0;
+    const int page_b = ROWS ? table_entry<false>(a.table, min(pb_last, max(page_hi - 1, 0))) : 0;
     const int pg = table_entry<PRE>(a.table, min(pb0 + wave + rot * WAVES, max(page_hi - 1, 0)));
     load_k<KK>(kr, a, pg, kvh, lane);
     if constexpr (MQ) load_v<KK>(vr, a, pg, kvh, lane);
@@ -258,7 +288,33 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
             }
         });
     }
-    if (appends) {
+    if constexpr (ROWS) {
+        if (appends) {
+#pragma unroll
+            for (int u = 0; u < MU; ++u) {
+                const int e = tid + u * THREADS, r = e / (P / 4), d = e % (P / 4) * 4;
+                if (r < C) {
+                    uint2 kb, vb;
+                    kb.x = bf16_bits(k_unit[u][0]) | (uint32_t)bf16_bits(k_unit[u][1]) << 16;
+                    kb.y = bf16_bits(k_unit[u][2]) | (uint32_t)bf16_bits(k_unit[u][3]) << 16;
+                    vb.x = bf16_bits(v_unit[u][0]) | (uint32_t)bf16_bits(v_unit[u][1]) << 16;
+                    vb.y = bf16_bits(v_unit[u][2]) | (uint32_t)bf16_bits(v_unit[u][3]) << 16;
+                    *reinterpret_cast<uint2 *>(new_k + r * P + d) = kb;
+                    *reinterpret_cast<uint2 *>(new_v + r * P + d) = vb;
+                    const int pb = (s_new + r) >> 4, row = (s_new + r) & 15;
+                    if (stores && pb >= pb0 && pb < pb1 && d < g.head_dim) {
+                        const long tile_at = (long)(pb == pb_new ? page_a : page_b) * g.page_elems + (long)kvh * g.tile_elems;
+                        // (a unit across head_dim stores the padding's zeros again)
+                        *reinterpret_cast<uint2 *>(const_cast<uint16_t *>(a.k_pool) + tile_at + k_index(P, row, d)) = kb;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            if (d + i < g.head_dim)
+                                const_cast<uint16_t *>(a.v_pool)[tile_at + v_index(P, row, d + i)] = (uint16_t)((i < 2 ? vb.x : vb.y) >> (16 * (i & 1)));
+                    }
+                }
+            }
+        }
+    } else if (appends) {
         const long tile_at = new_tile();
 #pragma unroll
         for (int u = 0; u < NE; ++u) {
@@ -388,14 +444,43 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
 
     // the page that receives the appended row takes it from LDS instead of memory
     auto patch_k = [&](int pb) __attribute__((always_inline)) {
-        if (appends && pb == pb_new && n == r_new) {
+        if constexpr (ROWS) {
+            if (!appends || pb < pb_new || pb > pb_last) return; // uniform
+            const int r = pb * 16 + n - s_new;
+            if (r >= 0 && r < C) {
+#pragma unroll
+                for (int kk = 0; kk < KK; ++kk)
+                    kr[kk] = *reinterpret_cast<const uint4 *>(new_k + r * P + kk * 32 + j * 8);
+            }
+        } else if (appends && pb == pb_new && n == r_new) {
 #pragma unroll
             for (int kk = 0; kk < KK; ++kk)
                 kr[kk] = *reinterpret_cast<const uint4 *>(new_k + kk * 32 + j * 8);
         }
     };
     auto patch_v = [&](int pb) __attribute__((always_inline)) {
-        if (appends && pb == pb_new && j == (r_new >> 2)) {
+        if constexpr (ROWS) {
+            if (!appends || pb < pb_new || pb > pb_last) return; // uniform
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int r = pb * 16 + j * 4 + i - s_new;
+                if (r < 0 || r >= C) continue;
+                const uint32_t keep = (i & 1) ? 0x0000ffffu : 0xffff0000u;
+                const int sh = (i & 1) * 16;
+#pragma unroll
+                for (int kk = 0; kk < KK; ++kk) {
+                    const uint32_t b0 = (uint32_t)new_v[r * P + kk * 32 + n] << sh;
+                    const uint32_t b1 = (uint32_t)new_v[r * P + kk * 32 + 16 + n] << sh;
+                    if (i < 2) {
+                        vr[kk].x = (vr[kk].x & keep) | b0;
+                        vr[kk].z = (vr[kk].z & keep) | b1;
+                    } else {
+                        vr[kk].y = (vr[kk].y & keep) | b0;
+                        vr[kk].w = (vr[kk].w & keep) | b1;
+                    }
+                }
+            }
+        } else if (appends && pb == pb_new && j == (r_new >> 2)) {
             const int i = r_new & 3;
             const uint32_t keep = (i & 1) ? 0x0000ffffu : 0xffff0000u;
             const int sh = (i & 1) * 16;
@@ -544,9 +629,9 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
     }
 }
 
-template <int P, int WAVES, bool MQ, bool PRE>
+template <int P, int WAVES, bool MQ, bool PRE, bool ROWS>
 __global__ __launch_bounds__(WAVES * 64) void decode_split_kernel(DecodeArgs a) {
-    decode_split_body<P, WAVES, MQ, PRE>(a, blockIdx.x, blockIdx.y, blockIdx.z);
+    decode_split_body<P, WAVES, MQ, PRE, ROWS>(a, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // Several independent sequences of the same model layer in one launch: grid z is the
@@ -801,10 +886,11 @@ __global__ __launch_bounds__(128) void decode_merge_wave_batch_kernel(DecodeBatc
     merge_wave_body<PER>(a, kvh, (int)blockIdx.y - kvh * d.g.gqa, cg);
 }
 
-template <int P, int WAVES, bool MQ, bool PRE>
+template <int P, int WAVES, bool MQ, bool PRE, bool ROWS = false>
 static hipError_t launch_split_mq(const DecodeArgs &a, hipStream_t s) {
     constexpr int KK = P / 32;
-    size_t stage = (size_t)2 * KK * 64 * sizeof(uint4) + 2 * P * sizeof(uint16_t);
+    if (a.k_new && a.n_queries > (ROWS ? MQ_APPEND_ROWS : 1)) return hipErrorInvalidValue;
+    size_t stage = (size_t)2 * KK * 64 * sizeof(uint4) + 2 * P * sizeof(uint16_t) * (ROWS ? a.n_queries : 1);
     if (PRE) stage += PreKvStage<P, WAVES * 64>::LDS_FLOATS * sizeof(float);
     const int n_slots = a.n_queries * a.g.gqa;
     const int rows = n_slots < 16 ? n_slots : 16;
@@ -814,13 +900,13 @@ static hipError_t launch_split_mq(const DecodeArgs &a, hipStream_t s) {
     const size_t lds = apart ? stage16 + xchg : (stage > xchg ? stage : xchg);
     static std::atomic<uint64_t> lds_ok{0}; // per instantiation
     {
-        hipError_t e = allow_full_lds(reinterpret_cast<const void *>(&decode_split_kernel<P, WAVES, MQ, PRE>), lds_ok);
+        hipError_t e = allow_full_lds(reinterpret_cast<const void *>(&decode_split_kernel<P, WAVES, MQ, PRE, ROWS>), lds_ok);
         if (e != hipSuccess) return e;
     }
     DecodeArgs b = a;
     b.xchg_off = apart ? (int)stage16 : 0;
     dim3 grid((unsigned)a.splits, (unsigned)a.g.kv_heads, (unsigned)((n_slots + 15) / 16));
-    hipLaunchKernelGGL((decode_split_kernel<P, WAVES, MQ, PRE>), grid, dim3(WAVES * 64), lds, s, b);
+    hipLaunchKernelGGL((decode_split_kernel<P, WAVES, MQ, PRE, ROWS>), grid, dim3(WAVES * 64), lds, s, b);
     return hipGetLastError();
 }
 
@@ -829,7 +915,8 @@ static hipError_t launch_split(const DecodeArgs &a, hipStream_t s) {
     // the decode specialisation assumes a single tile of query slots
     if (a.n_queries > 1 || a.g.gqa > 16) {
         if (a.pre) return hipErrorInvalidValue; // the caller keeps the fused step to single-tile decode
-        return launch_split_mq<P, WAVES, true, false>(a, s);
+        return a.k_new && a.n_queries > 1 ? launch_split_mq<P, WAVES, true, false, true>(a, s)
+                                          : launch_split_mq<P, WAVES, true, false>(a, s);
     }
     return a.pre ? launch_split_mq<P, WAVES, false, true>(a, s) : launch_split_mq<P, WAVES, false, false>(a, s);
 }
@@ -841,7 +928,8 @@ static hipError_t launch_split(const DecodeArgs &a, hipStream_t s) {
 static hipError_t launch_split_wide(const DecodeArgs &a, hipStream_t s) {
     if (a.n_queries > 1 || a.g.gqa > 16) {
         if (a.pre) return hipErrorInvalidValue;
-        return launch_split_mq<512, 4, true, false>(a, s);
+        return a.k_new && a.n_queries > 1 ? launch_split_mq<512, 4, true, false, true>(a, s)
+                                          : launch_split_mq<512, 4, true, false>(a, s);
     }
     return a.pre ? launch_split_mq<512, 4, false, true>(a, s) : launch_split_mq<512, 4, false, false>(a, s);
 }

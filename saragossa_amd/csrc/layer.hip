@@ -1252,6 +1252,23 @@ int32_t skv_prefill_chunk_device(skv_layer *L, skv_stream stream, const float *q
             out += c * q_dim;
             continue;
         }
+        // a few rows over a full bf16 layer (a speculative verify, the rest of a prompt): the multi-query launch
+        // appends them itself, as a decode step's does (its last query tile stores them: all of them have to
+        // lie in that tile's window)
+        if (c > 1 && c <= (size_t)MQ_APPEND_ROWS && ring == 0 && (L->window == 0 || L->window >= c) && !L->g.f32 && tuning().fused_append &&
+            !takes_tile_kernel(L->g, c * (size_t)L->g.gqa, (L->len + c + 15) / 16)) {
+            L->len += c;
+            rc = encode_attention(L, as_stream(stream), q, out, 0, k, v, c);
+            if (rc) {
+                L->len -= c;
+                return rc;
+            }
+            q += c * q_dim;
+            k += c * kv_dim;
+            v += c * kv_dim;
+            out += c * q_dim;
+            continue;
+        }
         rc = encode_append(L, as_stream(stream), k, v, c);
         if (rc) return rc;
         const size_t ws_base = L->g.ring_rows > 0 ? L->floor_pos : 0;

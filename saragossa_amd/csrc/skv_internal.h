@@ -366,6 +366,9 @@ norm_rope_unit(__attribute__((ext_vector_type(4))) float x, __attribute__((ext_v
 }
 #endif
 
+// Rows of a chunk that the decode kernel's multi-query mode can append itself.
+constexpr int MQ_APPEND_ROWS = 16;
+
 // One decode step of the same model layer for several independent sequences.
 constexpr int SKV_MAX_BATCH = 16;
 struct DecodeBatchArgs {

@@ -141,3 +141,35 @@ def test_chunks_that_quarters_take(state, head_dim, window, base, rows):
         want[:, cols] = torch.softmax(s.masked_fill(hidden, -float("inf")), -1) @ v[:, cols]
     # queries and probabilities in two 8-bit terms: 2^-16 of scores up to 6, and of the probabilities
     assert (got.double() - want).abs().max() <= 7 * 2.0 ** -16 * want.abs().max()
+
+
+@pytest.mark.parametrize("dims,window,start,counts", [
+    ((8, 2, 64), 0, 0, (2, 16, 15, 7, 16)),     # from an empty cache, across and up to page edges
+    ((16, 2, 256), 0, 1021, (6, 16, 3, 16)),    # several query tiles, whose last one stores; rows in two splits' pages
+    ((32, 8, 128), 0, 2300, (12, 2, 16)),
+    ((20, 1, 128), 0, 40, (5, 1, 16)),          # more heads a group than a tile has slots
+    ((3, 1, 18), 0, 30, (4, 16)),               # no 16-byte loads, padded head
+    ((4, 2, 320), 0, 333, (16, 5)),             # several units a thread
+    ((8, 2, 64), 10, 20, (9, 12)),              # a window shorter than the chunk (appended by a launch of its own)
+])
+def test_few_rows_are_appended_by_the_attention_launch(state, dims, window, start, counts):
+    q_heads, kv_heads, head_dim = dims
+    rng = np.random.default_rng(start + head_dim)
+    kv = state.full_attention_bf16(start + sum(counts), q_heads, kv_heads, head_dim, window=window)
+    kv.set_block_table(rng.permutation(kv.pages()).astype(np.int32))
+    lay = oracle.layout(q_heads, kv_heads, head_dim, sliding_window=window)
+    cache = oracle.LayerKvCache("bf16r")
+    kv_dim = kv_heads * head_dim
+    if start:
+        k, v = (rng.standard_normal((start, kv_dim), dtype=np.float32) for _ in range(2))
+        kv.seed(k, v, start)
+        cache.append_batch(k, v, lay)
+    for c in counts:
+        q = rng.standard_normal((c, q_heads * head_dim), dtype=np.float32)
+        k, v = (rng.standard_normal((c, kv_dim), dtype=np.float32) for _ in range(2))
+        got = kv.prefill_rows(q, k, v)
+        want = oracle.cached_attention_prefill_rows(q, k, v, cache, lay)
+        assert np.abs(got - want).max() <= 1e-4, c
+    first = max(0, kv.len() - window) if window else 0
+    gk, gv = kv.read_rows_f32(first, kv.len() - first)
+    assert np.array_equal(gk, cache.keys()[first:]) and np.array_equal(gv, cache.values()[first:])
