@@ -3,6 +3,7 @@
 #include <type_traits>
 
 #include "chunk_pages.h"
+#include "f32_terms.h"
 
 namespace skv {
 
@@ -13,35 +14,8 @@ typedef __attribute__((ext_vector_type(4))) unsigned int u4;
 namespace {
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-// upper halves of two words, the first in the low half
-__device__ __forceinline__ uint32_t upper_halves(uint32_t x, uint32_t y) { return __builtin_amdgcn_perm(y, x, 0x07060302u); }
-__device__ __forceinline__ uint32_t bf16_pair(float x, float y) {
-    typedef __attribute__((ext_vector_type(2))) float f2;
-    typedef __attribute__((ext_vector_type(2))) __bf16 b2;
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{x, y}, b2));
-}
-// Two f32 values as three bf16 terms each, x = t0 + t1 + t2 exactly (24 bits in 8 + 8 + 8): the upper
-// half cut off (so that the largest finite values do not round to infinity), the remainder rounded
-// to nearest (so that what the products below leave out has no sign of its own), the rest. A
-// term can be inexact only where it is below the smallest bf16, 2^-133.
-__device__ __forceinline__ void three_terms(float x, float y, uint32_t &t0, uint32_t &t1, uint32_t &t2) {
-    const uint32_t xb = __float_as_uint(x), yb = __float_as_uint(y);
-    t0 = upper_halves(xb, yb);
-    const float x1 = x - __uint_as_float(xb & 0xffff0000u), y1 = y - __uint_as_float(yb & 0xffff0000u);
-    t1 = bf16_pair(x1, y1);
-    t2 = upper_halves(__float_as_uint(x1 - __uint_as_float(t1 << 16)), __float_as_uint(y1 - __uint_as_float(t1 & 0xffff0000u)));
-}
-
-// The products of two factors of three terms that are kept, (left term, right term); the even ones
-// go to one accumulator, the odd ones to another. The three left out are below 2^-24 of it, less than the rounding of
-// one f32 product, and of either sign.
-struct TermPair {
-    int l, r;
-};
 // steps of `n` done before beat b, spread over the beats [from, to)
 __host__ __device__ constexpr int done_before(int b, int n, int from, int to) { return b <= from ? 0 : b >= to ? n : (b - from) * n / (to - from); }
-
-constexpr TermPair TERMS[6] = {{0, 0}, {0, 1}, {1, 0}, {1, 1}, {2, 0}, {0, 2}};
 
 } // namespace
 
@@ -51,8 +25,8 @@ constexpr TermPair TERMS[6] = {{0, 0}, {0, 1}, {1, 0}, {1, 1}, {2, 0}, {0, 2}};
 // pair's accumulation). Six bf16 products of three-term factors replace one f32 product: the f32
 // instruction does 4 keys' or dims' worth in the cycles in which the bf16 one does 64, so six
 // are 2.6 times as fast (157 TFLOP/s against 2.5 PFLOP/s / 6), and no less exact: the factors are
-// split without a rounding, what is left out is below 2^-24 of a product, and sums are in f32
-// in both.
+// split without a rounding, what is left out is at most 2^-24 of a product (f32_terms.h), and sums are
+// in f32 in both.
 //
 // Pages come through registers, where all threads split each value once for the whole
 // workgroup, and go to LDS as three planes of bf16 operands. K and V have one buffer each: V of a

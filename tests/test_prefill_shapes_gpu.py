@@ -173,3 +173,38 @@ def test_few_rows_are_appended_by_the_attention_launch(state, dims, window, star
     first = max(0, kv.len() - window) if window else 0
     gk, gv = kv.read_rows_f32(first, kv.len() - first)
     assert np.array_equal(gk, cache.keys()[first:]) and np.array_equal(gv, cache.values()[first:])
+
+
+def test_f32_scores_of_one_product_each(state, shape):
+    """Factors just below a bf16 value or one, one product a score, scores of a thousand: no further off
+    than the kernel of f32 products (a margin of 1.5 for the order of the sums). With the terms cut off instead of
+    rounded, what the products leave out is largest for these, and several times the rounding of f32 ones."""
+    q_heads, kv_heads, head_dim, base, n = 2, 1, 32, 500, 64
+    rng = np.random.default_rng(8)
+    k = np.zeros((base + n, head_dim), np.float32)
+    k[:, 3] = 16 * (1.5 - np.where(rng.random(base + n) < 0.5, 0, rng.integers(0x81, 0xa0, base + n)) * 2.0 ** -23)
+    # queries whose products with the kernel's scale, 1 / sqrt(head_dim) in base 2, lie there
+    scale = np.float32(1) / np.sqrt(np.float32(head_dim)) * np.float32(1.4426950408889634)
+    some = (rng.uniform(240, 250, 1 << 20)).astype(np.float32)
+    low = (some * scale).view(np.uint32) & 0xffff
+    q = np.zeros((n, q_heads * head_dim), np.float32)
+    q[:, 3::head_dim] = some[(low >= 0xff60) & (low < 0xff80)][:n * q_heads].reshape(n, q_heads)
+    v = rng.standard_normal((base + n, head_dim), dtype=np.float32)
+    want = np.empty((n, q_heads * head_dim))
+    for h in range(q_heads):
+        cols = slice(h * head_dim, (h + 1) * head_dim)
+        s = q[:, cols].astype(np.float64) @ k.astype(np.float64).T / np.sqrt(head_dim)
+        s[np.arange(base + n)[None] > base + np.arange(n)[:, None]] = -np.inf
+        p = np.exp(s - s.max(1, keepdims=True))
+        want[:, cols] = p / p.sum(1, keepdims=True) @ v
+
+    def run():
+        kv = state.full_attention_f32(base + n, q_heads, kv_heads, head_dim)
+        kv.seed(k[:base], v[:base], base)
+        out = kv.prefill_rows(q, k[base:], v[base:])
+        kv.close()
+        return np.linalg.norm(out - want)
+    terms = run()
+    os.environ["SKV_PREFILL_TILES"] = "0"
+    skv.flags.reload()
+    assert terms <= 1.5 * run()
