@@ -578,7 +578,7 @@ __device__ __forceinline__ void merge_rows_body(const DecodeArgs &a, const int k
         float4_t v[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            const int sp = min(sp0 + u, a.splits_total - 1); // a repeat of the last one weighs zero below
+            const int sp = min(sp0 + u, a.splits_total - 1); // a repeat of the last one is left out below
             const long pidx = base + (long)sp * n_slots;
             w[u] = a.part_m[pidx];
             lp[u] = a.part_l[pidx];
@@ -596,7 +596,8 @@ __device__ __forceinline__ void merge_rows_body(const DecodeArgs &a, const int k
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            const float wu = sp0 + u < a.splits_total ? fast_exp2(w[u] - m_safe) : 0.0f;
+            if (sp0 + u >= a.splits_total) continue; // uniform (a repeat: 0 x Inf would be NaN)
+            const float wu = fast_exp2(w[u] - m_safe);
             lsum += wu * lp[u];
 #pragma unroll
             for (int i = 0; i < 4; ++i) acc[i] += wu * v[u][i];

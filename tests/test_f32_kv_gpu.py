@@ -286,3 +286,21 @@ def test_flash_sdpa_off_uses_the_plain_kernel_on_f32_rows(state, dims, n):
     matrix = kv.attention_decode(q)
     assert np.abs(plain - want).max() <= 2e-6
     assert np.abs(plain - matrix).max() <= TOL
+
+
+@pytest.mark.parametrize("rows", [4, 40])
+def test_infinite_row_in_the_last_of_three_splits(state, rows):
+    """The merge of a chunk's partials takes four splits a round: the round's empty place must not weigh the
+    last split's infinity by zero."""
+    q_heads, kv_heads, head_dim, base = 4, 2, 64, 300
+    rng = np.random.default_rng(rows)
+    k, v = (rng.standard_normal((base + rows, kv_heads * head_dim), dtype=np.float32) for _ in range(2))
+    q = rng.standard_normal((rows, q_heads * head_dim), dtype=np.float32)
+    v[base - 5, 7] = -np.inf
+    kv = state.full_attention_f32(base + rows, q_heads, kv_heads, head_dim)
+    kv.seed(k[:base], v[:base], base)
+    got = kv.prefill_rows(q, k[base:], v[base:])
+    assert np.isneginf(got[:, [7, head_dim + 7]]).all()
+    got[:, [7, head_dim + 7]] = 0
+    assert np.isfinite(got).all()
+    kv.close()
