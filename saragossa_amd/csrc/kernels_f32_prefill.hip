@@ -458,24 +458,144 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
         }
     }
 
+    // One slot again, in f32 products, by the whole wavefront. An infinite factor has no three terms (an
+    // infinity times its own remainder, or times the second term of the other factor, is NaN), and in V
+    // it reaches the slots that do not attend its row as 0 x NaN; so the slots whose sums are not
+    // numbers come here, where keys outside the slot's range are left out and an infinity does what it does in
+    // f32. What is NaN then stays NaN. Lane (n, j) holds key n's dims 4j .. 4j+3 of every 16, then dim n's keys
+    // 4j .. 4j+3. Rare and not fast: a few registers, so that the kernel above keeps its own, and VT tiles of 16
+    // dims of V at a time, the scores taken again for each VT.
+    const DecodeArgs &args = a;
+    const ChunkPages &pages = c;
+    auto plain_slot = [&](int slot, float *dst, bool whole, long pidx) {
+        // Up to head_dim 128 the arguments come again from the launch's memory: kept for this place they
+        // spill scalar registers around the loop above (1500 rows through 36 layers of q32/kv8/hd128: 840 us as
+        // it is, 850 with them kept, 835 without this function). At 256, where reading them again makes the
+        // compiler spill vector registers inside the loop, they are kept (512 rows of q16/kv2/hd256 over 8192 rows: 0.5 % for the
+        // function as it is, 3.4 % with the arguments read again).
+        const char *mem = reinterpret_cast<const char *>(&args);
+        if constexpr (P <= 128) {
+            mem = (const char *)__builtin_amdgcn_kernarg_segment_ptr();
+            asm("" : "+s"(mem)); // (not known to be what has been read before)
+        }
+        const DecodeArgs &a = *reinterpret_cast<const DecodeArgs *>(mem);
+        const ChunkPages &c = P <= 128 ? *reinterpret_cast<const ChunkPages *>(mem + sizeof(DecodeArgs)) : pages;
+        const Geom &g = a.g;
+        const int G = g.gqa;
+        auto limit_of = [&](int slot) { return a.q_pos0 + slot / G; };
+        auto ws_of = [&](int slot) { return a.window > 0 ? max(a.window_start, limit_of(slot) + 1 - a.window) : a.window_start; };
+        constexpr int VT = NT < 8 ? NT : 8, KT = NT < 4 ? NT : 4;
+        const float *qrow = a.q + ((long)(slot / G) * g.q_heads + kvh * G + slot % G) * g.head_dim;
+        const int lo0 = ws_of(slot), hi0 = limit_of(slot);
+#pragma unroll 1
+        for (int v0 = 0; v0 < NT; v0 += VT) {
+            float acc[VT], m = -INFINITY, sum = 0.0f; // sum: of the keys n of every page
+#pragma unroll
+            for (int u = 0; u < VT; ++u) acc[u] = 0.0f;
+#pragma unroll 1
+            for (int e = pb0; e < pb1; ++e) {
+                const int pos0 = entry_pos<RING>(c, e);
+                const int lo = max(lo0, entry_lo<RING>(c, e)), hi = min(hi0, entry_hi<RING>(c, e));
+                if (pos0 + 15 < lo || pos0 > hi) continue; // uniform
+                const uint32_t at = entry_tile<RING>(a, c, e, kvh);
+                const bool own = RING && e >= c.n_old;
+                const float4_t *kt = reinterpret_cast<const float4_t *>(own ? c.k_new : a.k_pool) + at + lane;
+                const float4_t *vt = reinterpret_cast<const float4_t *>(own ? c.v_new : a.v_pool) + at + lane + v0 * 64;
+                float sc = 0.0f;
+#pragma unroll 1
+                for (int k0 = 0; k0 < NT; k0 += KT) {
+#pragma unroll
+                    for (int u = 0; u < KT; ++u) {
+                        const float4_t x = kt[(k0 + u) * 64];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const int d = (k0 + u) * 16 + j * 4 + i;
+                            const float y = qrow[min(d, g.head_dim - 1)] * a.qscale;
+                            sc += x[i] * (d < g.head_dim ? y : 0.0f); // (K is zero there)
+                        }
+                    }
+                }
+                sc = rows_sum(sc);
+                sc = pos0 + n >= lo && pos0 + n <= hi ? sc : -INFINITY;
+                float top = sc;
+#pragma unroll
+                for (int x = 1; x < 16; x *= 2) top = fmaxf(top, __shfl_xor(top, x, 64));
+                const float m_new = fmaxf(m, top), m_safe = m_new == -INFINITY ? 0.0f : m_new;
+                const float alpha = fast_exp2(m - m_safe), pk = fast_exp2(sc - m_safe);
+                m = m_new;
+                sum = sum * alpha + pk;
+#pragma unroll
+                for (int u = 0; u < VT; ++u) acc[u] *= alpha;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float pi = __shfl(pk, j * 4 + i, 64);
+                    const bool in = pos0 + j * 4 + i >= lo && pos0 + j * 4 + i <= hi;
+#pragma unroll
+                    for (int u = 0; u < VT; ++u) {
+                        const float x = vt[u * 64][i];
+                        acc[u] += in ? pi * x : 0.0f;
+                    }
+                }
+                if (__builtin_amdgcn_ballot_w64(sum != sum)) break; // a weight that is NaN: nothing is a number any more
+            }
+#pragma unroll
+            for (int x = 1; x < 16; x *= 2) sum += __shfl_xor(sum, x, 64);
+            if (!whole && lane == 0) {
+                a.part_m[pidx] = m;
+                a.part_l[pidx] = sum;
+            }
+            // (a NaN sum: the rows that were not looked at any more are NaN too)
+            const float scale = whole ? 1.0f / sum : sum != sum ? sum : 1.0f;
+#pragma unroll
+            for (int u = 0; u < VT; ++u) {
+                const float x = rows_sum(acc[u]) * scale;
+                const int col = (v0 + u) * 16 + n;
+                if (j == 0 && col < g.head_dim) dst[col] = x;
+            }
+        }
+    };
+
     // ---- every wavefront writes its own slots -------------------------------------------
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
         const float l = rows_sum(l_run[t]);
-        const int slot = wg_slot0 + (tw * TILES + t) * 16 + n;
-        if (!t_on[t] || slot >= n_slots) continue;
-        float *dst;
-        float scale = 1.0f;
-        if (a.splits_total == 1) {
-            scale = 1.0f / l;
-            dst = a.out + ((long)(slot / G) * g.q_heads + kvh * G + slot % G) * g.head_dim;
-        } else {
-            const long pidx = ((long)kvh * a.splits_total + a.split_base + split) * n_slots + slot;
-            dst = a.part_o + pidx * g.head_dim;
-            if (j == 0) {
-                a.part_m[pidx] = thr[t] == -INFINITY ? -INFINITY : m_base[t];
-                a.part_l[pidx] = l;
+        const int slot0 = wg_slot0 + (tw * TILES + t) * 16;
+        if (!t_on[t]) continue;
+        const bool whole = a.splits_total == 1;
+        auto partial_of = [&](int slot) { return ((long)kvh * a.splits_total + a.split_base + split) * n_slots + slot; };
+        auto dst_of = [&](int slot) {
+            return whole ? a.out + ((long)(slot / G) * g.q_heads + kvh * G + slot % G) * g.head_dim
+                         : a.part_o + partial_of(slot) * g.head_dim;
+        };
+        // slots whose sums are not all numbers (columns past head_dim are none of theirs)
+        float zero = 0.0f * l;
+        if (g.head_dim == P) { // uniform
+#pragma unroll
+            for (int u = 0; u < NT; ++u) {
+                const float4_t z = o[t][u];
+                zero = fmaf(z[0], 0.0f, fmaf(z[1], 0.0f, fmaf(z[2], 0.0f, fmaf(z[3], 0.0f, zero))));
             }
+        } else {
+#pragma unroll
+            for (int u = 0; u < NT; ++u) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    zero = fmaf(word_f32(f32_word(o[t][u][i]) & (uint32_t)((u * 16 + j * 4 + i - g.head_dim) >> 31)), 0.0f, zero);
+            }
+        }
+        const uint64_t lanes = __builtin_amdgcn_ballot_w64(!(zero == 0.0f));
+        const uint32_t odd = (uint32_t)(lanes | lanes >> 16 | lanes >> 32 | lanes >> 48) & 0xffffu;
+        for (uint32_t left = odd; left; left &= left - 1) {
+            const int slot = slot0 + __builtin_ctz(left);
+            if (slot < n_slots) plain_slot(slot, dst_of(slot), whole, partial_of(slot));
+        }
+        const int slot = slot0 + n;
+        if (slot >= n_slots || (odd >> n & 1)) continue;
+        float *dst = dst_of(slot);
+        const float scale = whole ? 1.0f / l : 1.0f;
+        if (!whole && j == 0) {
+            a.part_m[partial_of(slot)] = thr[t] == -INFINITY ? -INFINITY : m_base[t];
+            a.part_l[partial_of(slot)] = l;
         }
         const bool vec_ok = (g.head_dim & 3) == 0;
 #pragma unroll

@@ -175,6 +175,39 @@ def test_few_rows_are_appended_by_the_attention_launch(state, dims, window, star
     assert np.array_equal(gk, cache.keys()[first:]) and np.array_equal(gv, cache.values()[first:])
 
 
+@pytest.mark.parametrize("head_dim,window,base", [(64, 0, 61), (128, 0, 900), (256, 0, 61), (256, 0, 900), (40, 0, 900),
+                                                  (64, 70, 61), (128, 900, 1200)])  # one split, several; rings
+def test_infinite_rows_of_an_f32_chunk(state, shape, head_dim, window, base):
+    """A live f32 row with an infinity gives what f32 products give, and only to the rows that attend it: an
+    infinite V element that column of their contexts, an infinite K element weight zero or a NaN context as the
+    query's sign there has it, an infinite query element its own head's context."""
+    q_heads, kv_heads, rows = 4, 2, 150
+    kv_dim, q_dim = kv_heads * head_dim, q_heads * head_dim
+    rng = np.random.default_rng(head_dim + window)
+    kv = state.full_attention_f32(base + rows, q_heads, kv_heads, head_dim, window=window)
+    kv.set_block_table(rng.permutation(kv.pages()).astype(np.int32))
+    lay = oracle.layout(q_heads, kv_heads, head_dim, sliding_window=window)
+    cache = oracle.LayerKvCache("f32")
+    k0, v0 = (rng.standard_normal((base, kv_dim), dtype=np.float32) for _ in range(2))
+    kv.seed(k0, v0, base)
+    cache.append_batch(k0, v0, lay)
+    q = rng.standard_normal((rows, q_dim), dtype=np.float32)
+    k, v = (rng.standard_normal((rows, kv_dim), dtype=np.float32) for _ in range(2))
+    v[20, 3], v[100, head_dim + 7] = np.inf, -np.inf
+    v[60, 5] = np.float32(3.4e38)      # finite: its first term, rounded, is not
+    k[40, 9], k[120, head_dim + 2] = np.inf, -np.inf
+    q[:, 9] = -np.abs(q[:, 9])         # head 0 gives that key weight zero; head 1 by its own sign
+    q[140, 2 * head_dim + 1] = np.inf
+    got = kv.prefill_rows(q, k, v)
+    with np.errstate(all="ignore"):
+        want = oracle.cached_attention_prefill_rows(q, k, v, cache, lay)
+    assert not np.isfinite(want).all() and np.isfinite(want[:20]).all()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
+    ok = np.isfinite(want)
+    assert (np.abs(got - want)[ok] <= 2e-5 * np.maximum(np.abs(want[ok]), 1.0)).all()
+
+
 def test_f32_scores_of_one_product_each(state, shape):
     """Factors just below a bf16 value or one, one product a score, scores of a thousand: no further off
     than the kernel of f32 products (a margin of 1.5 for the order of the sums). With the terms cut off instead of
