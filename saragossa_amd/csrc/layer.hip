@@ -376,11 +376,16 @@ int32_t multi_query_partials(skv_layer *L, hipStream_t s, size_t n_sets, size_t 
         }
         void *p = nullptr;
         SKV_HIP(hipMalloc(&p, need));
-        std::lock_guard<std::mutex> lk(c->arena_mu);
-        skv_ctx::MqScratch &slot = c->mq_scratch[s];
-        slot.ptr = p;
-        slot.bytes = need;
-        slot.used = ++c->mq_clock;
+        try {
+            std::lock_guard<std::mutex> lk(c->arena_mu);
+            skv_ctx::MqScratch &slot = c->mq_scratch[s];
+            slot.ptr = p;
+            slot.bytes = need;
+            slot.used = ++c->mq_clock;
+        } catch (...) {
+            (void)hipFree(p);
+            throw;
+        }
         buf = p;
     }
     if (pages) *pages = buf;
@@ -611,6 +616,19 @@ void appended(skv_layer *L, size_t n_rows) {
     if (L->g.ring_rows > 0 && L->len > (size_t)L->g.ring_rows)
         L->floor_pos = std::max(L->floor_pos, L->len - (size_t)L->g.ring_rows);
 }
+
+// A layer that counts n rows ahead of the launch that writes them, until the end of the scope unless they are written by
+// then: an error, or an exception on the way (a launch's scratch may have to grow), leaves it as it was.
+struct RowsAhead {
+    skv_layer *L;
+    size_t n;
+    bool written = false;
+    RowsAhead(skv_layer *layer, size_t rows) : L(layer), n(rows) { L->len += n; }
+    RowsAhead(const RowsAhead &) = delete;
+    ~RowsAhead() {
+        if (!written) L->len -= n;
+    }
+};
 
 int32_t encode_append(skv_layer *L, hipStream_t s, const float *k_dev, const float *v_dev,
                       size_t n_rows) {
@@ -1140,9 +1158,10 @@ static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const flo
     const size_t pool_bytes = n_new * (size_t)g.page_elems * sizeof(uint16_t); // of K and of V
 
     DecodeArgs a{};
-    L->len += c; // the queries are the last c rows
-    fill_decode_args(L, q, out, L->floor_pos, nullptr, nullptr, c, tuning().prefill_wgs, a);
-    L->len -= c;
+    {
+        RowsAhead ahead(L, c); // the queries are the last c rows
+        fill_decode_args(L, q, out, L->floor_pos, nullptr, nullptr, c, tuning().prefill_wgs, a);
+    }
     // pages a workgroup of one tile row walks: the window and the workgroup's own rows
     const size_t walked = std::min<size_t>((size_t)pages.n_old + n_new, L->window / 16 + 2);
     const TileShape shape = prefill_shape(g, c * (size_t)g.gqa, walked);
@@ -1257,12 +1276,10 @@ int32_t skv_prefill_chunk_device(skv_layer *L, skv_stream stream, const float *q
         // lie in that tile's window)
         if (c > 1 && c <= (size_t)MQ_APPEND_ROWS && ring == 0 && (L->window == 0 || L->window >= c) && !L->g.f32 && tuning().fused_append &&
             !takes_tile_kernel(L->g, c * (size_t)L->g.gqa, (L->len + c + 15) / 16)) {
-            L->len += c;
+            RowsAhead ahead(L, c);
             rc = encode_attention(L, as_stream(stream), q, out, 0, k, v, c);
-            if (rc) {
-                L->len -= c;
-                return rc;
-            }
+            if (rc) return rc;
+            ahead.written = true;
             q += c * q_dim;
             k += c * kv_dim;
             v += c * kv_dim;

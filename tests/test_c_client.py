@@ -12,6 +12,7 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SRC = os.path.join(ROOT, "tests", "native", "kv_c_client.c")
 EXE = os.path.join(ROOT, "tests", "native", "kv_c_client")
+EXE_THROW = os.path.join(ROOT, "tests", "native", "kv_throw_client")
 EXE_REMEMBER = os.path.join(ROOT, "tests", "native", "kv_c_remember")
 
 
@@ -32,7 +33,7 @@ def test_header_is_strict_c11_and_cxx17():
 @pytest.mark.skipif(shutil.which("gcc") is None, reason="gcc not available")
 def test_c_client_compiles_and_links_against_the_library():
     compile_c_client()
-    assert os.path.exists(EXE) and os.path.exists(EXE_REMEMBER)
+    assert all(os.path.exists(exe) for exe in (EXE, EXE_REMEMBER, EXE_THROW))
 
 
 @pytest.mark.gpu
@@ -58,3 +59,14 @@ def test_c_remember_client_caches_every_block_one_call_per_boundary():
     rep = json.loads(run.stdout.strip().splitlines()[-1])
     assert rep["calls"] == 256 and rep["cached"] == 256
     assert rep["host_us_per_call"] < 40.0, rep
+
+
+@pytest.mark.gpu
+def test_rows_are_not_counted_when_memory_runs_out_on_the_way():
+    """A chunk of few rows is appended by its attention launch, whose scratch may have to grow first: where the host has
+    no memory for that, the call returns a status and the layer counts no row that nobody wrote."""
+    if not os.path.exists(EXE_THROW):
+        compile_c_client()
+    run = subprocess.run([EXE_THROW], capture_output=True, text=True, timeout=120)
+    assert run.returncode == 0, (run.stdout[-500:], run.stderr[-2000:])
+    assert run.stdout.strip().endswith("ok")
