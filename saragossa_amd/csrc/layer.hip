@@ -1138,6 +1138,18 @@ int32_t skv_decode_step_static_device(skv_layer *L, skv_stream stream, const voi
     return skv::fail_exception();
 }
 
+// Whether a chunk's context is to lie over its K or V rows (a caller's activations that share a buffer): every row
+// then has to be in the cache before the first context is written.
+static bool context_over_rows(const skv_layer *L, size_t c, const float *out, const float *k, const float *v) {
+    const size_t n = c * skv_kv_dim(L) * sizeof(float), m = c * (size_t)L->g.q_heads * L->g.head_dim * sizeof(float);
+    const uintptr_t o = reinterpret_cast<uintptr_t>(out);
+    for (const float *p : {k, v}) {
+        const uintptr_t r = reinterpret_cast<uintptr_t>(p);
+        if (o < r + n && r < o + m) return true;
+    }
+    return false;
+}
+
 // A chunk of c > 1 rows on a ring layer (bf16, or f32 where the f32 chunk kernel serves the head_dim). The ring holds little more than the window, so the
 // chunk's own rows overwrite rows its first queries still attend. They are therefore first
 // written to pages of the context's scratch; one launch attends the ring's rows and them, in the
@@ -1167,6 +1179,9 @@ static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const flo
     const TileShape shape = prefill_shape(g, c * (size_t)g.gqa, walked);
     const bool halves = g.f32 && f32_halves(g, c * (size_t)g.gqa, walked);
     a.splits = chunk_splits(g, c, (size_t)(g.f32 ? f32_prefill_slots(g.P, halves) : prefill_tile_slots(g.P, shape)), walked);
+    // a context over the chunk's own rows is written once they are in the ring: by the merge, so there has to be one
+    const bool over_rows = context_over_rows(L, c, out, k, v);
+    if (over_rows) a.splits = std::max(a.splits, 2);
     a.splits_total = a.splits;
     void *scratch = nullptr;
     int32_t rc = multi_query_partials(L, s, a.splits > 1 ? (size_t)a.splits : 0, c, a, 2 * pool_bytes, &scratch);
@@ -1185,6 +1200,12 @@ static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const flo
     pages.v_new = w.v_pool;
     SKV_HIP(g.f32 ? launch_f32_prefill(a, pages, halves, s) : launch_prefill_tiles(a, pages, shape, s));
     if (a.splits == 1) return encode_append(L, s, k, v, c);
+    if (over_rows) {
+        rc = encode_append(L, s, k, v, c);
+        if (rc) return rc;
+        SKV_HIP(launch_merge_rows(a, s));
+        return SKV_OK;
+    }
     SKV_HIP(launch_merge_append(a, append_args(L, k, v, c), s)); // (the caller has checked the capacity)
     appended(L, c);
     return SKV_OK;
@@ -1275,7 +1296,7 @@ int32_t skv_prefill_chunk_device(skv_layer *L, skv_stream stream, const float *q
         // appends them itself, as a decode step's does (its last query tile stores them: all of them have to
         // lie in that tile's window)
         if (c > 1 && c <= (size_t)MQ_APPEND_ROWS && ring == 0 && (L->window == 0 || L->window >= c) && !L->g.f32 && tuning().fused_append &&
-            !takes_tile_kernel(L->g, c * (size_t)L->g.gqa, (L->len + c + 15) / 16)) {
+            !context_over_rows(L, c, out, k, v) && !takes_tile_kernel(L->g, c * (size_t)L->g.gqa, (L->len + c + 15) / 16)) {
             RowsAhead ahead(L, c);
             rc = encode_attention(L, as_stream(stream), q, out, 0, k, v, c);
             if (rc) return rc;

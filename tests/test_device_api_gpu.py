@@ -343,3 +343,41 @@ def test_measurement_probes_leave_the_cache_untouched(state):
         assert np.array_equal(before[0], after[0]) and np.array_equal(before[1], after[1])
         assert np.array_equal(attend(), want)
         kv.close()
+
+
+@pytest.mark.parametrize("element", ["bf16", "f32"])
+@pytest.mark.parametrize("heads,head_dim,window,base,rows", [
+    ((4, 4), 64, 48, 100, 90),       # ring, one split: the rows go into it after the attention
+    ((4, 2), 64, 1500, 1700, 70),    # ring, several splits: with the merge
+    ((32, 8), 64, 0, 300, 6),        # few rows, appended by the attention launch; several query tiles
+    ((4, 4), 64, 0, 300, 40),
+])
+@pytest.mark.parametrize("over", ["k", "v"])
+def test_context_of_a_chunk_over_its_own_rows(state, element, heads, head_dim, window, base, rows, over):
+    """The context may be written where the chunk's K or V rows lay (a caller's activations share a buffer):
+    the rows are in the cache, and the context is the same."""
+    kv_dim, q_dim = heads[1] * head_dim, heads[0] * head_dim
+    gen = torch.Generator().manual_seed(base + rows)
+    k0, v0 = (torch.randn(base, kv_dim, generator=gen).numpy() for _ in range(2))
+    q, k, v = (torch.randn(rows, d, generator=gen).cuda() for d in (q_dim, kv_dim, kv_dim))
+    results = []
+    for shared in (False, True):
+        make = state.full_attention_f32 if element == "f32" else state.full_attention_bf16
+        kv = make(base + rows, *heads, head_dim, window=window)
+        kv.seed(k0, v0, base)
+        arena = torch.zeros(rows * q_dim, device="cuda")
+        kc, vc = k.clone(), v.clone()
+        if shared:
+            arena[-rows * kv_dim:] = (k if over == "k" else v).flatten()
+        at = arena.data_ptr() + rows * (q_dim - kv_dim) * 4 if shared else None
+        kv.encode_prefill_rows(_stream(), q.data_ptr(), at if shared and over == "k" else kc.data_ptr(),
+                               at if shared and over == "v" else vc.data_ptr(), rows, arena.data_ptr())
+        torch.cuda.synchronize()
+        first = max(0, kv.len() - window) if window else 0
+        results.append((arena.cpu().numpy(), *kv.read_rows_f32(first, kv.len() - first)))
+        kv.close()
+    (apart, *rows_apart), (shared, *rows_shared) = results
+    # (a ring's chunk of one split is then two and a merge: probabilities of 16 bits on bf16 layers, sums in another order on f32)
+    assert np.abs(apart - shared).max() <= (1e-4 if element == "bf16" else 2e-5)
+    for a, b in zip(rows_apart, rows_shared):
+        assert np.array_equal(a, b)

@@ -115,3 +115,31 @@ def test_prefill_chunk_under_knobs(state, knobs, element, tol, dims, start, chun
     assert np.abs(got - want).max() <= tol
     gk, gv = kv.read_rows_f32()
     assert np.array_equal(gk, cache.keys()) and np.array_equal(gv, cache.values())
+
+
+@pytest.mark.parametrize("element,tiles", [("f32", "2"), ("bf16", "0"), ("bf16", "2")])
+@pytest.mark.parametrize("knob", [{"RETI_RUST_SDPA_2PASS_MIN_LEN": "100000"}, {"SKV_DECODE_WGS": "1"},
+                                  {"SKV_DECODE_MIN_PAGES": "4096"}], ids=lambda k: next(iter(k)))
+def test_split_knobs_reach_every_chunk_kernel(state, element, tiles, knob):
+    """A chunk over a context that the knobs forbid to split is the launch without splits, bit for bit."""
+    q_heads, kv_heads, head_dim, base, rows = 8, 2, 64, 3000, 20
+    rng = np.random.default_rng(4)
+    k, v = (rng.standard_normal((base + rows, kv_heads * head_dim), dtype=np.float32) for _ in range(2))
+    q = rng.standard_normal((rows, q_heads * head_dim), dtype=np.float32)
+
+    def run(**env):
+        env["SKV_PREFILL_TILES"] = tiles
+        saved = {name: os.environ.get(name) for name in env}
+        os.environ.update(env)
+        skv.flags.reload()
+        try:
+            kv = (state.full_attention_f32 if element == "f32" else state.full_attention_bf16)(base + rows, q_heads, kv_heads, head_dim)
+            kv.seed(k[:base], v[:base], base)
+            return kv.prefill_rows(q, k[base:], v[base:])
+        finally:
+            for name, was in saved.items():
+                os.environ.pop(name) if was is None else os.environ.__setitem__(name, was)
+            skv.flags.reload()
+    whole = run(RETI_RUST_SDPA_2PASS="0")
+    assert not np.array_equal(run(), whole)     # several splits by default
+    assert np.array_equal(run(**knob), whole)
