@@ -476,7 +476,8 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
         if (attn_scalar > 0.0f) a.qscale = (1.0f / std::sqrt(attn_scalar)) * 1.4426950408889634f;
         if (n_queries > 1 && takes_f32_chunk_kernel(g, n_queries * (size_t)g.gqa, (size_t)a.n_pages)) {
             const bool halves = f32_halves(g, n_queries * (size_t)g.gqa, (size_t)a.n_pages);
-            a.splits = chunk_splits(g, n_queries, (size_t)f32_prefill_slots(g.P, halves), (size_t)a.n_pages);
+            // (choose_splits' number, which the split knobs of decode launches bound, is the larger one unless they do)
+            a.splits = std::min(a.splits, chunk_splits(g, n_queries, (size_t)f32_prefill_slots(g.P, halves), (size_t)a.n_pages));
             a.splits_total = a.splits;
             if (a.splits > 1) {
                 int32_t rc2 = multi_query_partials(L, s, (size_t)a.splits, n_queries, a);
@@ -559,7 +560,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
             // eight; 256 rows of q16/kv2/hd256: 14.2/30.1 and 13.5/24.6)
             const size_t slot_tiles = (n_queries * (size_t)g.gqa + 15) / 16 * (size_t)g.kv_heads;
             a.waves = g.P <= 128 && slot_tiles >= 512 ? 4 : 8;
-            a.splits = choose_splits(L, a.n_pages, L->len - window_start, a.waves, 256);
+            a.splits = choose_splits(L, a.n_pages, L->len - window_start, a.waves, decode_target_wgs());
         }
         const size_t per_wg = use_tiles ? (size_t)prefill_tile_slots(g.P, shape) : 16;
         const size_t tiles = (n_queries * (size_t)g.gqa + per_wg - 1) / per_wg * (size_t)g.kv_heads;
