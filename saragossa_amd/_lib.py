@@ -208,14 +208,21 @@ def lib():
     return _lib
 
 
+class _ThroughCtypes:
+    """Stands for the module of csrc/calls.c where it cannot be loaded: every function leaves the call to ctypes."""
+
+    def __getattr__(self, name):
+        return lambda *args: -1
+
+
 def calls():
-    """The module of csrc/calls.c: the per-token calls without ctypes, on the same library."""
+    """The module of csrc/calls.c: the per-token calls without ctypes, on the same library. Built for one
+    interpreter; another one, or a build of the library alone, makes the same calls through ctypes."""
     lib()
     try:
         from . import _calls
-    except ImportError as e:
-        raise DeviceError(f"saragossa_amd/_calls.so cannot be loaded ({e}): build it with `python -c "
-                          "'import __graft_entry__ as g; g.build()'`") from e
+    except ImportError:
+        return _ThroughCtypes()
     return _calls
 
 

@@ -230,3 +230,24 @@ def test_calls_module_stands_for_ctypes(name, symbol):
         odd = [True, "1", 2.0, np.int64(3)] if k is not ctypes.c_float else [1, None, "1"]
         for x in odd + ([None] if k is ctypes.c_size_t else []):
             assert fast(*null[:i], x, *null[i + 1:]) == -1, (i, x)
+
+
+def test_without_the_calls_module_every_call_goes_through_ctypes(monkeypatch):
+    """Another interpreter than the one it was built for, or a build of the library alone."""
+    monkeypatch.setitem(sys.modules, "saragossa_amd._calls", None)   # its import raises ImportError
+    monkeypatch.delattr(skv, "_calls", raising=False)
+    rc = _lib.calls().decode_step(None, None, None, 0, None, 0, None, None)
+    with pytest.raises(skv.DeviceError, match="nul"):                # the library's own refusal of a null layer
+        _lib.settle(rc, skv.lib().skv_decode_step_device, None, None, None, 0, None, 0, None, None)
+
+
+def test_calls_module_is_named_for_its_interpreter():
+    import sysconfig
+    assert _lib.calls().__file__.endswith("_calls" + sysconfig.get_config_var("EXT_SUFFIX"))
+
+
+def test_library_builds_without_python_headers():
+    """`make` without an interpreter's headers asks for the library and nothing else."""
+    csrc = os.path.join(ROOT, "saragossa_amd", "csrc")
+    run = subprocess.run(["make", "-n", "-B", "-C", csrc, "PYTHON=false"], capture_output=True, text=True, timeout=60)
+    assert run.returncode == 0 and "libsaragossa_kv.so" in run.stdout and "calls.c" not in run.stdout
