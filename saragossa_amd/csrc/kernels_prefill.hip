@@ -653,7 +653,8 @@ hipError_t launch_merge_append(const DecodeArgs &a, const AppendArgs &w, hipStre
 // Query slots one workgroup of the kernel covers for a padded head_dim.
 int prefill_tile_slots(int P, TileShape shape) {
     if (P > 256) return 64; // four wavefronts, one per SIMD (the accumulators and query halves are 256 registers)
-    return shape == TileShape::two_tiles && P <= 128 ? 256 : shape == TileShape::halves || shape == TileShape::quarters ? 64 : 128;
+    if (shape == TileShape::two_tiles && P <= 128) return 256;
+    return shape == TileShape::halves || (shape == TileShape::quarters && P == 128) ? 64 : 128;
 }
 
 template <int P, int TILES, int SP, int WAVES, int HALVES, bool RING>

@@ -193,6 +193,11 @@ size_t decode_target_wgs() { return tuning().target_wgs; }
 // 37.6/45.0/38.9/38.5, 1024 rows over 4096, 16384 36.3/41.9/37.2/37.4, 85.9/82.7/109/92.6; q16/kv2/hd256 (one tile /
 // halves), 512 rows over 512, 2048, 4096, 8192 38.6/37.5, 57.1/56.7, 82.0/82.4, 131/134, 1024 rows over 2048, 8192
 // 101/91.0, 245/246.
+// Quarters from 208 workgroups of 64 slots on: up to 204, two-tile workgroups fill the device in five splits; from there to
+// 256 only four fit, and up to 48 compute units stay idle. 400 rows (200 workgroups) of q32/kv8/hd128 at walks of 55000, 75000,
+// 98000, two tiles / quarters 76.4/74.0, 93.0/93.7, 113/118; 416 rows (208) 73.5/70.6, 90.2/90.0, 110/113; 448 (224) 71.1/67.2,
+// 86.0/84.8, 105/107; 480 (240) 70.2/63.8, 84.6/80.2, 102/101; 512 (256) 67.1/60.6, 82.5/77.2, 98.4/97.0 (halves 58.6, 77.1,
+// 108). At head_dim 96 they are up to 4 % behind the better of one and two tiles (q30/kv10, 448 rows 62.1/62.5 and 88.7/92.0).
 TileShape prefill_shape(const Geom &g, size_t n_slots, size_t n_pages) {
     if (g.P > 256) return TileShape::one_tile;
     const long knob = tuning().prefill_tiles2_min_pages;
@@ -1151,8 +1156,8 @@ static bool context_over_rows(const skv_layer *L, size_t c, const float *out, co
     return false;
 }
 
-// A chunk of c > 1 rows on a ring layer (bf16, or f32 where the f32 chunk kernel serves the head_dim). The ring holds little more than the window, so the
-// chunk's own rows overwrite rows its first queries still attend. They are therefore first
+// A chunk of c > 1 rows on a ring layer (bf16, or f32 where the f32 chunk kernel serves the head_dim). The
+// ring holds little more than the window, so the chunk's own rows overwrite rows its first queries still attend. They are therefore first
 // written to pages of the context's scratch; one launch attends the ring's rows and them, in the
 // order of positions, each workgroup only the pages its slots' windows touch; then the rows go
 // into the ring. (Two launches around the append, over the old rows and over the new ones,
@@ -1212,8 +1217,8 @@ static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const flo
     return SKV_OK;
 }
 
-// The same on an f32 ring layer of wider heads, c <= ring_rows, attended in two phases around the append: first every query over the rows
-// already in the ring (capped at the last old position), then, once the chunk is appended,
+// The same on an f32 ring layer of wider heads, c <= ring_rows, attended in two phases around the append:
+// first every query over the rows already in the ring (capped at the last old position), then, once the chunk is appended,
 // over the chunk's own rows (from its first position up to each query's own). Both phases
 // leave (o, m, l) partials; one merge produces the context. c <= ring_rows.
 static int32_t ring_chunk_f32(skv_layer *L, hipStream_t s, const float *q, const float *k, const float *v,
@@ -1294,9 +1299,8 @@ int32_t skv_prefill_chunk_device(skv_layer *L, skv_stream stream, const float *q
             continue;
         }
         // a few rows over a full bf16 layer (a speculative verify, the rest of a prompt): the multi-query launch
-        // appends them itself, as a decode step's does (its last query tile stores them: all of them have to
-        // lie in that tile's window)
-        if (c > 1 && c <= (size_t)MQ_APPEND_ROWS && ring == 0 && (L->window == 0 || L->window >= c) && !L->g.f32 && tuning().fused_append &&
+        // appends them itself, as a decode step's does (its last query tile, which sees all of them, stores them)
+        if (c > 1 && c <= (size_t)MQ_APPEND_ROWS && ring == 0 && !L->g.f32 && tuning().fused_append &&
             !context_over_rows(L, c, out, k, v) && !takes_tile_kernel(L->g, c * (size_t)L->g.gqa, (L->len + c + 15) / 16)) {
             RowsAhead ahead(L, c);
             rc = encode_attention(L, as_stream(stream), q, out, 0, k, v, c);

@@ -150,7 +150,7 @@ def test_chunks_that_quarters_take(state, head_dim, window, base, rows):
     ((20, 1, 128), 0, 40, (5, 1, 16)),          # more heads a group than a tile has slots
     ((3, 1, 18), 0, 30, (4, 16)),               # no 16-byte loads, padded head
     ((4, 2, 320), 0, 333, (16, 5)),             # several units a thread
-    ((8, 2, 64), 10, 20, (9, 12)),              # a window shorter than the chunk (appended by a launch of its own)
+    ((8, 2, 64), 10, 20, (9, 12)),              # a ring layer: appended by a launch of its own
 ])
 def test_few_rows_are_appended_by_the_attention_launch(state, dims, window, start, counts):
     q_heads, kv_heads, head_dim = dims
