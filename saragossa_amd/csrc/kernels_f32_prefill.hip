@@ -272,11 +272,11 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
             if (__builtin_amdgcn_ballot_w64(mx > thr[t])) {
                 const float top = rows_max(mx);
                 const bool unseen = thr[t] == -INFINITY;
-                const float d = unseen ? (top == -INFINITY ? 0.0f : top) : fmaxf(top, 0.0f);
+                const float d = top > thr[t] ? top + 8.0f : 0.0f;
                 const float alpha = unseen ? 1.0f : fast_exp2(-d);
                 m_base[t] += d;
                 neg_m[t] = float4_t{-m_base[t], -m_base[t], -m_base[t], -m_base[t]};
-                thr[t] = unseen && top == -INFINITY ? -INFINITY : 8.0f;
+                thr[t] = unseen && top == -INFINITY ? -INFINITY : 0.0f;
                 l_run[t] *= alpha;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
@@ -454,7 +454,7 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
 #pragma unroll
             for (int u = 0; u < NT; ++u) o[t][u] = o[t][u] * w0 + xo[(t * (NT + 1) + u) * 64] * w1;
             m_base[t] = m_safe;
-            thr[t] = mx == -INFINITY ? -INFINITY : 8.0f;
+            thr[t] = mx == -INFINITY ? -INFINITY : 0.0f;
         }
     }
 
@@ -465,21 +465,14 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
     // f32. What is NaN then stays NaN. Lane (n, j) holds key n's dims 4j .. 4j+3 of every 16, then dim n's keys
     // 4j .. 4j+3. Rare and not fast: a few registers, so that the kernel above keeps its own, and VT tiles of 16
     // dims of V at a time, the scores taken again for each VT.
-    const DecodeArgs &args = a;
-    const ChunkPages &pages = c;
     auto plain_slot = [&](int slot, float *dst, bool whole, long pidx) {
-        // Up to head_dim 128 the arguments come again from the launch's memory: kept for this place they
-        // spill scalar registers around the loop above (1500 rows through 36 layers of q32/kv8/hd128: 840 us as
-        // it is, 850 with them kept, 835 without this function). At 256, where reading them again makes the
-        // compiler spill vector registers inside the loop, they are kept (512 rows of q16/kv2/hd256 over 8192 rows: 0.5 % for the
-        // function as it is, 3.4 % with the arguments read again).
-        const char *mem = reinterpret_cast<const char *>(&args);
-        if constexpr (P <= 128) {
-            mem = (const char *)__builtin_amdgcn_kernarg_segment_ptr();
-            asm("" : "+s"(mem)); // (not known to be what has been read before)
-        }
+        // The arguments come again from the launch's memory: kept in registers for this place they spill
+        // around the loop above (this function costs 1500 rows through 36 layers of q32/kv8/hd128, 838 us, 1.2 % so
+        // and 0.5 % as it is; 512 rows of q16/kv2/hd256 over 8192 rows nothing).
+        const char *mem = (const char *)__builtin_amdgcn_kernarg_segment_ptr();
+        asm("" : "+s"(mem)); // (not known to be what has been read before)
         const DecodeArgs &a = *reinterpret_cast<const DecodeArgs *>(mem);
-        const ChunkPages &c = P <= 128 ? *reinterpret_cast<const ChunkPages *>(mem + sizeof(DecodeArgs)) : pages;
+        const ChunkPages &c = *reinterpret_cast<const ChunkPages *>(mem + sizeof(DecodeArgs));
         const Geom &g = a.g;
         const int G = g.gqa;
         auto limit_of = [&](int slot) { return a.q_pos0 + slot / G; };

@@ -44,11 +44,12 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // were in their vector phases at the same time: four pairs at head_dim 128 took 4.4 us by
 // time stamps where they take 3.4 now, of which the products are 1.75.)
 //
-// The softmax runs in base 2 against a base m per slot that is not the running maximum but
-// within 2^8 of it: the score accumulators start at -m, so the products deliver s - m and the
-// exponential needs no subtraction, and only a score above m + 8 makes the wavefront move the
-// bases and rescale its sums. Probabilities stay below 2^8 and are split relatively, so
-// nothing is lost; partials carry (o, base, l) and any base serves the merge.
+// The softmax runs in base 2 against a base m per slot that is not the running maximum but up to 8
+// above it: the score accumulators start at -m, so the products deliver s - m and the exponential
+// needs no subtraction, and only a score above m makes the wavefront move the bases (to 8 above that
+// score) and rescale its sums. Probabilities are at most one, so that sums of large values are no larger than
+// against the maximum, and are split relatively, so nothing is lost; partials carry (o, base, l) and any base
+// serves the merge.
 // With HALVES = 2 (or 4) the wavefronts are two halves (four quarters) that hold the same slots and take
 // the page pairs in turn; the others' (o, m, l) join the first's through LDS at the end. Otherwise there is
 // no merge inside the workgroup; with several splits the partials go to merge_rows_kernel.
@@ -268,7 +269,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
 
     float4_t o[TILES][NT];
     float4_t neg_m[TILES];             // -m in all four: what the score accumulators start from
-    float m_base[TILES], thr[TILES];   // base of the slot; a score above base + thr moves it (-inf: no key yet)
+    float m_base[TILES], thr[TILES];   // base of the slot; a score above base + thr moves it: 0, or -inf (no key yet)
     float l_run[TILES];                // this lane's share of the slot's sum
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
@@ -325,11 +326,11 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
             if (__builtin_amdgcn_ballot_w64(mx > thr[t])) {
                 const float top = rows_max(mx); // of the slot, relative to its base
                 const bool unseen = thr[t] == -INFINITY;
-                const float d = unseen ? (top == -INFINITY ? 0.0f : top) : fmaxf(top, 0.0f);
+                const float d = top > thr[t] ? top + 8.0f : 0.0f;
                 const float alpha = unseen ? 1.0f : fast_exp2(-d);
                 m_base[t] += d;
                 neg_m[t] = float4_t{-m_base[t], -m_base[t], -m_base[t], -m_base[t]};
-                thr[t] = unseen && top == -INFINITY ? -INFINITY : 8.0f;
+                thr[t] = unseen && top == -INFINITY ? -INFINITY : 0.0f;
                 l_run[t] *= alpha;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
@@ -508,7 +509,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
 #pragma unroll
                 for (int u = 0; u < NT; ++u) o[t][u] = o[t][u] * w0 + src[u * 64] * w1;
                 m_base[t] = m_safe;
-                thr[t] = mx == -INFINITY ? -INFINITY : 8.0f;
+                thr[t] = mx == -INFINITY ? -INFINITY : 0.0f;
             }
         }
     }

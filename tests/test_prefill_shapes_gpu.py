@@ -71,7 +71,7 @@ def test_chunks_in_every_shape(state, shape, element, tol, dims, window, base, c
 @pytest.mark.parametrize("element", ["bf16", "f32"])
 def test_scores_that_climb(state, shape, element):
     """Keys that grow along the context move the softmax base again and again (it follows a slot's
-    scores only once they pass it by 2^8), and fall below it by far more."""
+    scores only once they pass it), and fall below it by far more."""
     rng = np.random.default_rng(3)
     q_heads, kv_heads, head_dim, n = 8, 2, 64, 300
     make = state.full_attention_f32 if element == "f32" else state.full_attention_bf16
@@ -241,3 +241,22 @@ def test_f32_scores_of_one_product_each(state, shape):
     os.environ["SKV_PREFILL_TILES"] = "0"
     skv.flags.reload()
     assert terms <= 1.5 * run()
+
+
+@pytest.mark.parametrize("element", ["bf16", "f32"])
+def test_values_near_the_top_of_the_range(state, shape, element):
+    """Weights are never above one, so a context of 300 rows of 5e35 does not pass through an infinity: also where
+    scores rise by less than what moves the softmax base."""
+    rng = np.random.default_rng(6)
+    q_heads, kv_heads, head_dim, n = 8, 2, 64, 300
+    make = state.full_attention_f32 if element == "f32" else state.full_attention_bf16
+    kv = make(n, q_heads, kv_heads, head_dim)
+    lay = oracle.layout(q_heads, kv_heads, head_dim)
+    cache = oracle.LayerKvCache("f32" if element == "f32" else "bf16r")
+    q = np.ones((n, q_heads * head_dim), np.float32)
+    k = np.repeat(np.linspace(0.0, 0.6, n, dtype=np.float32)[:, None], kv_heads * head_dim, 1)   # scores 0 to 4.8, 6.9 in base 2
+    v = (5e35 * (1.0 + 0.1 * rng.random((n, kv_heads * head_dim)))).astype(np.float32)
+    got = kv.prefill_rows(q, k, v)
+    want = oracle.cached_attention_prefill_rows(q, k, v, cache, lay)
+    assert np.isfinite(want).all() and np.isfinite(got).all()
+    assert (np.abs(got - want) <= (1e-4 if element == "bf16" else 2e-5) * want).all()
