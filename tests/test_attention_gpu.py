@@ -207,6 +207,73 @@ def test_normal_inputs_config0(state):
     assert delta.max() <= 1e-4, delta.max()
 
 
+# ---- chunked prefill over the cache (multi-query, matrix cores) ----------------------------
+CHUNK_KERNELS = {
+    "by-shape": {},
+    "multi-query": {"SKV_PREFILL_TILES": "0"},
+    "halves": {"SKV_PREFILL_TILES": "2"},
+    "one-tile": {"SKV_PREFILL_TILES": "2", "SKV_PREFILL_TILES2_MIN_PAGES": "1000000000"},
+    "two-tiles": {"SKV_PREFILL_TILES": "2", "SKV_PREFILL_TILES2_MIN_PAGES": "0"},
+}
+
+
+@pytest.fixture(params=CHUNK_KERNELS, ids=str)
+def chunk_kernel(request):
+    """The library picks the decode kernel's multi-query mode or the LDS-shared prefill kernel, and the latter's
+    shape (halves, one or two 16-slot query tiles per wavefront), by the chunk's slots and the pages they walk; the
+    knobs force each for chunks of 64 slots and more, so that contexts a test can afford reach all of them."""
+    env = CHUNK_KERNELS[request.param]
+    saved = {k: os.environ.get(k) for k in env}
+    os.environ.update(env)
+    skv.flags.reload()
+    yield request.param
+    for k, v in saved.items():
+        os.environ.pop(k) if v is None else os.environ.__setitem__(k, v)
+    skv.flags.reload()
+
+
+@pytest.mark.parametrize("dims,start,chunk,window", [
+    ((32, 8, 128), 0, 64, 0),        # first chunk from an empty cache
+    ((32, 8, 128), 300, 200, 0),     # later chunk, crosses page boundaries
+    ((16, 2, 256), 1000, 37, 0),     # head_dim 256, ragged chunk
+    ((16, 2, 256), 5, 3, 0),         # speculative-verify sized chunk (split over the context)
+    ((4, 2, 16), 0, 50, 0),
+    ((6, 1, 40), 17, 33, 0),         # head_dim padded to 64, GQA 6
+    # 64 query slots and more: the LDS-shared kernel where the knobs force it, by shape the first two only
+    ((16, 2, 256), 5000, 600, 0),    # several workgroups per kv head, split context, ragged tail
+    ((32, 8, 128), 0, 1000, 0),      # from an empty cache: early tiles see few pages (empty splits)
+    ((6, 1, 40), 100, 100, 0),       # rows too short for 16-byte query loads, padded head_dim
+    ((8, 1, 32), 33, 77, 0),         # head_dim 32, odd page count
+    ((40, 1, 64), 10, 9, 0),         # GQA 40: 360 slots from 9 rows
+    ((8, 2, 512), 100, 70, 0),       # head_dim 512: four wavefronts, 64 slots per workgroup
+    ((4, 1, 512), 700, 300, 0),      # head_dim 512, several workgroups and splits
+    ((4, 1, 320), 0, 33, 0),         # padded to 512
+])
+def test_prefill_rows_match_per_row_oracle(state, chunk_kernel, dims, start, chunk, window):
+    """One launch == the reference's per-row loop (append, then cached_attention_one)."""
+    q_heads, kv_heads, head_dim = dims
+    kv_dim, q_dim = kv_heads * head_dim, q_heads * head_dim
+    rng = np.random.default_rng(start * 7 + chunk)
+    lay = oracle.layout(q_heads, kv_heads, head_dim, sliding_window=window)
+    cache = oracle.LayerKvCache("bf16r")
+    kv = state.full_attention_bf16(start + chunk, q_heads, kv_heads, head_dim)
+    kv.set_block_table(rng.permutation(kv.pages()).astype(np.int32))
+    if start:
+        k0 = rng.standard_normal((start, kv_dim), dtype=np.float32)
+        v0 = rng.standard_normal((start, kv_dim), dtype=np.float32)
+        kv.seed(k0, v0, start)
+        cache.append_batch(k0, v0, lay)
+    q = rng.standard_normal((chunk, q_dim), dtype=np.float32)
+    k = rng.standard_normal((chunk, kv_dim), dtype=np.float32)
+    v = rng.standard_normal((chunk, kv_dim), dtype=np.float32)
+    got = kv.prefill_rows(q, k, v)
+    want = oracle.cached_attention_prefill_rows(q, k, v, cache, lay)
+    assert kv.len() == len(cache) == start + chunk
+    assert np.abs(got - want).max() <= 1e-4, np.abs(got - want).max()
+    gk, gv = kv.read_rows_f32()
+    assert np.array_equal(gk, cache.keys()) and np.array_equal(gv, cache.values())
+
+
 @pytest.mark.parametrize("q_scale,k_scale,v_scale,tol", [
     # Scores in the hundreds and thousands: softmax is nearly one-hot and near-tied keys
     # trade weight on the last bits of their scores. Against an fp64 evaluation of the same
@@ -218,7 +285,7 @@ def test_normal_inputs_config0(state):
     (1e-3, 1e-3, 1e4, 8e-4),     # scores ~ 0: uniform weights over large values
     (8.0, 8.0, 1e-6, 8e-4),      # peaked weights over tiny values (no flush to zero in the product)
 ])
-def test_attention_extreme_magnitudes(state, q_scale, k_scale, v_scale, tol):
+def test_attention_extreme_magnitudes(state, chunk_kernel, q_scale, k_scale, v_scale, tol):
     """The online softmax (running maximum, base-2 exponent) and the hi/lo operand split must
     neither overflow nor lose the answer when scores are huge, vanish, or values are tiny:
     decode (split context) and a prefill chunk against the CPU path, error relative to the
@@ -247,72 +314,12 @@ def test_attention_extreme_magnitudes(state, q_scale, k_scale, v_scale, tol):
     assert np.abs(got - want).max() <= tol * v_scale, np.abs(got - want).max()
 
 
-# ---- chunked prefill over the cache (multi-query, matrix cores) ----------------------------
-@pytest.fixture(params=["by-shape", "one-tile", "two-tiles"])
-def tiles_per_wavefront(request):
-    """The LDS-shared prefill kernel holds one or two 16-slot query tiles per wavefront; the
-    library picks by head_dim and context length (two only for long contexts), the knob forces
-    either so that contexts a test can afford reach both instantiations."""
-    if request.param == "by-shape":
-        yield request.param
-        return
-    os.environ["SKV_PREFILL_TILES2_MIN_PAGES"] = "0" if request.param == "two-tiles" else "1000000000"
-    skv.flags.reload()
-    try:
-        yield request.param
-    finally:
-        os.environ.pop("SKV_PREFILL_TILES2_MIN_PAGES", None)
-        skv.flags.reload()
-
-
-@pytest.mark.parametrize("dims,start,chunk,window", [
-    ((32, 8, 128), 0, 64, 0),        # first chunk from an empty cache
-    ((32, 8, 128), 300, 200, 0),     # later chunk, crosses page boundaries
-    ((16, 2, 256), 1000, 37, 0),     # head_dim 256, ragged chunk
-    ((16, 2, 256), 5, 3, 0),         # speculative-verify sized chunk (split over the context)
-    ((4, 2, 16), 0, 50, 0),
-    ((6, 1, 40), 17, 33, 0),         # head_dim padded to 64, GQA 6
-    # chunks of 64 query slots and more take the kernel that shares K/V pages through LDS
-    ((16, 2, 256), 5000, 600, 0),    # several workgroups per kv head, split context, ragged tail
-    ((32, 8, 128), 0, 1000, 0),      # from an empty cache: early tiles see few pages (empty splits)
-    ((6, 1, 40), 100, 100, 0),       # rows too short for 16-byte query loads, padded head_dim
-    ((8, 1, 32), 33, 77, 0),         # head_dim 32, odd page count
-    ((40, 1, 64), 10, 9, 0),         # GQA 40: 360 slots from 9 rows
-    ((8, 2, 512), 100, 70, 0),       # head_dim 512: four wavefronts, 64 slots per workgroup
-    ((4, 1, 512), 700, 300, 0),      # head_dim 512, several workgroups and splits
-    ((4, 1, 320), 0, 33, 0),         # padded to 512
-])
-def test_prefill_rows_match_per_row_oracle(state, tiles_per_wavefront, dims, start, chunk, window):
-    """One launch == the reference's per-row loop (append, then cached_attention_one)."""
-    q_heads, kv_heads, head_dim = dims
-    kv_dim, q_dim = kv_heads * head_dim, q_heads * head_dim
-    rng = np.random.default_rng(start * 7 + chunk)
-    lay = oracle.layout(q_heads, kv_heads, head_dim, sliding_window=window)
-    cache = oracle.LayerKvCache("bf16r")
-    kv = state.full_attention_bf16(start + chunk, q_heads, kv_heads, head_dim)
-    kv.set_block_table(rng.permutation(kv.pages()).astype(np.int32))
-    if start:
-        k0 = rng.standard_normal((start, kv_dim), dtype=np.float32)
-        v0 = rng.standard_normal((start, kv_dim), dtype=np.float32)
-        kv.seed(k0, v0, start)
-        cache.append_batch(k0, v0, lay)
-    q = rng.standard_normal((chunk, q_dim), dtype=np.float32)
-    k = rng.standard_normal((chunk, kv_dim), dtype=np.float32)
-    v = rng.standard_normal((chunk, kv_dim), dtype=np.float32)
-    got = kv.prefill_rows(q, k, v)
-    want = oracle.cached_attention_prefill_rows(q, k, v, cache, lay)
-    assert kv.len() == len(cache) == start + chunk
-    assert np.abs(got - want).max() <= 1e-4, np.abs(got - want).max()
-    gk, gv = kv.read_rows_f32()
-    assert np.array_equal(gk, cache.keys()) and np.array_equal(gv, cache.values())
-
-
 @pytest.mark.parametrize("window,chunks,heads", [
     (32, [40, 7, 64], (8, 2)), (20, [5, 30, 3], (8, 2)),
-    (250, [7, 300, 20], (32, 2)),   # 7-row steps of 16 heads per group: the LDS-shared kernel on a ring
+    (250, [7, 300, 20], (32, 2)),   # 7 rows of 16 heads per group: whole chunks from scratch pages
     (100, [130, 50], (64, 4)),
 ])
-def test_prefill_rows_on_ring_layer(state, tiles_per_wavefront, window, chunks, heads):
+def test_prefill_rows_on_ring_layer(state, chunk_kernel, window, chunks, heads):
     """A ring that holds exactly its window advances row by row; results equal the oracle's
     sliding-window attention."""
     (q_heads, kv_heads), head_dim = heads, 64
@@ -331,8 +338,8 @@ def test_prefill_rows_on_ring_layer(state, tiles_per_wavefront, window, chunks, 
 
 
 def test_prefill_rows_on_ring_layer_head_dim_512(state):
-    """head_dim 512 on a ring layer: whole chunks in two phases around the append, on the
-    four-wavefront shape of the prefill kernel."""
+    """head_dim 512 on a ring layer, on the four-wavefront shape of the prefill kernel: a chunk that wraps the ring
+    is attended from scratch pages and enters it afterwards."""
     q_heads, kv_heads, head_dim, window = 4, 2, 512, 40
     kv_dim, q_dim = kv_heads * head_dim, q_heads * head_dim
     rng = np.random.default_rng(77)
@@ -469,13 +476,13 @@ def test_first_chunk_matches_causal_attention_divide_form(state, dims, chunk, el
     kv.close()
 
 
-def test_non_finite_row_in_a_chunk_stays_inside_its_launch_tile(state):
+def test_non_finite_row_in_a_chunk_stays_inside_its_launch_tile(state, chunk_kernel):
     """bf16 rounding of a finite f32 at or above 3.39e38 is an infinity (the reference's rounding
     has no special case, src/decode_resident/utils.rs:55-60), so a live row of a chunk can hold
     one. The reference's causal loop never reads a later row; a multi-query launch shares each
     V page among the query slots of a workgroup and masks by the workgroup's range, so there
-    0 x Inf can reach the contexts of earlier query rows of the SAME workgroup tile (at most
-    256 query slots). What is asserted: rows that attend the infinite row are non-finite in
+    0 x Inf can reach the contexts of earlier query rows of the SAME workgroup tile (16
+    query slots in the multi-query mode, 64 to 256 in the LDS-shared kernel). What is asserted: rows that attend the infinite row are non-finite in
     both; every row of an earlier workgroup tile equals the oracle's finite context; the
     infinity is stored as the reference stores it."""
     q_heads, kv_heads, head_dim = 16, 2, 64
@@ -503,8 +510,9 @@ def test_non_finite_row_in_a_chunk_stays_inside_its_launch_tile(state):
     gqa = q_heads // kv_heads
     cols = [h * head_dim + 5 for h in range(gqa)]           # kv head 0 serves query heads 0..gqa-1
     assert not np.isfinite(want[bad:][:, cols]).any() and not np.isfinite(got[bad:][:, cols]).any()
-    # a workgroup tile holds at most 256 query slots = 256 / gqa rows: rows before that are untouched
-    safe = bad - 256 // gqa
+    # rows before the workgroup's are untouched (by shape, this chunk takes the multi-query mode)
+    slots = {"by-shape": 16, "multi-query": 16, "halves": 64, "one-tile": 128, "two-tiles": 256}[chunk_kernel]
+    safe = bad - slots // gqa
     assert np.isfinite(got[:safe]).all()
     assert np.abs(got[:safe] - want[:safe]).max() <= 1e-4
     kv.close()

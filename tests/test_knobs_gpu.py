@@ -20,8 +20,9 @@ KNOBS = [
     {"SKV_FUSED_APPEND": "0"},
     {"SKV_Q_VEC": "0"},
     {"SKV_PREFILL_TILES": "0"},
-    {"SKV_PREFILL_TILES2_MIN_PAGES": "0", "SKV_PREFILL_WGS": "64"},
-    {"SKV_PREFILL_MAX_SPLITS": "1"},
+    {"SKV_PREFILL_TILES": "2"},
+    {"SKV_PREFILL_TILES": "2", "SKV_PREFILL_TILES2_MIN_PAGES": "0", "SKV_PREFILL_WGS": "64"},
+    {"SKV_PREFILL_TILES": "2", "SKV_PREFILL_MAX_SPLITS": "1"},
 ]
 
 
@@ -102,7 +103,8 @@ def test_batch_step_under_knobs(state, knobs, element, tol):
 
 
 @pytest.mark.parametrize("element,tol", [("bf16", 1e-4), ("f32", 2e-5)])
-@pytest.mark.parametrize("dims,start,chunk", [((16, 2, 256), 700, 90), ((32, 8, 128), 0, 130), ((6, 1, 40), 50, 5)])
+@pytest.mark.parametrize("dims,start,chunk", [((16, 2, 256), 700, 90), ((32, 8, 128), 0, 130), ((6, 1, 40), 50, 5),
+                                               ((16, 2, 256), 2700, 130)])  # past the line where bf16 chunks share pages by themselves
 def test_prefill_chunk_under_knobs(state, knobs, element, tol, dims, start, chunk):
     rng = np.random.default_rng(start + chunk)
     kv, cache, lay = _layer(state, element, dims, start, 0, start + chunk, rng)
