@@ -467,7 +467,7 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
     // dims of V at a time, the scores taken again for each VT.
     auto plain_slot = [&](int slot, float *dst, bool whole, long pidx) {
         // The arguments come again from the launch's memory: kept in registers for this place they spill
-        // around the loop above (this function costs 1500 rows through 36 layers of q32/kv8/hd128, 838 us, 1.2 % so
+        // around the loop above (this function costs 1500 rows through 4 layers of q32/kv8/hd128, 838 us, 1.2 % so
         // and 0.5 % as it is; 512 rows of q16/kv2/hd256 over 8192 rows nothing).
         const char *mem = (const char *)__builtin_amdgcn_kernarg_segment_ptr();
         asm("" : "+s"(mem)); // (not known to be what has been read before)

@@ -230,17 +230,23 @@ bool takes_tile_kernel(const Geom &g, size_t n_slots, size_t n_pages) {
 }
 
 // The same questions for f32 layers: the kernel that splits its factors into bf16 terms (head_dim up to
-// 256) or the one that streams pages into the f32 instruction, 16 slots a workgroup. Whole chunks, streaming /
-// one tile / halves, in us: q32/kv8/hd128, 32 rows over 2048, 8192 rows 28.9/37.5/32.6, 59.7/50.3/49.3; 128 rows
+// 256) or the one that streams pages into the f32 instruction, 16 slots a workgroup. The line is in (16 slots,
+// page) pairs as a chunk's rows walk them on the average, each up to its own position: half of the pages of a
+// first chunk (counted by all pages, 384 rows of q16/kv2/hd256 over 100 took the first kernel, 82.5 us, where
+// streaming takes 52.2, and 512 over none 58.8 where it takes 51.1). Over 953 chunks of 4 to 1024 rows over 0 to
+// 16000 in eleven geometries it is nowhere more than 14 % slower than streaming alone (60 % by all pages). Whole chunks,
+// streaming / one tile / halves, in us: q32/kv8/hd128, 32 rows over 2048, 8192 rows 28.9/37.5/32.6, 59.7/50.3/49.3; 128 rows
 // over 512, 2048: 28.7/39.0/31.9, 60.7/45.6/45.1; 512 rows over 0, 512, 2048, 8192: 44.0/45.5/39.4, 82.5/63.7/62.2,
 // 197/122/131, 656/354/405; q16/kv2/hd256, 64 rows over 2048, 8192: 54.2/60.7, 119/76.6; 256 rows over 0, 512, 2048:
 // 34.1/49.8, 58.7/57.9, 119/71.9; q8/kv2/hd64, 256 rows over 2048, 8192: 24.1/28.0/26.6, 54.6/45.3/45.3; 512 rows over
 // 512, 2048: 22.1/25.1/21.8, 37.5/32.8/31.2.
-bool takes_f32_chunk_kernel(const Geom &g, size_t n_slots, size_t n_pages) {
+bool takes_f32_chunk_kernel(const Geom &g, size_t n_queries, size_t n_pages) {
+    const size_t n_slots = n_queries * (size_t)g.gqa;
     if (f32_prefill_slots(g.P, false) == 0 || n_slots < 64 || tuning().prefill_tiles == 0) return false;
     if (tuning().prefill_tiles > 1) return true;
-    const size_t limit = g.P <= 64 ? 25000 : g.P == 128 ? 16000 : 11500;
-    return (n_slots + 15) / 16 * (size_t)g.kv_heads * n_pages >= limit;
+    const size_t limit = g.P <= 64 ? 26000 : g.P == 128 ? 16200 : 12200;
+    const size_t walked = n_pages > n_queries / 32 ? n_pages - n_queries / 32 : 1;
+    return (n_slots + 15) / 16 * (size_t)g.kv_heads * walked >= limit;
 }
 bool f32_halves(const Geom &g, size_t n_slots, size_t n_pages) {
     if (tuning().prefill_tiles2_min_pages >= 0) return false;
@@ -479,7 +485,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
             a.q_head_stride = pre->q_head_stride;
         }
         if (attn_scalar > 0.0f) a.qscale = (1.0f / std::sqrt(attn_scalar)) * 1.4426950408889634f;
-        if (n_queries > 1 && takes_f32_chunk_kernel(g, n_queries * (size_t)g.gqa, (size_t)a.n_pages)) {
+        if (n_queries > 1 && takes_f32_chunk_kernel(g, n_queries, (size_t)a.n_pages)) {
             const bool halves = f32_halves(g, n_queries * (size_t)g.gqa, (size_t)a.n_pages);
             // (choose_splits' number, which the split knobs of decode launches bound, is the larger one unless they do)
             a.splits = std::min(a.splits, chunk_splits(g, n_queries, (size_t)f32_prefill_slots(g.P, halves), (size_t)a.n_pages));
@@ -495,7 +501,10 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
         }
         if (n_queries > 1) {
             const size_t tiles = (n_queries * (size_t)g.gqa + 15) / 16 * (size_t)g.kv_heads;
-            const size_t want = std::max<size_t>(2 * decode_target_wgs() / tiles, 1);
+            size_t want = std::max<size_t>(2 * decode_target_wgs() / tiles, 1);
+            // a chunk that a ring holds without wrapping: whole eights of pages a split (130 rows of q16/kv8/hd256 on an empty
+            // ring: 22.3 us with one, 29.7 with two and a merge)
+            if (g.ring_rows > 0) want = std::min(want, std::max<size_t>((size_t)a.n_pages / 8, 1));
             a.splits = (int)std::min<size_t>((size_t)a.splits, want);
             a.splits_total = a.splits;
             if (a.splits > 1) {
