@@ -274,7 +274,7 @@ int32_t skv_decode_step_static_device(skv_layer *layer, skv_stream stream, const
  * the layer's sliding window: cached_attention_prefill_rows
  * (src/decoder/attention_ops.rs:976-1017) as one launch on the matrix cores instead of
  * the reference's per-row loop (src/decode_resident/layers.rs:1113-1118). out_dev is
- * [n_rows, q_dim] f32. */
+ * [n_rows, q_dim] f32; up to 4096 rows a call it may lie over k_dev or v_dev. */
 int32_t skv_prefill_chunk_device(skv_layer *layer, skv_stream stream, const float *q_dev,
                                  const void *k_dev, const void *v_dev, size_t n_rows,
                                  float *out_dev);
