@@ -477,6 +477,7 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
         asm("" : "+s"(mem)); // (not known to be what has been read before)
         const DecodeArgs &a = *reinterpret_cast<const DecodeArgs *>(mem);
         const ChunkPages &c = *reinterpret_cast<const ChunkPages *>(mem + sizeof(DecodeArgs));
+        static_assert(sizeof(DecodeArgs) % alignof(ChunkPages) == 0, "the launch's memory holds the two side by side");
         const Geom &g = a.g;
         const int G = g.gqa;
         auto limit_of = [&](int slot) { return a.q_pos0 + slot / G; };
