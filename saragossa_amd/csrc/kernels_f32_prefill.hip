@@ -222,7 +222,13 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
         }
     }
 
-    float4_t o[TILES][NT];
+    // Up to head_dim 128 the leading products and the other five, 2^-8 of them, have sums of their own: an
+    // addition cuts off what is far below its sum. Errors against 64 bits, sums apart / together / the kernel of f32
+    // products: 512 rows of q32/kv8/hd128 over 1536 3.1e-7/5.3e-7/4.5e-7, over none 2.0e-7/2.4e-7/2.1e-7, of q8/kv2/hd64
+    // over 2000 2.1e-7/3.3e-7/3.6e-7. At 256, where there are no registers for it (together / f32 products):
+    // q16/kv2 over 4000 6.4e-7/6.8e-7, q16/kv8 on a ring of 1024 4.4e-7/4.0e-7.
+    constexpr bool APART = P <= 128;
+    float4_t o[TILES][NT], o_low[TILES][APART ? NT : 1];
     // The base of a slot's softmax lags up to 8 behind its largest score, so weights reach 2^8 and the
     // accumulators start close to zero, where their sums are most exact (512 rows of q32/kv8/hd128 over 1536: errors of 5.3e-7 against 64
     // bits, 1.3e-6 with the base 8 ahead). Sums of values near the top of the range that pass
@@ -233,6 +239,8 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
     for (int t = 0; t < TILES; ++t) {
 #pragma unroll
         for (int u = 0; u < NT; ++u) o[t][u] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < (APART ? NT : 0); ++u) o_low[t][u] = float4_t{0.f, 0.f, 0.f, 0.f};
         m_base[t] = 0.0f;
         neg_m[t] = float4_t{0.f, 0.f, 0.f, 0.f};
         thr[t] = -INFINITY;
@@ -290,6 +298,8 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
                 if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
 #pragma unroll
                     for (int u = 0; u < NT; ++u) o[t][u] *= alpha;
+#pragma unroll
+                    for (int u = 0; u < (APART ? NT : 0); ++u) o_low[t][u] *= alpha;
                 }
             }
         }
@@ -389,8 +399,10 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
                 __builtin_amdgcn_sched_barrier(0);
                 const bf16x8_t vv = __builtin_bit_cast(bf16x8_t, op[at][TERMS[b].l]);
 #pragma unroll
-                for (int t = 0; t < TILES; ++t)
-                    o[t][at] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv, p[t][TERMS[b].r], o[t][at], 0, 0, 0);
+                for (int t = 0; t < TILES; ++t) {
+                    float4_t &sum = APART && b > 0 ? o_low[t][APART ? at : 0] : o[t][at];
+                    sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv, p[t][TERMS[b].r], sum, 0, 0, 0);
+                }
                 constexpr int S_FROM = SHARE ? BEATS / 2 : 0;
                 const int beat = at * 6 + b, ss = done_before(beat, SPLIT_STEPS, S_FROM, BEATS);
                 if (done_before(beat + 1, SPLIT_STEPS, S_FROM, BEATS) > ss) split_step(ss, false);
@@ -433,6 +445,14 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
         __syncthreads();
     }
 
+    if constexpr (APART) {
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+#pragma unroll
+            for (int u = 0; u < NT; ++u) o[t][u] += o_low[t][u];
+        }
+    }
+
     // ---- the second half's states join the first's through LDS -----------------------------
     if constexpr (HALVES > 1) {
         static_assert(HALVES == 2 && TW * TILES * (NT + 1) * 64 <= 2 * V_AT, "the second half's states fit the page buffers");
@@ -469,14 +489,20 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
     // f32. What is NaN then stays NaN. Lane (n, j) holds key n's dims 4j .. 4j+3 of every 16, then dim n's keys
     // 4j .. 4j+3. Rare and not fast: a few registers, so that the kernel above keeps its own, and VT tiles of 16
     // dims of V at a time, the scores taken again for each VT.
+    const DecodeArgs &args = a;
+    const ChunkPages &pages = c;
     auto plain_slot = [&](int slot, float *dst, bool whole, long pidx) {
-        // The arguments come again from the launch's memory: kept in registers for this place they spill
-        // around the loop above (this function costs 1500 rows through 4 layers of q32/kv8/hd128, 838 us, 1.2 % so
-        // and 0.5 % as it is; 512 rows of q16/kv2/hd256 over 8192 rows nothing).
-        const char *mem = (const char *)__builtin_amdgcn_kernarg_segment_ptr();
-        asm("" : "+s"(mem)); // (not known to be what has been read before)
+        // Up to head_dim 128 the arguments come again from the launch's memory: kept in registers for this place
+        // they spill around the loop above (this function costs 1500 rows through 4 layers of q32/kv8/hd128,
+        // 838 us, 1.2 % so and 0.5 % as it is). At 256, where reading them again makes the compiler spill inside the
+        // loop, they are kept (512 rows of q16/kv2/hd256 over 8192 rows: 0.5 %, and 2.7 % with them read again).
+        const char *mem = reinterpret_cast<const char *>(&args);
+        if constexpr (P <= 128) {
+            mem = (const char *)__builtin_amdgcn_kernarg_segment_ptr();
+            asm("" : "+s"(mem)); // (not known to be what has been read before)
+        }
         const DecodeArgs &a = *reinterpret_cast<const DecodeArgs *>(mem);
-        const ChunkPages &c = *reinterpret_cast<const ChunkPages *>(mem + sizeof(DecodeArgs));
+        const ChunkPages &c = P <= 128 ? *reinterpret_cast<const ChunkPages *>(mem + sizeof(DecodeArgs)) : pages;
         static_assert(sizeof(DecodeArgs) % alignof(ChunkPages) == 0, "the launch's memory holds the two side by side");
         const Geom &g = a.g;
         const int G = g.gqa;
