@@ -8,6 +8,7 @@
 namespace skv {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
 typedef __attribute__((ext_vector_type(4))) short short4_t;
 typedef __attribute__((ext_vector_type(4))) float float4_t;
 typedef __attribute__((ext_vector_type(4))) unsigned int u4;
@@ -36,7 +37,8 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // in registers as bf16 hi + lo halves (pre-scaled by log2(e)/sqrt(head_dim)). Per pair:
 //   window 1: S^T(p+1) = K . Q^T of the NEXT pair (16x16x32 products over the head dims) with the
 //             exponentials and the hi + lo split of this pair's probabilities between the products;
-//   window 2: O^T += V^T . P^T(p), 16x16x32 products over the pair's 32 keys.
+//   window 2: O^T += V^T . P^T(p), 16x16x32 products over the pair's 32 keys, with the next operands' halves put side by
+//             side and the search for the largest of the next pair's scores between the products.
 // A product occupies the matrix pipe for 16 cycles and its wavefront for 4; the vector work of
 // the softmax therefore costs nothing where it is issued between products that do not depend on
 // it, and a pair's softmax never depends on the next pair's scores. (With the softmax between the
@@ -59,20 +61,32 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // the other and copied through registers: q32/kv8/hd128 over 0, 1536, 4700, 16384 rows 34.5 -> 21.7,
 // 57.2 -> 41.1, 106 -> 86.5, 256 -> 225; q16/kv2/hd256 40.0 -> 24.3, 55.7 -> 50.5, 97.9 -> 89.0, 247 -> 225 (where
 // the matrix pipes alone need 130).
+// A wavefront issues an instruction in four to five cycles, so every one beside the products counts: with a tile per
+// wavefront to copy, the moves that put operands together and the search for the maximum between products, and the second
+// terms of the probabilities by a dot product, chunks of 512 rows on layers that are in no cache went, in us, for q32/kv8/hd128
+// over 4700, 16384 from 87.7 to 83.2, 223.5 to 220.5; for q16/kv8/hd256 on a ring of 1024 rows from 46.1 to 44.4. (Three
+// wavefronts per SIMD, twelve in thirds at 154 registers, were no faster than two; two tiles per wavefront at
+// head_dim 256, four wavefronts at 400 registers, 11 to 40 % slower.)
 // ------------------------------------------------------------------------------------
 
 // 64 x 16 bytes straight from memory to LDS, lane l's to lds + 16 l (`lds` the same in every lane), no
 // register in between. In assembly because the compiler, which cannot tell the two halves of the
 // double buffer apart, would make every LDS read wait for a copy it knows of; the kernel
 // waits for all of them itself (copies_landed) in front of the barrier that hands the buffer over.
-__device__ __forceinline__ void copy_to_lds(const void *base, uint32_t lane_offset, uint32_t lds) {
+// `kib`: a constant, that many KiB further at both ends (an immediate of the instruction).
+__device__ __forceinline__ void copy_to_lds(const void *base, uint32_t lane_offset, uint32_t lds, int kib = 0) {
     // (both are the same in every lane: said so, whatever the compiler can prove)
     const uint64_t b = reinterpret_cast<uint64_t>(base);
     const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
     const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
     const uint64_t from = ((uint64_t)hi << 32) | lo;
     const uint32_t to = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds);
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(lane_offset), "s"(from) : "m0");
+    switch (kib) {
+    case 0: asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(lane_offset), "s"(from) : "m0"); break;
+    case 1: asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 offset:1024" ::"s"(to), "v"(lane_offset), "s"(from) : "m0"); break;
+    case 2: asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 offset:2048" ::"s"(to), "v"(lane_offset), "s"(from) : "m0"); break;
+    default: asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 offset:3072" ::"s"(to), "v"(lane_offset), "s"(from) : "m0"); break;
+    }
 }
 __device__ __forceinline__ void copies_landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
@@ -90,10 +104,12 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
     constexpr int THREADS = WAVES * 64;
     constexpr int KK = P / 32;
     constexpr int NT = P / 16;
+    // Vector work is held in its place between the products; a wavefront alone on its SIMD (head_dim above 256) does better
+    // where the compiler places it (256 rows of q8/kv2/hd512 over 4096: 61.0 us against 66.0)
+    constexpr bool PINNED = P <= 256;
     constexpr int TILE_U4 = KK * 64;                           // 16-byte units of one K (or V) tile
     constexpr int GP = 2 * HALVES;                             // pages of a group: a pair for each half
-    constexpr int CU = SP * GP * TILE_U4 / THREADS;            // units of K, and of V, a thread copies per step
-    static_assert(SP * GP * TILE_U4 % THREADS == 0 && TILE_U4 % 64 == 0, "a wavefront copies whole KiB of one page");
+    static_assert(TILE_U4 % 64 == 0, "a wavefront copies whole KiB of one page");
     extern __shared__ __attribute__((aligned(16))) u4 kv_lds[]; // [2 buffers][K of SP pairs | V of SP pairs]
     constexpr int HALF_U4 = SP * GP * TILE_U4;
     constexpr int BUF_U4 = 2 * HALF_U4;
@@ -150,28 +166,38 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
     };
     ask_ids(0);
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)kv_lds;
-    const uint32_t lane_at = (uint32_t)(tid & (TILE_U4 - 1)) * 16; // where in its page a lane's units lie, in bytes
-    // unit u of a step's K (v = false) or V into the buffer half at unit `dst` of LDS; it0: see tile_of
-    auto copy_unit = [&](int u, bool v, int it0, int dst) __attribute__((always_inline)) {
-        const int i0 = wave * 64 + u * THREADS; // the wavefront's first unit
-        const int pg = i0 / TILE_U4;
-        const uint32_t off = THREADS % TILE_U4 == 0 ? lane_at : lane_at + (uint32_t)((u * THREADS) & (TILE_U4 - 1)) * 16;
-        copy_to_lds(tile_of(it0, v ? pg : pg + GP, v), off, lds0 + (uint32_t)(dst + i0) * 16);
+    const uint32_t lane_at = (uint32_t)lane * 16;
+    // A wavefront copies whole tiles, TPW of a step's K and then V tiles, a KiB an instruction: one place in the page
+    // list and one address for four instructions (with the KiBs of a step dealt out to the wavefronts in turn, each had
+    // a place, an address and an LDS address of its own: nine instructions a copy, seventy of a step's four hundred).
+    constexpr int TPW = 2 * SP * GP / WAVES, CPT = TILE_U4 / 64;
+    static_assert(2 * SP * GP % WAVES == 0, "a wavefront copies whole tiles");
+    const u4 *from[TPW];
+    auto find_tiles = [&](int it0) __attribute__((always_inline)) { // it0: see tile_of; the step's first V page
+#pragma unroll
+        for (int i = 0; i < TPW; ++i) {
+            const int ti = wave * TPW + i;
+            const bool v = ti >= SP * GP;
+            from[i] = tile_of(it0, v ? ti - SP * GP : ti + GP, v);
+        }
+    };
+    // KiB i of the wavefront's copies, to the buffer half at unit `dst` of LDS
+    auto copy_kib = [&](int i, int dst) __attribute__((always_inline)) {
+        const int quad = i % CPT / 4 * 256;
+        copy_to_lds(from[i / CPT] + quad, lane_at, lds0 + (uint32_t)(dst + (wave * TPW + i / CPT) * TILE_U4 + quad) * 16, i % CPT % 4);
     };
     // The copies of a step are spread over the K-steps of the first half of its products (512 rows of
     // q16/kv2/hd256 over 16384 rows: 243 us against 265 with all of them in front of one window; 223
     // with copies straight to LDS instead of through registers, which took stores besides).
     constexpr int COPY_SPAN = KK * SP;
     auto copy_slot = [&](int slot, int step) __attribute__((always_inline)) {
-        const int it0 = (step + 1) * SP * GP; // first page of the V copy, a group before the K copy's
-        const int dst = ((step + 1) & 1) * BUF_U4;
+        if (slot == 0) {
+            find_tiles((step + 1) * SP * GP); // first page of the V copy, a group before the K copy's
+            ask_ids((step + 2) * SP * GP);
+        }
 #pragma unroll
-        for (int i = 0; i < 2 * CU; ++i)
-            if (i * COPY_SPAN / (2 * CU) == slot) {
-                if (i < CU) copy_unit(i, false, it0, dst);
-                else copy_unit(i - CU, true, it0, dst + HALF_U4);
-                if (i == 2 * CU - 1) ask_ids((step + 2) * SP * GP);
-            }
+        for (int i = 0; i < TPW * CPT; ++i)
+            if (i * COPY_SPAN / (TPW * CPT) == slot) copy_kib(i, ((step + 1) & 1) * BUF_U4);
     };
     // V rows of the pages from first_page on that nobody attends, cleared in the buffer half at `v`
     const Inner wg_in = inner_entries<RING>(c, pb0, pb1, wg_ws_lo, wg_lim_hi);
@@ -198,15 +224,11 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
     for (int u = 0; u < (GP * TILE_U4 + THREADS - 1) / THREADS; ++u) {
         const int i0 = wave * 64 + u * THREADS;
         if (GP * TILE_U4 % THREADS == 0 || i0 < GP * TILE_U4)
-            copy_to_lds(tile_of(0, i0 / TILE_U4, false),
-                        THREADS % TILE_U4 == 0 ? lane_at : lane_at + (uint32_t)((u * THREADS) & (TILE_U4 - 1)) * 16,
-                        lds0 + (uint32_t)(BUF_U4 + i0) * 16);
+            copy_to_lds(tile_of(0, i0 / TILE_U4, false) + (i0 & (TILE_U4 - 1)), lane_at, lds0 + (uint32_t)(BUF_U4 + i0) * 16);
     }
+    find_tiles(0);
 #pragma unroll
-    for (int u = 0; u < CU; ++u) {
-        copy_unit(u, false, 0, 0);
-        copy_unit(u, true, 0, HALF_U4);
-    }
+    for (int i = 0; i < TPW * CPT; ++i) copy_kib(i, 0);
     // ---- this wavefront's query tiles ------------------------------------------------
     int my_limit[TILES], my_ws[TILES];
     int t_ws_hi[TILES], t_lim_lo[TILES]; // per tile extremes
@@ -270,7 +292,11 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
 
     float4_t o[TILES][NT];
     float4_t neg_m[TILES];             // -m in all four: what the score accumulators start from
-    float m_base[TILES], thr[TILES];   // base of the slot; a score above base + thr moves it: 0, or -inf (no key yet)
+    // base of the slot; a score whose bits reach thr_i moves it: SEEN (any above the base), or, for a slot without a key
+    // so far, UNSEEN (whatever it is)
+    constexpr int UNSEEN = INT32_MIN, SEEN = 1;
+    float m_base[TILES];
+    int thr_i[TILES];
     float l_run[TILES];                // this lane's share of the slot's sum
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
@@ -278,7 +304,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
         for (int u = 0; u < NT; ++u) o[t][u] = float4_t{0.f, 0.f, 0.f, 0.f};
         m_base[t] = 0.0f;
         neg_m[t] = float4_t{0.f, 0.f, 0.f, 0.f};
-        thr[t] = -INFINITY;
+        thr_i[t] = UNSEEN;
         l_run[t] = 0.0f;
     }
 
@@ -286,7 +312,9 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
     float4_t sa[TILES], sb[TILES];
     // probabilities of the pair being accumulated, as two bf16 terms
     bf16x8_t ph[TILES], pl[TILES];
-    constexpr int DEPTH = KK < 2 || TILES > 1 ? 1 : 2; // K-steps an operand is asked for ahead of its products
+    // K-steps an operand is asked for ahead of its products (of V's a step more, which the moves take)
+    constexpr int DEPTH = KK < 2 || TILES > 1 ? 1 : 2;
+    constexpr int DEPTH_V = KK < 4 || P > 256 ? DEPTH : DEPTH + 1;
 
     // the half's pairs are the page pairs HALVES * group + half.
     // pairs whose keys every slot of the wavefront attends: [in0, in1) and, of new pages, [in2, in3)
@@ -304,34 +332,50 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
         in2 = (r.n0 - pb0 + 1) >> 1;
         in3 = (r.n1 - pb0) >> 1;
     }
-    // scores of keys outside the slot's range become -inf; then, where a score passes the base by more
-    // than thr, the wavefront's bases move
-    auto settle = [&](int pair) __attribute__((always_inline)) {
+    // scores of keys outside the slot's range become -inf
+    auto mask = [&](int pair) __attribute__((always_inline)) {
+        if ((pair >= in0 && pair < in1) || (RING && pair >= in2 && pair < in3)) return; // uniform
+        const int it = 2 * pair;
+        const int ea = entry(it), eb = entry(it + 1);
+        const int pos_a = entry_pos<RING>(c, ea), pos_b = entry_pos<RING>(c, eb);
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
-            if (!((pair >= in0 && pair < in1) || (RING && pair >= in2 && pair < in3))) { // uniform
-                const int it = 2 * pair;
-                const int ea = entry(it), eb = entry(it + 1);
-                const int pos_a = entry_pos<RING>(c, ea), pos_b = entry_pos<RING>(c, eb);
-                const int lo_a = max(my_ws[t], entry_lo<RING>(c, ea)), hi_a = min(my_limit[t], entry_hi<RING>(c, ea));
-                const int lo_b = max(my_ws[t], entry_lo<RING>(c, eb)), hi_b = min(my_limit[t], entry_hi<RING>(c, eb));
+            const int lo_a = max(my_ws[t], entry_lo<RING>(c, ea)), hi_a = min(my_limit[t], entry_hi<RING>(c, ea));
+            const int lo_b = max(my_ws[t], entry_lo<RING>(c, eb)), hi_b = min(my_limit[t], entry_hi<RING>(c, eb));
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int pa = pos_a + j * 4 + e, pb = pos_b + j * 4 + e;
-                    sa[t][e] = it < n_it && pa >= lo_a && pa <= hi_a ? sa[t][e] : -INFINITY;
-                    sb[t][e] = it + 1 < n_it && pb >= lo_b && pb <= hi_b ? sb[t][e] : -INFINITY;
-                }
+            for (int e = 0; e < 4; ++e) {
+                const int pa = pos_a + j * 4 + e, pb = pos_b + j * 4 + e;
+                sa[t][e] = it < n_it && pa >= lo_a && pa <= hi_a ? sa[t][e] : -INFINITY;
+                sb[t][e] = it + 1 < n_it && pb >= lo_b && pb <= hi_b ? sb[t][e] : -INFINITY;
             }
-            const float mx = fmaxf(fmaxf(fmaxf(sa[t][0], sa[t][1]), fmaxf(sa[t][2], sa[t][3])),
-                                   fmaxf(fmaxf(sb[t][0], sb[t][1]), fmaxf(sb[t][2], sb[t][3])));
-            if (__builtin_amdgcn_ballot_w64(mx > thr[t])) {
+        }
+    };
+    // Whether a score is above its slot's base is whether the largest of the scores' bits, as integers, is positive (a
+    // positive float is a positive integer, and every other one is zero or negative): v_max3_i32, where maxima of
+    // floats cost an instruction more per operand, to quiet what is no number.
+    int mi[TILES];
+    auto top_step = [&](int q) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            const float4_t &x = q < 2 ? sa[t] : sb[t];
+            const int m = max(__float_as_int(x[q & 1 ? 2 : 0]), __float_as_int(x[q & 1 ? 3 : 1]));
+            mi[t] = q == 0 ? m : max(m, mi[t]);
+        }
+    };
+    // where a score passes the base, the wavefront's bases move
+    auto settle = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            if (__builtin_amdgcn_ballot_w64(mi[t] >= thr_i[t])) {
+                const float mx = fmaxf(fmaxf(fmaxf(sa[t][0], sa[t][1]), fmaxf(sa[t][2], sa[t][3])),
+                                       fmaxf(fmaxf(sb[t][0], sb[t][1]), fmaxf(sb[t][2], sb[t][3])));
                 const float top = rows_max(mx); // of the slot, relative to its base
-                const bool unseen = thr[t] == -INFINITY;
-                const float d = top > thr[t] ? top + 4.0f : 0.0f;
+                const bool unseen = thr_i[t] < 0;
+                const float d = top > (unseen ? -INFINITY : 0.0f) ? top + 4.0f : 0.0f;
                 const float alpha = unseen ? 1.0f : fast_exp2(-d);
                 m_base[t] += d;
                 neg_m[t] = float4_t{-m_base[t], -m_base[t], -m_base[t], -m_base[t]};
-                thr[t] = unseen && top == -INFINITY ? -INFINITY : 0.0f;
+                thr_i[t] = unseen && top == -INFINITY ? UNSEEN : SEEN;
                 l_run[t] *= alpha;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
@@ -349,8 +393,11 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
     // probabilities of the settled scores, in nine small steps per tile so that they can stand
     // between products: step q takes the exponential of score q and splits that of score q - 1
     float pr_[TILES];                  // exponential of the last step
-    float rest[TILES][2];
-    uint32_t pbits[TILES][2], hi4[TILES][4], lo4[TILES][4];
+    float pr2[TILES][2];
+    // (in registers: as an immediate of the instruction the first one is taken for the second)
+    uint32_t minus_first = 0x0000bf80u, minus_second = 0xbf800000u;
+    asm("" : "+s"(minus_first), "+s"(minus_second));
+    uint32_t hi4[TILES][4], lo4[TILES][4];
     auto prob_step = [&](int q) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
@@ -359,14 +406,18 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
             if (q > 0) {
                 const int e = q - 1;
                 l_run[t] += prev;
-                pbits[t][e & 1] = __float_as_uint(prev);
+                pr2[t][e & 1] = prev;
                 // p = hi + lo with hi the upper 16 bits of p (cut off) and lo the exact remainder rounded to
                 // nearest: 2^-17 relative, of either sign (512 rows of q32/kv8/hd128 over 1536: errors of 5.4e-6
                 // against 64 bits; lo cut off as well, always too small, 9.9e-6)
-                rest[t][e & 1] = prev - __uint_as_float(pbits[t][e & 1] & 0xffff0000u);
+                // (a difference is a product of the pair of high terms with -1 and 0, exact, one instruction)
                 if (e & 1) {
-                    hi4[t][e >> 1] = __builtin_amdgcn_perm(pbits[t][1], pbits[t][0], 0x07060302u);
-                    lo4[t][e >> 1] = bf16_pair(rest[t][0], rest[t][1]);
+                    const uint32_t hi = __builtin_amdgcn_perm(__float_as_uint(prev), __float_as_uint(pr2[t][0]), 0x07060302u);
+                    hi4[t][e >> 1] = hi;
+                    const bf16x2_t h2 = __builtin_bit_cast(bf16x2_t, hi);
+                    lo4[t][e >> 1] = bf16_pair(__builtin_amdgcn_fdot2_f32_bf16(h2, __builtin_bit_cast(bf16x2_t, minus_first), pr2[t][0], false),
+                                               __builtin_amdgcn_fdot2_f32_bf16(h2, __builtin_bit_cast(bf16x2_t, minus_second), prev, false));
+                    if (PINNED) asm volatile("" : "+v"(hi4[t][e >> 1]), "+v"(lo4[t][e >> 1])); // (here, between the products, not behind them)
                 }
             }
         }
@@ -399,7 +450,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
         for (int kk = 0; kk < KK; ++kk) {
             if (kk + DEPTH < KK) ask_k(kt, kk + DEPTH);
             copies(kk);
-            if (PROBS && kk + DEPTH >= KK) ask_v(vt, kk + DEPTH - KK);
+            if (PROBS && kk + DEPTH_V >= KK) ask_v(vt, kk + DEPTH_V - KK);
             const bf16x8_t ka = __builtin_bit_cast(bf16x8_t, ra[kk]);
             const bf16x8_t kb = __builtin_bit_cast(bf16x8_t, rb[kk]);
 #pragma unroll
@@ -425,29 +476,60 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
         if (PROBS) probs_done();
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
+            if (PROBS && PINNED) asm volatile("" : "+v"(l_run[t])); // (the sum's additions stay between the products)
             sa[t] = na[t];
             sb[t] = nb[t];
         }
     };
-    // window 2: O^T += V^T . P^T over the 32 keys of the pair
+    // A lane's unit holds four keys of dims n and n + 16: both pages' halves side by side are the 32-key operands of
+    // the two dim tiles.
+    auto v_first = [&](int kk, bf16x8_t &v) __attribute__((always_inline)) {
+        u4 x = {rva[kk].x, rva[kk].y, rvb[kk].x, rvb[kk].y};
+        if (PINNED) asm volatile("" : "+v"(x)); // (put together here, not in front of the product that takes it)
+        v = __builtin_bit_cast(bf16x8_t, x);
+    };
+    auto v_second = [&](int kk, bf16x8_t &v) __attribute__((always_inline)) {
+        u4 x = {rva[kk].z, rva[kk].w, rvb[kk].z, rvb[kk].w};
+        if (PINNED) asm volatile("" : "+v"(x));
+        v = __builtin_bit_cast(bf16x8_t, x);
+    };
+    // window 2: O^T += V^T . P^T over the 32 keys of the pair; between the products the next operands are put
+    // together and the largest of the settled pair's scores is found
     auto accumulate = [&](const u4 *vt, auto copies) __attribute__((always_inline)) {
+        auto fence = [&]() __attribute__((always_inline)) {
+            if (PINNED) __builtin_amdgcn_sched_barrier(0);
+        };
+        bf16x8_t v0, v1, w0, w1;
+        v_first(0, v0);
+        v_second(0, v1);
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) {
-            if (kk + DEPTH < KK) ask_v(vt, kk + DEPTH);
+            if (kk + DEPTH_V < KK) ask_v(vt, kk + DEPTH_V);
             copies(kk);
             __builtin_amdgcn_sched_barrier(0);
-            // a lane's unit holds four keys of dims n and n + 16: both pages' halves side by side are the
-            // 32-key operands of the two dim tiles
-            const bf16x8_t v0 = __builtin_bit_cast(bf16x8_t, u4{rva[kk].x, rva[kk].y, rvb[kk].x, rvb[kk].y});
-            const bf16x8_t v1 = __builtin_bit_cast(bf16x8_t, u4{rva[kk].z, rva[kk].w, rvb[kk].z, rvb[kk].w});
 #pragma unroll
-            for (int t = 0; t < TILES; ++t) {
-                o[t][2 * kk] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v0, ph[t], o[t][2 * kk], 0, 0, 0);
-                o[t][2 * kk + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v1, ph[t], o[t][2 * kk + 1], 0, 0, 0);
-                o[t][2 * kk] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v0, pl[t], o[t][2 * kk], 0, 0, 0);
-                o[t][2 * kk + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v1, pl[t], o[t][2 * kk + 1], 0, 0, 0);
+            for (int h = 0; h < 2; ++h) {
+#pragma unroll
+                for (int t = 0; t < TILES; ++t) {
+                    const bf16x8_t pt = h ? pl[t] : ph[t];
+                    fence();
+                    o[t][2 * kk] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v0, pt, o[t][2 * kk], 0, 0, 0);
+                    fence();
+                    if (h == 0 && t == 0 && kk + 1 < KK) v_first(kk + 1, w0);
+                    if (h == 1 && t == 0) {
+#pragma unroll
+                        for (int q = 0; q < 4; ++q)
+                            if (PINNED && q * KK / 4 == kk) top_step(q);
+                    }
+                    fence();
+                    o[t][2 * kk + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v1, pt, o[t][2 * kk + 1], 0, 0, 0);
+                    fence();
+                    if (h == 0 && t == 0 && kk + 1 < KK) v_second(kk + 1, w1);
+                }
             }
             __builtin_amdgcn_sched_barrier(0);
+            v0 = w0;
+            v1 = w1;
         }
     };
 
@@ -459,7 +541,10 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
 #pragma unroll
     for (int kk = 0; kk < DEPTH; ++kk) ask_k(kv_lds + BUF_U4 + half * 2 * TILE_U4, kk);
     scores(kv_lds + BUF_U4 + half * 2 * TILE_U4, nullptr, std::false_type{}, [](int) {});
-    settle(half);
+    mask(half);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) top_step(q);
+    settle();
     __syncthreads(); // the second buffer is free
 
     for (int step = 0; step < n_steps; ++step) {
@@ -474,8 +559,14 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
             for (int kk = 0; kk < DEPTH; ++kk) ask_k(kt, kk);
             // (after the last step the copies re-read its pages into the idle buffer)
             scores(kt, vt, std::true_type{}, [&](int kk) __attribute__((always_inline)) { copy_slot(2 * KK * pp + kk, step); });
+            if (PINNED) mask((group + 1) * HALVES + half);
             accumulate(vt, [&](int kk) __attribute__((always_inline)) { copy_slot(2 * KK * pp + KK + kk, step); });
-            settle((group + 1) * HALVES + half);
+            if (!PINNED) {
+                mask((group + 1) * HALVES + half);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) top_step(q);
+            }
+            settle();
         }
         copies_landed();
         __syncthreads();
@@ -493,7 +584,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
                 float4_t *dst = xo + (half - 1) * STATES + t * (NT + 1) * 64;
 #pragma unroll
                 for (int u = 0; u < NT; ++u) dst[u * 64] = o[t][u];
-                dst[NT * 64] = float4_t{thr[t] == -INFINITY ? -INFINITY : m_base[t], l_run[t], 0.f, 0.f};
+                dst[NT * 64] = float4_t{thr_i[t] < 0 ? -INFINITY : m_base[t], l_run[t], 0.f, 0.f};
             }
         }
         __syncthreads();
@@ -504,7 +595,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
             for (int h = 0; h < HALVES - 1; ++h) {
                 const float4_t *src = xo + h * STATES + t * (NT + 1) * 64;
                 const float4_t ml = src[NT * 64];
-                const float m0 = thr[t] == -INFINITY ? -INFINITY : m_base[t], m1 = ml[0];
+                const float m0 = thr_i[t] < 0 ? -INFINITY : m_base[t], m1 = ml[0];
                 const float mx = fmaxf(m0, m1);
                 const float m_safe = mx == -INFINITY ? 0.0f : mx;
                 const float w0 = fast_exp2(m0 - m_safe), w1 = fast_exp2(m1 - m_safe);
@@ -512,7 +603,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
 #pragma unroll
                 for (int u = 0; u < NT; ++u) o[t][u] = o[t][u] * w0 + src[u * 64] * w1;
                 m_base[t] = m_safe;
-                thr[t] = mx == -INFINITY ? -INFINITY : 0.0f;
+                thr_i[t] = mx == -INFINITY ? UNSEEN : SEEN;
             }
         }
     }
@@ -532,7 +623,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
             const long pidx = ((long)kvh * a.splits_total + a.split_base + split) * n_slots + slot;
             dst = a.part_o + pidx * g.head_dim;
             if (j == 0) {
-                a.part_m[pidx] = thr[t] == -INFINITY ? -INFINITY : m_base[t];
+                a.part_m[pidx] = thr_i[t] < 0 ? -INFINITY : m_base[t];
                 a.part_l[pidx] = l;
             }
         }
