@@ -218,22 +218,12 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
         __syncthreads();
     };
 
-    // the first group's K (into the second buffer) and the first step's pages are on their way while
-    // the queries are prepared
-#pragma unroll
-    for (int u = 0; u < (GP * TILE_U4 + THREADS - 1) / THREADS; ++u) {
-        const int i0 = wave * 64 + u * THREADS;
-        if (GP * TILE_U4 % THREADS == 0 || i0 < GP * TILE_U4)
-            copy_to_lds(tile_of(0, i0 / TILE_U4, false) + (i0 & (TILE_U4 - 1)), lane_at, lds0 + (uint32_t)(BUF_U4 + i0) * 16);
-    }
-    find_tiles(0);
-#pragma unroll
-    for (int i = 0; i < TPW * CPT; ++i) copy_kib(i, 0);
     // ---- this wavefront's query tiles ------------------------------------------------
     int my_limit[TILES], my_ws[TILES];
     int t_ws_hi[TILES], t_lim_lo[TILES]; // per tile extremes
     bool t_on[TILES];
     bf16x8_t qh[TILES][KK], ql[TILES][KK];
+    float qv[TILES][KK][8];
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
         const int s0 = wg_slot0 + (tw * TILES + t) * 16;
@@ -248,7 +238,6 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
         // eight consecutive dims of the slot's row per k-step: all loads first (two 16-byte
         // loads per step when the row allows), unconditional from clamped addresses, so that
         // they are one round trip; dims past head_dim are zeroed afterwards
-        float qv[KK][8];
         if (a.q_vec) {
 #pragma unroll
             for (int kk = 0; kk < KK; ++kk) {
@@ -257,17 +246,27 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
                 const float4_t x0 = qp[0], x1 = qp[1];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    qv[kk][e] = x0[e];
-                    qv[kk][4 + e] = x1[e];
+                    qv[t][kk][e] = x0[e];
+                    qv[t][kk][4 + e] = x1[e];
                 }
             }
         } else {
 #pragma unroll
             for (int kk = 0; kk < KK; ++kk) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) qv[kk][e] = qrow[min(kk * 32 + j * 8 + e, g.head_dim - 1)];
+                for (int e = 0; e < 8; ++e) qv[t][kk][e] = qrow[min(kk * 32 + j * 8 + e, g.head_dim - 1)];
             }
         }
+    }
+    // the first group's K, into the second buffer
+#pragma unroll
+    for (int u = 0; u < (GP * TILE_U4 + THREADS - 1) / THREADS; ++u) {
+        const int i0 = wave * 64 + u * THREADS;
+        if (GP * TILE_U4 % THREADS == 0 || i0 < GP * TILE_U4)
+            copy_to_lds(tile_of(0, i0 / TILE_U4, false) + (i0 & (TILE_U4 - 1)), lane_at, lds0 + (uint32_t)(BUF_U4 + i0) * 16);
+    }
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) {
             const int d0 = kk * 32 + j * 8;
@@ -276,7 +275,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
             const float scale = !a.q_vec || d0 < g.head_dim ? a.qscale : 0.0f;
 #pragma unroll
             for (int e2 = 0; e2 < 4; ++e2) {
-                float x0 = qv[kk][e2 * 2] * scale, x1 = qv[kk][e2 * 2 + 1] * scale;
+                float x0 = qv[t][kk][e2 * 2] * scale, x1 = qv[t][kk][e2 * 2 + 1] * scale;
                 if (!a.q_vec) {
                     x0 = d0 + e2 * 2 < g.head_dim ? x0 : 0.0f;
                     x1 = d0 + e2 * 2 + 1 < g.head_dim ? x1 : 0.0f;
@@ -288,6 +287,14 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
             ql[t][kk] = __builtin_bit_cast(bf16x8_t, u4{lo[0], lo[1], lo[2], lo[3]});
         }
     }
+    // The first scores wait for the queries and that K alone; the first step's pages are on their way meanwhile. (The compiler
+    // waits for the queries as if there were no copies behind them: with all copies in front of the queries, that wait
+    // was for the last page. First scores done, in us after a launch's start: q32/kv8/hd128 over 1024 5.4 -> 5.0,
+    // q16/kv8/hd256 on a ring 9.6 -> 8.3; whole chunks of 512 rows 39.7 -> 38.8 over 1536 and 44.3 -> 43.9.)
+    copies_landed();
+    find_tiles(0);
+#pragma unroll
+    for (int i = 0; i < TPW * CPT; ++i) copy_kib(i, 0);
     ask_ids(SP * GP);
 
     float4_t o[TILES][NT];
@@ -535,9 +542,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
 
     // ---- first pair's scores
     const int n_steps = (n_groups + SP - 1) / SP;
-    copies_landed();
     __syncthreads();
-    clear_v(0, kv_lds + HALF_U4);
 #pragma unroll
     for (int kk = 0; kk < DEPTH; ++kk) ask_k(kv_lds + BUF_U4 + half * 2 * TILE_U4, kk);
     scores(kv_lds + BUF_U4 + half * 2 * TILE_U4, nullptr, std::false_type{}, [](int) {});
@@ -545,7 +550,9 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
 #pragma unroll
     for (int q = 0; q < 4; ++q) top_step(q);
     settle();
-    __syncthreads(); // the second buffer is free
+    copies_landed();
+    __syncthreads(); // the second buffer is free, the first one full
+    clear_v(0, kv_lds + HALF_U4);
 
     for (int step = 0; step < n_steps; ++step) {
         const u4 *buf = kv_lds + (step & 1) * BUF_U4;
