@@ -51,21 +51,14 @@ int decode_max_splits() { return DEC_MAX_SPLITS; }
 // row (the per-row loop of cached_attention_prefill_rows,
 // src/decoder/attention_ops.rs:976-1017, as one launch).
 // ------------------------------------------------------------------------------------
-template <int KK>
-__device__ __forceinline__ void load_k(uint4 (&k)[KK], const DecodeArgs &a, int page, int kvh,
-                                       int lane) {
-    const long tile = (long)page * a.g.page_elems + (long)kvh * a.g.tile_elems;
-    const u32x4_t *kp = reinterpret_cast<const u32x4_t *>(a.k_pool + tile) + lane;
+// One tile of K or V. SHARED: other workgroups (of further query tiles) ask for it as well, and it should be in
+// their L2; otherwise it is read once per launch.
+template <int KK, bool SHARED>
+__device__ __forceinline__ void load_tile(uint4 (&x)[KK], const uint16_t *pool, const Geom &g, int page, int kvh, int lane) {
+    const long tile = (long)page * g.page_elems + (long)kvh * g.tile_elems;
+    const u32x4_t *p = reinterpret_cast<const u32x4_t *>(pool + tile) + lane;
 #pragma unroll
-    for (int kk = 0; kk < KK; ++kk) k[kk] = __builtin_bit_cast(uint4, __builtin_nontemporal_load(kp + kk * 64));
-}
-template <int KK>
-__device__ __forceinline__ void load_v(uint4 (&v)[KK], const DecodeArgs &a, int page, int kvh,
-                                       int lane) {
-    const long tile = (long)page * a.g.page_elems + (long)kvh * a.g.tile_elems;
-    const u32x4_t *vp = reinterpret_cast<const u32x4_t *>(a.v_pool + tile) + lane;
-#pragma unroll
-    for (int kk = 0; kk < KK; ++kk) v[kk] = __builtin_bit_cast(uint4, __builtin_nontemporal_load(vp + kk * 64));
+    for (int kk = 0; kk < KK; ++kk) x[kk] = __builtin_bit_cast(uint4, SHARED ? p[kk * 64] : __builtin_nontemporal_load(p + kk * 64));
 }
 
 // MQ = false is the decode case (one query row, at most 16 heads per group): query slot ==
@@ -76,7 +69,10 @@ __device__ __forceinline__ void load_v(uint4 (&v)[KK], const DecodeArgs &a, int 
 // the rows it uses, in LDS, while its first page is in flight.
 // ROWS: a chunk's few rows, which the launch appends (compiled apart: the larger chunks of the multi-query mode,
 // 512 rows of q32/kv8/hd128 over none, lose 2 us of 18 with it).
-template <int P, int WAVES, bool MQ, bool PRE, bool ROWS = false>
+// SHARED: the launch has many tiles of query slots, whose workgroups ask for the same pages: plain loads instead of
+// non-temporal ones (whole chunks on layers that are in no cache, in us: 50 rows over 4000 of q16/kv2/hd256, 25 tiles, 29.0 -> 25.5;
+// 128 rows over 1000 of q32/kv8/hd128, 32 tiles, 15.2 -> 15.3; but 32 rows over 4700, 8 tiles, 20.4 -> 21.2, 12 rows 13.1 -> 13.3).
+template <int P, int WAVES, bool MQ, bool PRE, bool ROWS = false, bool SHARED = false>
 __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int split, const int kvh,
                                                   const int tile_z) {
     constexpr int THREADS = WAVES * 64;
@@ -246,8 +242,8 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
     const int page_a = ROWS ? table_entry<false>(a.table, min(pb_new, max(page_hi - 1, 0))) : 0;
     const int page_b = ROWS ? table_entry<false>(a.table, min(pb_last, max(page_hi - 1, 0))) : 0;
     const int pg = table_entry<PRE>(a.table, min(pb0 + wave + rot * WAVES, max(page_hi - 1, 0)));
-    load_k<KK>(kr, a, pg, kvh, lane);
-    if constexpr (MQ) load_v<KK>(vr, a, pg, kvh, lane);
+    load_tile<KK, SHARED>(kr, a.k_pool, g, pg, kvh, lane);
+    if constexpr (MQ) load_tile<KK, SHARED>(vr, a.v_pool, g, pg, kvh, lane);
     // the appended row's tile; its page's physical id comes with the arguments: a table lookup would wait for
     // every load issued before it, the first K page included
     auto new_tile = [&]() __attribute__((always_inline)) { return (long)a.new_page * g.page_elems + (long)kvh * g.tile_elems; };
@@ -260,7 +256,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
         __syncthreads();
         Pre::scales(pre_lds, a, rows, n_rows, tid);
         __syncthreads();
-        load_v<KK>(vr, a, pg, kvh, lane);
+        load_tile<KK, SHARED>(vr, a.v_pool, g, pg, kvh, lane);
         // finished queries go straight to their operand layout (hi and lo halves), the finished k row to the
         // pool and to LDS
         Pre::each(pre_lds, a, rows, n_rows, tid, [&](int r, int c4, float4_t v) __attribute__((always_inline)) {
@@ -360,7 +356,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
         }
     }
     __syncthreads();
-    if constexpr (!MQ && !PRE) load_v<KK>(vr, a, pg, kvh, lane);
+    if constexpr (!MQ && !PRE) load_tile<KK, SHARED>(vr, a.v_pool, g, pg, kvh, lane);
 
     float4_t o[NT];
 #pragma unroll
@@ -535,13 +531,13 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
         const int next = page_id(it + 1);
         patch_k(pb);
         const float4_t s = qk();
-        load_k<KK>(kr, a, next, kvh, lane);
+        load_tile<KK, SHARED>(kr, a.k_pool, g, next, kvh, lane);
         short4_t ph, pl;
         softmax_step(s, pb, ph, pl);
         patch_v(pb);
         mask_v(pb);
         pv(ph, pl);
-        load_v<KK>(vr, a, next, kvh, lane);
+        load_tile<KK, SHARED>(vr, a.v_pool, g, next, kvh, lane);
     }
     if (n_it > 0) {
         const int pb = pb0 + wave + turned(n_it - 1) * WAVES;
@@ -629,9 +625,9 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
     }
 }
 
-template <int P, int WAVES, bool MQ, bool PRE, bool ROWS>
+template <int P, int WAVES, bool MQ, bool PRE, bool ROWS, bool SHARED>
 __global__ __launch_bounds__(WAVES * 64) void decode_split_kernel(DecodeArgs a) {
-    decode_split_body<P, WAVES, MQ, PRE, ROWS>(a, blockIdx.x, blockIdx.y, blockIdx.z);
+    decode_split_body<P, WAVES, MQ, PRE, ROWS, SHARED>(a, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // Several independent sequences of the same model layer in one launch: grid z is the
@@ -886,7 +882,7 @@ __global__ __launch_bounds__(128) void decode_merge_wave_batch_kernel(DecodeBatc
     merge_wave_body<PER>(a, kvh, (int)blockIdx.y - kvh * d.g.gqa, cg);
 }
 
-template <int P, int WAVES, bool MQ, bool PRE, bool ROWS = false>
+template <int P, int WAVES, bool MQ, bool PRE, bool ROWS = false, bool SHARED = false>
 static hipError_t launch_split_mq(const DecodeArgs &a, hipStream_t s) {
     constexpr int KK = P / 32;
     if (a.k_new && a.n_queries > (ROWS ? MQ_APPEND_ROWS : 1)) return hipErrorInvalidValue;
@@ -900,24 +896,29 @@ static hipError_t launch_split_mq(const DecodeArgs &a, hipStream_t s) {
     const size_t lds = apart ? stage16 + xchg : (stage > xchg ? stage : xchg);
     static std::atomic<uint64_t> lds_ok{0}; // per instantiation
     {
-        hipError_t e = allow_full_lds(reinterpret_cast<const void *>(&decode_split_kernel<P, WAVES, MQ, PRE, ROWS>), lds_ok);
+        hipError_t e = allow_full_lds(reinterpret_cast<const void *>(&decode_split_kernel<P, WAVES, MQ, PRE, ROWS, SHARED>), lds_ok);
         if (e != hipSuccess) return e;
     }
     DecodeArgs b = a;
     b.xchg_off = apart ? (int)stage16 : 0;
     dim3 grid((unsigned)a.splits, (unsigned)a.g.kv_heads, (unsigned)((n_slots + 15) / 16));
-    hipLaunchKernelGGL((decode_split_kernel<P, WAVES, MQ, PRE, ROWS>), grid, dim3(WAVES * 64), lds, s, b);
+    hipLaunchKernelGGL((decode_split_kernel<P, WAVES, MQ, PRE, ROWS, SHARED>), grid, dim3(WAVES * 64), lds, s, b);
     return hipGetLastError();
+}
+
+// Query rows over the cache, 16 slots a workgroup (a chunk's few rows are appended by the launch itself).
+template <int P, int WAVES>
+static hipError_t launch_split_rows(const DecodeArgs &a, hipStream_t s) {
+    if (a.pre) return hipErrorInvalidValue; // the caller keeps the fused step to single-tile decode
+    if (a.n_queries * a.g.gqa > 240 && !a.k_new) return launch_split_mq<P, WAVES, true, false, false, true>(a, s);
+    return a.k_new && a.n_queries > 1 ? launch_split_mq<P, WAVES, true, false, true>(a, s)
+                                      : launch_split_mq<P, WAVES, true, false>(a, s);
 }
 
 template <int P, int WAVES>
 static hipError_t launch_split(const DecodeArgs &a, hipStream_t s) {
     // the decode specialisation assumes a single tile of query slots
-    if (a.n_queries > 1 || a.g.gqa > 16) {
-        if (a.pre) return hipErrorInvalidValue; // the caller keeps the fused step to single-tile decode
-        return a.k_new && a.n_queries > 1 ? launch_split_mq<P, WAVES, true, false, true>(a, s)
-                                          : launch_split_mq<P, WAVES, true, false>(a, s);
-    }
+    if (a.n_queries > 1 || a.g.gqa > 16) return launch_split_rows<P, WAVES>(a, s);
     return a.pre ? launch_split_mq<P, WAVES, false, true>(a, s) : launch_split_mq<P, WAVES, false, false>(a, s);
 }
 
@@ -926,11 +927,7 @@ static hipError_t launch_split(const DecodeArgs &a, hipStream_t s) {
 // four wavefronts, one per SIMD with 512 registers each (two row elements per thread in the
 // fused pre-KV step and the fused append).
 static hipError_t launch_split_wide(const DecodeArgs &a, hipStream_t s) {
-    if (a.n_queries > 1 || a.g.gqa > 16) {
-        if (a.pre) return hipErrorInvalidValue;
-        return a.k_new && a.n_queries > 1 ? launch_split_mq<512, 4, true, false, true>(a, s)
-                                          : launch_split_mq<512, 4, true, false>(a, s);
-    }
+    if (a.n_queries > 1 || a.g.gqa > 16) return launch_split_rows<512, 4>(a, s);
     return a.pre ? launch_split_mq<512, 4, false, true>(a, s) : launch_split_mq<512, 4, false, false>(a, s);
 }
 

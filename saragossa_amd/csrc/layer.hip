@@ -265,6 +265,18 @@ int chunk_splits(const Geom &g, size_t n_queries, size_t per_wg, size_t n_pages)
     return (int)std::min<size_t>(want, tuning().prefill_max_splits);
 }
 
+// Splits of a launch in which the workgroups of several query tiles walk the same pages. Workgroup ids, the split fastest,
+// then the kv head, go to the eight XCDs in turn: where splits x kv heads are whole eights, all tiles of a
+// (split, kv head) run on one XCD and its L2 has a page from memory once. Worth up to a tenth of the splits: rows of
+// q16/kv2/hd256 as whole chunks on layers in no cache, in us, splits as they are / in whole eights, 6 over 8192 (42/40)
+// 15.6/14.7, over 20000 22.5/19.9, 12 over 8192 (21/20) 21.0/17.1; with plain loads 18 over 4000 (14/12) 16.9/17.6, 23 (11/8)
+// 17.5/17.8, 36 (7/4) 20.5/22.7. On f32 layers (42/40 and 21/20) 6 over 20000 88.5/80.4, 12 over 8192 61.6/58.5.
+int xcd_splits(int splits, int kv_heads) {
+    int unit = 8;
+    for (int h = kv_heads; unit > 1 && h % 2 == 0; h /= 2) unit /= 2;
+    return splits % unit * 10 <= splits ? splits - splits % unit : splits;
+}
+
 int choose_splits(const skv_layer *L, int n_pages_scan, size_t rows, int waves, size_t target_wgs) {
     const Tuning &t = tuning();
     if (!skv_flag_sdpa_2pass_enabled() || rows < t.split_min_len) return 1;
@@ -506,6 +518,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
             // ring: 22.3 us with one, 29.7 with two and a merge)
             if (g.ring_rows > 0) want = std::min(want, std::max<size_t>((size_t)a.n_pages / 8, 1));
             a.splits = (int)std::min<size_t>((size_t)a.splits, want);
+            if (tiles > (size_t)g.kv_heads) a.splits = xcd_splits(a.splits, g.kv_heads);
             a.splits_total = a.splits;
             if (a.splits > 1) {
                 int32_t rc2 = multi_query_partials(L, s, (size_t)a.splits, n_queries, a);
@@ -584,6 +597,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
             want = std::min<size_t>(want, tuning().prefill_max_splits);
         }
         a.splits = (int)std::min<size_t>((size_t)a.splits, want);
+        if (!use_tiles && tiles > (size_t)g.kv_heads) a.splits = xcd_splits(a.splits, g.kv_heads);
         a.splits_total = a.splits;
         if (a.splits > 1) {
             int32_t rc2 = multi_query_partials(L, s, (size_t)a.splits, n_queries, a);

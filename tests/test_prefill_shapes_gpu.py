@@ -175,6 +175,32 @@ def test_few_rows_are_appended_by_the_attention_launch(state, dims, window, star
     assert np.array_equal(gk, cache.keys()[first:]) and np.array_equal(gv, cache.values()[first:])
 
 
+@pytest.mark.parametrize("element,tol", [("bf16", 1e-4), ("f32", 2e-5)])
+@pytest.mark.parametrize("dims,base,counts", [
+    ((16, 2, 256), 700, (30, 31)),  # 240 slots, and the first number that makes pages shared by many tiles
+    ((16, 2, 256), 5000, (6, 12)),  # 42 and 21 splits over two kv heads: taken in whole eights, 40 and 20
+    ((6, 3, 48), 3100, (20, 130)),  # no power of two of kv heads
+])
+def test_rows_whose_tiles_share_pages(state, element, tol, dims, base, counts):
+    q_heads, kv_heads, head_dim = dims
+    rng = np.random.default_rng(base + head_dim)
+    make = state.full_attention_f32 if element == "f32" else state.full_attention_bf16
+    kv = make(base + sum(counts), q_heads, kv_heads, head_dim)
+    kv.set_block_table(rng.permutation(kv.pages()).astype(np.int32))
+    lay = oracle.layout(q_heads, kv_heads, head_dim)
+    cache = oracle.LayerKvCache("f32" if element == "f32" else "bf16r")
+    kv_dim = kv_heads * head_dim
+    k, v = (rng.standard_normal((base, kv_dim), dtype=np.float32) for _ in range(2))
+    kv.seed(k, v, base)
+    cache.append_batch(k, v, lay)
+    for c in counts:
+        q = rng.standard_normal((c, q_heads * head_dim), dtype=np.float32)
+        k, v = (rng.standard_normal((c, kv_dim), dtype=np.float32) for _ in range(2))
+        got = kv.prefill_rows(q, k, v)
+        want = oracle.cached_attention_prefill_rows(q, k, v, cache, lay)
+        assert np.abs(got - want).max() <= tol, c
+
+
 @pytest.mark.parametrize("head_dim,window,base", [(64, 0, 61), (128, 0, 900), (256, 0, 61), (256, 0, 900), (40, 0, 900),
                                                   (64, 70, 61), (128, 900, 1200)])  # one split, several; rings
 def test_infinite_rows_of_an_f32_chunk(state, shape, head_dim, window, base):
