@@ -142,6 +142,8 @@ struct Tuning {
     size_t prefill_tiles;   // 0 = never, 1 = by shape, 2 = every chunk of 64 query slots and more
     size_t prefill_wgs, prefill_max_splits;
     long prefill_tiles2_min_pages; // -1 = by head_dim
+    size_t f32_terms;       // f32 chunks: 0 = every workgroup splits its pages into terms, 1 = by shape, 2 = a launch of its own does
+    size_t f32_terms_max;   // bytes of terms held at a time
 };
 
 const Tuning &tuning() {
@@ -160,6 +162,8 @@ const Tuning &tuning() {
         t.prefill_max_splits = std::max<size_t>(env_usize("SKV_PREFILL_MAX_SPLITS", 512), 1);
         t.prefill_tiles2_min_pages = std::getenv("SKV_PREFILL_TILES2_MIN_PAGES")
                                          ? (long)env_usize("SKV_PREFILL_TILES2_MIN_PAGES", 0) : -1;
+        t.f32_terms = env_usize("SKV_F32_TERMS", 1);
+        t.f32_terms_max = std::min<size_t>(std::max<size_t>(env_usize("SKV_F32_TERMS_MB", 512), 1), 1 << 20) << 20;
         seen = epoch;
     }
     return t;
@@ -433,6 +437,120 @@ ChunkPages layer_pages(const skv_layer *L, size_t lo, size_t end) {
     return c;
 }
 
+// The launch arguments that append n_rows rows at the layer's length.
+AppendArgs append_args(const skv_layer *L, const float *k_dev, const float *v_dev, size_t n_rows) {
+    AppendArgs a{};
+    a.k_src = k_dev;
+    a.v_src = v_dev;
+    a.k_pool = L->k_pool;
+    a.v_pool = L->v_pool;
+    a.table = L->table_dev;
+    a.first_pos = (long)L->len;
+    a.n_rows = (int)n_rows;
+    a.g = L->g;
+    if (L->g.ring_rows > 0 && n_rows > (size_t)L->g.ring_rows) {
+        // only the last ring_rows rows survive; skip the ones that would be overwritten
+        const size_t skip = n_rows - (size_t)L->g.ring_rows;
+        const size_t kv_dim = (size_t)L->g.kv_heads * L->g.head_dim;
+        a.k_src += skip * kv_dim;
+        a.v_src += skip * kv_dim;
+        a.first_pos += (long)skip;
+        a.n_rows = L->g.ring_rows;
+    }
+    return a;
+}
+
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return true; // a stream that cannot say so takes no scratch
+    }
+    return status != hipStreamCaptureStatusNone;
+}
+
+// Whether a chunk on f32 pages has them split into terms by a launch of its own, once for all workgroups, instead of by each
+// workgroup for its slots. That launch moves 10 bytes per value of the whole context (19 us at 4600 rows of 8 x 128) and stores
+// the chunk's rows on the way; the attention behind it takes a quarter less on short walks and 5 to 10 % on long ones. So it pays
+// where many slots share a page, and on rings, whose context is short and whose rows otherwise take a launch to pages of
+// their own. Whole chunks on layers that are in no cache, in us, split by the workgroup / by a launch: q32/kv8/hd128, 512 rows over 0, 512,
+// 1024, 2048, 4096 39.4/33.0, 59.2/51.3, 81.2/68.3, 116/108, 194/185, 256 rows (1024 slots) over 500, 2048, 8192 37.4/36.4, 64.0/65.2,
+// 178/190, 64 rows over 8192 63.3/81.6; q28/kv4/hd128, 160 rows over 3000 56.2/57.1, 512 over 16000 611/556; q12/kv4/hd96, 512 rows
+// (1536 slots) over 2000 57.2/55.7; q8/kv2/hd64, 512 rows over 2048, 4096 30.3/27.5, 42.1/38.9, 300 over 10000 54.5/55.7; q16/kv2/hd256,
+// 128 rows (1024 slots) over 4096 71.1/70.3, 256 106/102, 512 190/174, over 16000 256 320/304; q16/kv8/hd256, 512 rows
+// (1024 slots) over 1000 84.2/85.2. Rings: q16/kv8/hd256 of 1024 rows, 64, 256, 512, 1024 rows 62.3/57.0, 67.7/62.5, 76.3/75.9, 120/120;
+// q32/kv8/hd128 of 512 and 1024, 64, 512 rows 32.4/27.7, 48.2/41.2, 128, 256 34.7/33.6, 48.2/43.4; q8/kv2/hd64 128 rows 22.4/19.0.
+bool f32_terms_pay(const Geom &g, size_t n_queries) {
+    if (tuning().f32_terms != 1) return tuning().f32_terms > 1;
+    return g.ring_rows > 0 || n_queries * (size_t)g.gqa >= (g.P > 128 ? 2048u : 1536u);
+}
+
+// Such a chunk. The scratch holds at most so many bytes of terms (512 MiB); longer contexts are taken in segments, each with
+// splits of its own (512 rows of q32/kv8/hd128 over 16384, 40000, in us, segments of 128 MiB / 1 GiB 657/643, 1562/1532; over 8192,
+// where two segments of 64 MiB take 357, one takes 340).
+struct F32Plan {
+    int first, last;    // pairs of entries of the page list
+    int entries;        // of the list
+    int segments, held; // pairs of a segment
+    int splits;         // of a segment
+    bool halves;
+    int sets() const { return segments * splits; }
+    // The terms' scratch. A layer of up to `pairs` pairs asks for all of them at once while that is 128 MiB at most, then for twice
+    // as much each time, so that the chunks of a growing context seldom replace it.
+    size_t bytes(const Geom &g, size_t pairs) const {
+        const size_t one = f32_terms_bytes(g), most = std::max<size_t>(tuning().f32_terms_max / one, 1);
+        size_t n = std::max<size_t>(((size_t)128 << 20) / one, 1);
+        while (n < (size_t)held) n *= 2;
+        return std::max(std::min({n, pairs, most}), (size_t)held) * one;
+    }
+};
+// walked: pages that a workgroup walks of all segments
+F32Plan plan_f32_chunk(const Geom &g, size_t n_queries, int first_entry, int entries, int walked, int max_splits) {
+    F32Plan p{};
+    p.first = first_entry / 2;
+    p.last = (entries + 1) / 2;
+    p.entries = entries;
+    const int pairs = p.last - p.first, most = (int)std::max<size_t>(tuning().f32_terms_max / f32_terms_bytes(g), 1);
+    p.segments = (pairs + most - 1) / most;
+    p.held = (pairs + p.segments - 1) / p.segments;
+    // Halves cover half the slots and walk two pairs at a time: the same time per workgroup with half as many splits, so fewer
+    // partials, but they copy each page for half as many slots, which costs more on long walks. Whole chunks, one tile / halves, in us: q32/kv8/hd128, 512 rows
+    // over 512, 1024, 2048, 6000, 8192 (two splits / one) 59.1/51.2, 74.5/68.5, 114/109, 262/265, 340/349; q8/kv2/hd64, 512 rows over 2048, 4096,
+    // 10000 (eight / four) 32.2/28.0, 42.5/40.0, 74.0/72.7; but q28/kv4/hd128, 300 rows over 3000 (three / one) 91.2/115,
+    // q12/kv4/hd96, 512 rows over 2000 (five / two) 56.1/60.3.
+    const size_t pages = (size_t)walked / (size_t)p.segments;
+    const int one = chunk_splits(g, n_queries, (size_t)f32_prefill_slots(g.P, false), pages);
+    const int two = chunk_splits(g, n_queries, (size_t)f32_prefill_slots(g.P, true), pages);
+    p.halves = g.P <= 128 && tuning().prefill_tiles2_min_pages < 0 && 2 * two >= one && walked <= 300;
+    // (choose_splits' number, which the split knobs of decode launches bound, is the larger one unless they do)
+    p.splits = std::min(max_splits, p.halves ? two : one);
+    return p;
+}
+int32_t run_f32_chunk(const F32Plan &p, DecodeArgs a, const ChunkPages &pages, void *terms, int pos_lo, const float *k_new,
+                      const float *v_new, hipStream_t s, bool merge = true) {
+    a.splits = p.splits;
+    a.splits_total = p.sets();
+    a.k_new = a.v_new = nullptr;
+    for (int seg = 0; seg < p.segments; ++seg) {
+        TermPairs t;
+        t.terms = terms;
+        t.first = p.first + seg * p.held;
+        t.held = std::min(p.held, p.last - t.first);
+        t.entries = p.entries;
+        t.pos_lo = pos_lo;
+        t.pos_hi = a.q_pos0 + a.n_queries - 1;
+        t.k_src = k_new;
+        t.v_src = v_new;
+        t.new_pos = k_new ? a.q_pos0 : INT32_MAX;
+        t.vec = k_new && (reinterpret_cast<uintptr_t>(k_new) & 15) == 0 && a.g.head_dim % 4 == 0;
+        a.split_base = seg * p.splits;
+        SKV_HIP(launch_f32_terms(a, pages, t, s));
+        SKV_HIP(launch_f32_prefill(a, pages, &t, p.halves, s));
+    }
+    if (merge && a.splits_total > 1) SKV_HIP(launch_merge_rows(a, s));
+    return SKV_OK;
+}
+
 // k_new / v_new non-null: the row at position len-1 has not been written yet and the
 // attention kernel appends it itself (the host bookkeeping has already advanced).
 // n_queries > 1: chunked prefill over the cache; the last n_queries rows are the new ones
@@ -483,7 +601,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
         // can append the row (and norm and rotate q and k) itself
         DecodeArgs a{};
         fill_decode_args(L, q_dev, out_dev, window_start, k_new, v_new, n_queries, decode_target_wgs(), a);
-        if ((k_new || v_new || pre) && !f32_decode_kernel_serves(a))
+        if ((k_new || v_new || pre) && n_queries == 1 && !f32_decode_kernel_serves(a))
             return fail(SKV_ERR_CONFIG, "KV f32: étape fusionnée non construite pour cette forme");
         if (pre) {
             a.pre = 1;
@@ -498,6 +616,27 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
         }
         if (attn_scalar > 0.0f) a.qscale = (1.0f / std::sqrt(attn_scalar)) * 1.4426950408889634f;
         if (n_queries > 1 && takes_f32_chunk_kernel(g, n_queries, (size_t)a.n_pages)) {
+            const size_t lo = std::max(window_start, skv_window_start(L->len - n_queries, L->window));
+            const ChunkPages pages = layer_pages(L, lo, L->len); // (a ring's list begins at `lo`, a full layer's at 0)
+            // A captured launch must not hold on to scratch that a later call may replace, and a card without room
+            // for it still has the other way, which needs none.
+            if (f32_terms_pay(g, n_queries) && !capturing(s)) {
+                const F32Plan plan = g.ring_rows > 0 ? plan_f32_chunk(g, n_queries, 0, pages.n_old, pages.n_old, a.splits)
+                                                     : plan_f32_chunk(g, n_queries, (int)(lo / 16), a.n_pages, a.n_pages, a.splits);
+                void *terms = nullptr;
+                DecodeArgs b = a;
+                b.splits_total = plan.sets();
+                if (multi_query_partials(L, s, plan.sets() > 1 ? (size_t)plan.sets() : 0, n_queries, b,
+                                         plan.bytes(g, (size_t)(L->n_pages + 1) / 2), &terms) == SKV_OK)
+                    return run_f32_chunk(plan, b, pages, terms, (int)lo, k_new, v_new, s);
+                (void)hipGetLastError();
+            }
+            if (k_new) { // rows that the terms' launch would have stored
+                AppendArgs w = append_args(L, k_new, v_new, n_queries);
+                w.first_pos -= (long)n_queries; // (counted already)
+                SKV_HIP(launch_append(w, s));
+                a.k_new = a.v_new = nullptr;
+            }
             const bool halves = f32_halves(g, n_queries * (size_t)g.gqa, (size_t)a.n_pages);
             // (choose_splits' number, which the split knobs of decode launches bound, is the larger one unless they do)
             a.splits = std::min(a.splits, chunk_splits(g, n_queries, (size_t)f32_prefill_slots(g.P, halves), (size_t)a.n_pages));
@@ -506,8 +645,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
                 int32_t rc2 = multi_query_partials(L, s, (size_t)a.splits, n_queries, a);
                 if (rc2) return rc2;
             }
-            const size_t lo = std::max(window_start, skv_window_start(L->len - n_queries, L->window));
-            SKV_HIP(launch_f32_prefill(a, layer_pages(L, lo, L->len), halves, s));
+            SKV_HIP(launch_f32_prefill(a, pages, nullptr, halves, s));
             if (a.splits > 1) SKV_HIP(launch_merge_rows(a, s));
             return SKV_OK;
         }
@@ -618,28 +756,6 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
     return SKV_OK;
 }
 
-// The launch arguments that append n_rows rows at the layer's length.
-AppendArgs append_args(const skv_layer *L, const float *k_dev, const float *v_dev, size_t n_rows) {
-    AppendArgs a{};
-    a.k_src = k_dev;
-    a.v_src = v_dev;
-    a.k_pool = L->k_pool;
-    a.v_pool = L->v_pool;
-    a.table = L->table_dev;
-    a.first_pos = (long)L->len;
-    a.n_rows = (int)n_rows;
-    a.g = L->g;
-    if (L->g.ring_rows > 0 && n_rows > (size_t)L->g.ring_rows) {
-        // only the last ring_rows rows survive; skip the ones that would be overwritten
-        const size_t skip = n_rows - (size_t)L->g.ring_rows;
-        const size_t kv_dim = (size_t)L->g.kv_heads * L->g.head_dim;
-        a.k_src += skip * kv_dim;
-        a.v_src += skip * kv_dim;
-        a.first_pos += (long)skip;
-        a.n_rows = L->g.ring_rows;
-    }
-    return a;
-}
 void appended(skv_layer *L, size_t n_rows) {
     L->len += n_rows;
     if (L->g.ring_rows > 0 && L->len > (size_t)L->g.ring_rows)
@@ -1206,29 +1322,50 @@ static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const flo
     // pages a workgroup of one tile row walks: the window and the workgroup's own rows
     const size_t walked = std::min<size_t>((size_t)pages.n_old + n_new, L->window / 16 + 2);
     const TileShape shape = prefill_shape(g, c * (size_t)g.gqa, walked);
+    // f32 pages as terms, made by a launch of their own (see encode_attention), or split by each workgroup
+    bool made = g.f32 && f32_terms_pay(g, c) && !capturing(s);
+    F32Plan plan{};
     const bool halves = g.f32 && f32_halves(g, c * (size_t)g.gqa, walked);
-    a.splits = chunk_splits(g, c, (size_t)(g.f32 ? f32_prefill_slots(g.P, halves) : prefill_tile_slots(g.P, shape)), walked);
     // a context over the chunk's own rows is written once they are in the ring: by the merge, so there has to be one
     const bool over_rows = context_over_rows(L, c, out, k, v);
-    if (over_rows) a.splits = std::max(a.splits, 2);
-    a.splits_total = a.splits;
     void *scratch = nullptr;
-    int32_t rc = multi_query_partials(L, s, a.splits > 1 ? (size_t)a.splits : 0, c, a, 2 * pool_bytes, &scratch);
-    if (rc) return rc;
-    AppendArgs w{};
-    w.k_src = k;
-    w.v_src = v;
-    w.k_pool = static_cast<uint16_t *>(scratch);
-    w.v_pool = w.k_pool + pool_bytes / sizeof(uint16_t);
-    w.first_pos = (long)(base % 16);
-    w.n_rows = (int)c;
-    w.g = g;
-    w.g.ring_rows = 0;
-    SKV_HIP(launch_append(w, s));
-    pages.k_new = w.k_pool;
-    pages.v_new = w.v_pool;
-    SKV_HIP(g.f32 ? launch_f32_prefill(a, pages, halves, s) : launch_prefill_tiles(a, pages, shape, s));
-    if (a.splits == 1) return encode_append(L, s, k, v, c);
+    int32_t rc = SKV_OK;
+    if (made) {
+        plan = plan_f32_chunk(g, c, 0, (int)((size_t)pages.n_old + n_new), (int)walked, INT32_MAX);
+        if (over_rows) plan.splits = std::max(plan.splits, 2);
+        a.splits = plan.splits;
+        a.splits_total = plan.sets();
+        if (multi_query_partials(L, s, a.splits_total > 1 ? (size_t)a.splits_total : 0, c, a, plan.bytes(g, 0), &scratch) != SKV_OK) {
+            (void)hipGetLastError();
+            made = false;
+        }
+    }
+    if (!made) {
+        a.splits = chunk_splits(g, c, (size_t)(g.f32 ? f32_prefill_slots(g.P, halves) : prefill_tile_slots(g.P, shape)), walked);
+        if (over_rows) a.splits = std::max(a.splits, 2);
+        a.splits_total = a.splits;
+        rc = multi_query_partials(L, s, a.splits > 1 ? (size_t)a.splits : 0, c, a, 2 * pool_bytes, &scratch);
+        if (rc) return rc;
+    }
+    if (made) {
+        rc = run_f32_chunk(plan, a, pages, scratch, (int)lo, k, v, s, false);
+        if (rc) return rc;
+    } else {
+        AppendArgs w{};
+        w.k_src = k;
+        w.v_src = v;
+        w.k_pool = static_cast<uint16_t *>(scratch);
+        w.v_pool = w.k_pool + pool_bytes / sizeof(uint16_t);
+        w.first_pos = (long)(base % 16);
+        w.n_rows = (int)c;
+        w.g = g;
+        w.g.ring_rows = 0;
+        SKV_HIP(launch_append(w, s));
+        pages.k_new = w.k_pool;
+        pages.v_new = w.v_pool;
+        SKV_HIP(g.f32 ? launch_f32_prefill(a, pages, nullptr, halves, s) : launch_prefill_tiles(a, pages, shape, s));
+    }
+    if (a.splits_total == 1) return encode_append(L, s, k, v, c);
     if (over_rows) {
         rc = encode_append(L, s, k, v, c);
         if (rc) return rc;
@@ -1325,6 +1462,19 @@ int32_t skv_prefill_chunk_device(skv_layer *L, skv_stream stream, const float *q
         // appends them itself, as a decode step's does (its last query tile, which sees all of them, stores them)
         if (c > 1 && c <= (size_t)MQ_APPEND_ROWS && ring == 0 && !L->g.f32 && tuning().fused_append &&
             !context_over_rows(L, c, out, k, v) && !takes_tile_kernel(L->g, c * (size_t)L->g.gqa, (L->len + c + 15) / 16)) {
+            RowsAhead ahead(L, c);
+            rc = encode_attention(L, as_stream(stream), q, out, 0, k, v, c);
+            if (rc) return rc;
+            ahead.written = true;
+            q += c * q_dim;
+            k += c * kv_dim;
+            v += c * kv_dim;
+            out += c * q_dim;
+            continue;
+        }
+        // a chunk that the f32 chunk kernel takes: its rows are stored by the launch that splits its pages into terms
+        if (c > 1 && ring == 0 && L->g.f32 && tuning().fused_append && f32_terms_pay(L->g, c) &&
+            takes_f32_chunk_kernel(L->g, c, (L->len + c + 15) / 16)) {
             RowsAhead ahead(L, c);
             rc = encode_attention(L, as_stream(stream), q, out, 0, k, v, c);
             if (rc) return rc;

@@ -172,8 +172,23 @@ struct ChunkPages {
     int ring_pages;      // 0 = not a ring
     int new_pos0;        // first new position (INT32_MAX = none)
     int new_first;       // position of the first new page's first row
-    const uint16_t *k_new; // tiles of the new pages, in order
+    const uint16_t *k_new; // tiles of the new pages, in order (null: their rows lie in the caller's memory, TermPairs)
     const uint16_t *v_new;
+};
+
+// Pages of a chunk's list as three bf16 terms a value (f32 layers): pairs [first, first + held) of entries (2i, 2i + 1), per kv head
+// and pair K, then V, three planes each (kernels_f32_prefill.hip).
+struct TermPairs {
+    void *terms;
+    int first, held;
+    int entries;        // of the whole list
+    int pos_lo, pos_hi; // positions that some query attends
+    // the chunk's own rows [kv_dim], from position new_pos to pos_hi: on a full layer to be stored into its pages, on a
+    // ring the rows of the list's new entries (new_pos INT32_MAX: all rows are in the layer's pages)
+    const float *k_src;
+    const float *v_src;
+    int new_pos;
+    int vec;            // K rows may be read 16 bytes at a time
 };
 
 // How a workgroup of the prefill tile kernel divides its work among its wavefronts: one 16-slot
@@ -403,7 +418,9 @@ hipError_t launch_f32_split_batch(const DecodeBatchArgs &b, int n_seq, int max_s
 hipError_t launch_merge(const DecodeArgs &a, hipStream_t s);        // split-K partials -> context
 hipError_t launch_prefill_tiles(const DecodeArgs &a, const ChunkPages &c, TileShape shape, hipStream_t s); // chunked prefill, no merge
 int prefill_tile_slots(int P, TileShape shape);
-hipError_t launch_f32_prefill(const DecodeArgs &a, const ChunkPages &c, bool halves, hipStream_t s); // the same on f32 pages
+hipError_t launch_f32_terms(const DecodeArgs &a, const ChunkPages &c, const TermPairs &t, hipStream_t s); // f32 pages -> terms
+size_t f32_terms_bytes(const Geom &g); // of one pair of pages, all kv heads
+hipError_t launch_f32_prefill(const DecodeArgs &a, const ChunkPages &c, const TermPairs *t, bool halves, hipStream_t s); // chunked prefill over them (null: over the f32 pages)
 int f32_prefill_slots(int P, bool halves); // query slots of a workgroup, 0 = head_dim not served
 hipError_t launch_merge_rows(const DecodeArgs &a, hipStream_t s);    // the same merge for many query slots
 hipError_t launch_merge_append(const DecodeArgs &a, const AppendArgs &w, hipStream_t s); // that and an append nobody waits for in it
