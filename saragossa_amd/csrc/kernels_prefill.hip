@@ -9,7 +9,6 @@
 namespace skv {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
-typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
 typedef __attribute__((ext_vector_type(4))) short short4_t;
 typedef __attribute__((ext_vector_type(4))) float float4_t;
 typedef __attribute__((ext_vector_type(4))) unsigned int u4;
@@ -63,9 +62,11 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // 57.2 -> 41.1, 106 -> 86.5, 256 -> 225; q16/kv2/hd256 40.0 -> 24.3, 55.7 -> 50.5, 97.9 -> 89.0, 247 -> 225 (where
 // the matrix pipes alone need 130).
 // A wavefront issues an instruction in four to five cycles, so every one beside the products counts: with a tile per
-// wavefront to copy, the moves that put operands together and the search for the maximum between products, and the second
-// terms of the probabilities by a dot product, chunks of 512 rows on layers that are in no cache went, in us, for q32/kv8/hd128
-// over 4700, 16384 from 87.7 to 83.2, 223.5 to 220.5; for q16/kv8/hd256 on a ring of 1024 rows from 46.1 to 44.4. (Three
+// wavefront to copy and the moves that put operands together and the search for the maximum between products, chunks of 512
+// rows on layers that are in no cache went, in us, for q32/kv8/hd128 over 4700, 16384 from 88.0 to 80.5, 224 to 213; for
+// q16/kv8/hd256 on a ring of 1024 rows from 47.2 to 44.1. (Second terms of the probabilities as dot products of the pair of
+// first terms with -1 and 0, an instruction less each, took longer: 1024 rows of q24/kv8/hd128 over 4000 139.4 against 132.2.
+// Three
 // wavefronts per SIMD, twelve in thirds at 154 registers, were no faster than two; two tiles per wavefront at
 // head_dim 256, four wavefronts at 400 registers, 11 to 40 % slower.)
 // ------------------------------------------------------------------------------------
@@ -84,9 +85,10 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
     constexpr int THREADS = WAVES * 64;
     constexpr int KK = P / 32;
     constexpr int NT = P / 16;
-    // Vector work is held in its place between the products; a wavefront alone on its SIMD (head_dim above 256) does better
-    // where the compiler places it (256 rows of q8/kv2/hd512 over 4096: 61.0 us against 66.0)
-    constexpr bool PINNED = P <= 256;
+    // Vector work is held in its place between the products; a wavefront alone on its SIMD (head_dim above 256), and one with
+    // few products to a pair (up to 64), does better where the compiler places it (256 rows of q8/kv2/hd512 over 4096: 61.0 us
+    // against 66.0; 1024 of q8/kv2/hd64 over 8000: 53.0 against 55.7)
+    constexpr bool PINNED = KK >= 4 && P <= 256;
     constexpr int TILE_U4 = KK * 64;                           // 16-byte units of one K (or V) tile
     constexpr int GP = 2 * HALVES;                             // pages of a group: a pair for each half
     static_assert(TILE_U4 % 64 == 0, "a wavefront copies whole KiB of one page");
@@ -381,9 +383,6 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
     // between products: step q takes the exponential of score q and splits that of score q - 1
     float pr_[TILES];                  // exponential of the last step
     float pr2[TILES][2];
-    // (in registers: as an immediate of the instruction the first one is taken for the second)
-    uint32_t minus_first = 0x0000bf80u, minus_second = 0xbf800000u;
-    asm("" : "+s"(minus_first), "+s"(minus_second));
     uint32_t hi4[TILES][4], lo4[TILES][4];
     auto prob_step = [&](int q) __attribute__((always_inline)) {
 #pragma unroll
@@ -397,13 +396,10 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
                 // p = hi + lo with hi the upper 16 bits of p (cut off) and lo the exact remainder rounded to
                 // nearest: 2^-17 relative, of either sign (512 rows of q32/kv8/hd128 over 1536: errors of 5.4e-6
                 // against 64 bits; lo cut off as well, always too small, 9.9e-6)
-                // (a difference is a product of the pair of high terms with -1 and 0, exact, one instruction)
                 if (e & 1) {
                     const uint32_t hi = __builtin_amdgcn_perm(__float_as_uint(prev), __float_as_uint(pr2[t][0]), 0x07060302u);
                     hi4[t][e >> 1] = hi;
-                    const bf16x2_t h2 = __builtin_bit_cast(bf16x2_t, hi);
-                    lo4[t][e >> 1] = bf16_pair(__builtin_amdgcn_fdot2_f32_bf16(h2, __builtin_bit_cast(bf16x2_t, minus_first), pr2[t][0], false),
-                                               __builtin_amdgcn_fdot2_f32_bf16(h2, __builtin_bit_cast(bf16x2_t, minus_second), prev, false));
+                    lo4[t][e >> 1] = bf16_pair(pr2[t][0] - __uint_as_float(hi << 16), prev - __uint_as_float(hi & 0xffff0000u));
                     if (PINNED) asm volatile("" : "+v"(hi4[t][e >> 1]), "+v"(lo4[t][e >> 1])); // (here, between the products, not behind them)
                 }
             }
