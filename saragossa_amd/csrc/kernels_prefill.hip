@@ -427,6 +427,10 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
     auto scores = [&](const u4 *kt, const u4 *vt, auto with_probs, auto copies) __attribute__((always_inline)) {
         constexpr bool PROBS = decltype(with_probs)::value;
         constexpr int BEATS = 2 * KK; // (k-step, hi or lo half)
+        // The SIMD's other wavefront may be in its second window, which is products almost alone and so gets on with the cycles that
+        // are left (1024 rows of q24/kv8/hd128 over 4000 132.2 -> 128.9 us, of q8/kv2/hd64 over 8000 51.7 -> 50.0; 512 of
+        // q32/kv8/hd128 over 16384 212 -> 208; raised in the second window instead: half of that)
+        __builtin_amdgcn_s_setprio(1);
         float4_t na[TILES], nb[TILES];
         int q = 0;
 #pragma unroll
@@ -456,6 +460,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
             }
         }
         __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(0);
         if (PROBS) probs_done();
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
