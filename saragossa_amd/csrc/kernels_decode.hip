@@ -938,6 +938,7 @@ hipError_t launch_decode(const DecodeArgs &a, hipStream_t s) {
     case 512: e = launch_split_wide(a, s); break;
     case 32: e = w8 ? launch_split<32, 8>(a, s) : launch_split<32, 4>(a, s); break;
     case 64: e = w8 ? launch_split<64, 8>(a, s) : launch_split<64, 4>(a, s); break;
+    case 96: e = w8 ? launch_split<96, 8>(a, s) : launch_split<96, 4>(a, s); break;
     case 128: e = w8 ? launch_split<128, 8>(a, s) : launch_split<128, 4>(a, s); break;
     case 256: e = w8 ? launch_split<256, 8>(a, s) : launch_split<256, 4>(a, s); break;
     default: break;
@@ -1036,6 +1037,7 @@ hipError_t launch_decode_batch(const DecodeBatchArgs &b, int n_seq, hipStream_t 
     case 512: e = launch_split_batch<512, 4>(b, n_seq, max_splits, s); break;
     case 32: e = w8 ? launch_split_batch<32, 8>(b, n_seq, max_splits, s) : launch_split_batch<32, 4>(b, n_seq, max_splits, s); break;
     case 64: e = w8 ? launch_split_batch<64, 8>(b, n_seq, max_splits, s) : launch_split_batch<64, 4>(b, n_seq, max_splits, s); break;
+    case 96: e = w8 ? launch_split_batch<96, 8>(b, n_seq, max_splits, s) : launch_split_batch<96, 4>(b, n_seq, max_splits, s); break;
     case 128: e = w8 ? launch_split_batch<128, 8>(b, n_seq, max_splits, s) : launch_split_batch<128, 4>(b, n_seq, max_splits, s); break;
     case 256: e = w8 ? launch_split_batch<256, 8>(b, n_seq, max_splits, s) : launch_split_batch<256, 4>(b, n_seq, max_splits, s); break;
     default: break;

@@ -878,6 +878,7 @@ hipError_t launch_f32_split(const DecodeArgs &a, hipStream_t s) {
         switch (a.g.P) {
         case 32: return w8 ? launch_f32_decode<32, 8>(a, grid, s) : launch_f32_decode<32, 4>(a, grid, s);
         case 64: return w8 ? launch_f32_decode<64, 8>(a, grid, s) : launch_f32_decode<64, 4>(a, grid, s);
+        case 96: return w8 ? launch_f32_decode<96, 8>(a, grid, s) : launch_f32_decode<96, 4>(a, grid, s);
         case 128: return w8 ? launch_f32_decode<128, 8>(a, grid, s) : launch_f32_decode<128, 4>(a, grid, s);
         case 256: return w8 ? launch_f32_decode<256, 8>(a, grid, s) : launch_f32_decode<256, 4>(a, grid, s);
         default: break;
@@ -887,6 +888,7 @@ hipError_t launch_f32_split(const DecodeArgs &a, hipStream_t s) {
     switch (a.g.P) {
     case 32: return launch_f32<32>(a, grid, s);
     case 64: return launch_f32<64>(a, grid, s);
+    case 96: return launch_f32<96>(a, grid, s);
     case 128: return launch_f32<128>(a, grid, s);
     case 256: return launch_f32<256>(a, grid, s);
     case 512: return launch_f32<512>(a, grid, s);
@@ -918,6 +920,7 @@ hipError_t launch_f32_split_batch(const DecodeBatchArgs &b, int n_seq, int max_s
     switch (a0.g.P) {
     case 32: return w8 ? launch_f32_batch<32, 8>(b, n_seq, max_splits, s) : launch_f32_batch<32, 4>(b, n_seq, max_splits, s);
     case 64: return w8 ? launch_f32_batch<64, 8>(b, n_seq, max_splits, s) : launch_f32_batch<64, 4>(b, n_seq, max_splits, s);
+    case 96: return w8 ? launch_f32_batch<96, 8>(b, n_seq, max_splits, s) : launch_f32_batch<96, 4>(b, n_seq, max_splits, s);
     case 128: return w8 ? launch_f32_batch<128, 8>(b, n_seq, max_splits, s) : launch_f32_batch<128, 4>(b, n_seq, max_splits, s);
     case 256: return w8 ? launch_f32_batch<256, 8>(b, n_seq, max_splits, s) : launch_f32_batch<256, 4>(b, n_seq, max_splits, s);
     default: return hipErrorInvalidValue;

@@ -81,7 +81,7 @@ __global__ __launch_bounds__(256) void f32_terms_kernel(DecodeArgs a, ChunkPages
             }
         } else {
             // dims d0 .. d0 + 7 of a row: two units of its tile, 16 apart
-            const int du = i & (PLANE / 2 - 1), pg = i / (PLANE / 2), d0 = (du >> 4) * 8;
+            const int pg = i / (PLANE / 2), du = i - pg * (PLANE / 2), d0 = (du >> 4) * 8;
             const float *k = (pg ? tile[1] : tile[0]) + ((du >> 5) * 64 + ((du >> 4) & 1) * 32 + (du & 15)) * 4;
             const int p = (pg ? pos[1] : pos[0]) + (du & 15);
             const bool nw = fresh && is_new(pg, p);
@@ -168,7 +168,13 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
     constexpr int ITEM = HALVES * 3 * PLANE;     // units of a group's K (or V): [half][term][PLANE]
     constexpr int GP = 2 * HALVES;               // pages of a group: a pair for each half
     constexpr int NBUF = f32_prefill_buffers(P, MADE);
-    constexpr int CPW = (ITEM / 64 + WAVES - 1) / WAVES; // MADE: KiB of an item that a wavefront copies
+    constexpr int HALF_KIB = 3 * PLANE / 64;
+    // MADE: KiB of an item that a wavefront copies (of two pairs: a number that divides a pair's)
+    constexpr int CPW = [] {
+        int n = (ITEM / 64 + WAVES - 1) / WAVES;
+        while (HALVES > 1 && HALF_KIB % n != 0) ++n;
+        return n;
+    }();
     constexpr int CU = (HALVES * PLANE + THREADS - 1) / THREADS; // else: units of K, and of V, a thread makes per group
     constexpr bool FULL = HALVES * PLANE % THREADS == 0;
     extern __shared__ __attribute__((aligned(16))) u4 kv_planes[]; // [NBUF][ITEM] (not MADE: K, V)
@@ -215,7 +221,6 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
     // item 2 g + 1. Pairs past the end are the last one again, unused.
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)kv_planes;
     const uint32_t lane_at = (uint32_t)lane * 16;
-    constexpr int HALF_KIB = 3 * PLANE / 64;
     static_assert(!MADE || HALF_KIB % CPW == 0 || HALVES == 1, "a wavefront copies from one pair");
     const int kib0 = min(wave * CPW, ITEM / 64 - CPW); // (the last ones may copy the same)
     const u4 *const terms_kvh = reinterpret_cast<const u4 *>(terms.terms) + (size_t)kvh * terms.held * 2 * 3 * PLANE;
@@ -261,7 +266,7 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
         for (int u = 0; u < CU; ++u) {
             const int i = tid + u * THREADS;
             const int pg = min(__builtin_amdgcn_readfirstlane(i / (PLANE / 2)), GP - 1);
-            const int du = i & (PLANE / 2 - 1);
+            const int du = i % (PLANE / 2);
             const float4_t *t = tile_of(it0, d + pg, false) + (du >> 5) * 64 + ((du >> 4) & 1) * 32 + (du & 15);
             kx[u][0] = t[0];
             kx[u][1] = t[16];
@@ -272,8 +277,8 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
         for (int u = 0; u < CU; ++u) {
             const int i = tid + u * THREADS;
             const int pr = min(__builtin_amdgcn_readfirstlane(i / PLANE), HALVES - 1);
-            vx[u][0] = tile_of(it0, d + 2 * pr, true)[i & (PLANE - 1)];
-            vx[u][1] = tile_of(it0, d + 2 * pr + 1, true)[i & (PLANE - 1)];
+            vx[u][0] = tile_of(it0, d + 2 * pr, true)[i % PLANE];
+            vx[u][1] = tile_of(it0, d + 2 * pr + 1, true)[i % PLANE];
         }
     };
     // Keys that no slot of the workgroup attends: zero probability, but 0 x NaN is NaN, so on the
@@ -312,7 +317,7 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
             // K: [half][term][page of the pair][P/2 * 4 units]; V: [half][term][PLANE]
             const int h = i / PLANE;
             if (FULL || h < HALVES) {
-                u4 *dst = kv_planes + (v ? V_AT : 0) + h * 3 * PLANE + (i & (PLANE - 1));
+                u4 *dst = kv_planes + (v ? V_AT : 0) + h * 3 * PLANE + i % PLANE;
                 dst[0] = u4{t0[0], t0[1], t0[2], t0[3]};
                 dst[PLANE] = u4{t1[0], t1[1], t1[2], t1[3]};
                 dst[2 * PLANE] = u4{t2[0], t2[1], t2[2], t2[3]};
@@ -753,7 +758,8 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
         const int G = g.gqa;
         auto limit_of = [&](int slot) { return a.q_pos0 + slot / G; };
         auto ws_of = [&](int slot) { return a.window > 0 ? max(a.window_start, limit_of(slot) + 1 - a.window) : a.window_start; };
-        constexpr int VT = NT < 8 ? NT : 8, KT = NT < 4 ? NT : 4;
+        constexpr int VT = NT < 8 ? NT : 8, KT = NT % 4 == 0 ? 4 : NT % 3 == 0 ? 3 : NT;
+        static_assert(NT % VT == 0 && NT % KT == 0, "whole steps");
         const float *qrow = a.q + ((long)(slot / G) * g.q_heads + kvh * G + slot % G) * g.head_dim;
         const int lo0 = ws_of(slot), hi0 = limit_of(slot);
 #pragma unroll 1
@@ -914,6 +920,7 @@ hipError_t launch_f32_terms(const DecodeArgs &a, const ChunkPages &c, const Term
         break
         SKV_TERMS(32);
         SKV_TERMS(64);
+        SKV_TERMS(96);
         SKV_TERMS(128);
         SKV_TERMS(256);
 #undef SKV_TERMS
@@ -951,6 +958,7 @@ hipError_t launch_f32_prefill(const DecodeArgs &a, const ChunkPages &c, const Te
     switch (a.g.P) {
     case 32: return halves ? launch_f32_prefill_p<32, 1, 8, 2>(a, c, t, grid, s) : launch_f32_prefill_p<32, 1, 8, 1>(a, c, t, grid, s);
     case 64: return halves ? launch_f32_prefill_p<64, 1, 8, 2>(a, c, t, grid, s) : launch_f32_prefill_p<64, 1, 8, 1>(a, c, t, grid, s);
+    case 96: return halves ? launch_f32_prefill_p<96, 1, 8, 2>(a, c, t, grid, s) : launch_f32_prefill_p<96, 1, 8, 1>(a, c, t, grid, s);
     case 128: return halves ? launch_f32_prefill_p<128, 1, 8, 2>(a, c, t, grid, s) : launch_f32_prefill_p<128, 1, 8, 1>(a, c, t, grid, s);
     case 256: return launch_f32_prefill_p<256, 1, 8, 1>(a, c, t, grid, s);
     default: return hipErrorInvalidValue;

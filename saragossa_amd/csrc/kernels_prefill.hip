@@ -245,7 +245,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
     for (int u = 0; u < (GP * TILE_U4 + THREADS - 1) / THREADS; ++u) {
         const int i0 = wave * 64 + u * THREADS;
         if (GP * TILE_U4 % THREADS == 0 || i0 < GP * TILE_U4)
-            copy_to_lds(tile_of(0, i0 / TILE_U4, false) + (i0 & (TILE_U4 - 1)), lane_at, lds0 + (uint32_t)(BUF_U4 + i0) * 16);
+            copy_to_lds(tile_of(0, i0 / TILE_U4, false) + i0 % TILE_U4, lane_at, lds0 + (uint32_t)(BUF_U4 + i0) * 16);
     }
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
@@ -737,7 +737,7 @@ hipError_t launch_merge_append(const DecodeArgs &a, const AppendArgs &w, hipStre
 int prefill_tile_slots(int P, TileShape shape) {
     if (P > 256) return 64; // four wavefronts, one per SIMD (the accumulators and query halves are 256 registers)
     if (shape == TileShape::two_tiles && P <= 128) return 256;
-    return shape == TileShape::halves || (shape == TileShape::quarters && P == 128) ? 64 : 128;
+    return shape == TileShape::halves || (shape == TileShape::quarters && P > 64 && P <= 128) ? 64 : 128;
 }
 
 template <int P, int TILES, int SP, int WAVES, int HALVES, bool RING>
@@ -770,6 +770,10 @@ hipError_t launch_prefill_tiles(const DecodeArgs &a, const ChunkPages &c, TileSh
     case 64:
         if (halves) return launch_tiles<64, 1, 2, 8, 2>(a, c, grid, s);
         return two ? launch_tiles<64, 2, 4>(a, c, grid, s) : launch_tiles<64, 1, 4>(a, c, grid, s);
+    case 96:
+        if (shape == TileShape::quarters) return launch_tiles<96, 2, 1, 8, 4>(a, c, grid, s);
+        if (halves) return launch_tiles<96, 1, 2, 8, 2>(a, c, grid, s);
+        return two ? launch_tiles<96, 2, 2>(a, c, grid, s) : launch_tiles<96, 1, 4>(a, c, grid, s);
     case 128:
         if (shape == TileShape::quarters) return launch_tiles<128, 2, 1, 8, 4>(a, c, grid, s);
         if (halves) return launch_tiles<128, 1, 2, 8, 2>(a, c, grid, s);

@@ -116,10 +116,18 @@ hipError_t static_scratch_ptr(int device, void **ptr) {
     return hipSuccess;
 }
 
+// Dims of a tile's row: whole K-steps of 32, where kernels are built for them. (96 for the heads of 65 to 96 dims: with 128, a
+// quarter of their bytes and products was padding.)
 int padded_head_dim(size_t hd) {
-    for (int p : {32, 64, 128, 256, 512})
+    for (int p : {32, 64, 96, 128, 256, 512})
         if ((size_t)p >= hd) return p;
     return 0;
+}
+// Elements of a row that a layer's pools have room for: a power of two, as callers who budget by skv_layer_bytes know it.
+size_t pool_head_dim(size_t hd) {
+    size_t p = 32;
+    while (p < hd) p *= 2;
+    return p;
 }
 
 size_t env_usize(const char *name, size_t dflt) {
@@ -192,8 +200,7 @@ size_t decode_target_wgs() { return tuning().target_wgs; }
 // tiles / halves / quarters, in us on one MI355X: 512 rows of q32/kv8/hd128 over 512, 2048, 4096, 8192 rows
 // 34.7/40.1/25.8/30.3, 54.9/58.2/51.7/51.5, 81.7/82.2/84.5/78.5, 135/129/149/133; 256 rows over 2048, 4096, 16384
 // 36.9/43.9/35.9/39.1, 50.3/55.5/52.1/52.2, 131/127/151/132; 1024 rows over 4096, 8192 145/149/161/157,
-// 252/244/282/266; q12/kv4/hd96, 512 rows over 4096 43.1/49.1/51.7/51.1, 1024 rows over 2048, 4096
-// 56.8/55.2/53.8/55.3, 81.5/72.6/90.5/81.5; q8/kv2/hd64, 256 rows over 4096, 16384 24.9/29.5/21.6/24.9,
+// 252/244/282/266; q12/kv4/hd96, 512 rows over 4096, 16000 36.5/40.9/45.2/41.0, 82.7/80.4/129/101; q8/kv2/hd64, 256 rows over 4096, 16384 24.9/29.5/21.6/24.9,
 // 37.6/45.0/38.9/38.5, 1024 rows over 4096, 16384 36.3/41.9/37.2/37.4, 85.9/82.7/109/92.6; q16/kv2/hd256 (one tile /
 // halves), 512 rows over 512, 2048, 4096, 8192 38.6/37.5, 57.1/56.7, 82.0/82.4, 131/134, 1024 rows over 2048, 8192
 // 101/91.0, 245/246.
@@ -201,16 +208,20 @@ size_t decode_target_wgs() { return tuning().target_wgs; }
 // 256 only four fit, and up to 48 compute units stay idle. 400 rows (200 workgroups) of q32/kv8/hd128 at walks of 55000, 75000,
 // 98000, two tiles / quarters 76.4/74.0, 93.0/93.7, 113/118; 416 rows (208) 73.5/70.6, 90.2/90.0, 110/113; 448 (224) 71.1/67.2,
 // 86.0/84.8, 105/107; 480 (240) 70.2/63.8, 84.6/80.2, 102/101; 512 (256) 67.1/60.6, 82.5/77.2, 98.4/97.0 (halves 58.6, 77.1,
-// 108). At head_dim 96 they are up to 4 % behind the better of one and two tiles (q30/kv10, 448 rows 62.1/62.5 and 88.7/92.0).
+// 108). Heads of 65 to 96 dims walk a pair in less time, so that joining the states weighs more and the reads of LDS less: quarters from
+// shorter walks on, to shorter ones. q12/kv4/hd96, 1024 rows (192) over 300, 1000, 2048, 4096 31.6/35.5/25.1/26.8,
+// 37.5/39.8/34.7/33.2, 46.5/45.9/48.3/42.9, 64.9/58.6/75.5/62.1; q30/kv10/hd96, 448 rows (210) over 500, 1200, 3000, 5000
+// 27.7/33.0/22.8/24.7, 33.8/37.2/32.3/31.1, 51.0/51.8/56.9/48.7, 69.8/68.9/85.7/68.8.
 TileShape prefill_shape(const Geom &g, size_t n_slots, size_t n_pages) {
     if (g.P > 256) return TileShape::one_tile;
     const long knob = tuning().prefill_tiles2_min_pages;
     if (knob >= 0) return g.P <= 128 && (long)n_pages >= knob ? TileShape::two_tiles : TileShape::one_tile;
     const size_t wgs = (n_slots + 63) / 64 * (size_t)g.kv_heads, walk = wgs * n_pages;
-    if (g.P == 128 && wgs <= 256) {
+    if (g.P > 64 && g.P <= 128 && wgs <= 256) {
         if (wgs < 192) return walk < 20000 ? TileShape::halves : walk < 95000 ? TileShape::one_tile : TileShape::two_tiles;
-        if (walk < 41000) return TileShape::halves;
-        return wgs >= 208 && walk < 100000 ? TileShape::quarters : TileShape::two_tiles;
+        if (walk < (g.P == 96 ? 24000u : 41000u)) return TileShape::halves;
+        const size_t quarters_to = g.P == 96 ? (wgs >= 208 ? 75000 : 50000) : wgs >= 208 ? 100000 : 0;
+        return walk < quarters_to ? TileShape::quarters : TileShape::two_tiles;
     }
     if (wgs <= 256 && walk < (wgs >= 192 ? 110000u : 40000u)) return TileShape::halves;
     return g.P <= 128 && walk >= (wgs <= 256 ? 110000u : 250000u) ? TileShape::two_tiles : TileShape::one_tile;
@@ -229,7 +240,7 @@ TileShape prefill_shape(const Geom &g, size_t n_slots, size_t n_pages) {
 // 1024, 2048: 17.0/16.0, 19.1/19.8; 512 rows over 512, 1024: 16.6/15.1, 17.7/19.0.
 bool takes_tile_kernel(const Geom &g, size_t n_slots, size_t n_pages) {
     if (tuning().prefill_tiles != 1 || n_slots < 64) return tuning().prefill_tiles > 1 && n_slots >= 64;
-    const size_t limit = g.P <= 64 ? 18000 : g.P == 128 ? 42000 : g.P == 256 ? 22000 : 6000;
+    const size_t limit = g.P <= 64 ? 18000 : g.P <= 128 ? 42000 : g.P == 256 ? 22000 : 6000;
     return (n_slots + 15) / 16 * (size_t)g.kv_heads * n_pages >= limit;
 }
 
@@ -248,7 +259,7 @@ bool takes_f32_chunk_kernel(const Geom &g, size_t n_queries, size_t n_pages) {
     const size_t n_slots = n_queries * (size_t)g.gqa;
     if (f32_prefill_slots(g.P, false) == 0 || n_slots < 64 || tuning().prefill_tiles == 0) return false;
     if (tuning().prefill_tiles > 1) return true;
-    const size_t limit = g.P <= 64 ? 26000 : g.P == 128 ? 16200 : 12200;
+    const size_t limit = g.P <= 64 ? 26000 : g.P <= 128 ? 16200 : 12200;
     const size_t walked = n_pages > n_queries / 32 ? n_pages - n_queries / 32 : 1;
     return (n_slots + 15) / 16 * (size_t)g.kv_heads * walked >= limit;
 }
@@ -476,7 +487,7 @@ bool capturing(hipStream_t s) {
 // their own. Whole chunks on layers that are in no cache, in us, split by the workgroup / by a launch: q32/kv8/hd128, 512 rows over 0, 512,
 // 1024, 2048, 4096 39.4/33.0, 59.2/51.3, 81.2/68.3, 116/108, 194/185, 256 rows (1024 slots) over 500, 2048, 8192 37.4/36.4, 64.0/65.2,
 // 178/190, 64 rows over 8192 63.3/81.6; q28/kv4/hd128, 160 rows over 3000 56.2/57.1, 512 over 16000 611/556; q12/kv4/hd96, 512 rows
-// (1536 slots) over 2000 57.2/55.7; q8/kv2/hd64, 512 rows over 2048, 4096 30.3/27.5, 42.1/38.9, 300 over 10000 54.5/55.7; q16/kv2/hd256,
+// (1536 slots) over 2000 50.7/50.6; q8/kv2/hd64, 512 rows over 2048, 4096 30.3/27.5, 42.1/38.9, 300 over 10000 54.5/55.7; q16/kv2/hd256,
 // 128 rows (1024 slots) over 4096 71.1/70.3, 256 106/102, 512 190/174, over 16000 256 320/304; q16/kv8/hd256, 512 rows
 // (1024 slots) over 1000 84.2/85.2. Rings: q16/kv8/hd256 of 1024 rows, 64, 256, 512, 1024 rows 62.3/57.0, 67.7/62.5, 76.3/75.9, 120/120;
 // q32/kv8/hd128 of 512 and 1024, 64, 512 rows 32.4/27.7, 48.2/41.2, 128, 256 34.7/33.6, 48.2/43.4; q8/kv2/hd64 128 rows 22.4/19.0.
@@ -516,8 +527,7 @@ F32Plan plan_f32_chunk(const Geom &g, size_t n_queries, int first_entry, int ent
     // Halves cover half the slots and walk two pairs at a time: the same time per workgroup with half as many splits, so fewer
     // partials, but they copy each page for half as many slots, which costs more on long walks. Whole chunks, one tile / halves, in us: q32/kv8/hd128, 512 rows
     // over 512, 1024, 2048, 6000, 8192 (two splits / one) 59.1/51.2, 74.5/68.5, 114/109, 262/265, 340/349; q8/kv2/hd64, 512 rows over 2048, 4096,
-    // 10000 (eight / four) 32.2/28.0, 42.5/40.0, 74.0/72.7; but q28/kv4/hd128, 300 rows over 3000 (three / one) 91.2/115,
-    // q12/kv4/hd96, 512 rows over 2000 (five / two) 56.1/60.3.
+    // 10000 (eight / four) 32.2/28.0, 42.5/40.0, 74.0/72.7; but q28/kv4/hd128, 300 rows over 3000 (three / one) 91.2/115.
     const size_t pages = (size_t)walked / (size_t)p.segments;
     const int one = chunk_splits(g, n_queries, (size_t)f32_prefill_slots(g.P, false), pages);
     const int two = chunk_splits(g, n_queries, (size_t)f32_prefill_slots(g.P, true), pages);
@@ -907,7 +917,7 @@ static int32_t plan_layer(size_t capacity, size_t q_heads, size_t kv_heads, size
         rows = ring;
     }
     p.n_pages = (int)((rows + 15) / 16);
-    p.pool_bytes = (size_t)p.n_pages * g.page_elems * sizeof(uint16_t);
+    p.pool_bytes = (size_t)p.n_pages * kv_heads * pool_head_dim(head_dim) * 16 * (f32 ? sizeof(float) : sizeof(uint16_t));
     p.max_splits = std::min(decode_max_splits(), std::max(1, p.n_pages));
     const size_t n_part = (size_t)kv_heads * p.max_splits * g.gqa;
     p.table_bytes = (size_t)p.n_pages * sizeof(int32_t);

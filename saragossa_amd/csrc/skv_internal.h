@@ -51,7 +51,7 @@ int32_t fail_hip(hipError_t e, const char *what);
 //   V tile [P/32][4 row-quads][16 cols][2][4 rows]  element (row r, dim d) at
 //          ((((d/32)*4 + r/4)*16 + d%16)*2 + (d%32)/16)*4 + r%4
 //
-// P is head_dim rounded up to 32, 64, 128, 256 or 512; dims in [head_dim, P) stay zero.
+// P is head_dim rounded up to 32, 64, 96, 128, 256 or 512; dims in [head_dim, P) stay zero.
 struct Geom {
     int q_heads;
     int kv_heads;
@@ -286,7 +286,7 @@ __device__ __forceinline__ float head_inv_rms(const float *row, int head_dim, fl
     return 1.0f / sqrtf(mean_square + eps);
 }
 // The same from the squares, already taken (x * x, rounded) and padded with zeros to PADDED entries
-// (32, 64 or a multiple of 128) at a 16-byte aligned address: the adds stay in index order, the
+// (32, 64, 96 or a multiple of 128) at a 16-byte aligned address: the adds stay in index order, the
 // 16-byte loads of a round are asked for before the adds of the round before (asked for four at a time and
 // waited for, the LDS's latency was as long again as the adds). The loop stays a loop: unrolled, every
 // load moves to its top and the page registers of the caller spill.
@@ -294,8 +294,9 @@ template <int PADDED>
 __device__ __forceinline__ float head_inv_rms_sq(const float *sq, int head_dim, float eps) {
 #pragma clang fp contract(off)
     typedef __attribute__((ext_vector_type(4))) float f4;
-    constexpr int R = PADDED <= 64 ? PADDED / 8 : PADDED <= 128 ? 8 : 4; // units of a round
-    constexpr int N = PADDED / (8 * R);                                  // pairs of rounds
+    constexpr int R = PADDED <= 64 ? PADDED / 8 : PADDED == 96 ? 6 : PADDED <= 128 ? 8 : 4; // units of a round
+    constexpr int N = PADDED / (8 * R);                                                     // pairs of rounds
+    static_assert(N * 8 * R == PADDED, "every square is added");
     const f4 *p = reinterpret_cast<const f4 *>(sq);
     float sum = 0.0f;
     f4 x[R], y[R];
