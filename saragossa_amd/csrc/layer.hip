@@ -227,21 +227,31 @@ TileShape prefill_shape(const Geom &g, size_t n_slots, size_t n_pages) {
     return g.P <= 128 && walk >= (wgs <= 256 ? 110000u : 250000u) ? TileShape::two_tiles : TileShape::one_tile;
 }
 
-// Whether a chunk of n_slots query slots per kv head over n_pages pages takes the kernel that shares each
-// page among 64 to 256 slots through LDS, or the decode kernel's multi-query mode (speculative verify rows,
-// short chunks over short contexts): one workgroup per 16 slots that streams the pages into its own
-// registers, without a prologue to speak of, but asks for every page once per 16 slots. The line is
-// the number of (16 slots, page) pairs where those requests cost what the tile kernel's start does.
-// Whole chunks, tile kernel / multi-query mode, in us on one MI355X: q32/kv8/hd128, 32 rows over 2048,
-// 8192, 32000 rows: 21.5/15.6, 32.1/25.9, 53.9/80.2; 256 rows over 1024, 2048: 28.5/24.1, 35.3/35.7; 512 rows over
-// 0, 512: 19.7/19.4, 26.8/32.5; q16/kv2/hd256, 16 rows over 8192, 32000: 37.5/19.7, 58.0/44.9; 64 rows over
-// 2048, 8192: 29.8/25.2, 41.7/40.5; 256 rows over 1024, 2048: 34.5/30.1, 39.2/44.6; q8/kv2/hd512, 64 rows over 2048,
-// 8192: 43.4/36.6, 55.6/77.5; 128 rows over 1024, 2048: 43.4/42.3, 46.1/54.7; q8/kv2/hd64, 256 rows over
-// 1024, 2048: 17.0/16.0, 19.1/19.8; 512 rows over 512, 1024: 16.6/15.1, 17.7/19.0.
-bool takes_tile_kernel(const Geom &g, size_t n_slots, size_t n_pages) {
+// Whether a chunk of n_queries rows over n_pages pages takes the kernel that shares each page among 64 to 256 query slots
+// through LDS, or the decode kernel's multi-query mode (speculative verify rows, short chunks over short contexts): one workgroup
+// per 16 slots that streams the pages into its own registers, without a prologue to speak of, but asks for every page once per 16
+// slots. The line is the number of (16 slots, page) pairs, as a chunk's rows walk them on the average, where those requests cost
+// what the tile kernel's start does; and that start is one workgroup's on every compute unit, with no split and no merge, where
+// the chunk's 64-slot workgroups are 208 to 256. Over 136 chunks of 32 to 2048 rows over 0 to 16000 the kernel chosen is at most 12 %
+// slower than the other but for one (256 rows of q8/kv2/hd512 over none, 38.3/30.1), 0.9 % on the average (by all pages, and lower
+// lines, 51 % and 3.5 %). Whole chunks, multi-query mode / tile
+// kernel, in us on one MI355X, with the pairs they walk in thousands: q32/kv8/hd128, 512 rows over 0, 100, 300 (16, 24, 36; 256
+// workgroups) 19.1/18.3, 22.6/20.4, 28.0/23.3; 128 over 2000 (33) 21.4/26.3; 256 over 1000, 1500 (36, 53) 25.4/27.6, 32.1/31.3;
+// q28/kv4/hd128, 512 over 500 (43) 31.6/25.4, 128 over 4000 (57) 31.9/31.8; q16/kv2/hd256, 512 over 500, 1000 (25, 40) 33.0/36.8, 43.7/42.7,
+// 256 over 1000, 2000 (18, 34) 23.9/32.0, 35.0/38.3, 64 over 4000, 8000 (16, 32) 28.6/33.3, 40.5/38.9, 850 over none (24; 214) 42.7/33.1;
+// q12/kv4/hd96, 512 over 1000, 2000 (30, 54) 19.5/23.6, 27.3/30.8, 128 over 8000 (48) 33.4/28.8; q8/kv2/hd64, 512 over 1000, 2000 (20, 36)
+// 12.9/16.0, 16.4/18.1, 256 over 4000 (33) 19.5/19.6; q32/kv8/hd64, 512 over 0, 400 (16, 42; 256) 13.7/13.0, 20.8/17.9; q8/kv2/hd512, 64
+// over 1000 (2) 29.9/36.5, 512 over none (4) 37.3/40.3; q16/kv8/hd512, 64 over 1000 (4) 41.6/39.0.
+bool takes_tile_kernel(const Geom &g, size_t n_queries, size_t n_pages) {
+    const size_t n_slots = n_queries * (size_t)g.gqa;
     if (tuning().prefill_tiles != 1 || n_slots < 64) return tuning().prefill_tiles > 1 && n_slots >= 64;
-    const size_t limit = g.P <= 64 ? 18000 : g.P <= 128 ? 42000 : g.P == 256 ? 22000 : 6000;
-    return (n_slots + 15) / 16 * (size_t)g.kv_heads * n_pages >= limit;
+    const size_t wgs = (n_slots + 63) / 64 * (size_t)g.kv_heads;
+    const size_t walked = n_pages > n_queries / 32 ? n_pages - n_queries / 32 : 1;
+    size_t line = g.P <= 32 ? 32500 : g.P <= 64 ? 38000 : g.P <= 96 ? 42000 : g.P <= 128 ? 40000 : g.P <= 256 ? 30000 : 4100;
+    // (on a ring that has not wrapped yet the multi-query mode looks at the position of every key: 512 rows of q16/kv8/hd256 over 400,
+    // 512 (21, 25) 36.9/37.8, 40.0/38.8)
+    if (g.ring_rows > 0) line = line / 4 * 3;
+    return (n_slots + 15) / 16 * (size_t)g.kv_heads * walked >= (wgs >= 208 && wgs <= 256 ? std::min<size_t>(line, 12000) : line);
 }
 
 // The same questions for f32 layers: the kernel that splits its factors into bf16 terms (head_dim up to
@@ -722,7 +732,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
         a.gate = pre->gate;
         a.q_head_stride = pre->q_head_stride;
     }
-    const bool use_tiles = n_queries > 1 && takes_tile_kernel(g, n_queries * (size_t)g.gqa, (size_t)a.n_pages);
+    const bool use_tiles = n_queries > 1 && takes_tile_kernel(g, n_queries, (size_t)a.n_pages);
     TileShape shape = TileShape::one_tile;
     if (n_queries > 1) {
         // split the context only while the query tiles alone leave compute units idle, and
@@ -1471,7 +1481,7 @@ int32_t skv_prefill_chunk_device(skv_layer *L, skv_stream stream, const float *q
         // a few rows over a full bf16 layer (a speculative verify, the rest of a prompt): the multi-query launch
         // appends them itself, as a decode step's does (its last query tile, which sees all of them, stores them)
         if (c > 1 && c <= (size_t)MQ_APPEND_ROWS && ring == 0 && !L->g.f32 && tuning().fused_append &&
-            !context_over_rows(L, c, out, k, v) && !takes_tile_kernel(L->g, c * (size_t)L->g.gqa, (L->len + c + 15) / 16)) {
+            !context_over_rows(L, c, out, k, v) && !takes_tile_kernel(L->g, c, (L->len + c + 15) / 16)) {
             RowsAhead ahead(L, c);
             rc = encode_attention(L, as_stream(stream), q, out, 0, k, v, c);
             if (rc) return rc;
