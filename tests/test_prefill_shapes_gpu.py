@@ -149,26 +149,28 @@ def test_chunks_that_quarters_take(state, head_dim, window, base, rows):
     (27, 96, 0, 37, 481),    # 216, whose last ones are half full
     (32, 40, 1024, 0, 511),  # 256, on a ring that has not wrapped
 ])
-def test_first_chunks_of_a_workgroup_to_each_compute_unit(state, heads, head_dim, window, base, rows):
+@pytest.mark.parametrize("element", ["bf16", "f32"])
+def test_first_chunks_of_a_workgroup_to_each_compute_unit(state, element, heads, head_dim, window, base, rows):
     """Short walks of as many slots as the compute units take at once, on both sides of the line between the kernels."""
     import torch
     n = base + rows
     gen = torch.Generator().manual_seed(n)
     k, v = (torch.randn(n, heads * head_dim, generator=gen) for _ in range(2))
     q = torch.randn(rows, heads * head_dim, generator=gen)
-    kv = state.full_attention_bf16(n, heads, heads, head_dim, window=window)
+    make = state.full_attention_f32 if element == "f32" else state.full_attention_bf16
+    kv = make(n, heads, heads, head_dim, window=window)
     if base:
         kv.seed(k[:base].numpy(), v[:base].numpy(), base)
     got = torch.from_numpy(kv.prefill_rows(q.numpy(), k[base:].numpy(), v[base:].numpy()))
     hidden = torch.arange(n)[None] > base + torch.arange(rows)[:, None]
-    k, v = (x.bfloat16().double() for x in (k, v))
+    k, v = (x.double() if element == "f32" else x.bfloat16().double() for x in (k, v))
     want = torch.empty(rows, heads * head_dim, dtype=torch.float64)
     for h in range(heads):
         cols = slice(h * head_dim, (h + 1) * head_dim)
         s = q[:, cols].double() @ k[:, cols].T.contiguous() / head_dim ** 0.5
         want[:, cols] = torch.softmax(s.masked_fill(hidden, -float("inf")), -1) @ v[:, cols]
-    # queries and probabilities in two 8-bit terms: 2^-16 of scores up to 6, and of the probabilities
-    assert (got.double() - want).abs().max() <= 7 * 2.0 ** -16 * want.abs().max()
+    # bf16: queries and probabilities in two 8-bit terms, 2^-16 of scores up to 6, and of the probabilities; f32: sums of up to 600 products
+    assert (got.double() - want).abs().max() <= (2e-5 if element == "f32" else 7 * 2.0 ** -16 * want.abs().max())
 
 
 @pytest.mark.parametrize("dims,window,start,counts", [
