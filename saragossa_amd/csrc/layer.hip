@@ -196,35 +196,39 @@ size_t decode_target_wgs() { return tuning().target_wgs; }
 // the device with fewer splits, or with none where 128-slot workgroups need two and a merge; they
 // copy each page for half as many slots. Quarters (head_dim 65 to 128) read LDS half as often per product as
 // halves but walk eight pages at a time and join four states. Two tiles read LDS half as often too, and need
-// the most splits: they pay on long walks. Whole chunks over layers that are not in any cache, one tile / two
-// tiles / halves / quarters, in us on one MI355X: 512 rows of q32/kv8/hd128 over 512, 2048, 4096, 8192 rows
-// 34.7/40.1/25.8/30.3, 54.9/58.2/51.7/51.5, 81.7/82.2/84.5/78.5, 135/129/149/133; 256 rows over 2048, 4096, 16384
-// 36.9/43.9/35.9/39.1, 50.3/55.5/52.1/52.2, 131/127/151/132; 1024 rows over 4096, 8192 145/149/161/157,
-// 252/244/282/266; q12/kv4/hd96, 512 rows over 4096, 16000 36.5/40.9/45.2/41.0, 82.7/80.4/129/101; q8/kv2/hd64, 256 rows over 4096, 16384 24.9/29.5/21.6/24.9,
-// 37.6/45.0/38.9/38.5, 1024 rows over 4096, 16384 36.3/41.9/37.2/37.4, 85.9/82.7/109/92.6; q16/kv2/hd256 (one tile /
-// halves), 512 rows over 512, 2048, 4096, 8192 38.6/37.5, 57.1/56.7, 82.0/82.4, 131/134, 1024 rows over 2048, 8192
-// 101/91.0, 245/246.
-// Quarters from 208 workgroups of 64 slots on: up to 204, two-tile workgroups fill the device in five splits; from there to
-// 256 only four fit, and up to 48 compute units stay idle. 400 rows (200 workgroups) of q32/kv8/hd128 at walks of 55000, 75000,
-// 98000, two tiles / quarters 76.4/74.0, 93.0/93.7, 113/118; 416 rows (208) 73.5/70.6, 90.2/90.0, 110/113; 448 (224) 71.1/67.2,
-// 86.0/84.8, 105/107; 480 (240) 70.2/63.8, 84.6/80.2, 102/101; 512 (256) 67.1/60.6, 82.5/77.2, 98.4/97.0 (halves 58.6, 77.1,
-// 108). Heads of 65 to 96 dims walk a pair in less time, so that joining the states weighs more and the reads of LDS less: quarters from
-// shorter walks on, to shorter ones. q12/kv4/hd96, 1024 rows (192) over 300, 1000, 2048, 4096 31.6/35.5/25.1/26.8,
-// 37.5/39.8/34.7/33.2, 46.5/45.9/48.3/42.9, 64.9/58.6/75.5/62.1; q30/kv10/hd96, 448 rows (210) over 500, 1200, 3000, 5000
-// 27.7/33.0/22.8/24.7, 33.8/37.2/32.3/31.1, 51.0/51.8/56.9/48.7, 69.8/68.9/85.7/68.8.
+// the most splits: they pay on long walks. Above 256 workgroups of 64 slots the device is full in any shape. The lines are in pages walked
+// by all 64-slot workgroups, where whole chunks cost the same in two shapes, between layers that are not in any cache and those that are, as a
+// short prompt's, where halves stay ahead for longer (512 rows of q32/kv8/hd64 over 2000, halves / two tiles 29.5/36.1 in
+// caches, 34.8/36.2 not; of q32/kv8/hd128 over 1024, halves / quarters 34.5/34.9 and 34.4/36.3, over 2048 46.8/47.6 and 50.5/46.8). Over 134
+// chunks of 128 to 1024 rows over 500 to 12000 the shape chosen is at most 11 % slower than the best, 1 % on the average (31 % and
+// 2.4 % with fewer, wider lines). One tile / two tiles / halves / quarters, in us on one MI355X, in no cache, with workgroups, walk in thousands: q32/kv8/hd128, 400 rows over 500, 1500, 3000, 6000 (200; 11, 24, 43,
+// 80) 32.5/37.2/25.0/27.2, 42.7/44.5/40.0/37.6, 59.5/59.7/64.0/55.0, 94.4/90.2/110/87.9, 512 over 1500, 6000 (256; 32, 104)
+// 48.0/49.8/42.8/40.8, 106/100/114/96.2; q28/kv4/hd128, 400 over 500, 1500, 6000 (176; 10, 21, 70) 31.8/36.6/23.8/26.3, 42.6/43.2/38.6/36.4,
+// 92.2/79.1/107/85.1; q24/kv8/hd128, 400 over 1500, 3000, 6000 (152; 18, 32, 61) 35.7/41.2/39.6/37.0, 48.5/51.5/63.4/54.3, 74.8/74.5/109/87.2, 512
+// over 3000, 6000 (192; 42, 78) 60.7/58.6/65.3/56.4, 94.9/84.8/112/89.1, 1024 over 1500 (384) 71.6/77.6/75.8/76.9; q32/kv8/hd64, 400 over 1500, 3000,
+// 6000 (200; 24, 43, 80) 29.8/31.7/28.2, 40.7/40.5/45.0, 63.2/57.8/75.8, 256 over 3000, 12000 (128; 26, 98) 29.1/32.5/30.5, 63.0/61.5/79.0;
+// q16/kv2/hd256 (one tile / halves), 400 over 3000, 6000 (100; 21, 40) 60.8/59.9, 87.5/92.4, 1024 over 1500, 6000 (256; 40, 112) 85.9/73.7, 191/186.
+// (Two tiles fill the device in five splits up to 204 workgroups; from there to 256 only four fit, and up to 48 compute units stay idle:
+// quarters stay ahead of them for longer there.) Heads of 65 to 96 dims walk a pair in less time, so that joining the states weighs more and the
+// reads of LDS less. q12/kv4/hd96, 512 rows over 4096, 16000 (96; 28, 98) 36.5/40.9/45.2/41.0, 82.7/80.4/129/101, 1024 rows over 300, 1000, 2048, 4096
+// (192; 16, 24, 37, 61) 31.6/35.5/25.1/26.8, 37.5/39.8/34.7/33.2, 46.5/45.9/48.3/42.9, 64.9/58.6/75.5/62.1; q30/kv10/hd96, 448 over 500, 1200, 3000, 5000
+// (210; 13, 22, 45, 72) 27.7/33.0/22.8/24.7, 33.8/37.2/32.3/31.1, 51.0/51.8/56.9/48.7, 69.8/68.9/85.7/68.8.
 TileShape prefill_shape(const Geom &g, size_t n_slots, size_t n_pages) {
     if (g.P > 256) return TileShape::one_tile;
     const long knob = tuning().prefill_tiles2_min_pages;
     if (knob >= 0) return g.P <= 128 && (long)n_pages >= knob ? TileShape::two_tiles : TileShape::one_tile;
     const size_t wgs = (n_slots + 63) / 64 * (size_t)g.kv_heads, walk = wgs * n_pages;
-    if (g.P > 64 && g.P <= 128 && wgs <= 256) {
-        if (wgs < 192) return walk < 20000 ? TileShape::halves : walk < 95000 ? TileShape::one_tile : TileShape::two_tiles;
-        if (walk < (g.P == 96 ? 24000u : 41000u)) return TileShape::halves;
-        const size_t quarters_to = g.P == 96 ? (wgs >= 208 ? 75000 : 50000) : wgs >= 208 ? 100000 : 0;
-        return walk < quarters_to ? TileShape::quarters : TileShape::two_tiles;
+    if (wgs > 256) return g.P <= 128 && walk >= 250000 ? TileShape::two_tiles : TileShape::one_tile;
+    if (g.P <= 64) {
+        if (walk < (wgs >= 192 ? 46000u : 26500u)) return TileShape::halves;
+        return wgs >= 192 || walk >= 90000 ? TileShape::two_tiles : TileShape::one_tile;
     }
-    if (wgs <= 256 && walk < (wgs >= 192 ? 110000u : 40000u)) return TileShape::halves;
-    return g.P <= 128 && walk >= (wgs <= 256 ? 110000u : 250000u) ? TileShape::two_tiles : TileShape::one_tile;
+    if (g.P > 128) return walk < (wgs >= 192 ? 130000u : 40000u) ? TileShape::halves : TileShape::one_tile;
+    const bool p96 = g.P <= 96;
+    if (wgs < (p96 ? 192u : 172u)) return walk < (p96 ? 20000u : 16000u) ? TileShape::halves : walk < 70000 ? TileShape::one_tile : TileShape::two_tiles;
+    if (walk < (p96 ? 24000u : wgs >= 208 ? 30000u : 19000u)) return TileShape::halves;
+    const size_t quarters_to = p96 ? (wgs >= 208 ? 75000 : 50000) : wgs >= 208 ? 105000 : wgs >= 196 ? 85000 : 55000;
+    return walk < quarters_to ? TileShape::quarters : TileShape::two_tiles;
 }
 
 // Whether a chunk of n_queries rows over n_pages pages takes the kernel that shares each page among 64 to 256 query slots
