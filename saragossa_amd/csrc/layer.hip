@@ -251,10 +251,7 @@ bool takes_tile_kernel(const Geom &g, size_t n_queries, size_t n_pages) {
     if (tuning().prefill_tiles != 1 || n_slots < 64) return tuning().prefill_tiles > 1 && n_slots >= 64;
     const size_t wgs = (n_slots + 63) / 64 * (size_t)g.kv_heads;
     const size_t walked = n_pages > n_queries / 32 ? n_pages - n_queries / 32 : 1;
-    size_t line = g.P <= 32 ? 32500 : g.P <= 64 ? 38000 : g.P <= 96 ? 42000 : g.P <= 128 ? 40000 : g.P <= 256 ? 30000 : 4100;
-    // (on a ring that has not wrapped yet the multi-query mode looks at the position of every key: 512 rows of q16/kv8/hd256 over 400,
-    // 512 (21, 25) 36.9/37.8, 40.0/38.8)
-    if (g.ring_rows > 0) line = line / 4 * 3;
+    const size_t line = g.P <= 32 ? 32500 : g.P <= 64 ? 38000 : g.P <= 96 ? 42000 : g.P <= 128 ? 40000 : g.P <= 256 ? 30000 : 4100;
     return (n_slots + 15) / 16 * (size_t)g.kv_heads * walked >= (wgs >= 208 && wgs <= 256 ? std::min<size_t>(line, 12000) : line);
 }
 
@@ -350,8 +347,12 @@ bool wide_f32_heads(const skv_layer *L) { return L->g.f32 && L->g.P > 256; }
 // Arguments of the matrix-core attention kernel for the layer's current length.
 void fill_decode_args(const skv_layer *L, const float *q_dev, float *out_dev, size_t window_start,
                       const float *k_new, const float *v_new, size_t n_queries, size_t target_wgs,
-                      DecodeArgs &a) {
-    const Geom &g = L->g;
+                      DecodeArgs &a, bool keep_ring = false) {
+    Geom g = L->g;
+    // A ring that has not wrapped is a full layer: every position in its own slot, no page but those in the queries' reach to walk and
+    // no position to work out (512 rows of q16/kv8/hd256 on an empty ring of 1056 27.4 -> 23.2 us, over 512 38.6 -> 33.2, f32 over none
+    // 66.5 -> 52.3; 256 rows of q32/kv8/hd128 over 700 25.9 -> 21.5).
+    if (!keep_ring && L->len <= (size_t)g.ring_rows) g.ring_rows = 0;
     a.q = q_dev;
     a.out = out_dev;
     a.k_pool = L->k_pool;
@@ -453,14 +454,14 @@ int32_t multi_query_partials(skv_layer *L, hipStream_t s, size_t n_sets, size_t 
 
 // The layer's pages as the queries of a chunk walk them: from position 0 on on a full layer, from
 // position `lo` to the last row before `end` on a ring.
-ChunkPages layer_pages(const skv_layer *L, size_t lo, size_t end) {
+ChunkPages layer_pages(const Geom &g, size_t lo, size_t end) {
     ChunkPages c{};
     c.n_old = INT32_MAX;
     c.new_pos0 = INT32_MAX;
-    if (L->g.ring_rows > 0) {
+    if (g.ring_rows > 0) {
         c.n_old = lo < end ? (int)((end - 1) / 16 - lo / 16) + 1 : 0;
         c.first_pos = (int)(lo / 16 * 16);
-        c.ring_pages = L->g.ring_rows / 16;
+        c.ring_pages = g.ring_rows / 16;
         c.start = (int)(lo / 16 % (size_t)c.ring_pages);
     }
     return c;
@@ -645,12 +646,12 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
         if (attn_scalar > 0.0f) a.qscale = (1.0f / std::sqrt(attn_scalar)) * 1.4426950408889634f;
         if (n_queries > 1 && takes_f32_chunk_kernel(g, n_queries, (size_t)a.n_pages)) {
             const size_t lo = std::max(window_start, skv_window_start(L->len - n_queries, L->window));
-            const ChunkPages pages = layer_pages(L, lo, L->len); // (a ring's list begins at `lo`, a full layer's at 0)
+            const ChunkPages pages = layer_pages(a.g, lo, L->len); // (a ring's list begins at `lo`, a full layer's at 0)
             // A captured launch must not hold on to scratch that a later call may replace, and a card without room
             // for it still has the other way, which needs none.
-            if (f32_terms_pay(g, n_queries) && !capturing(s)) {
-                const F32Plan plan = g.ring_rows > 0 ? plan_f32_chunk(g, n_queries, 0, pages.n_old, pages.n_old, a.splits)
-                                                     : plan_f32_chunk(g, n_queries, (int)(lo / 16), a.n_pages, a.n_pages, a.splits);
+            if (f32_terms_pay(a.g, n_queries) && !capturing(s)) {
+                const F32Plan plan = a.g.ring_rows > 0 ? plan_f32_chunk(g, n_queries, 0, pages.n_old, pages.n_old, a.splits)
+                                                     : plan_f32_chunk(g, n_queries, (int)(lo / 16), a.page_first + a.n_pages, a.n_pages, a.splits);
                 void *terms = nullptr;
                 DecodeArgs b = a;
                 b.splits_total = plan.sets();
@@ -682,7 +683,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
             size_t want = std::max<size_t>(2 * decode_target_wgs() / tiles, 1);
             // a chunk that a ring holds without wrapping: whole eights of pages a split (130 rows of q16/kv8/hd256 on an empty
             // ring: 22.3 us with one, 29.7 with two and a merge)
-            if (g.ring_rows > 0) want = std::min(want, std::max<size_t>((size_t)a.n_pages / 8, 1));
+            if (L->g.ring_rows > 0) want = std::min(want, std::max<size_t>((size_t)a.n_pages / 8, 1));
             a.splits = (int)std::min<size_t>((size_t)a.splits, want);
             if (tiles > (size_t)g.kv_heads) a.splits = xcd_splits(a.splits, g.kv_heads);
             a.splits_total = a.splits;
@@ -740,7 +741,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
         a.gate = pre->gate;
         a.q_head_stride = pre->q_head_stride;
     }
-    const bool use_tiles = n_queries > 1 && takes_tile_kernel(g, n_queries, (size_t)a.n_pages);
+    const bool use_tiles = n_queries > 1 && takes_tile_kernel(a.g, n_queries, (size_t)a.n_pages);
     TileShape shape = TileShape::one_tile;
     if (n_queries > 1) {
         // split the context only while the query tiles alone leave compute units idle, and
@@ -776,7 +777,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
     }
     if (use_tiles) {
         const size_t lo = std::max(window_start, skv_window_start(L->len - n_queries, L->window));
-        SKV_HIP(launch_prefill_tiles(a, layer_pages(L, lo, L->len), shape, s));
+        SKV_HIP(launch_prefill_tiles(a, layer_pages(a.g, lo, L->len), shape, s));
         if (a.splits > 1) SKV_HIP(launch_merge_rows(a, s));
         return SKV_OK;
     }
@@ -1336,7 +1337,7 @@ static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const flo
     const size_t base = L->len;
     // the rows in the ring that the first query attends (it attends the most of them)
     const size_t lo = std::max(L->floor_pos, skv_window_start(base, L->window));
-    ChunkPages pages = layer_pages(L, lo, base);
+    ChunkPages pages = layer_pages(g, lo, base);
     pages.new_pos0 = (int)base;
     pages.new_first = (int)(base / 16 * 16);
     const size_t n_new = (base + c - 1) / 16 - base / 16 + 1;
@@ -1422,7 +1423,7 @@ static int32_t ring_chunk_f32(skv_layer *L, hipStream_t s, const float *q, const
     DecodeArgs a1{}, a3{};
     int s1 = 0;
     if (base > 0) { // phase 1, prepared against the ring as it is now
-        fill_decode_args(L, q, out, L->floor_pos, nullptr, nullptr, c, tuning().prefill_wgs, a1);
+        fill_decode_args(L, q, out, L->floor_pos, nullptr, nullptr, c, tuning().prefill_wgs, a1, true);
         a1.q_pos0 = (int)base;
         a1.limit_cap = (int)base - 1;
         s1 = splits_for(a1.n_pages);
@@ -1440,7 +1441,7 @@ static int32_t ring_chunk_f32(skv_layer *L, hipStream_t s, const float *q, const
     }
     int32_t rc = encode_append(L, s, k, v, c);
     if (rc) return rc;
-    fill_decode_args(L, q, out, std::max(base, L->floor_pos), nullptr, nullptr, c, tuning().prefill_wgs, a3);
+    fill_decode_args(L, q, out, std::max(base, L->floor_pos), nullptr, nullptr, c, tuning().prefill_wgs, a3, true);
     a3.q_pos0 = (int)base;
     a3.splits = s3;
     a3.split_base = s1;
