@@ -80,6 +80,17 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // attended range their V values are cleared in LDS, behind a barrier of its own, so the bits of
 // such a row never reach a context (the reference never reads those rows,
 // src/decode_resident/kernels.rs:11-88).
+// 16-byte units of LDS: two buffers of a step's pages, [K of SP pairs | V of SP pairs] each. The parts of a workgroup, which hold the same
+// query tiles, make their operands together (QUERIES units, behind the first group's K in the second buffer).
+template <int P, int TILES, int SP, int WAVES, int HALVES>
+struct TileLds {
+    static constexpr int KK = P / 32, TILE = KK * 64, GP = 2 * HALVES;
+    static constexpr int BUF = 2 * SP * GP * TILE;
+    static constexpr bool TOGETHER = HALVES > 1 && KK > 1;
+    static constexpr int QUERIES_AT = BUF + GP * TILE, QUERIES = TOGETHER ? WAVES / HALVES * TILES * KK * 2 * 64 : 0;
+    static constexpr int UNITS = 2 * BUF > QUERIES_AT + QUERIES ? 2 * BUF : QUERIES_AT + QUERIES;
+};
+
 template <int P, int TILES, int SP, int WAVES, int HALVES, bool RING>
 __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, ChunkPages c) {
     constexpr int THREADS = WAVES * 64;
@@ -205,7 +216,14 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
     int t_ws_hi[TILES], t_lim_lo[TILES]; // per tile extremes
     bool t_on[TILES];
     bf16x8_t qh[TILES][KK], ql[TILES][KK];
-    float qv[TILES][KK][8];
+    // The parts load a share of their tiles' K-steps each and find the others' in LDS behind the first barrier. (A load whose lanes all
+    // hit lines of their own takes 64 cycles; with all of them loaded by every wavefront, 128 such loads a compute unit at
+    // head_dim 256, chunks of 512 rows took, in us: q16/kv8/hd256 on a ring 44.5 against 42.0, q32/kv8/hd128 over 0, 1024, 4700
+    // 18.3/17.2, 34.5/33.3, 80.7/78.4.)
+    using Lds = TileLds<P, TILES, SP, WAVES, HALVES>;
+    constexpr int QK = Lds::TOGETHER ? (KK + HALVES - 1) / HALVES : KK; // K-steps of a tile that this wavefront loads
+    auto share = [&](int i) { return Lds::TOGETHER ? min(half * QK + i, KK - 1) : i; }; // (the last part may make one again)
+    float qv[TILES][QK][8];
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
         const int s0 = wg_slot0 + (tw * TILES + t) * 16;
@@ -222,8 +240,8 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
         // they are one round trip; dims past head_dim are zeroed afterwards
         if (a.q_vec) {
 #pragma unroll
-            for (int kk = 0; kk < KK; ++kk) {
-                const int d0 = kk * 32 + j * 8;
+            for (int kk = 0; kk < QK; ++kk) {
+                const int d0 = share(kk) * 32 + j * 8;
                 const float4_t *qp = reinterpret_cast<const float4_t *>(qrow + min(d0, g.head_dim - 8));
                 const float4_t x0 = qp[0], x1 = qp[1];
 #pragma unroll
@@ -234,12 +252,13 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
             }
         } else {
 #pragma unroll
-            for (int kk = 0; kk < KK; ++kk) {
+            for (int kk = 0; kk < QK; ++kk) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) qv[t][kk][e] = qrow[min(kk * 32 + j * 8 + e, g.head_dim - 1)];
+                for (int e = 0; e < 8; ++e) qv[t][kk][e] = qrow[min(share(kk) * 32 + j * 8 + e, g.head_dim - 1)];
             }
         }
     }
+    u4 *const queries = kv_lds + Lds::QUERIES_AT + tw * TILES * KK * 2 * 64 + lane; // of this wavefront's tiles
     // the first group's K, into the second buffer
 #pragma unroll
     for (int u = 0; u < (GP * TILE_U4 + THREADS - 1) / THREADS; ++u) {
@@ -250,8 +269,8 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
 #pragma unroll
-        for (int kk = 0; kk < KK; ++kk) {
-            const int d0 = kk * 32 + j * 8;
+        for (int kk = 0; kk < QK; ++kk) {
+            const int d0 = share(kk) * 32 + j * 8;
             uint32_t hi[4], lo[4];
             // (with 16-byte loads head_dim is a multiple of 8: the lane's eight dims are all inside or all padding)
             const float scale = !a.q_vec || d0 < g.head_dim ? a.qscale : 0.0f;
@@ -265,8 +284,14 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
                 hi[e2] = bf16_pair(x0, x1);
                 lo[e2] = bf16_pair(x0 - __uint_as_float(hi[e2] << 16), x1 - __uint_as_float(hi[e2] & 0xffff0000u));
             }
-            qh[t][kk] = __builtin_bit_cast(bf16x8_t, u4{hi[0], hi[1], hi[2], hi[3]});
-            ql[t][kk] = __builtin_bit_cast(bf16x8_t, u4{lo[0], lo[1], lo[2], lo[3]});
+            if constexpr (Lds::TOGETHER) {
+                u4 *at = queries + (t * KK + share(kk)) * 2 * 64;
+                at[0] = u4{hi[0], hi[1], hi[2], hi[3]};
+                at[64] = u4{lo[0], lo[1], lo[2], lo[3]};
+            } else {
+                qh[t][kk] = __builtin_bit_cast(bf16x8_t, u4{hi[0], hi[1], hi[2], hi[3]});
+                ql[t][kk] = __builtin_bit_cast(bf16x8_t, u4{lo[0], lo[1], lo[2], lo[3]});
+            }
         }
     }
     // The first scores wait for the queries and that K alone; the first step's pages are on their way meanwhile. (The compiler
@@ -524,6 +549,16 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
     // ---- first pair's scores
     const int n_steps = (n_groups + SP - 1) / SP;
     __syncthreads();
+    if constexpr (Lds::TOGETHER) {
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) {
+                qh[t][kk] = __builtin_bit_cast(bf16x8_t, queries[(t * KK + kk) * 2 * 64]);
+                ql[t][kk] = __builtin_bit_cast(bf16x8_t, queries[(t * KK + kk) * 2 * 64 + 64]);
+            }
+        }
+    }
 #pragma unroll
     for (int kk = 0; kk < DEPTH; ++kk) ask_k(kv_lds + BUF_U4 + half * 2 * TILE_U4, kk);
     scores(kv_lds + BUF_U4 + half * 2 * TILE_U4, nullptr, std::false_type{}, [](int) {});
@@ -742,7 +777,7 @@ int prefill_tile_slots(int P, TileShape shape) {
 
 template <int P, int TILES, int SP, int WAVES, int HALVES, bool RING>
 static hipError_t launch_tiles_of(const DecodeArgs &a, const ChunkPages &c, dim3 grid, hipStream_t s) {
-    constexpr size_t lds = (size_t)2 * 2 * SP * HALVES * 2 * (P / 32) * 64 * sizeof(uint4);
+    constexpr size_t lds = (size_t)TileLds<P, TILES, SP, WAVES, HALVES>::UNITS * sizeof(uint4);
     static_assert(lds <= 160 * 1024, "two steps of pages share the LDS of a compute unit");
     static std::atomic<uint64_t> lds_ok{0}; // per instantiation
     {
