@@ -17,6 +17,15 @@ namespace {
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 // LDS buffers of a group's K or V
 __host__ __device__ constexpr int f32_prefill_buffers(int P, bool made) { return made && P <= 128 ? 3 : 2; }
+// whether the halves of a workgroup, which hold the same query tiles, make their operands together
+__host__ __device__ constexpr bool f32_together(int P, int halves) { return halves > 1 && P > 32; }
+// units of those operands, and whether they have LDS of their own; else they lie in the last of three buffers until it is needed
+__host__ __device__ constexpr int f32_query_units(int P, int tiles, int waves, int halves) {
+    return f32_together(P, halves) ? waves / halves * tiles * (P / 32) * 3 * 64 : 0;
+}
+__host__ __device__ constexpr bool f32_queries_apart(int P, int tiles, int waves, int halves, bool made) {
+    return f32_prefill_buffers(P, made) * halves * 3 * 4 * P + f32_query_units(P, tiles, waves, halves) <= 10240;
+}
 // steps of `n` done before beat b, spread over the beats [from, to)
 __host__ __device__ constexpr int done_before(int b, int n, int from, int to) { return b <= from ? 0 : b >= to ? n : (b - from) * n / (to - from); }
 
@@ -177,6 +186,11 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
     }();
     constexpr int CU = (HALVES * PLANE + THREADS - 1) / THREADS; // else: units of K, and of V, a thread makes per group
     constexpr bool FULL = HALVES * PLANE % THREADS == 0;
+    constexpr bool TOGETHER = f32_together(P, HALVES);
+    static_assert(!TOGETHER || P <= 128, "all three terms are in registers");
+    constexpr bool Q_APART = f32_queries_apart(P, TILES, WAVES, HALVES, MADE);
+    constexpr int Q_AT = Q_APART ? NBUF * ITEM : 2 * ITEM;
+    static_assert(Q_APART || (NBUF == 3 && f32_query_units(P, TILES, WAVES, HALVES) <= ITEM), "the queries fit the buffer that is free");
     extern __shared__ __attribute__((aligned(16))) u4 kv_planes[]; // [NBUF][ITEM] (not MADE: K, V)
     constexpr int V_AT = ITEM;
 
@@ -336,7 +350,12 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
     // (at head_dim 256 the third terms, used once per K-step and page, live in LDS behind the planes)
     constexpr int QT = P > 128 ? 2 : 3;
     bf16x8_t q[TILES][KK][QT];
-    float qv[TILES][KK][8];
+    // Halves load a half of their tiles' K-steps each and find the others' in LDS behind the first barrier (see prefill_tile_kernel; 512 rows
+    // of q32/kv8/hd128 over 0, 512 30.9 -> 30.1, 51.7 -> 51.0 us, of q8/kv2/hd64 over 2000 28.4 -> 27.9).
+    constexpr int QK = TOGETHER ? (KK + HALVES - 1) / HALVES : KK;
+    auto share = [&](int i) { return TOGETHER ? min(half * QK + i, KK - 1) : i; }; // (the last part may make one again)
+    u4 *const queries = kv_planes + Q_AT + tw * TILES * KK * 3 * 64 + lane; // of this wavefront's tiles
+    float qv[TILES][QK][8];
     u4 *q_third = kv_planes + NBUF * ITEM + wave * TILES * KK * 64 + lane; // the wavefront's own
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
@@ -351,8 +370,8 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
         const float *qrow = a.q + ((long)(my_slot / G) * g.q_heads + kvh * G + my_slot % G) * g.head_dim;
         if (a.q_vec) {
 #pragma unroll
-            for (int kk = 0; kk < KK; ++kk) {
-                const float4_t *qp = reinterpret_cast<const float4_t *>(qrow + min(kk * 32 + j * 8, g.head_dim - 8));
+            for (int kk = 0; kk < QK; ++kk) {
+                const float4_t *qp = reinterpret_cast<const float4_t *>(qrow + min(share(kk) * 32 + j * 8, g.head_dim - 8));
                 const float4_t x0 = qp[0], x1 = qp[1];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
@@ -362,9 +381,9 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
             }
         } else {
 #pragma unroll
-            for (int kk = 0; kk < KK; ++kk) {
+            for (int kk = 0; kk < QK; ++kk) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) qv[t][kk][e] = qrow[min(kk * 32 + j * 8 + e, g.head_dim - 1)];
+                for (int e = 0; e < 8; ++e) qv[t][kk][e] = qrow[min(share(kk) * 32 + j * 8 + e, g.head_dim - 1)];
             }
         }
     }
@@ -376,17 +395,22 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
 #pragma unroll
-        for (int kk = 0; kk < KK; ++kk) {
+        for (int kk = 0; kk < QK; ++kk) {
             uint32_t w[3][4];
 #pragma unroll
             for (int e2 = 0; e2 < 4; ++e2) {
-                const int d = kk * 32 + j * 8 + e2 * 2;
+                const int d = share(kk) * 32 + j * 8 + e2 * 2;
                 const float x = d < g.head_dim ? qv[t][kk][e2 * 2] * a.qscale : 0.0f;
                 const float y = d + 1 < g.head_dim ? qv[t][kk][e2 * 2 + 1] * a.qscale : 0.0f;
                 three_terms(x, y, w[0][e2], w[1][e2], w[2][e2]);
             }
+            if constexpr (TOGETHER) {
 #pragma unroll
-            for (int k = 0; k < QT; ++k) q[t][kk][k] = __builtin_bit_cast(bf16x8_t, u4{w[k][0], w[k][1], w[k][2], w[k][3]});
+                for (int k = 0; k < 3; ++k) queries[((t * KK + share(kk)) * 3 + k) * 64] = u4{w[k][0], w[k][1], w[k][2], w[k][3]};
+            } else {
+#pragma unroll
+                for (int k = 0; k < QT; ++k) q[t][kk][k] = __builtin_bit_cast(bf16x8_t, u4{w[k][0], w[k][1], w[k][2], w[k][3]});
+            }
             if constexpr (QT == 2) q_third[(t * KK + kk) * 64] = u4{w[2][0], w[2][1], w[2][2], w[2][3]};
         }
     }
@@ -633,6 +657,17 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
         if constexpr (!SHARE) load_v(0, 0);
     }
     __syncthreads();
+    if constexpr (TOGETHER) {
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) {
+#pragma unroll
+                for (int k = 0; k < 3; ++k) q[t][kk][k] = __builtin_bit_cast(bf16x8_t, queries[((t * KK + kk) * 3 + k) * 64]);
+            }
+        }
+        if constexpr (!Q_APART) __syncthreads(); // (the next copies go there)
+    }
     scores(planes, !MADE ? none : NBUF == 3 ? item_of(0, true, 2) : item_of(1, false, 1), std::true_type{});
     mask(half);
 #pragma unroll
@@ -931,7 +966,8 @@ hipError_t launch_f32_terms(const DecodeArgs &a, const ChunkPages &c, const Term
 
 template <int P, int TILES, int WAVES, int HALVES, bool RING, bool MADE>
 static hipError_t launch_f32_prefill_of(const DecodeArgs &a, const ChunkPages &c, const TermPairs &t, dim3 grid, hipStream_t s) {
-    constexpr size_t lds = ((size_t)f32_prefill_buffers(P, MADE) * HALVES * 3 * 4 * P + (P > 128 ? WAVES * TILES * (P / 32) * 64 : 0)) * sizeof(u4);
+    constexpr size_t lds = ((size_t)f32_prefill_buffers(P, MADE) * HALVES * 3 * 4 * P + (P > 128 ? WAVES * TILES * (P / 32) * 64 : 0) +
+                                   (f32_queries_apart(P, TILES, WAVES, HALVES, MADE) ? f32_query_units(P, TILES, WAVES, HALVES) : 0)) * sizeof(u4);
     static_assert(lds <= 160 * 1024, "a group's K and V (and the queries' third terms) share the LDS of a compute unit");
     static std::atomic<uint64_t> lds_ok{0}; // per instantiation
     {
