@@ -49,11 +49,17 @@ typedef struct skv_hot skv_hot;
  * The *_device entry points only queue work on that stream: they neither wait for the
  * device nor switch devices, so the stream must belong to the context's device and that
  * device must be current on the calling thread (the *_host entry points and the create /
- * destroy calls make it current themselves). Two exceptions allocate, after a device
- * synchronisation: a chunked-prefill call whose split partials need more scratch than any
+ * destroy calls make it current themselves). Two exceptions allocate, and may wait for the stream or the device: a
+ * chunked-prefill call whose scratch (split partials, on a ring layer pages of its own rows) needs more than any
  * call before it on the same context and stream (one buffer per stream, which only grows: calls
- * on different streams never share partials), and the first attention call of a
- * layer on the plain kernel (RETI_RUST_FLASH_SDPA=0), which creates its score buffer. Host-side bookkeeping (len, ring position)
+ * on different streams never share one), and the first attention call of a
+ * layer on the plain kernel (RETI_RUST_FLASH_SDPA=0), which creates its score buffer.
+ * A call on a stream that is being captured is recorded with the lengths of that moment. A chunked-prefill call whose
+ * scratch would then have to grow returns SKV_ERR_DEVICE without having queued its attention: run the same call
+ * once before the capture, on the same stream. The scratch that a captured call uses stays where it is until the
+ * context is destroyed; it is also that of the stream's later calls, so replays of such graphs have to be ordered with
+ * each other and with chunked-prefill calls on the captured stream, as work on one stream is.
+ * Host-side bookkeeping (len, ring position)
  * advances when the call returns, before the device has run the work, exactly like the
  * reference's encode-time `len += 1` (src/decode_resident/attention.rs:993); buffers handed
  * to a *_device call must stay valid until the stream has passed that work. */

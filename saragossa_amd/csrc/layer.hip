@@ -61,12 +61,22 @@ void arena_put(skv_ctx *ctx, void *ptr, size_t bytes) {
     (void)hipFree(ptr);
 }
 
+// The device as a context's scratch sees it. A failed call leaves no error behind for the next launch to report.
+static struct HipScratch final : ScratchDevice {
+    static int status(hipError_t e) {
+        if (e != hipSuccess) (void)hipGetLastError();
+        return (int)e;
+    }
+    int alloc(void **p, size_t bytes) override { return status(hipMalloc(p, bytes)); }
+    int free(void *p) override { return status(hipFree(p)); }
+    int wait_stream(void *stream) override { return status(hipStreamSynchronize(static_cast<hipStream_t>(stream))); }
+    int wait_device() override { return status(hipDeviceSynchronize()); }
+} hip_scratch;
+
 // Frees what the context holds on the device; the caller has synchronised the device.
 static void ctx_drain(skv_ctx *ctx) {
+    ctx->scratch.drain(hip_scratch);
     std::lock_guard<std::mutex> lk(ctx->arena_mu);
-    for (auto &kv : ctx->mq_scratch)
-        if (kv.second.ptr) (void)hipFree(kv.second.ptr);
-    ctx->mq_scratch.clear();
     for (auto &kv : ctx->arena_free) (void)hipFree(kv.second);
     ctx->arena_free.clear();
     ctx->arena_bytes = 0;
@@ -75,7 +85,7 @@ static void ctx_drain(skv_ctx *ctx) {
 void ctx_release(skv_ctx *ctx) {
     if (ctx->refs.fetch_sub(1, std::memory_order_acq_rel) != 1) return;
     // a layer that outlived skv_ctx_destroy may have grown the multi-query scratch again
-    if (!ctx->mq_scratch.empty()) {
+    if (!ctx->scratch.empty()) {
         (void)hipSetDevice(ctx->device);
         (void)hipDeviceSynchronize();
         ctx_drain(ctx);
@@ -391,60 +401,29 @@ void fill_decode_args(const skv_layer *L, const float *q_dev, float *out_dev, si
     a.g = g;
 }
 
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return true; // what cannot be told is taken for the one that holds on to its scratch
+    }
+    return status != hipStreamCaptureStatusNone;
+}
+
 // Split partials of a multi-query launch live in the context's scratch, grown on demand:
 // [kv_heads][n_sets][n_queries * gqa] of (o[head_dim], m, l); in front of them `page_bytes` for
-// pages of the chunk's own rows (*pages, a multiple of 256).
+// pages of the chunk's own rows (*pages, a multiple of 256). The lease is the caller's until it has queued its launches.
 int32_t multi_query_partials(skv_layer *L, hipStream_t s, size_t n_sets, size_t n_queries, DecodeArgs &a,
-                             size_t page_bytes = 0, void **pages = nullptr) {
+                             StreamScratch::Lease &lease, size_t page_bytes = 0, void **pages = nullptr) {
     const Geom &g = L->g;
     const size_t n_part = (size_t)g.kv_heads * n_sets * n_queries * g.gqa;
     const size_t need = page_bytes + n_part * ((size_t)g.head_dim + 2) * sizeof(float);
-    skv_ctx *c = L->ctx;
     void *buf = nullptr;
-    void *old = nullptr;     // this stream's buffer, too small: freed once the stream has drained
-    void *evicted = nullptr; // another stream's buffer, pushed out of the bounded map
-    {
-        std::lock_guard<std::mutex> lk(c->arena_mu);
-        auto it = c->mq_scratch.find(s);
-        if (it != c->mq_scratch.end() && it->second.bytes >= need) {
-            it->second.used = ++c->mq_clock;
-            buf = it->second.ptr;
-        } else if (it != c->mq_scratch.end()) {
-            old = it->second.ptr;
-            c->mq_scratch.erase(it); // nobody else uses this stream's entry (one thread per stream)
-        } else if (c->mq_scratch.size() >= skv_ctx::MQ_SCRATCH_STREAMS) {
-            auto lru = c->mq_scratch.begin();
-            for (auto j = c->mq_scratch.begin(); j != c->mq_scratch.end(); ++j)
-                if (j->second.used < lru->second.used) lru = j;
-            evicted = lru->second.ptr;
-            c->mq_scratch.erase(lru);
-        }
-    }
-    if (!buf) {
-        // waits, frees and the allocation outside the lock: other threads' arena_get / arena_put
-        // and launches on other streams go on meanwhile
-        if (old) {
-            SKV_HIP(hipStreamSynchronize(s)); // work queued on the stream may still read it
-            SKV_HIP(hipFree(old));
-        }
-        if (evicted) {
-            SKV_HIP(hipDeviceSynchronize()); // its stream may be gone: wait for everything
-            SKV_HIP(hipFree(evicted));
-        }
-        void *p = nullptr;
-        SKV_HIP(hipMalloc(&p, need));
-        try {
-            std::lock_guard<std::mutex> lk(c->arena_mu);
-            skv_ctx::MqScratch &slot = c->mq_scratch[s];
-            slot.ptr = p;
-            slot.bytes = need;
-            slot.used = ++c->mq_clock;
-        } catch (...) {
-            (void)hipFree(p);
-            throw;
-        }
-        buf = p;
-    }
+    const int status = L->ctx->scratch.get(hip_scratch, s, need, capturing(s), lease, &buf);
+    if (status == StreamScratch::REFUSED)
+        return fail(SKV_ERR_DEVICE, "prefill chunk: flux en capture, le tampon du flux est plus petit que les " +
+                                        std::to_string(need) + " o requis (même appel d'abord hors capture)");
+    if (status != 0) return fail_hip((hipError_t)status, "prefill chunk: tampon des partiels");
     if (pages) *pages = buf;
     a.part_o = reinterpret_cast<float *>(static_cast<char *>(buf) + page_bytes);
     a.part_m = a.part_o + n_part * g.head_dim;
@@ -488,15 +467,6 @@ AppendArgs append_args(const skv_layer *L, const float *k_dev, const float *v_de
         a.n_rows = L->g.ring_rows;
     }
     return a;
-}
-
-bool capturing(hipStream_t s) {
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &status) != hipSuccess) {
-        (void)hipGetLastError();
-        return true; // a stream that cannot say so takes no scratch
-    }
-    return status != hipStreamCaptureStatusNone;
 }
 
 // Whether a chunk on f32 pages has them split into terms by a launch of its own, once for all workgroups, instead of by each
@@ -624,6 +594,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
     const Geom &g = L->g;
     if (static_partials && (n_queries != 1 || !uses_flash(L)))
         return fail(SKV_ERR_CONFIG, "decode_step_static: une ligne de requête, noyau matriciel seulement");
+    StreamScratch::Lease lease;
     if (g.f32 && (uses_flash(L) || n_queries > 1)) {
         // the f32 element's matrix kernels: 16 query slots per workgroup, the context split while
         // that leaves compute units idle; one query row of narrow heads takes the kernel that
@@ -655,7 +626,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
                 void *terms = nullptr;
                 DecodeArgs b = a;
                 b.splits_total = plan.sets();
-                if (multi_query_partials(L, s, plan.sets() > 1 ? (size_t)plan.sets() : 0, n_queries, b,
+                if (multi_query_partials(L, s, plan.sets() > 1 ? (size_t)plan.sets() : 0, n_queries, b, lease,
                                          plan.bytes(g, (size_t)(L->n_pages + 1) / 2), &terms) == SKV_OK)
                     return run_f32_chunk(plan, b, pages, terms, (int)lo, k_new, v_new, s);
                 (void)hipGetLastError();
@@ -671,7 +642,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
             a.splits = std::min(a.splits, chunk_splits(g, n_queries, (size_t)f32_prefill_slots(g.P, halves), (size_t)a.n_pages));
             a.splits_total = a.splits;
             if (a.splits > 1) {
-                int32_t rc2 = multi_query_partials(L, s, (size_t)a.splits, n_queries, a);
+                int32_t rc2 = multi_query_partials(L, s, (size_t)a.splits, n_queries, a, lease);
                 if (rc2) return rc2;
             }
             SKV_HIP(launch_f32_prefill(a, pages, nullptr, halves, s));
@@ -688,7 +659,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
             if (tiles > (size_t)g.kv_heads) a.splits = xcd_splits(a.splits, g.kv_heads);
             a.splits_total = a.splits;
             if (a.splits > 1) {
-                int32_t rc2 = multi_query_partials(L, s, (size_t)a.splits, n_queries, a);
+                int32_t rc2 = multi_query_partials(L, s, (size_t)a.splits, n_queries, a, lease);
                 if (rc2) return rc2;
             }
         }
@@ -767,7 +738,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
         if (!use_tiles && tiles > (size_t)g.kv_heads) a.splits = xcd_splits(a.splits, g.kv_heads);
         a.splits_total = a.splits;
         if (a.splits > 1) {
-            int32_t rc2 = multi_query_partials(L, s, (size_t)a.splits, n_queries, a);
+            int32_t rc2 = multi_query_partials(L, s, (size_t)a.splits, n_queries, a, lease);
             if (rc2) return rc2;
         }
     }
@@ -1357,6 +1328,7 @@ static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const flo
     const bool halves = g.f32 && f32_halves(g, c * (size_t)g.gqa, walked);
     // a context over the chunk's own rows is written once they are in the ring: by the merge, so there has to be one
     const bool over_rows = context_over_rows(L, c, out, k, v);
+    StreamScratch::Lease lease;
     void *scratch = nullptr;
     int32_t rc = SKV_OK;
     if (made) {
@@ -1364,7 +1336,7 @@ static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const flo
         if (over_rows) plan.splits = std::max(plan.splits, 2);
         a.splits = plan.splits;
         a.splits_total = plan.sets();
-        if (multi_query_partials(L, s, a.splits_total > 1 ? (size_t)a.splits_total : 0, c, a, plan.bytes(g, 0), &scratch) != SKV_OK) {
+        if (multi_query_partials(L, s, a.splits_total > 1 ? (size_t)a.splits_total : 0, c, a, lease, plan.bytes(g, 0), &scratch) != SKV_OK) {
             (void)hipGetLastError();
             made = false;
         }
@@ -1373,7 +1345,7 @@ static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const flo
         a.splits = chunk_splits(g, c, (size_t)(g.f32 ? f32_prefill_slots(g.P, halves) : prefill_tile_slots(g.P, shape)), walked);
         if (over_rows) a.splits = std::max(a.splits, 2);
         a.splits_total = a.splits;
-        rc = multi_query_partials(L, s, a.splits > 1 ? (size_t)a.splits : 0, c, a, 2 * pool_bytes, &scratch);
+        rc = multi_query_partials(L, s, a.splits > 1 ? (size_t)a.splits : 0, c, a, lease, 2 * pool_bytes, &scratch);
         if (rc) return rc;
     }
     if (made) {
@@ -1420,6 +1392,7 @@ static int32_t ring_chunk_f32(skv_layer *L, hipStream_t s, const float *q, const
         want = std::min<size_t>(want, std::max<size_t>((size_t)n_pages / 8, 1));
         return (int)std::min<size_t>(want, tuning().prefill_max_splits);
     };
+    StreamScratch::Lease lease;
     DecodeArgs a1{}, a3{};
     int s1 = 0;
     if (base > 0) { // phase 1, prepared against the ring as it is now
@@ -1435,7 +1408,7 @@ static int32_t ring_chunk_f32(skv_layer *L, hipStream_t s, const float *q, const
         a1.splits = s1;
         a1.split_base = 0;
         a1.splits_total = total;
-        int32_t rc = multi_query_partials(L, s, (size_t)total, c, a1);
+        int32_t rc = multi_query_partials(L, s, (size_t)total, c, a1, lease);
         if (rc) return rc;
         SKV_HIP(launch_f32_split(a1, s));
     }
@@ -1447,7 +1420,7 @@ static int32_t ring_chunk_f32(skv_layer *L, hipStream_t s, const float *q, const
     a3.split_base = s1;
     a3.splits_total = total;
     if (total > 1) {
-        rc = multi_query_partials(L, s, (size_t)total, c, a3);
+        rc = multi_query_partials(L, s, (size_t)total, c, a3, lease);
         if (rc) return rc;
     }
     SKV_HIP(launch_f32_split(a3, s));
