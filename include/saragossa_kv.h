@@ -54,6 +54,11 @@ typedef struct skv_hot skv_hot;
  * call before it on the same context and stream (one buffer per stream, which only grows: calls
  * on different streams never share one), and the first attention call of a
  * layer on the plain kernel (RETI_RUST_FLASH_SDPA=0), which creates its score buffer.
+ * Chunked-prefill calls on f32 layers also keep room for their pages as bf16 terms, 6 bytes per K and per V value of
+ * the context they walk: in one buffer per stream, replaced by a larger one as contexts grow (which waits for the stream), in
+ * all of a context's buffers at most SKV_F32_TERMS_MB (environment, 512 MiB by default), until the context is destroyed.
+ * skv_layer_bytes does not count it. It is never required: where there is no memory for it, and in a
+ * stream that is being captured, a call does without.
  * A call on a stream that is being captured is recorded with the lengths of that moment. A chunked-prefill call whose
  * scratch would then have to grow returns SKV_ERR_DEVICE without having queued its attention: run the same call
  * once before the capture, on the same stream. The scratch that a captured call uses stays where it is until the

@@ -16,7 +16,7 @@ struct skv_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     void *static_scratch = nullptr; // this device's copy of the library's static scratch array
-    // Split-K partials of multi-query launches (chunked prefill) and pages of a ring chunk's own rows.
+    // Split-K partials of multi-query launches (chunked prefill) and pages of a ring chunk's own rows; terms of f32 pages.
     skv::StreamScratch scratch;
     // Device buffers of destroyed layers, kept for the next layer that needs about as much:
     // the stand-in for the arena DecodeResidentState leases its buffers from

@@ -50,6 +50,7 @@ hipError_t arena_get(skv_ctx *ctx, size_t bytes, void **ptr, size_t *got) {
 
 void arena_put(skv_ctx *ctx, void *ptr, size_t bytes) {
     if (!ptr) return;
+    ctx->scratch.freed(); // (or about to be, in a layer's end: worth another question at most)
     {
         std::lock_guard<std::mutex> lk(ctx->arena_mu);
         if (!ctx->closed && ctx->arena_bytes + bytes <= ctx->arena_cap) {
@@ -71,6 +72,7 @@ static struct HipScratch final : ScratchDevice {
     int free(void *p) override { return status(hipFree(p)); }
     int wait_stream(void *stream) override { return status(hipStreamSynchronize(static_cast<hipStream_t>(stream))); }
     int wait_device() override { return status(hipDeviceSynchronize()); }
+    bool full(int status) override { return status == (int)hipErrorOutOfMemory; }
 } hip_scratch;
 
 // Frees what the context holds on the device; the caller has synchronised the device.
@@ -161,7 +163,7 @@ struct Tuning {
     size_t prefill_wgs, prefill_max_splits;
     long prefill_tiles2_min_pages; // -1 = by head_dim
     size_t f32_terms;       // f32 chunks: 0 = every workgroup splits its pages into terms, 1 = by shape, 2 = a launch of its own does
-    size_t f32_terms_max;   // bytes of terms held at a time
+    size_t f32_terms_max;   // bytes of terms that a context holds
 };
 
 const Tuning &tuning() {
@@ -181,7 +183,7 @@ const Tuning &tuning() {
         t.prefill_tiles2_min_pages = std::getenv("SKV_PREFILL_TILES2_MIN_PAGES")
                                          ? (long)env_usize("SKV_PREFILL_TILES2_MIN_PAGES", 0) : -1;
         t.f32_terms = env_usize("SKV_F32_TERMS", 1);
-        t.f32_terms_max = std::min<size_t>(std::max<size_t>(env_usize("SKV_F32_TERMS_MB", 512), 1), 1 << 20) << 20;
+        t.f32_terms_max = std::min<size_t>(env_usize("SKV_F32_TERMS_MB", 512), 1 << 20) << 20;
         seen = epoch;
     }
     return t;
@@ -413,21 +415,29 @@ bool capturing(hipStream_t s) {
 // Split partials of a multi-query launch live in the context's scratch, grown on demand:
 // [kv_heads][n_sets][n_queries * gqa] of (o[head_dim], m, l); in front of them `page_bytes` for
 // pages of the chunk's own rows (*pages, a multiple of 256). The lease is the caller's until it has queued its launches.
-int32_t multi_query_partials(skv_layer *L, hipStream_t s, size_t n_sets, size_t n_queries, DecodeArgs &a,
-                             StreamScratch::Lease &lease, size_t page_bytes = 0, void **pages = nullptr) {
+int try_partials(skv_layer *L, hipStream_t s, size_t n_sets, size_t n_queries, DecodeArgs &a, StreamScratch::Lease &lease,
+                 size_t page_bytes = 0, void **pages = nullptr, bool optional = false, size_t *asked = nullptr) {
     const Geom &g = L->g;
     const size_t n_part = (size_t)g.kv_heads * n_sets * n_queries * g.gqa;
     const size_t need = page_bytes + n_part * ((size_t)g.head_dim + 2) * sizeof(float);
     void *buf = nullptr;
-    const int status = L->ctx->scratch.get(hip_scratch, s, need, capturing(s), lease, &buf);
-    if (status == StreamScratch::REFUSED)
-        return fail(SKV_ERR_DEVICE, "prefill chunk: flux en capture, le tampon du flux est plus petit que les " +
-                                        std::to_string(need) + " o requis (même appel d'abord hors capture)");
-    if (status != 0) return fail_hip((hipError_t)status, "prefill chunk: tampon des partiels");
+    const int status = L->ctx->scratch.get(hip_scratch, s, need, capturing(s), lease, &buf, optional);
+    if (asked) *asked = need;
+    if (status != 0) return status;
     if (pages) *pages = buf;
     a.part_o = reinterpret_cast<float *>(static_cast<char *>(buf) + page_bytes);
     a.part_m = a.part_o + n_part * g.head_dim;
     a.part_l = a.part_m + n_part;
+    return 0;
+}
+int32_t multi_query_partials(skv_layer *L, hipStream_t s, size_t n_sets, size_t n_queries, DecodeArgs &a,
+                             StreamScratch::Lease &lease, size_t page_bytes = 0, void **pages = nullptr) {
+    size_t need = 0;
+    const int status = try_partials(L, s, n_sets, n_queries, a, lease, page_bytes, pages, false, &need);
+    if (status == StreamScratch::REFUSED)
+        return fail(SKV_ERR_DEVICE, "prefill chunk: flux en capture, le tampon du flux est plus petit que les " +
+                                        std::to_string(need) + " o requis (même appel d'abord hors capture)");
+    if (status != 0) return fail_hip((hipError_t)status, "prefill chunk: tampon des partiels");
     return SKV_OK;
 }
 
@@ -485,7 +495,19 @@ bool f32_terms_pay(const Geom &g, size_t n_queries) {
     return g.ring_rows > 0 || n_queries * (size_t)g.gqa >= (g.P > 128 ? 2048u : 1536u);
 }
 
-// Such a chunk. The scratch holds at most so many bytes of terms (512 MiB); longer contexts are taken in segments, each with
+// Scratch for the terms of a chunk that walks `pairs` pairs of pages, of a layer of up to `layer_pairs`: the number of pairs it holds, 0 =
+// none. A layer asks for all of its pairs at once while that is 128 MiB at most, then for twice as much each time, so that
+// the chunks of a growing context seldom replace it. A quarter of what the chunk walks will do, the context is then taken in
+// segments, each with partials of its own (four of them, 512 rows of q32/kv8/hd128 over 40000, cost 2 %; terms gain 5 to 10).
+size_t terms_scratch(skv_layer *L, hipStream_t s, size_t pairs, size_t layer_pairs, StreamScratch::Lease &lease, void **terms) {
+    const size_t one = f32_terms_bytes(L->g), limit = tuning().f32_terms_max, most = limit / one;
+    size_t n = std::max<size_t>(((size_t)128 << 20) / one, 1);
+    while (n < pairs) n *= 2;
+    const size_t want = std::min(std::max(std::min(n, layer_pairs), pairs), most), least = (std::min(pairs, most) + 3) / 4;
+    return want == 0 ? 0 : L->ctx->scratch.terms(hip_scratch, s, want * one, least * one, limit, lease, terms) / one;
+}
+
+// Such a chunk. Contexts of more pairs than the terms' scratch holds are taken in segments, each with
 // splits of its own (512 rows of q32/kv8/hd128 over 16384, 40000, in us, segments of 128 MiB / 1 GiB 657/643, 1562/1532; over 8192,
 // where two segments of 64 MiB take 357, one takes 340).
 struct F32Plan {
@@ -495,24 +517,16 @@ struct F32Plan {
     int splits;         // of a segment
     bool halves;
     int sets() const { return segments * splits; }
-    // The terms' scratch. A layer of up to `pairs` pairs asks for all of them at once while that is 128 MiB at most, then for twice
-    // as much each time, so that the chunks of a growing context seldom replace it.
-    size_t bytes(const Geom &g, size_t pairs) const {
-        const size_t one = f32_terms_bytes(g), most = std::max<size_t>(tuning().f32_terms_max / one, 1);
-        size_t n = std::max<size_t>(((size_t)128 << 20) / one, 1);
-        while (n < (size_t)held) n *= 2;
-        return std::max(std::min({n, pairs, most}), (size_t)held) * one;
-    }
 };
-// walked: pages that a workgroup walks of all segments
-F32Plan plan_f32_chunk(const Geom &g, size_t n_queries, int first_entry, int entries, int walked, int max_splits) {
+// walked: pages that a workgroup walks of all segments; most: pairs that the scratch holds
+F32Plan plan_f32_chunk(const Geom &g, size_t n_queries, int first_entry, int entries, int walked, int max_splits, size_t most) {
     F32Plan p{};
     p.first = first_entry / 2;
     p.last = (entries + 1) / 2;
     p.entries = entries;
-    const int pairs = p.last - p.first, most = (int)std::max<size_t>(tuning().f32_terms_max / f32_terms_bytes(g), 1);
-    p.segments = (pairs + most - 1) / most;
-    p.held = (pairs + p.segments - 1) / p.segments;
+    const size_t pairs = (size_t)(p.last - p.first);
+    p.segments = (int)((pairs + most - 1) / most);
+    p.held = (int)((pairs + (size_t)p.segments - 1) / (size_t)p.segments);
     // Halves cover half the slots and walk two pairs at a time: the same time per workgroup with half as many splits, so fewer
     // partials, but they copy each page for half as many slots, which costs more on long walks. Whole chunks, one tile / halves, in us: q32/kv8/hd128, 512 rows
     // over 512, 1024, 2048, 6000, 8192 (two splits / one) 59.1/51.2, 74.5/68.5, 114/109, 262/265, 340/349; q8/kv2/hd64, 512 rows over 2048, 4096,
@@ -615,28 +629,36 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
             a.q_head_stride = pre->q_head_stride;
         }
         if (attn_scalar > 0.0f) a.qscale = (1.0f / std::sqrt(attn_scalar)) * 1.4426950408889634f;
-        if (n_queries > 1 && takes_f32_chunk_kernel(g, n_queries, (size_t)a.n_pages)) {
+        const bool by_terms = n_queries > 1 && takes_f32_chunk_kernel(g, n_queries, (size_t)a.n_pages);
+        const auto store_rows = [&]() -> int32_t { // rows that the terms' launch would have stored
+            if (n_queries == 1 || !k_new) return SKV_OK;
+            AppendArgs w = append_args(L, k_new, v_new, n_queries);
+            w.first_pos -= (long)n_queries; // (counted already)
+            SKV_HIP(launch_append(w, s));
+            a.k_new = a.v_new = nullptr;
+            return SKV_OK;
+        };
+        if (by_terms) {
             const size_t lo = std::max(window_start, skv_window_start(L->len - n_queries, L->window));
             const ChunkPages pages = layer_pages(a.g, lo, L->len); // (a ring's list begins at `lo`, a full layer's at 0)
-            // A captured launch must not hold on to scratch that a later call may replace, and a card without room
-            // for it still has the other way, which needs none.
+            // (a captured launch makes no terms: their scratch is replaced and dropped)
             if (f32_terms_pay(a.g, n_queries) && !capturing(s)) {
-                const F32Plan plan = a.g.ring_rows > 0 ? plan_f32_chunk(g, n_queries, 0, pages.n_old, pages.n_old, a.splits)
-                                                     : plan_f32_chunk(g, n_queries, (int)(lo / 16), a.page_first + a.n_pages, a.n_pages, a.splits);
+                const bool ring = a.g.ring_rows > 0;
+                const int first = ring ? 0 : (int)(lo / 16), entries = ring ? pages.n_old : a.page_first + a.n_pages;
+                StreamScratch::Lease terms_lease;
                 void *terms = nullptr;
-                DecodeArgs b = a;
-                b.splits_total = plan.sets();
-                if (multi_query_partials(L, s, plan.sets() > 1 ? (size_t)plan.sets() : 0, n_queries, b, lease,
-                                         plan.bytes(g, (size_t)(L->n_pages + 1) / 2), &terms) == SKV_OK)
-                    return run_f32_chunk(plan, b, pages, terms, (int)lo, k_new, v_new, s);
-                (void)hipGetLastError();
+                const size_t most = terms_scratch(L, s, (size_t)((entries + 1) / 2 - first / 2), (size_t)(L->n_pages + 1) / 2, terms_lease, &terms);
+                if (most > 0) {
+                    const F32Plan plan = plan_f32_chunk(g, n_queries, first, entries, ring ? entries : a.n_pages, a.splits, most);
+                    DecodeArgs b = a;
+                    b.splits_total = plan.sets();
+                    if (plan.sets() == 1 || try_partials(L, s, (size_t)plan.sets(), n_queries, b, lease, 0, nullptr, true) == 0)
+                        return run_f32_chunk(plan, b, pages, terms, (int)lo, k_new, v_new, s);
+                }
+                // no memory for them: the other way needs none
             }
-            if (k_new) { // rows that the terms' launch would have stored
-                AppendArgs w = append_args(L, k_new, v_new, n_queries);
-                w.first_pos -= (long)n_queries; // (counted already)
-                SKV_HIP(launch_append(w, s));
-                a.k_new = a.v_new = nullptr;
-            }
+            rc = store_rows();
+            if (rc) return rc;
             const bool halves = f32_halves(g, n_queries * (size_t)g.gqa, (size_t)a.n_pages);
             // (choose_splits' number, which the split knobs of decode launches bound, is the larger one unless they do)
             a.splits = std::min(a.splits, chunk_splits(g, n_queries, (size_t)f32_prefill_slots(g.P, halves), (size_t)a.n_pages));
@@ -650,6 +672,8 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
             return SKV_OK;
         }
         if (n_queries > 1) {
+            rc = store_rows(); // (a knob that turned between the caller's look at it and this one)
+            if (rc) return rc;
             const size_t tiles = (n_queries * (size_t)g.gqa + 15) / 16 * (size_t)g.kv_heads;
             size_t want = std::max<size_t>(2 * decode_target_wgs() / tiles, 1);
             // a chunk that a ring holds without wrapping: whole eights of pages a split (130 rows of q16/kv8/hd256 on an empty
@@ -1331,14 +1355,17 @@ static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const flo
     StreamScratch::Lease lease;
     void *scratch = nullptr;
     int32_t rc = SKV_OK;
+    StreamScratch::Lease terms_lease;
     if (made) {
-        plan = plan_f32_chunk(g, c, 0, (int)((size_t)pages.n_old + n_new), (int)walked, INT32_MAX);
-        if (over_rows) plan.splits = std::max(plan.splits, 2);
-        a.splits = plan.splits;
-        a.splits_total = plan.sets();
-        if (multi_query_partials(L, s, a.splits_total > 1 ? (size_t)a.splits_total : 0, c, a, lease, plan.bytes(g, 0), &scratch) != SKV_OK) {
-            (void)hipGetLastError();
-            made = false;
+        const int entries = (int)((size_t)pages.n_old + n_new);
+        const size_t most = terms_scratch(L, s, (size_t)(entries + 1) / 2, 0, terms_lease, &scratch);
+        made = most > 0;
+        if (made) {
+            plan = plan_f32_chunk(g, c, 0, entries, (int)walked, INT32_MAX, most);
+            if (over_rows) plan.splits = std::max(plan.splits, 2);
+            a.splits = plan.splits;
+            a.splits_total = plan.sets();
+            made = a.splits_total == 1 || try_partials(L, s, (size_t)a.splits_total, c, a, lease, 0, nullptr, true) == 0;
         }
     }
     if (!made) {

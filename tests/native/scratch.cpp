@@ -46,6 +46,7 @@ struct Device final : skv::ScratchDevice {
         ++waits;
         return failing_waits > 0 ? (--failing_waits, 3) : 0;
     }
+    bool full(int status) override { return status == 2; }
     int calls() const { return allocs + frees + waits; }
 };
 
@@ -167,11 +168,97 @@ static void random_calls() {
     }
 }
 
+static size_t terms(StreamScratch &s, Device &d, int i, size_t want, size_t least, size_t limit, void **out = nullptr) {
+    StreamScratch::Lease lease;
+    void *p = nullptr;
+    const size_t n = s.terms(d, stream(i), want, least, limit, lease, &p);
+    CHECK(n <= want && (n == 0) == (p == nullptr) && (n == 0 || (n >= least && d.live.at(p) >= n)));
+    if (out) *out = p;
+    return n;
+}
+
+static void terms_beside_partials() {
+    Device d;
+    StreamScratch s;
+    void *partials = got(s, d, 1, 1000), *a = nullptr, *b = nullptr;
+    CHECK(terms(s, d, 1, 500, 100, 10000, &a) == 500 && a != partials);
+    CHECK(terms(s, d, 1, 300, 300, 10000, &b) == 300 && b == a);
+    CHECK(terms(s, d, 1, 5000, 600, 10000, &b) == 5000 && !d.live.count(a) && d.live.count(partials));
+    CHECK(got(s, d, 1, 1000) == partials); // never replaced for terms
+    // no memory: what there is serves, nothing is freed or waited for, and the size is asked for once
+    d.room = d.held + 100;
+    const int frees = d.frees, waits = d.waits;
+    CHECK(terms(s, d, 1, 9000, 600, 10000) == 5000);
+    int allocs = d.allocs;
+    CHECK(terms(s, d, 1, 9000, 600, 10000) == 5000 && d.allocs == allocs);
+    CHECK(terms(s, d, 1, 9500, 5500, 10000) == 0 && d.allocs == allocs);
+    CHECK(terms(s, d, 2, 4000, 4000, 10000) == 0);
+    allocs = d.allocs;
+    CHECK(terms(s, d, 2, 4000, 4000, 10000) == 0 && d.allocs == allocs);
+    StreamScratch::Lease lease;
+    void *p = nullptr;
+    CHECK(s.get(d, stream(1), 4100, false, lease, &p, true) != 0 && d.allocs == allocs); // optional partials: not tried either
+    CHECK(s.get(d, stream(1), 1500, false, lease, &p, true) != 0 && d.allocs == allocs + 1);
+    CHECK(s.get(d, stream(1), 1500, false, lease, &p, true) != 0 && d.allocs == allocs + 1);
+    CHECK(got(s, d, 1, 1000) == partials && d.frees == frees && d.waits == waits);
+    s.freed();
+    d.room = SIZE_MAX;
+    CHECK(terms(s, d, 1, 9000, 600, 10000) == 9000 && d.live.size() == 2);
+    CHECK(terms(s, d, 1, 700, 600, 10000, &a) == 700);
+    // half of what is wanted, or a quarter, where there is that
+    d.room = d.held + 450;
+    CHECK(terms(s, d, 3, 1000, 100, 20000, &b) == 500 / 2);
+    CHECK(d.live.at(b) == 250);
+    d.room = SIZE_MAX;
+    CHECK(terms(s, d, 3, 1000, 100, 20000) == 250); // still remembered
+    s.freed();
+    CHECK(terms(s, d, 3, 1000, 100, 20000) == 1000 && !d.live.count(b));
+}
+
+static void terms_of_many_streams() {
+    Device d;
+    StreamScratch s;
+    void *first = nullptr, *p = nullptr;
+    CHECK(terms(s, d, 1, 600, 100, 1000, &first) == 600);
+    CHECK(terms(s, d, 2, 600, 100, 1000) == 400); // what is left
+    CHECK(terms(s, d, 3, 600, 100, 1000) == 0 && d.held == 1000);
+    for (int i = 0; i < 100; ++i) CHECK(terms(s, d, 2, 600, 100, 1000) == 400); // (stream 1 is idle)
+    CHECK(terms(s, d, 3, 600, 100, 1000) == 600 && !d.live.count(first) && d.held == 1000);
+    {
+        StreamScratch::Lease lease; // a call of stream 3 that still queues launches
+        CHECK(s.terms(d, stream(3), 600, 100, 1000, lease, &p) == 600);
+        for (int i = 0; i < 100; ++i) CHECK(terms(s, d, 2, 400, 100, 1000) == 400);
+        CHECK(terms(s, d, 4, 600, 100, 1000) == 0 && d.live.count(p));
+    }
+    for (int i = 0; i < 100; ++i) CHECK(terms(s, d, 2, 400, 100, 1000) == 400);
+    CHECK(terms(s, d, 4, 600, 100, 1000) == 600 && !d.live.count(p));
+    CHECK(terms(s, d, 2, 300, 1, 0) == 300); // a lower limit takes nothing away
+    CHECK(terms(s, d, 2, 500, 450, 0) == 0);
+    for (int i = 10; i < 40; ++i) terms(s, d, i, 1, 1, 100000);
+    CHECK(d.live.size() == StreamScratch::STREAMS);
+    d.failing_waits = 1;
+    CHECK(terms(s, d, 2, 50000, 1, 100000) == 50000 && d.live.size() == StreamScratch::STREAMS + 1);
+    s.drain(d);
+    CHECK(d.live.empty() && s.empty());
+    std::mt19937 rng(9);
+    for (int call = 0; call < 20000; ++call) {
+        const size_t want = 1 + rng() % 3000;
+        d.room = rng() % 4 == 0 ? d.held + rng() % 2000 : SIZE_MAX;
+        if (rng() % 100 == 0) s.freed();
+        if (rng() % 3 == 0) d.room = SIZE_MAX, (void)got(s, d, (int)(rng() % 12), 1 + rng() % 100);
+        terms(s, d, (int)(rng() % 12), want, 1 + want / 8, 6000);
+    }
+    s.drain(d);
+    CHECK(d.live.empty() && s.empty());
+}
+
 int main() {
     captured_buffers_stay();
     oldest_goes();
     failures();
     random_calls();
+    terms_beside_partials();
+    terms_of_many_streams();
     std::puts("ok");
     return 0;
 }

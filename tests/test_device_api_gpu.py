@@ -278,9 +278,9 @@ def test_prefill_chunk_device_with_unaligned_query_pointer(state):
 
 
 def test_attention_launches_replay_correctly_from_a_hip_graph(state):
-    """The *_device entry points only queue kernels (no allocation, no synchronisation, no
-    memset), so a caller may capture them in a HIP graph; what is captured is the work at the
-    lengths of capture time. Several layers' attention captured once, replayed three times
+    """The attention calls of one row only queue kernels (no allocation, no synchronisation, no
+    memset), so a caller may capture them in a HIP graph (chunks: tests/test_captured_chunks_gpu.py); what is captured is the
+    work at the lengths of capture time. Several layers' attention captured once, replayed three times
     with eager work and synchronisations in between, each replay against the eager result
     (short context: single split; long context: split + merge)."""
     q_heads, kv_heads, head_dim = 16, 2, 256

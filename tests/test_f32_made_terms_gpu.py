@@ -28,7 +28,9 @@ def under(env, call):
 
 MADE = {"halves": {"SKV_F32_TERMS": "2"}, "one_tile": {"SKV_F32_TERMS": "2", "SKV_PREFILL_TILES2_MIN_PAGES": "1000000"},
         "segments": {"SKV_F32_TERMS": "2", "SKV_F32_TERMS_MB": "1"}, "no_split": {"SKV_F32_TERMS": "2", "SKV_PREFILL_MAX_SPLITS": "1"},
-        "own": {"SKV_F32_TERMS": "0"}}
+        "own": {"SKV_F32_TERMS": "0"},
+        # chosen, and then no memory for them: the call stores its rows and splits its pages another way
+        "refused": {"SKV_F32_TERMS": "2", "SKV_F32_TERMS_MB": "0"}}
 
 
 @pytest.mark.parametrize("mode", MADE)
@@ -68,7 +70,7 @@ def test_chunks_of_made_terms(state, mode, dims, window, base, chunks):
     assert np.array_equal(gk, cache.keys()[first:]) and np.array_equal(gv, cache.values()[first:])
 
 
-@pytest.mark.parametrize("mode", ["halves", "segments"])
+@pytest.mark.parametrize("mode", ["halves", "segments", "refused"])
 @pytest.mark.parametrize("head_dim,window,base", [(64, 0, 61), (128, 0, 900), (256, 0, 333), (64, 70, 61), (128, 900, 1200)])
 def test_infinities_as_in_the_other_way(state, mode, head_dim, window, base):
     """Rows with infinities, and rows that were rolled back and hold NaN: the same contexts either way, and no NaN from rows that
