@@ -275,12 +275,14 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
         if constexpr (SHARE) return kx;
         else return vx_own;
     }();
+    // (places as unsigned numbers: the remainder by a power of two of a signed one, which the compiler does not know to be positive, takes
+    // registers that head_dim 256 does not have: a ring chunk of 64 rows of q16/kv8/hd256 67.0 us against 62.2)
     auto load_k = [&](int it0, int d) __attribute__((always_inline)) { // pages it0 + d ..
 #pragma unroll
         for (int u = 0; u < CU; ++u) {
             const int i = tid + u * THREADS;
             const int pg = min(__builtin_amdgcn_readfirstlane(i / (PLANE / 2)), GP - 1);
-            const int du = i % (PLANE / 2);
+            const int du = (int)((unsigned)i % (PLANE / 2));
             const float4_t *t = tile_of(it0, d + pg, false) + (du >> 5) * 64 + ((du >> 4) & 1) * 32 + (du & 15);
             kx[u][0] = t[0];
             kx[u][1] = t[16];
@@ -291,8 +293,8 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
         for (int u = 0; u < CU; ++u) {
             const int i = tid + u * THREADS;
             const int pr = min(__builtin_amdgcn_readfirstlane(i / PLANE), HALVES - 1);
-            vx[u][0] = tile_of(it0, d + 2 * pr, true)[i % PLANE];
-            vx[u][1] = tile_of(it0, d + 2 * pr + 1, true)[i % PLANE];
+            vx[u][0] = tile_of(it0, d + 2 * pr, true)[(unsigned)i % PLANE];
+            vx[u][1] = tile_of(it0, d + 2 * pr + 1, true)[(unsigned)i % PLANE];
         }
     };
     // Keys that no slot of the workgroup attends: zero probability, but 0 x NaN is NaN, so on the
@@ -331,7 +333,7 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
             // K: [half][term][page of the pair][P/2 * 4 units]; V: [half][term][PLANE]
             const int h = i / PLANE;
             if (FULL || h < HALVES) {
-                u4 *dst = kv_planes + (v ? V_AT : 0) + h * 3 * PLANE + i % PLANE;
+                u4 *dst = kv_planes + (v ? V_AT : 0) + h * 3 * PLANE + (unsigned)i % PLANE;
                 dst[0] = u4{t0[0], t0[1], t0[2], t0[3]};
                 dst[PLANE] = u4{t1[0], t1[1], t1[2], t1[3]};
                 dst[2 * PLANE] = u4{t2[0], t2[1], t2[2], t2[3]};
@@ -543,6 +545,7 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
     };
 
     const u4 *const planes = kv_planes + half * 3 * PLANE + lane;
+    const u4 *const v_planes = kv_planes + V_AT + half * 3 * PLANE + lane; // not MADE
     constexpr int BEATS = 2 * KK * 6;
     static_assert(BEATS >= 9 && (MADE ? BEATS >= 2 * CPW : BEATS >= SPLIT_STEPS * (SHARE ? 2 : 1)), "at most one step of a kind between two products");
     // operand set `at` of a window, K-step at / 2 of page A or B, dim tile `at` of V: three terms
@@ -710,7 +713,7 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
             __syncthreads();
             if constexpr (!SHARE) load_v(it0, 0);
             if constexpr (!SHARE) ask_ids(it0 + GP);
-            accumulate(planes + V_AT, none);
+            accumulate(v_planes, none);
             if constexpr (SHARE) {
                 load_v(it0, 0);
                 ask_ids(it0 + GP);
