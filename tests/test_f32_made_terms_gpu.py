@@ -98,3 +98,63 @@ def test_infinities_as_in_the_other_way(state, mode, head_dim, window, base):
         assert np.array_equal(test(got), test(want))
     ok = np.isfinite(want)
     assert (np.abs(got[ok] - want[ok]) <= 2e-5 * np.maximum(np.abs(want[ok]), 1.0)).all()
+
+
+@pytest.mark.parametrize("mode", ["halves", "one_tile", "segments", "no_split", "refused"])
+@pytest.mark.parametrize("over", ["k", "v"])
+def test_context_over_the_rows_that_the_terms_launch_stores(state, mode, over):
+    """The context may lie where the chunk's K or V rows are (a caller's activations share a buffer)."""
+    torch = pytest.importorskip("torch")
+    q_heads, kv_heads, head_dim, base, rows = 8, 2, 64, 300, 200
+    kv_dim, q_dim = kv_heads * head_dim, q_heads * head_dim
+    rng = np.random.default_rng(rows)
+    k0, v0 = (rng.standard_normal((base, kv_dim), dtype=np.float32) for _ in range(2))
+    q, k, v = (rng.standard_normal((rows, d), dtype=np.float32) for d in (q_dim, kv_dim, kv_dim))
+    kv = state.full_attention_f32(base + rows, q_heads, kv_heads, head_dim)
+    kv.seed(k0, v0, base)
+    lay = oracle.layout(q_heads, kv_heads, head_dim)
+    cache = oracle.LayerKvCache("f32")
+    cache.append_batch(k0, v0, lay)
+    want = oracle.cached_attention_prefill_rows(q, k, v, cache, lay)
+    arena = torch.zeros(rows * q_dim, device="cuda")  # the context's; the rows lie in its end
+    shared = torch.from_numpy(k if over == "k" else v).cuda().flatten()
+    apart, qd = torch.from_numpy(v if over == "k" else k).cuda(), torch.from_numpy(q).cuda()
+    arena[-rows * kv_dim:] = shared
+    at = arena.data_ptr() + rows * (q_dim - kv_dim) * 4
+    stream = torch.cuda.current_stream().cuda_stream
+    under(MADE[mode], lambda: kv.encode_prefill_rows(stream, qd.data_ptr(), at if over == "k" else apart.data_ptr(),
+                                                     at if over == "v" else apart.data_ptr(), rows, arena.data_ptr()))
+    torch.cuda.synchronize()
+    assert np.abs(arena.cpu().numpy().reshape(rows, q_dim) - want).max() <= 2e-5
+    gk, gv = kv.read_rows_f32(0, kv.len())
+    assert np.array_equal(gk, cache.keys()) and np.array_equal(gv, cache.values())
+
+
+def test_chunks_of_made_terms_on_two_streams_in_turn(state):
+    """Two sequences of one context on streams of their own, whose chunks are in flight together: each has its terms to itself."""
+    torch = pytest.importorskip("torch")
+    q_heads, kv_heads, head_dim, steps = 16, 4, 64, 5
+    kv_dim, q_dim = kv_heads * head_dim, q_heads * head_dim
+    lay = oracle.layout(q_heads, kv_heads, head_dim)
+    work = []
+    for i, rows in enumerate((130, 96)):
+        gen = np.random.default_rng(i)
+        q, k, v = (gen.standard_normal((steps, rows, d), dtype=np.float32) for d in (q_dim, kv_dim, kv_dim))
+        work.append((state.full_attention_f32(steps * rows, q_heads, kv_heads, head_dim), torch.cuda.Stream(), rows, (q, k, v),
+                     [torch.from_numpy(x).cuda() for x in (q, k, v)], torch.empty(steps, rows, q_dim, device="cuda")))
+    torch.cuda.synchronize()
+
+    def run():
+        for step in range(steps):
+            for kv, stream, rows, _, (q, k, v), out in work:
+                kv.encode_prefill_rows(stream.cuda_stream, q[step].data_ptr(), k[step].data_ptr(), v[step].data_ptr(), rows, out[step].data_ptr())
+
+    under(MADE["halves"], run)
+    torch.cuda.synchronize()
+    for kv, _, rows, (q, k, v), _, out in work:
+        cache = oracle.LayerKvCache("f32")
+        for step in range(steps):
+            want = oracle.cached_attention_prefill_rows(q[step], k[step], v[step], cache, lay)
+            assert np.abs(out[step].cpu().numpy() - want).max() <= 2e-5, step
+        gk, gv = kv.read_rows_f32(0, kv.len())
+        assert np.array_equal(gk, cache.keys()) and np.array_equal(gv, cache.values())
