@@ -69,9 +69,8 @@ __device__ __forceinline__ void load_tile(uint4 (&x)[KK], const uint16_t *pool, 
 // the rows it uses, in LDS, while its first page is in flight.
 // ROWS: a chunk's few rows, which the launch appends (compiled apart: the larger chunks of the multi-query mode,
 // 512 rows of q32/kv8/hd128 over none, lose 2 us of 18 with it).
-// SHARED: the launch has many tiles of query slots, whose workgroups ask for the same pages: plain loads instead of
-// non-temporal ones (whole chunks on layers that are in no cache, in us: 50 rows over 4000 of q16/kv2/hd256, 25 tiles, 29.0 -> 25.5;
-// 128 rows over 1000 of q32/kv8/hd128, 32 tiles, 15.2 -> 15.3; but 32 rows over 4700, 8 tiles, 20.4 -> 21.2, 12 rows 13.1 -> 13.3).
+// SHARED: the workgroups of several tiles of query slots ask for the same pages from different XCDs: plain loads instead of
+// non-temporal ones (pages_shared).
 template <int P, int WAVES, bool MQ, bool PRE, bool ROWS = false, bool SHARED = false>
 __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int split, const int kvh,
                                                   const int tile_z) {
@@ -906,11 +905,23 @@ static hipError_t launch_split_mq(const DecodeArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 
+// Whether the launch's page loads are plain: the pages may stay in the caches for other tiles of query slots. Workgroup ids
+// go to the eight XCDs in turn, so where splits x kv heads are whole eights all tiles of a (split, kv head) run on one XCD at about the same time, and
+// its L2 serves them with non-temporal loads as well, which are the faster ones there. Elsewhere, and with very many tiles, plain loads are.
+// Whole chunks on layers in no cache, non-temporal / plain, in us on average over contexts of 400 to 12000: eights, 6 to 8 tiles a kv head of q32/kv8/hd128 or
+// hd64 1/1.06, 16 to 20 1/1.04, 32 1/1.02, 40 to 64 1/1.00, of q16/kv8/hd256 4 to 8 1/1.02, 64 1/0.98, 75 to 128 1/0.95 to 0.88; not eights,
+// q16/kv2/hd256 9 to 28 tiles 1/0.97 to 0.86 (10, 16 and 32, which are: 1/1.03, 1.03, 1.01), 80 to 128 1/0.88, q28/kv4/hd128 1/0.99 to 0.90
+// (13, 16, 28, which are: 1/1.05, 1.04, 1.03), q30/kv10/hd96 1/1.00 to 0.81 (6, which are: 1/1.08).
+static bool pages_shared(const DecodeArgs &a) {
+    const int tiles = (a.n_queries * a.g.gqa + 15) / 16;
+    return tiles > 64 || (tiles > 4 && a.splits * a.g.kv_heads % 8 != 0);
+}
+
 // Query rows over the cache, 16 slots a workgroup (a chunk's few rows are appended by the launch itself).
 template <int P, int WAVES>
 static hipError_t launch_split_rows(const DecodeArgs &a, hipStream_t s) {
     if (a.pre) return hipErrorInvalidValue; // the caller keeps the fused step to single-tile decode
-    if (a.n_queries * a.g.gqa > 240 && !a.k_new) return launch_split_mq<P, WAVES, true, false, false, true>(a, s);
+    if (!a.k_new && pages_shared(a)) return launch_split_mq<P, WAVES, true, false, false, true>(a, s);
     return a.k_new && a.n_queries > 1 ? launch_split_mq<P, WAVES, true, false, true>(a, s)
                                       : launch_split_mq<P, WAVES, true, false>(a, s);
 }
