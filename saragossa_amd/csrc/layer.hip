@@ -247,24 +247,40 @@ TileShape prefill_shape(const Geom &g, size_t n_slots, size_t n_pages) {
 // through LDS, or the decode kernel's multi-query mode (speculative verify rows, short chunks over short contexts): one workgroup
 // per 16 slots that streams the pages into its own registers, without a prologue to speak of, but asks for every page once per 16
 // slots. The line is the number of (16 slots, page) pairs, as a chunk's rows walk them on the average, where those requests cost
-// what the tile kernel's start does; and that start is one workgroup's on every compute unit, with no split and no merge, where
-// the chunk's 64-slot workgroups are 208 to 256. Over 136 chunks of 32 to 2048 rows over 0 to 16000 the kernel chosen is at most 12 %
-// slower than the other but for one (256 rows of q8/kv2/hd512 over none, 38.3/30.1), 0.9 % on the average (by all pages, and lower
-// lines, 51 % and 3.5 %). Whole chunks, multi-query mode / tile
-// kernel, in us on one MI355X, with the pairs they walk in thousands: q32/kv8/hd128, 512 rows over 0, 100, 300 (16, 24, 36; 256
-// workgroups) 19.1/18.3, 22.6/20.4, 28.0/23.3; 128 over 2000 (33) 21.4/26.3; 256 over 1000, 1500 (36, 53) 25.4/27.6, 32.1/31.3;
-// q28/kv4/hd128, 512 over 500 (43) 31.6/25.4, 128 over 4000 (57) 31.9/31.8; q16/kv2/hd256, 512 over 500, 1000 (25, 40) 33.0/36.8, 43.7/42.7,
-// 256 over 1000, 2000 (18, 34) 23.9/32.0, 35.0/38.3, 64 over 4000, 8000 (16, 32) 28.6/33.3, 40.5/38.9, 850 over none (24; 214) 42.7/33.1;
-// q12/kv4/hd96, 512 over 1000, 2000 (30, 54) 19.5/23.6, 27.3/30.8, 128 over 8000 (48) 33.4/28.8; q8/kv2/hd64, 512 over 1000, 2000 (20, 36)
-// 12.9/16.0, 16.4/18.1, 256 over 4000 (33) 19.5/19.6; q32/kv8/hd64, 512 over 0, 400 (16, 42; 256) 13.7/13.0, 20.8/17.9; q8/kv2/hd512, 64
-// over 1000 (2) 29.9/36.5, 512 over none (4) 37.3/40.3; q16/kv8/hd512, 64 over 1000 (4) 41.6/39.0.
+// what the tile kernel's start does. It depends on how the workgroups of either fall on the 256 compute units:
+// - the multi-query mode's, one to a compute unit: it loses early where two splits and their merge have to make up for few tiles (86 to 128 of
+//   16 slots), or where the last round of workgroups leaves more than a third of the device idle;
+// - the tile kernel's 64-slot ones: from 129 on they need no split and no merge, from 193 to 256 they fill the device in one round; above, they
+//   are of 128 slots.
+// Over 1955 chunks of 12 to 1024 rows around the lines in nineteen geometries, on layers in no cache, the kernel chosen is 0.6 % slower than the
+// better one on the average (P 512: 1 %), 17 % at most. Multi-query mode / tile kernel, in us on one MI355X, with the pairs they walk in thousands:
+// q32/kv8/hd128, no such trouble: 128 rows (256 tiles) 30 20.9/24.6, 54 30.9/30.5; two splits: 64 rows (128) 18 22/23.0, 30 28/26.5; a third idle:
+// 160 rows (320) 18 21.7/22.4, 30 28.4/25.6; unsplit tiles: 384 rows (192 workgroups of 64) 18 18.5/18.4, 37 25.8/24.4; one round:
+// 512 rows (256) 16 19.5/17.0, 37 27.9/22.7, q28/kv4/hd128, 448 rows (196) 12 18.0/16.5, 37 30.7/24.2; above: 600 rows (304) 31
+// 26.9/27.8, 44 33.1/32.3. q16/kv2/hd256, 256 rows (256 tiles) 18 23.6/30.2, 33 33.8/35.5; 128 rows (128) 9 27.6/26.7, 23 36.7/32.4; 320 rows
+// (320) 14 28.7/28.7, 23 37.1/31.6; 700 rows (176 workgroups) 16 31.0/27.3, 33 44.4/35.7. q8/kv2/hd512, 32 rows (16 tiles) 4.5 37.2/46.0; 128 rows
+// (64) 3.7 38.9/41.0, 5.6 46.8/41.7; 200 rows (100, two splits) 1.3 37.7/33.3; 320 rows (160) 3.2 36.8/42.2, 5.6 49.0/44.4; 600 (300) 6 56.8/44.9.
+// (With one line per size of head, 448 rows of q28/kv4/hd128 over 516 took 30.8, 100 rows of q16/kv8/hd256 over 4108 48.0, 32 of q8/kv2/hd512 over
+// 4500 46.1: now 24.2, 37.1, 36.9.)
 bool takes_tile_kernel(const Geom &g, size_t n_queries, size_t n_pages) {
     const size_t n_slots = n_queries * (size_t)g.gqa;
     if (tuning().prefill_tiles != 1 || n_slots < 64) return tuning().prefill_tiles > 1 && n_slots >= 64;
-    const size_t wgs = (n_slots + 63) / 64 * (size_t)g.kv_heads;
-    const size_t walked = n_pages > n_queries / 32 ? n_pages - n_queries / 32 : 1;
-    const size_t line = g.P <= 32 ? 32500 : g.P <= 64 ? 38000 : g.P <= 96 ? 42000 : g.P <= 128 ? 40000 : g.P <= 256 ? 30000 : 4100;
-    return (n_slots + 15) / 16 * (size_t)g.kv_heads * walked >= (wgs >= 208 && wgs <= 256 ? std::min<size_t>(line, 12000) : line);
+    const size_t wgs = (n_slots + 63) / 64 * (size_t)g.kv_heads, tiles = (n_slots + 15) / 16 * (size_t)g.kv_heads;
+    const size_t walked = n_pages > n_queries / 32 ? n_pages - n_queries / 32 : 1, pairs = tiles * walked;
+    if (g.P > 256) return pairs >= (tiles <= 36 ? 6000u : tiles <= 85 ? 4200u : tiles <= 128 ? 1100u : tiles <= 256 ? 5200u : 3000u);
+    struct Lines {
+        size_t full, two_splits, third_idle, unsplit, one_round, many;
+    };
+    const Lines l = g.P <= 32    ? Lines{44000, 35500, 29500, 15500, 12000, 32000}
+                    : g.P <= 64  ? Lines{51500, 34300, 34300, 17300, 12000, 34500}
+                    : g.P <= 96  ? Lines{50000, 25500, 31500, 25500, 12000, 33000}
+                    : g.P <= 128 ? Lines{44000, 30000, 26500, 18500, 12000, 37500}
+                                 : Lines{26000, 9000, 13700, 9000, 9000, 20000};
+    if (wgs > 256) return pairs >= l.many;
+    if (wgs > 192) return pairs >= l.one_round;
+    if (wgs > 128) return pairs >= l.unsplit;
+    if (tiles <= 128) return pairs >= (tiles > 85 ? l.two_splits : l.full);
+    return pairs >= (3 * tiles < 2 * 256 * ((tiles + 255) / 256) ? l.third_idle : l.full);
 }
 
 // The same questions for f32 layers: the kernel that splits its factors into bf16 terms (head_dim up to
