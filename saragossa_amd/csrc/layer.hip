@@ -328,16 +328,17 @@ int chunk_splits(const Geom &g, size_t n_queries, size_t per_wg, size_t n_pages)
 // (split, kv head) run on one XCD and its L2 has a page from memory once. Worth up to a tenth of the splits: rows of
 // q16/kv2/hd256 as whole chunks on layers in no cache, in us, splits as they are / in whole eights, 6 over 8192 (42/40)
 // 15.6/14.7, over 20000 22.5/19.9, 12 over 8192 (21/20) 21.0/17.1; with plain loads 18 over 4000 (14/12) 16.9/17.6, 23 (11/8)
-// 17.5/17.8, 36 (7/4) 20.5/22.7. On f32 layers (42/40 and 21/20) 6 over 20000 88.5/80.4, 12 over 8192 61.6/58.5.
+// 17.5/17.8, 36 (7/4) 20.5/22.7. On f32 layers (42/40 and 21/20) 6 over 20000 88.5/80.4, 12 over 8192 61.6/58.5, but 24 of q28/kv4/hd128
+// (11/10) over 1356, 3420 23.6/24.3, 32.0/33.1, 28 of q24/kv4/hd256 over 1356 1/1.10: there a sixteenth (`share`).
 // Not where the wavefronts of a workgroup are four (f32 layers, heads above 256 dims), have a page each and would walk a second one: 12
 // rows of q8/kv2/hd512 over 1300 (21/20 splits of 83 pages) 20.9/22.8, on f32 layers 35.7/42.9, 30 of q16/kv2/hd256 over 1042
 // (17/16 of 67) on f32 34.1/36.5. (Where they walk two already fewer splits gain: 12 rows of q8/kv2/hd512 on f32 over 2680 65.2/52.5; and
 // eight wavefronts gain in any case, 6 rows of q16/kv2/hd256 over 2630, 42/40 of 165, 13.6/12.9.)
-int xcd_splits(int splits, int kv_heads, int n_pages, int waves) {
+int xcd_splits(int splits, int kv_heads, int n_pages, int waves, int share) {
     int unit = 8;
     for (int h = kv_heads; unit > 1 && h % 2 == 0; h /= 2) unit /= 2;
     const int fewer = splits - splits % unit;
-    if (splits % unit * 10 > splits || (waves == 4 && n_pages <= splits * 4 && n_pages > fewer * 4)) return splits;
+    if (splits % unit * share > splits || (waves == 4 && n_pages <= splits * 4 && n_pages > fewer * 4)) return splits;
     return fewer;
 }
 
@@ -702,7 +703,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
             // ring: 22.3 us with one, 29.7 with two and a merge)
             if (L->g.ring_rows > 0) want = std::min(want, std::max<size_t>((size_t)a.n_pages / 8, 1));
             a.splits = (int)std::min<size_t>((size_t)a.splits, want);
-            if (tiles > (size_t)g.kv_heads) a.splits = xcd_splits(a.splits, g.kv_heads, a.n_pages, 4);
+            if (tiles > (size_t)g.kv_heads) a.splits = xcd_splits(a.splits, g.kv_heads, a.n_pages, 4, 16);
             a.splits_total = a.splits;
             if (a.splits > 1) {
                 int32_t rc2 = multi_query_partials(L, s, (size_t)a.splits, n_queries, a, lease);
@@ -781,7 +782,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
             want = std::min<size_t>(want, tuning().prefill_max_splits);
         }
         a.splits = (int)std::min<size_t>((size_t)a.splits, want);
-        if (!use_tiles && tiles > (size_t)g.kv_heads) a.splits = xcd_splits(a.splits, g.kv_heads, a.n_pages, a.waves);
+        if (!use_tiles && tiles > (size_t)g.kv_heads) a.splits = xcd_splits(a.splits, g.kv_heads, a.n_pages, a.waves, 10);
         a.splits_total = a.splits;
         if (a.splits > 1) {
             int32_t rc2 = multi_query_partials(L, s, (size_t)a.splits, n_queries, a, lease);
