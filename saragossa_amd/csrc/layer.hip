@@ -553,11 +553,12 @@ F32Plan plan_f32_chunk(const Geom &g, size_t n_queries, int first_entry, int ent
     // Halves cover half the slots and walk two pairs at a time: the same time per workgroup with half as many splits, so fewer
     // partials, but they copy each page for half as many slots, which costs more on long walks. Whole chunks, one tile / halves, in us: q32/kv8/hd128, 512 rows
     // over 512, 1024, 2048, 6000, 8192 (two splits / one) 59.1/51.2, 74.5/68.5, 114/109, 262/265, 340/349; q8/kv2/hd64, 512 rows over 2048, 4096,
-    // 10000 (eight / four) 32.2/28.0, 42.5/40.0, 74.0/72.7; but q28/kv4/hd128, 300 rows over 3000 (three / one) 91.2/115.
+    // 10000 (eight / four) 32.2/28.0, 42.5/40.0, 74.0/72.7, 448 over 1856, 3420 (nine / four) 31.1/26.5, 39.9/34.5; but q28/kv4/hd128, 300 rows over
+    // 3000 (three / one) 91.2/115. So a ninth of the workgroups may go.
     const size_t pages = (size_t)walked / (size_t)p.segments;
     const int one = chunk_splits(g, n_queries, (size_t)f32_prefill_slots(g.P, false), pages);
     const int two = chunk_splits(g, n_queries, (size_t)f32_prefill_slots(g.P, true), pages);
-    p.halves = g.P <= 128 && tuning().prefill_tiles2_min_pages < 0 && 2 * two >= one && walked <= 300;
+    p.halves = g.P <= 128 && tuning().prefill_tiles2_min_pages < 0 && 18 * two >= 8 * one && walked <= 300;
     // (choose_splits' number, which the split knobs of decode launches bound, is the larger one unless they do)
     p.splits = std::min(max_splits, p.halves ? two : one);
     return p;
