@@ -288,23 +288,31 @@ bool takes_tile_kernel(const Geom &g, size_t n_queries, size_t n_pages) {
 // page) pairs as a chunk's rows walk them on the average, each up to its own position: half of the pages of a
 // first chunk (counted by all pages, 384 rows of q16/kv2/hd256 over 100 took the first kernel, 82.5 us, where
 // streaming takes 52.2, and 512 over none 58.8 where it takes 51.1), lower where 64-slot workgroups fill the device without a split.
-// Over 85 chunks of 64 to 1024 rows over 0 to 8000 around the lines the kernel chosen is at most 14 % slower than the other, 0.5 % on
-// the average (32 % and 3 % with one line to a size of head and the lines where terms were not made by a launch). Whole chunks,
+// Over 937 chunks of 64 to 1024 rows around the lines in ten geometries the kernel chosen is 1 % slower than the other on the average, at most 27 % (384
+// rows of q32/kv8/hd128 over 52, 192 workgroups of 64 slots). Whole chunks,
 // streaming / the kernel of terms, in us, with the pairs they walk in thousands: q32/kv8/hd128, 512 rows over none (16; 256 workgroups)
 // 40.4/31.1, 416 (11; 208) 34.2/27.8, 64 over 1000, 2000 (8, 16) 25.7/30.7, 36.0/34.1, 128 over 300, 1000 (6, 17) 23.4/32.3, 37.5/33.4, 256 over
 // 300 (14) 31.3/34.5; q24/kv8/hd128, 128 over 1000 (13) 36.7/31.9; q12/kv4/hd96, 256 over 1000 (14) 30.7/26.9, 128 over 2000 (12) 27.6/28.5;
 // q8/kv8/hd80, 64 over 8000 (16) 36.1/40.3; q8/kv2/hd64, 256 over 2000, 4000 (17, 33) 22.0/24.7, 32.6/30.8, 512 over 300, 1000 (9, 20)
 // 18.1/20.9, 25.1/22.9; q32/kv8/hd64, 416 over none (11; 208) 19.8/18.6, 160 over 1000 (22) 30.7/26.1; q16/kv2/hd256, 128 over 1000, 2000
-// (9, 17) 50.7/61.5, 71.7/64.0; q32/kv8/hd32, 512 over none (16; 256) 14.7/15.7.
+// (9, 17) 50.7/61.5, 71.7/64.0; q32/kv8/hd32, 512 over none (16; 256) 14.7/15.7; where streaming fills its round, or is of few tiles, q32/kv8/hd128, 256
+// over 312 (14; 512 tiles) 31.8/34.2, 160 over 600 (14; 320) 38.6/30.9, q32/kv8/hd64, 350 over 312 (23; 704) 26.1/28.0, q8/kv2/hd64, 64 over
+// 11800 (24; 64) 32.3/34.2.
 bool takes_f32_chunk_kernel(const Geom &g, size_t n_queries, size_t n_pages) {
     const size_t n_slots = n_queries * (size_t)g.gqa;
     if (f32_prefill_slots(g.P, false) == 0 || n_slots < 64 || tuning().prefill_tiles == 0) return false;
     if (tuning().prefill_tiles > 1) return true;
     const size_t wgs = (n_slots + 63) / 64 * (size_t)g.kv_heads;
-    size_t line = g.P <= 32 ? 26000 : g.P <= 64 ? 21500 : g.P <= 96 ? 16200 : g.P <= 128 ? 12600 : 12200;
+    const size_t tiles = (n_slots + 15) / 16 * (size_t)g.kv_heads;
+    // (512 tiles of 16 slots are one full round of streaming workgroups, two to a compute unit)
+    size_t line = g.P <= 32    ? 26000
+                  : g.P <= 64  ? (tiles <= 85 || tiles > 384 ? 25000 : 21500)
+                  : g.P <= 96  ? 16200
+                  : g.P <= 128 ? (tiles > 448 && tiles <= 512 ? 15000 : 12600)
+                               : 12200;
     if (g.P > 32 && wgs >= 208 && wgs <= 256) line = std::min<size_t>(line, 10000);
     const size_t walked = n_pages > n_queries / 32 ? n_pages - n_queries / 32 : 1;
-    return (n_slots + 15) / 16 * (size_t)g.kv_heads * walked >= line;
+    return tiles * walked >= line;
 }
 bool f32_halves(const Geom &g, size_t n_slots, size_t n_pages) {
     if (tuning().prefill_tiles2_min_pages >= 0) return false;
