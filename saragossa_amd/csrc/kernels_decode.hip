@@ -907,14 +907,14 @@ static hipError_t launch_split_mq(const DecodeArgs &a, hipStream_t s) {
 
 // Whether the launch's page loads are plain: the pages may stay in the caches for other tiles of query slots. Workgroup ids
 // go to the eight XCDs in turn, so where splits x kv heads are whole eights all tiles of a (split, kv head) run on one XCD at about the same time, and
-// its L2 serves them with non-temporal loads as well, which are the faster ones there. Elsewhere, and with very many tiles, plain loads are.
+// its L2 serves them with non-temporal loads as well, which are the faster ones there. Elsewhere, and with many tiles, plain loads are.
 // Whole chunks on layers in no cache, non-temporal / plain, in us on average over contexts of 400 to 12000: eights, 6 to 8 tiles a kv head of q32/kv8/hd128 or
-// hd64 1/1.06, 16 to 20 1/1.04, 32 1/1.02, 40 to 64 1/1.00, of q16/kv8/hd256 4 to 8 1/1.02, 64 1/0.98, 75 to 128 1/0.95 to 0.88; not eights,
+// hd64 1/1.06, 16 to 20 1/1.04, 32 1/1.02, 40 to 64 1/1.00, of q16/kv8/hd256 4 to 16 1/1.02, 25 to 64 1/0.98, 75 to 128 1/0.95 to 0.88; not eights,
 // q16/kv2/hd256 9 to 28 tiles 1/0.97 to 0.86 (10, 16 and 32, which are: 1/1.03, 1.03, 1.01), 80 to 128 1/0.88, q28/kv4/hd128 1/0.99 to 0.90
 // (13, 16, 28, which are: 1/1.05, 1.04, 1.03), q30/kv10/hd96 1/1.00 to 0.81 (6, which are: 1/1.08).
 static bool pages_shared(const DecodeArgs &a) {
     const int tiles = (a.n_queries * a.g.gqa + 15) / 16;
-    return tiles > 64 || (tiles > 4 && a.splits * a.g.kv_heads % 8 != 0);
+    return tiles > 32 || (tiles > 4 && a.splits * a.g.kv_heads % 8 != 0);
 }
 
 // Query rows over the cache, 16 slots a workgroup (a chunk's few rows are appended by the launch itself).

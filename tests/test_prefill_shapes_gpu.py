@@ -209,7 +209,7 @@ def test_few_rows_are_appended_by_the_attention_launch(state, dims, window, star
 @pytest.mark.parametrize("dims,base,counts", [
     ((16, 2, 256), 700, (30, 31)),  # 15 and 16 tiles of 16 slots, three splits each
     ((16, 2, 256), 1500, (17, 31, 32)),  # 9 tiles in 14 splits, whose workgroups want a page on several XCDs; 16 in 8, on one
-    ((64, 8, 32), 5, (128, 130)),   # 64 tiles a kv head, and more
+    ((64, 8, 32), 5, (64, 66)),     # 32 tiles a kv head, and more
     ((16, 2, 256), 5000, (6, 12)),  # 42 and 21 splits over two kv heads: taken in whole eights, 40 and 20
     ((6, 3, 48), 3100, (20, 130)),  # no power of two of kv heads
 ])
