@@ -164,8 +164,8 @@ __global__ __launch_bounds__(256) void f32_terms_kernel(DecodeArgs a, ChunkPages
 // buffer each: V of a group of pairs is stored while the scores of the next group are computed, K of the group after
 // that while the accumulation runs, with a barrier behind each window; the loads are issued a window ahead.
 // Bound by the matrix pipes, which run at 1.4 PFLOP/s on long walks. 512 rows as one call on layers that are in no cache, in us on
-// one MI355X, split by the workgroup / made: q32/kv8/hd128 over 0, 512, 1024, 4096, 16384 rows 39.3/33.0, 59.0/50.8, 88/73,
-// 193/184, 655/636; q16/kv2/hd256 over 1024, 4096 81.6/75.5, 191/176. (f32_split_kernel, kernels_f32.hip, over 512, 16384 of the
+// one MI355X, split by the workgroup / made: q32/kv8/hd128 over 0, 512, 1024, 4096, 16384 rows 35.0/30.1, 57.8/50.3, 80.1/69.5,
+// 187/183, 632/627; q16/kv2/hd256 over 1024, 4096 80.7/75.0, 188/173. (f32_split_kernel, kernels_f32.hip, over 512, 16384 of the
 // former 83.5, 1267.) At head_dim 256 the third terms of the queries live in LDS: in registers they spill.
 // ------------------------------------------------------------------------------------
 template <int P, int TILES, int WAVES, int HALVES, bool RING, bool MADE>

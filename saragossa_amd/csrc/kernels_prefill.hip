@@ -65,10 +65,9 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // wavefront to copy and the moves that put operands together and the search for the maximum between products, chunks of 512
 // rows on layers that are in no cache went, in us, for q32/kv8/hd128 over 4700, 16384 from 88.0 to 80.5, 224 to 213; for
 // q16/kv8/hd256 on a ring of 1024 rows from 47.2 to 44.1. (Second terms of the probabilities as dot products of the pair of
-// first terms with -1 and 0, an instruction less each, took longer: 1024 rows of q24/kv8/hd128 over 4000 139.4 against 132.2.
-// Three
-// wavefronts per SIMD, twelve in thirds at 154 registers, were no faster than two; two tiles per wavefront at
-// head_dim 256, four wavefronts at 400 registers, 11 to 40 % slower.)
+// first terms with -1 and 0, an instruction less each, took longer: 1024 rows of q24/kv8/hd128 over 4000 139.4 against 132.2. Three
+// wavefronts per SIMD, twelve in thirds at 154 registers, were no faster than two; two tiles per wavefront at head_dim 256, four
+// wavefronts at 400 registers, 11 to 40 % slower.)
 // ------------------------------------------------------------------------------------
 
 // LDS order of a step, SP pairs: [SP][K tile of page A | K tile of page B], then V the same way, tiles
@@ -97,8 +96,8 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
     constexpr int KK = P / 32;
     constexpr int NT = P / 16;
     // Vector work is held in its place between the products; a wavefront alone on its SIMD (head_dim above 256), and one with
-    // few products to a pair (up to 64), does better where the compiler places it (256 rows of q8/kv2/hd512 over 4096: 61.0 us
-    // against 66.0; 1024 of q8/kv2/hd64 over 8000: 53.0 against 55.7)
+    // few products to a pair (up to 96), does better where the compiler places it (256 rows of q8/kv2/hd512 over 4096: 61.0 us
+    // against 66.0; 1024 of q8/kv2/hd64 over 8000: 53.0 against 55.7; heads of 65 to 96 dims 1 to 3 %)
     constexpr bool PINNED = KK >= 4 && P <= 256;
     constexpr int TILE_U4 = KK * 64;                           // 16-byte units of one K (or V) tile
     constexpr int GP = 2 * HALVES;                             // pages of a group: a pair for each half

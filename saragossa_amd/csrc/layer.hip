@@ -211,9 +211,11 @@ size_t decode_target_wgs() { return tuning().target_wgs; }
 // the most splits: they pay on long walks. Above 256 workgroups of 64 slots the device is full in any shape. The lines are in pages walked
 // by all 64-slot workgroups, where whole chunks cost the same in two shapes, between layers that are not in any cache and those that are, as a
 // short prompt's, where halves stay ahead for longer (512 rows of q32/kv8/hd64 over 2000, halves / two tiles 29.5/36.1 in
-// caches, 34.8/36.2 not; of q32/kv8/hd128 over 1024, halves / quarters 34.5/34.9 and 34.4/36.3, over 2048 46.8/47.6 and 50.5/46.8). Over 134
-// chunks of 128 to 1024 rows over 500 to 12000 the shape chosen is at most 11 % slower than the best, 1 % on the average (31 % and
-// 2.4 % with fewer, wider lines). One tile / two tiles / halves / quarters, in us on one MI355X, in no cache, with workgroups, walk in thousands: q32/kv8/hd128, 400 rows over 500, 1500, 3000, 6000 (200; 11, 24, 43,
+// caches, 34.8/36.2 not; of q32/kv8/hd128 over 1024, halves / quarters 34.5/34.9 and 34.4/36.3, over 2048 46.8/47.6 and 50.5/46.8). On layers
+// in no cache, over 181 chunks of 64 to 1024 rows with up to 256 workgroups, the shape chosen is 1.7 % slower than the best on the average, at most 14 %
+// (400 to 600 rows of hd128 heads at walks of 20000 to 29000, where halves are up to 13 % behind quarters; in caches the two are even). Above 256
+// workgroups, over 33 chunks, 10 % and 42 %: the line of two tiles stands too high for 257 to 350 of them (700 rows of q28/kv4/hd128 over
+// 4000, 8000, one tile / two 119/92, 210/149). One tile / two tiles / halves / quarters, in us on one MI355X, in no cache, with workgroups, walk in thousands: q32/kv8/hd128, 400 rows over 500, 1500, 3000, 6000 (200; 11, 24, 43,
 // 80) 32.5/37.2/25.0/27.2, 42.7/44.5/40.0/37.6, 59.5/59.7/64.0/55.0, 94.4/90.2/110/87.9, 512 over 1500, 6000 (256; 32, 104)
 // 48.0/49.8/42.8/40.8, 106/100/114/96.2; q28/kv4/hd128, 400 over 500, 1500, 6000 (176; 10, 21, 70) 31.8/36.6/23.8/26.3, 42.6/43.2/38.6/36.4,
 // 92.2/79.1/107/85.1; q24/kv8/hd128, 400 over 1500, 3000, 6000 (152; 18, 32, 61) 35.7/41.2/39.6/37.0, 48.5/51.5/63.4/54.3, 74.8/74.5/109/87.2, 512
@@ -253,7 +255,7 @@ TileShape prefill_shape(const Geom &g, size_t n_slots, size_t n_pages) {
 // - the tile kernel's 64-slot ones: from 129 on they need no split and no merge, from 193 to 256 they fill the device in one round; above, they
 //   are of 128 slots.
 // Over 1955 chunks of 12 to 1024 rows around the lines in nineteen geometries, on layers in no cache, the kernel chosen is 0.6 % slower than the
-// better one on the average (P 512: 1 %), 17 % at most. Multi-query mode / tile kernel, in us on one MI355X, with the pairs they walk in thousands:
+// better one on the average (P 512: 1 %), 15 % at most. Multi-query mode / tile kernel, in us on one MI355X, with the pairs they walk in thousands:
 // q32/kv8/hd128, no such trouble: 128 rows (256 tiles) 30 20.9/24.6, 54 30.9/30.5; two splits: 64 rows (128) 18 22/23.0, 30 28/26.5; a third idle:
 // 160 rows (320) 18 21.7/22.4, 30 28.4/25.6; unsplit tiles: 384 rows (192 workgroups of 64) 18 18.5/18.4, 37 25.8/24.4; one round:
 // 512 rows (256) 16 19.5/17.0, 37 27.9/22.7, q28/kv4/hd128, 448 rows (196) 12 18.0/16.5, 37 30.7/24.2; above: 600 rows (304) 31
@@ -515,12 +517,12 @@ AppendArgs append_args(const skv_layer *L, const float *k_dev, const float *v_de
 // the chunk's rows on the way; the attention behind it takes a quarter less on short walks and 5 to 10 % on long ones. So it pays
 // where many slots share a page, and on rings, whose context is short and whose rows otherwise take a launch to pages of
 // their own. Whole chunks on layers that are in no cache, in us, split by the workgroup / by a launch: q32/kv8/hd128, 512 rows over 0, 512,
-// 1024, 2048, 4096 39.4/33.0, 59.2/51.3, 81.2/68.3, 116/108, 194/185, 256 rows (1024 slots) over 500, 2048, 8192 37.4/36.4, 64.0/65.2,
-// 178/190, 64 rows over 8192 63.3/81.6; q28/kv4/hd128, 160 rows over 3000 56.2/57.1, 512 over 16000 611/556; q12/kv4/hd96, 512 rows
-// (1536 slots) over 2000 50.7/50.6; q8/kv2/hd64, 512 rows over 2048, 4096 30.3/27.5, 42.1/38.9, 300 over 10000 54.5/55.7; q16/kv2/hd256,
-// 128 rows (1024 slots) over 4096 71.1/70.3, 256 106/102, 512 190/174, over 16000 256 320/304; q16/kv8/hd256, 512 rows
-// (1024 slots) over 1000 84.2/85.2. Rings: q16/kv8/hd256 of 1024 rows, 64, 256, 512, 1024 rows 62.3/57.0, 67.7/62.5, 76.3/75.9, 120/120;
-// q32/kv8/hd128 of 512 and 1024, 64, 512 rows 32.4/27.7, 48.2/41.2, 128, 256 34.7/33.6, 48.2/43.4; q8/kv2/hd64 128 rows 22.4/19.0.
+// 1024, 2048, 4096 35.0/30.1, 57.8/50.3, 80.1/69.5, 113/107, 187/183, 256 rows (1024 slots) over 500, 2048, 8192 36.9/35.6, 62.8/64.2,
+// 174/187, 64 rows over 8192 62.8/86.3; q28/kv4/hd128, 160 rows over 3000 54.7/56.9, 512 over 16000 587/540; q12/kv4/hd96, 512 rows
+// (1536 slots) over 2000 50.4/50.9; q8/kv2/hd64, 512 rows over 2048, 4096 30.4/28.2, 42.5/39.3, 300 over 10000 55.1/56.8; q16/kv2/hd256,
+// 128 rows (1024 slots) over 4096 71.1/70.2, 256 106/102, 512 188/173, over 16000 256 318/304; q16/kv8/hd256, 512 rows
+// (1024 slots) over 1000 83.8/84.6. Rings: q16/kv8/hd256 of 1024 rows, 64, 256, 512, 1024 rows 62.6/58.6, 68.7/64.5, 77.0/76.9, 127/123;
+// q32/kv8/hd128 of 512 rows, 64, 128 rows 32.3/28.9, 34.1/31.0, of 1024, 256, 512 48.4/44.4, 70.8/60.4; q8/kv2/hd64 of 1024, 128 rows 23.0/19.2.
 bool f32_terms_pay(const Geom &g, size_t n_queries) {
     if (tuning().f32_terms != 1) return tuning().f32_terms > 1;
     return g.ring_rows > 0 || n_queries * (size_t)g.gqa >= (g.P > 128 ? 2048u : 1536u);
@@ -560,9 +562,9 @@ F32Plan plan_f32_chunk(const Geom &g, size_t n_queries, int first_entry, int ent
     p.held = (int)((pairs + (size_t)p.segments - 1) / (size_t)p.segments);
     // Halves cover half the slots and walk two pairs at a time: the same time per workgroup with half as many splits, so fewer
     // partials, but they copy each page for half as many slots, which costs more on long walks. Whole chunks, one tile / halves, in us: q32/kv8/hd128, 512 rows
-    // over 512, 1024, 2048, 6000, 8192 (two splits / one) 59.1/51.2, 74.5/68.5, 114/109, 262/265, 340/349; q8/kv2/hd64, 512 rows over 2048, 4096,
-    // 10000 (eight / four) 32.2/28.0, 42.5/40.0, 74.0/72.7, 448 over 1856, 3420 (nine / four) 31.1/26.5, 39.9/34.5; but q28/kv4/hd128, 300 rows over
-    // 3000 (three / one) 91.2/115. So a ninth of the workgroups may go.
+    // over 0, 512, 1024, 2048, 6000, 8192, 16384 (two splits / one) 41.1/30.0, 58.4/50.1, 74.5/69.3, 111/106, 254/254, 333/336, 627/642; q8/kv2/hd64,
+    // 512 rows over 2048, 4096, 10000 (eight / four) 32.6/28.1, 43.0/39.1, 73.4/72.2, 448 over 1856, 3420 (nine / four) 31.1/26.5, 39.8/34.7; but
+    // q28/kv4/hd128, 300 rows over 3000 (three / one) 90.9/114. So a ninth of the workgroups may go.
     const size_t pages = (size_t)walked / (size_t)p.segments;
     const int one = chunk_splits(g, n_queries, (size_t)f32_prefill_slots(g.P, false), pages);
     const int two = chunk_splits(g, n_queries, (size_t)f32_prefill_slots(g.P, true), pages);
