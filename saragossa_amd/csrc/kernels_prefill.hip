@@ -417,11 +417,10 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
                 const int e = q - 1;
                 l_run[t] += prev;
                 pr2[t][e & 1] = prev;
-                // p = hi + lo with hi the upper 16 bits of p (cut off) and lo the exact remainder rounded to
-                // nearest: 2^-17 relative, of either sign (512 rows of q32/kv8/hd128 over 1536: errors of 5.4e-6
-                // against 64 bits; lo cut off as well, always too small, 9.9e-6)
+                // p = hi + lo, both rounded to nearest: 2^-18 relative, of either sign (512 rows of q8/kv2/hd64 over 2500: errors of 3.4e-6
+                // against 64 bits; with hi the upper 16 bits of p, cut off, as fast, 5.3e-6; both cut off, always too small, 9.9e-6)
                 if (e & 1) {
-                    const uint32_t hi = __builtin_amdgcn_perm(__float_as_uint(prev), __float_as_uint(pr2[t][0]), 0x07060302u);
+                    const uint32_t hi = bf16_pair(pr2[t][0], prev);
                     hi4[t][e >> 1] = hi;
                     lo4[t][e >> 1] = bf16_pair(pr2[t][0] - __uint_as_float(hi << 16), prev - __uint_as_float(hi & 0xffff0000u));
                     if (PINNED) asm volatile("" : "+v"(hi4[t][e >> 1]), "+v"(lo4[t][e >> 1])); // (here, between the products, not behind them)

@@ -173,6 +173,32 @@ def test_first_chunks_of_a_workgroup_to_each_compute_unit(state, element, heads,
     assert (got.double() - want).abs().max() <= (2e-5 if element == "f32" else 7 * 2.0 ** -16 * want.abs().max())
 
 
+@pytest.mark.parametrize("dims,base,rows", [((8, 2, 64), 1500, 70), ((28, 4, 128), 516, 448), ((12, 4, 96), 700, 200), ((16, 2, 256), 200, 300),
+                                            ((8, 2, 512), 32, 256)])
+def test_terms_of_queries_and_probabilities_are_rounded(state, shape, dims, base, rows):
+    """Two bf16 terms each, rounded to nearest: 2^-18 relative at most in a probability and in a query element, whose effects on a
+    context are of either sign. (A first term that is cut off doubles the largest error of a probability: 1.4 times 2^-18 in all.)"""
+    import torch
+    q_heads, kv_heads, head_dim = dims
+    n = base + rows
+    gen = torch.Generator().manual_seed(n)
+    k, v = (torch.randn(n, kv_heads * head_dim, generator=gen) for _ in range(2))
+    q = torch.randn(rows, q_heads * head_dim, generator=gen)
+    kv = state.full_attention_bf16(n, q_heads, kv_heads, head_dim)
+    kv.set_block_table(np.random.default_rng(base).permutation(kv.pages()).astype(np.int32))
+    kv.seed(k[:base].numpy(), v[:base].numpy(), base)
+    got = torch.from_numpy(kv.prefill_rows(q.numpy(), k[base:].numpy(), v[base:].numpy()))
+    hidden = torch.arange(n)[None] > base + torch.arange(rows)[:, None]
+    k, v = (x.bfloat16().double() for x in (k, v))
+    want = torch.empty(rows, q_heads * head_dim, dtype=torch.float64)
+    for h in range(q_heads):
+        own, group = slice(h * head_dim, (h + 1) * head_dim), h // (q_heads // kv_heads)
+        cols = slice(group * head_dim, (group + 1) * head_dim)
+        s = q[:, own].double() @ k[:, cols].T.contiguous() / head_dim ** 0.5
+        want[:, own] = torch.softmax(s.masked_fill(hidden, -float("inf")), -1) @ v[:, cols]
+    assert (got.double() - want).norm() <= 1.15 * 2.0 ** -18 * want.norm()
+
+
 @pytest.mark.parametrize("dims,window,start,counts", [
     ((8, 2, 64), 0, 0, (2, 16, 15, 7, 16)),     # from an empty cache, across and up to page edges
     ((16, 2, 256), 0, 1021, (6, 16, 3, 16)),    # several query tiles, whose last one stores; rows in two splits' pages
