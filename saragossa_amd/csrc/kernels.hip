@@ -389,6 +389,11 @@ __global__ __launch_bounds__(256) void norm_rope_rows_kernel(NormRopeArgs a) {
 // weights and rotations: one load of each instead of U, the loads through the cache having been as many as
 // five for every one of a row. Input rows not in a cache: 512 rows of 32 x 128 7.2 -> 6.4, of 8 x 128
 // 4.3 -> 3.9, of 16 x 256 8.3 -> 6.9, 2048 rows of 32 x 128 21.7 -> 15.6, 4096 rows of 16 x 256 41.7 -> 28.4.
+// All loads of a lane go out before any is waited for, and the ordered sum's reads alternate between two sets of registers (with
+// loads behind branches on what is there to load, and the next round's squares moved to the current one's registers, a move for
+// every addition): launches in a row, input rows not in a cache, 512 rows of 32 x 128 6.0 -> 5.3 (a copy of as many bytes: 3.9), of
+// 8 x 128 4.3 -> 3.6 (2.5), of 16 x 256 6.5 -> 5.7 (3.9), of 8 x 256 5.2 -> 4.4 (2.9), 6 rows of 16 x 256 3.6 -> 3.1 (2.2), 1024
+// rows of 32 x 128 9.2 -> 8.0 (7.8). Non-temporal loads of the rows: 0.2 slower up to 512 rows.
 // U: 16-byte units a lane holds. HD4: units of the widest head served; EXACT: head_dim is it.
 template <int HD4, int U, bool EXACT, bool ONE_ROW>
 __global__ __launch_bounds__(64) void norm_rope_wave_kernel(NormRopeArgs a) {
@@ -399,17 +404,20 @@ __global__ __launch_bounds__(64) void norm_rope_wave_kernel(NormRopeArgs a) {
     __shared__ f4 raw[PAIRS * (HD4 + 1)], sqs[PAIRS * (HD4 + 1)];
     const int lane = threadIdx.x;
     const int hd4 = EXACT ? HD4 : a.head_dim >> 2;
-    const int pair0 = (int)blockIdx.x * PAIRS;
-    const int here = min(PAIRS, a.n_rows * a.heads - pair0);
+    // ONE_ROW: grid (workgroups of a row, rows)
+    const int row0 = ONE_ROW ? (int)blockIdx.y : (int)blockIdx.x * PAIRS / a.heads;
+    const int pair0 = ONE_ROW ? row0 * a.heads + (int)blockIdx.x * PAIRS : (int)blockIdx.x * PAIRS;
+    const int head0 = pair0 - row0 * a.heads;
+    const int here = ONE_ROW ? PAIRS : min(PAIRS, a.n_rows * a.heads - pair0);
     const long row_elems = (long)a.heads * a.head_dim;
     const int hstride = a.x_head_stride > 0 ? a.x_head_stride : a.head_dim;
     const int half4 = a.rope_dims >> 3, rope4 = a.rope_dims >> 2;
-    const int row0 = pair0 / a.heads, head0 = pair0 - row0 * a.heads;
 
     // unit u of a lane: pair pr (past the end: the last one again, not stored), dims 4*c4 .. +3
     int pr[U], c4[U];
-    bool mine[U];
+    bool mine[U], rotated[U], is_first[U];
     f4 x[U], w[U], ow[U], r0[U], r1[U];
+    int oc4[U]; // the rotation's partner unit
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         if constexpr (EXACT) {
@@ -419,35 +427,29 @@ __global__ __launch_bounds__(64) void norm_rope_wave_kernel(NormRopeArgs a) {
             pr[u] = (int)__umulhi((unsigned)(lane + u * 64), a.hd4_magic);
             c4[u] = lane + u * 64 - pr[u] * hd4;
         }
-        mine[u] = pr[u] < here;
-        pr[u] = min(pr[u], here - 1);
+        mine[u] = ONE_ROW || pr[u] < here; // (ONE_ROW: heads are whole workgroups)
+        if (!ONE_ROW) pr[u] = min(pr[u], here - 1);
         const int at = head0 + pr[u];
         const int r = ONE_ROW ? 0 : a.heads > 1 ? (int)__umulhi((unsigned)at, a.heads_magic) : at;
         const int row = row0 + r, h = at - r * a.heads;
-        x[u] = *reinterpret_cast<const f4 *>(a.x + row * row_elems + (long)h * hstride + c4[u] * 4);
+        const float *head = a.x + row * row_elems + (long)h * hstride;
+        x[u] = *reinterpret_cast<const f4 *>(head + c4[u] * 4);
+        rotated[u] = a.rope && c4[u] < rope4;
+        is_first[u] = c4[u] < half4;
+        oc4[u] = !rotated[u] || a.rope_style == 1 ? c4[u] : is_first[u] ? c4[u] + half4 : c4[u] - half4;
         if (ONE_ROW && u > 0) { // the same dims of another head
             w[u] = w[0], ow[u] = ow[0], r0[u] = r0[0], r1[u] = r1[0];
             continue;
         }
-        const bool rotated = a.rope && c4[u] < rope4;
-        // the rotation's partner unit (halves) and the first of the unit's pairs
-        const int oc4 = c4[u] < half4 ? c4[u] + half4 : c4[u] - half4;
-        w[u] = ow[u] = f4{1.0f, 1.0f, 1.0f, 1.0f};
-        if (a.weight) {
-            w[u] = *reinterpret_cast<const f4 *>(a.weight + c4[u] * 4);
-            if (rotated) ow[u] = *reinterpret_cast<const f4 *>(a.weight + oc4 * 4);
-        }
-        r0[u] = r1[u] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-        if (rotated) {
-            const float *rt = a.rope + (long)row * a.rope_dims;
-            if (a.rope_style == 1) {
-                r0[u] = *reinterpret_cast<const f4 *>(rt + c4[u] * 4);
-            } else {
-                const int b = min(c4[u], oc4);
-                r0[u] = *reinterpret_cast<const f4 *>(rt + b * 8);
-                r1[u] = *reinterpret_cast<const f4 *>(rt + b * 8 + 4);
-            }
-        }
+        // Every load is unconditional, from the head itself where there is nothing to load: behind a branch the compiler waits for
+        // all that is in flight, and the loads were four trips to memory instead of one.
+        const float *wp = a.weight ? a.weight : head;
+        const float *rp = a.rope && rope4 > 0 ? a.rope + (long)row * a.rope_dims : head;
+        const int off = !rotated[u] ? 0 : a.rope_style == 1 ? c4[u] * 4 : min(c4[u], oc4[u]) * 8;
+        w[u] = *reinterpret_cast<const f4 *>(wp + c4[u] * 4);
+        ow[u] = *reinterpret_cast<const f4 *>(wp + oc4[u] * 4);
+        r0[u] = *reinterpret_cast<const f4 *>(rp + off);
+        r1[u] = *reinterpret_cast<const f4 *>(rp + (a.rope_style == 1 ? off : off + 4));
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
@@ -456,8 +458,13 @@ __global__ __launch_bounds__(64) void norm_rope_wave_kernel(NormRopeArgs a) {
             sqs[pr[u] * (HD4 + 1) + c4[u]] = x[u] * x[u];
         }
     __syncthreads();
+    f4 other[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) other[u] = raw[pr[u] * (HD4 + 1) + oc4[u]];
     float inv = 1.0f;
-    if (a.weight && lane < here) {
+    if (EXACT) {
+        if (a.weight && lane < here) inv = head_inv_rms_sq<HD4 * 4, false>(reinterpret_cast<const float *>(sqs + lane * (HD4 + 1)), HD4 * 4, a.eps);
+    } else if (a.weight && lane < here) {
         const f4 *row = sqs + lane * (HD4 + 1);
         constexpr int R = 8; // units per round
         float sum = 0.0f;
@@ -488,14 +495,14 @@ __global__ __launch_bounds__(64) void norm_rope_wave_kernel(NormRopeArgs a) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const float iv = __shfl(inv, pr[u], 64);
-        f4 n;
-        if (a.rope && c4[u] < rope4) {
-            const bool is_first = c4[u] < half4;
-            const int oc4 = a.rope_style == 1 ? c4[u] : is_first ? c4[u] + half4 : c4[u] - half4;
-            n = norm_rope_unit(x[u], raw[pr[u] * (HD4 + 1) + oc4], w[u], ow[u], r0[u], r1[u], iv, a.rope_style, is_first);
-        } else {
-            n = x[u] * iv;
-            n = n * w[u];
+        const f4 one = {1.0f, 1.0f, 1.0f, 1.0f};
+        const f4 wu = a.weight ? w[u] : one;
+        f4 n = x[u] * iv;
+        n = n * wu;
+        if (a.rope) { // uniform
+            const f4 t = norm_rope_unit(x[u], other[u], wu, a.weight ? ow[u] : one, r0[u], r1[u], iv, a.rope_style, is_first[u]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) n[e] = rotated[u] ? t[e] : n[e];
         }
         if (mine[u])
             *reinterpret_cast<f4 *>(a.out + ((long)(pair0 + pr[u]) * hd4 + c4[u]) * 4) = n;
@@ -519,7 +526,7 @@ static void launch_norm_rope_wave_u(const NormRopeArgs &a, hipStream_t s) {
     const dim3 grid((unsigned)((n_pairs + PAIRS - 1) / PAIRS));
     if constexpr (HD4 <= 64)
         if (a.head_dim == HD4 * 4 && a.heads % PAIRS == 0) {
-            hipLaunchKernelGGL((norm_rope_wave_kernel<HD4, U, true, true>), grid, dim3(64), 0, s, a);
+            hipLaunchKernelGGL((norm_rope_wave_kernel<HD4, U, true, true>), dim3((unsigned)(a.heads / PAIRS), (unsigned)a.n_rows), dim3(64), 0, s, a);
             return;
         }
     if (a.head_dim == HD4 * 4) hipLaunchKernelGGL((norm_rope_wave_kernel<HD4, U, true, false>), grid, dim3(64), 0, s, a);

@@ -288,9 +288,9 @@ __device__ __forceinline__ float head_inv_rms(const float *row, int head_dim, fl
 // The same from the squares, already taken (x * x, rounded) and padded with zeros to PADDED entries
 // (32, 64, 96 or a multiple of 128) at a 16-byte aligned address: the adds stay in index order, the
 // 16-byte loads of a round are asked for before the adds of the round before (asked for four at a time and
-// waited for, the LDS's latency was as long again as the adds). The loop stays a loop: unrolled, every
-// load moves to its top and the page registers of the caller spill.
-template <int PADDED>
+// waited for, the LDS's latency was as long again as the adds). LOOP: the loop stays a loop; unrolled, every
+// load moves to its top and the page registers of a decode kernel spill.
+template <int PADDED, bool LOOP = true>
 __device__ __forceinline__ float head_inv_rms_sq(const float *sq, int head_dim, float eps) {
 #pragma clang fp contract(off)
     typedef __attribute__((ext_vector_type(4))) float f4;
@@ -302,7 +302,7 @@ __device__ __forceinline__ float head_inv_rms_sq(const float *sq, int head_dim, 
     f4 x[R], y[R];
 #pragma unroll
     for (int i = 0; i < R; ++i) x[i] = p[i];
-#pragma unroll 1
+#pragma unroll LOOP ? 1 : N
     for (int k = 0; k < N; ++k) {
 #pragma unroll
         for (int i = 0; i < R; ++i) y[i] = p[(2 * k + 1) * R + i];

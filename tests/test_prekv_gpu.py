@@ -105,6 +105,8 @@ def test_rms_norm_rope_rows_is_bit_exact(state, heads, head_dim, rope_dims, thet
     (6, 256, 64, 3, 0, True, 0),      # the same, two heads, partial rotation
     (32, 128, 64, 1027, 0, True, 0),  # the same, four units a lane
     (12, 128, 128, 2731, 0, True, 0), # as many wavefronts, but eight heads would be of two rows
+    (8, 128, 0, 11, 0, True, 0),      # heads of one row, norm only
+    (4, 256, 4, 5, 1, False, 0),      # heads of one row, rotation only, of one unit
     (4, 64, 12, 6, 1, True, 0),       # interleaved, rotated dims of three units
     (4, 64, 12, 6, 0, True, 0),       # halves of one and a half units: the general kernel
     (8, 128, 128, 6, 0, True, 1),     # rows at an odd address: the general kernel
