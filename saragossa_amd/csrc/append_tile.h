@@ -30,16 +30,18 @@ __device__ __forceinline__ void append_tile(const AppendArgs &a, const int bx, c
     typedef __attribute__((ext_vector_type(4))) float f4;
     typedef __attribute__((ext_vector_type(4))) uint32_t w4;
     const Geom g = a.g;
-    const long pos0 = (a.first_pos / 16 + bx) * 16; // position of the page's first row
-    const long slot = slot_of(pos0, g.ring_rows);
-    const int page = a.table ? a.table[slot >> 4] : (int)(slot >> 4);
-    const long row0 = pos0 - a.first_pos; // batch row of the page's first row
-    const int r_lo = row0 < 0 ? (int)-row0 : 0, r_hi = (int)min(16l, a.n_rows - row0); // rows of the page in the batch
+    // The page's place is asked for in front of the rows and looked at behind them, by a vector load, because those come back in
+    // order: a scalar one is waited for together with every other, and the rows would be asked for after it.
+    int logical = a.first_page + bx;
+    if (a.ring_pages > 0 && logical >= a.ring_pages) logical -= a.ring_pages;
+    int at = a.table ? logical : 0;
+    asm("" : "+v"(at)); // (a vector register)
+    const int asked = (a.table ? a.table : reinterpret_cast<const int32_t *>(a.k_src))[at]; // (no table: some valid address)
+    const int row0 = bx * 16 - a.first_row; // batch row of the page's first row
+    const int r_lo = max(-row0, 0), r_hi = min(16, a.n_rows - row0); // rows of the page in the batch
     const int kv_dim = g.kv_heads * g.head_dim;
-    const float *ks = a.k_src + row0 * kv_dim + kvh * g.head_dim;
-    const float *vs = a.v_src + row0 * kv_dim + kvh * g.head_dim;
-    const long tile = (long)page * g.page_elems + (long)kvh * g.tile_elems;
-    w4 *kt = reinterpret_cast<w4 *>(a.k_pool + tile), *vt = reinterpret_cast<w4 *>(a.v_pool + tile);
+    const float *ks = a.k_src + (long)row0 * kv_dim + kvh * g.head_dim;
+    const float *vs = a.v_src + (long)row0 * kv_dim + kvh * g.head_dim;
     const int units = g.tile_elems >> 3;
     // K units past head_dim: a layer's pools are zero there from the start, scratch pages are not
     const int k_units = a.table ? ((g.head_dim + (F32 ? 3 : 7)) / (F32 ? 4 : 8)) * 16 : units;
@@ -58,10 +60,10 @@ __device__ __forceinline__ void append_tile(const AppendArgs &a, const int bx, c
         vr[i] = ((u >> 4) & 3) * 4;
         vd[i] = (u >> 6) * 16 * VD + (u & 15);
         const int row = min(max(kr[i], r_lo), r_hi - 1); // clamped: loads are unconditional, one round trip
-        if (a.vec && kd[i] + KE <= g.head_dim) {
+        if (a.vec) { // uniform
 #pragma unroll
             for (int e = 0; e < KE; e += 4) {
-                const f4 x = *reinterpret_cast<const f4 *>(ks + (long)row * kv_dim + kd[i] + e);
+                const f4 x = *reinterpret_cast<const f4 *>(ks + (long)row * kv_dim + min(kd[i] + e, g.head_dim - 4));
 #pragma unroll
                 for (int t = 0; t < 4; ++t) kx[i][e + t] = x[t];
             }
@@ -76,6 +78,9 @@ __device__ __forceinline__ void append_tile(const AppendArgs &a, const int bx, c
             for (int d = 0; d < VD; ++d) vx[i][r][d] = vs[(long)vrow * kv_dim + min(vd[i] + 16 * d, g.head_dim - 1)];
         }
     }
+    const int page = __builtin_amdgcn_readfirstlane(a.table ? asked : logical);
+    const long tile = (long)page * g.page_elems + (long)kvh * g.tile_elems;
+    w4 *kt = reinterpret_cast<w4 *>(a.k_pool + tile), *vt = reinterpret_cast<w4 *>(a.v_pool + tile);
 #pragma unroll
     for (int i = 0; i < UNITS; ++i) {
         const int u = (int)threadIdx.x + (bz * UNITS + i) * threads;
@@ -143,8 +148,14 @@ inline AppendGrid append_grid(const AppendArgs &a) {
     r.spread = r.pages * a.g.kv_heads * r.rounds <= 4096;
     return r;
 }
-inline int append_vec(const AppendArgs &a) { // 16-byte loads of K
-    return ((uintptr_t)a.k_src & 15) == 0 && (a.g.head_dim & 3) == 0;
+// What the launch wants to know of a: 16-byte loads of K, and the places of its pages
+inline AppendArgs append_placed(const AppendArgs &a) {
+    AppendArgs b = a;
+    b.vec = ((uintptr_t)a.k_src & 15) == 0 && (a.g.head_dim & 3) == 0;
+    b.first_page = (int)(slot_of(a.first_pos / 16 * 16, a.g.ring_rows) / 16);
+    b.first_row = (int)(a.first_pos % 16);
+    b.ring_pages = a.g.ring_rows / 16;
+    return b;
 }
 
 } // namespace skv

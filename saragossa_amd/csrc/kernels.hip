@@ -23,8 +23,7 @@ __global__ __launch_bounds__(256) void append_kernel(AppendArgs a) {
 
 hipError_t launch_append(const AppendArgs &a, hipStream_t s) {
     if (a.n_rows <= 0) return hipSuccess;
-    AppendArgs b = a;
-    b.vec = append_vec(a);
+    const AppendArgs b = append_placed(a);
     const AppendGrid r = append_grid(a);
     const int units = a.g.tile_elems >> 3, per = r.spread ? 1 : r.rounds;
     const dim3 grid((unsigned)r.pages, (unsigned)a.g.kv_heads, (unsigned)(r.spread ? r.rounds : 1));

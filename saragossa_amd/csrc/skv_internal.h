@@ -95,7 +95,10 @@ struct AppendArgs {
     const int32_t *table; // null = page i of the pools is page i of the positions
     long first_pos; // position of the first appended row
     int n_rows;
-    int vec;        // K rows may be read 16 bytes at a time (set by the launcher)
+    int vec;        // K rows may be read 16 bytes at a time (set by the launcher, like what follows)
+    int first_page; // logical page of the first row, of a ring the one it has come round to
+    int first_row;  // of that page
+    int ring_pages; // 0 = not a ring
     Geom g;
 };
 
