@@ -92,13 +92,13 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
     const int rows = min(16, n_slots - tile * 16); // query slots of this workgroup
     // this lane's query slot in the B and D operand layouts
     const int my_slot = min(tile * 16 + n, n_slots - 1);
-    const int my_q = MQ ? my_slot / G : 0;
+    const int my_q = MQ ? slot_row(g, my_slot) : 0;
     const int my_pos = a.q_pos0 + my_q;                 // position of the slot's query row
     const int my_limit = min(my_pos, a.limit_cap);      // last position the slot attends
     const int my_ws = a.window > 0 ? max(a.window_start, my_pos + 1 - a.window) : a.window_start;
     // extremes over the workgroup's slots
-    const int qrow_lo = MQ ? (tile * 16) / G : 0;
-    const int qrow_hi = MQ ? (tile * 16 + rows - 1) / G : 0;
+    const int qrow_lo = MQ ? slot_row(g, tile * 16) : 0;
+    const int qrow_hi = MQ ? slot_row(g, tile * 16 + rows - 1) : 0;
     const int lim_lo = min(a.q_pos0 + qrow_lo, a.limit_cap);
     const int lim_hi = min(a.q_pos0 + qrow_hi, a.limit_cap);
     const int ws_lo = a.window > 0 ? max(a.window_start, a.q_pos0 + qrow_lo + 1 - a.window) : a.window_start;
@@ -209,7 +209,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
         const int kk = idx >> 6;
         const int jj = (idx >> 4) & 3;
         const int qs = min(tile * 16 + (idx & 15), n_slots - 1);
-        const float *qrow = MQ ? a.q + ((long)(qs / G) * g.q_heads + kvh * G + qs % G) * g.head_dim
+        const float *qrow = MQ ? a.q + context_row(g, kvh, qs) * g.head_dim
                                : a.q + (long)(kvh * G + qs) * q_stride;
         if (a.q_vec) { // two 16-byte loads from a clamped address (dims past head_dim are zeroed below)
             const float4_t *qp = reinterpret_cast<const float4_t *>(qrow + min(kk * 32 + jj * 8, g.head_dim - 8));
@@ -602,7 +602,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
                 for (int i = 0; i < 4; ++i)
                     if (c4 + i < g.head_dim) acc[i] *= sigmoid_gate(gp[i]);
             }
-            dst = a.out + (MQ ? ((long)(slot / G) * g.q_heads + kvh * G + slot % G)
+            dst = a.out + (MQ ? context_row(g, kvh, slot)
                               : (long)(kvh * G + slot)) * g.head_dim + c4;
         } else {
             const long pidx = ((long)kvh * a.splits_total + a.split_base + split) * n_slots + slot;

@@ -89,7 +89,7 @@ __global__ __launch_bounds__(256) void f32_split_kernel(DecodeArgs a) {
     const int s_last = min(slot0 + 15, n_slots - 1);
     const int my_slot = min(slot0 + n, n_slots - 1);
 
-    auto pos_of = [&](int slot) { return a.q_pos0 + slot / G; };
+    auto pos_of = [&](int slot) { return a.q_pos0 + slot_row(a.g, slot); };
     auto limit_of = [&](int slot) { return min(pos_of(slot), a.limit_cap); };
     auto ws_of = [&](int slot) { return a.window > 0 ? max(a.window_start, pos_of(slot) + 1 - a.window) : a.window_start; };
     const int my_limit = limit_of(my_slot), my_ws = ws_of(my_slot);
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(256) void f32_split_kernel(DecodeArgs a) {
     // queries: lane (slot n, group j) holds dims 16m + 4j .. +3 of every block m
     float4_t qv[NT];
     {
-        const float *qrow = a.q + ((long)(my_slot / G) * g.q_heads + kvh * G + my_slot % G) * g.head_dim;
+        const float *qrow = a.q + context_row(g, kvh, my_slot) * g.head_dim;
         // all loads first, unconditional from clamped addresses (one round trip); dims past
         // head_dim are zeroed afterwards
         if (a.q_vec) {
@@ -402,7 +402,7 @@ __global__ __launch_bounds__(256) void f32_split_kernel(DecodeArgs a) {
     float scale = 1.0f;
     if (a.splits_total == 1) {
         scale = 1.0f / l;
-        dst = a.out + ((long)(slot / G) * g.q_heads + kvh * G + slot % G) * g.head_dim;
+        dst = a.out + context_row(g, kvh, slot) * g.head_dim;
     } else {
         const long pidx = ((long)kvh * a.splits_total + a.split_base + split) * n_slots + slot;
         dst = a.part_o + pidx * g.head_dim;

@@ -210,7 +210,7 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
     const int wg_slot0 = blockIdx.z * (TW * TILES * 16);
     const int wg_slot1 = min(n_slots, wg_slot0 + TW * TILES * 16) - 1;
 
-    auto limit_of = [&](int slot) { return a.q_pos0 + slot / G; };
+    auto limit_of = [&](int slot) { return a.q_pos0 + slot_row(a.g, slot); };
     auto ws_of = [&](int slot) { return a.window > 0 ? max(a.window_start, limit_of(slot) + 1 - a.window) : a.window_start; };
     const int wg_ws_lo = ws_of(wg_slot0);
     const int wg_lim_hi = limit_of(wg_slot1);
@@ -369,7 +369,7 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
         my_ws[t] = ws_of(my_slot);
         t_lim_lo[t] = limit_of(min(s0, n_slots - 1));
         t_ws_hi[t] = ws_of(s_last);
-        const float *qrow = a.q + ((long)(my_slot / G) * g.q_heads + kvh * G + my_slot % G) * g.head_dim;
+        const float *qrow = a.q + context_row(g, kvh, my_slot) * g.head_dim;
         if (a.q_vec) {
 #pragma unroll
             for (int kk = 0; kk < QK; ++kk) {
@@ -793,12 +793,11 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
         static_assert(sizeof(DecodeArgs) % alignof(ChunkPages) == 0 && (sizeof(DecodeArgs) + sizeof(ChunkPages)) % alignof(TermPairs) == 0,
                       "the launch's memory holds the three side by side");
         const Geom &g = a.g;
-        const int G = g.gqa;
-        auto limit_of = [&](int slot) { return a.q_pos0 + slot / G; };
+        auto limit_of = [&](int slot) { return a.q_pos0 + slot_row(a.g, slot); };
         auto ws_of = [&](int slot) { return a.window > 0 ? max(a.window_start, limit_of(slot) + 1 - a.window) : a.window_start; };
         constexpr int VT = NT < 8 ? NT : 8, KT = NT % 4 == 0 ? 4 : NT % 3 == 0 ? 3 : NT;
         static_assert(NT % VT == 0 && NT % KT == 0, "whole steps");
-        const float *qrow = a.q + ((long)(slot / G) * g.q_heads + kvh * G + slot % G) * g.head_dim;
+        const float *qrow = a.q + context_row(g, kvh, slot) * g.head_dim;
         const int lo0 = ws_of(slot), hi0 = limit_of(slot);
 #pragma unroll 1
         for (int v0 = 0; v0 < NT; v0 += VT) {
@@ -892,7 +891,7 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
         const bool whole = a.splits_total == 1;
         auto partial_of = [&](int slot) { return ((long)kvh * a.splits_total + a.split_base + split) * n_slots + slot; };
         auto dst_of = [&](int slot) {
-            return whole ? a.out + ((long)(slot / G) * g.q_heads + kvh * G + slot % G) * g.head_dim
+            return whole ? a.out + context_row(g, kvh, slot) * g.head_dim
                          : a.part_o + partial_of(slot) * g.head_dim;
         };
         // slots whose sums are not all numbers (columns past head_dim are none of theirs)

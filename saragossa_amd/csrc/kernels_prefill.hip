@@ -123,7 +123,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
     const int wg_slot1 = min(n_slots, wg_slot0 + TW * TILES * 16) - 1; // last slot of the workgroup
 
     // query slot -> position of its row (the last it attends), first position it attends
-    auto limit_of = [&](int slot) { return a.q_pos0 + slot / G; };
+    auto limit_of = [&](int slot) { return a.q_pos0 + slot_row(a.g, slot); };
     auto ws_of = [&](int slot) { return a.window > 0 ? max(a.window_start, limit_of(slot) + 1 - a.window) : a.window_start; };
 
     // entries of the page list any slot of the workgroup can see, divided among the splits
@@ -233,7 +233,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
         my_ws[t] = ws_of(my_slot);
         t_lim_lo[t] = limit_of(min(s0, n_slots - 1));
         t_ws_hi[t] = ws_of(s_last);
-        const float *qrow = a.q + ((long)(my_slot / G) * g.q_heads + kvh * G + my_slot % G) * g.head_dim;
+        const float *qrow = a.q + context_row(g, kvh, my_slot) * g.head_dim;
         // eight consecutive dims of the slot's row per k-step: all loads first (two 16-byte
         // loads per step when the row allows), unconditional from clamped addresses, so that
         // they are one round trip; dims past head_dim are zeroed afterwards
@@ -594,37 +594,49 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
         if (step + 1 < n_steps) clear_v((step + 1) * SP * GP, kv_lds + ((step + 1) & 1) * BUF_U4 + HALF_U4);
     }
 
-    // ---- the other parts' states join the first's through LDS -------------------------------
+    // ---- the parts join their states through LDS, each the columns that it then stores: part p the tiles u of 16 dims with
+    // owner(u) == p. (With all states joined and stored by the first part's wavefronts, FILL)
+    const auto owner = [](int u) { return HALVES == 2 ? 0 : u * HALVES / NT; };
     if constexpr (HALVES > 1) {
-        constexpr int STATES = TW * TILES * (NT + 1) * 64; // of a part
-        static_assert((HALVES - 1) * STATES <= 2 * BUF_U4, "the other parts' states fit the page buffers");
-        float4_t *xo = reinterpret_cast<float4_t *>(kv_lds) + (tw * TILES) * (NT + 1) * 64 + lane; // (the loop ends in a barrier)
-        if (half > 0) {
-#pragma unroll
-            for (int t = 0; t < TILES; ++t) {
-                float4_t *dst = xo + (half - 1) * STATES + t * (NT + 1) * 64;
-#pragma unroll
-                for (int u = 0; u < NT; ++u) dst[u * 64] = o[t][u];
-                dst[NT * 64] = float4_t{thr_i[t] < 0 ? -INFINITY : m_base[t], l_run[t], 0.f, 0.f};
-            }
-        }
-        __syncthreads();
-        if (half > 0) return;
+        constexpr int SETS = NT * (HALVES - 1) + HALVES; // of a tile: every u from the parts that do not own it; (m, l) of all
+        static_assert(TW * TILES * SETS * 64 <= 2 * BUF_U4, "the states fit the page buffers");
+        float4_t *xo = reinterpret_cast<float4_t *>(kv_lds) + (tw * TILES) * SETS * 64 + lane; // (the loop ends in a barrier)
+        const auto at = [&](int t, int u, int part) { return (t * SETS + u * (HALVES - 1) + (part < owner(u) ? part : part - 1)) * 64; };
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
-#pragma unroll 1
-            for (int h = 0; h < HALVES - 1; ++h) {
-                const float4_t *src = xo + h * STATES + t * (NT + 1) * 64;
-                const float4_t ml = src[NT * 64];
-                const float m0 = thr_i[t] < 0 ? -INFINITY : m_base[t], m1 = ml[0];
-                const float mx = fmaxf(m0, m1);
-                const float m_safe = mx == -INFINITY ? 0.0f : mx;
-                const float w0 = fast_exp2(m0 - m_safe), w1 = fast_exp2(m1 - m_safe);
-                l_run[t] = l_run[t] * w0 + ml[1] * w1;
 #pragma unroll
-                for (int u = 0; u < NT; ++u) o[t][u] = o[t][u] * w0 + src[u * 64] * w1;
-                m_base[t] = m_safe;
-                thr_i[t] = mx == -INFINITY ? UNSEEN : SEEN;
+            for (int u = 0; u < NT; ++u)
+                if (owner(u) != half) xo[at(t, u, half)] = o[t][u];
+            xo[(t * SETS + NT * (HALVES - 1) + half) * 64] = float4_t{thr_i[t] < 0 ? -INFINITY : m_base[t], l_run[t], 0.f, 0.f};
+        }
+        __syncthreads();
+        if (HALVES == 2 && half > 0) return;
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            float w[HALVES], l[HALVES], mx = -INFINITY;
+#pragma unroll
+            for (int h = 0; h < HALVES; ++h) {
+                const float4_t ml = xo[(t * SETS + NT * (HALVES - 1) + h) * 64];
+                w[h] = ml[0];
+                l[h] = ml[1];
+                mx = fmaxf(mx, w[h]);
+            }
+            const float m_safe = mx == -INFINITY ? 0.0f : mx;
+            l_run[t] = 0.0f;
+#pragma unroll
+            for (int h = 0; h < HALVES; ++h) {
+                w[h] = fast_exp2(w[h] - m_safe);
+                l_run[t] += l[h] * w[h];
+            }
+            m_base[t] = m_safe;
+            thr_i[t] = mx == -INFINITY ? UNSEEN : SEEN;
+#pragma unroll
+            for (int u = 0; u < NT; ++u) {
+                if (owner(u) != half) continue; // uniform
+                float4_t sum = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int h = 0; h < HALVES; ++h) sum += (h == owner(u) ? o[t][u] : xo[at(t, u, h)]) * w[h];
+                o[t][u] = sum;
             }
         }
     }
@@ -639,11 +651,11 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
         float scale = 1.0f;
         if (a.splits_total == 1) {
             scale = 1.0f / l;
-            dst = a.out + ((long)(slot / G) * g.q_heads + kvh * G + slot % G) * g.head_dim;
+            dst = a.out + context_row(g, kvh, slot) * g.head_dim;
         } else {
             const long pidx = ((long)kvh * a.splits_total + a.split_base + split) * n_slots + slot;
             dst = a.part_o + pidx * g.head_dim;
-            if (j == 0) {
+            if (j == 0 && half == 0) {
                 a.part_m[pidx] = thr_i[t] < 0 ? -INFINITY : m_base[t];
                 a.part_l[pidx] = l;
             }
@@ -651,6 +663,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_tile_kernel(DecodeArgs a, 
         const bool vec_ok = (g.head_dim & 3) == 0;
 #pragma unroll
         for (int u = 0; u < NT; ++u) {
+            if (owner(u) != half) continue; // uniform
             const int col = u * 16 + j * 4;
             const float4_t v = o[t][u] * scale;
             if (vec_ok) {
@@ -718,7 +731,7 @@ __device__ __forceinline__ void merge_rows_of(const DecodeArgs &a, const int kvh
             for (int i = 0; i < 4; ++i) acc[i] += wu * v[u][i];
         }
     }
-    float *dst = a.out + ((long)(slot / g.gqa) * g.q_heads + kvh * g.gqa + slot % g.gqa) * g.head_dim + c4;
+    float *dst = a.out + context_row(g, kvh, slot) * g.head_dim + c4;
     const float inv = 1.0f / lsum;
     if (vec_ok) {
         *reinterpret_cast<float4_t *>(dst) = float4_t{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};

@@ -947,7 +947,7 @@ static int32_t plan_layer(size_t capacity, size_t q_heads, size_t kv_heads, size
     g.kv_heads = (int)kv_heads;
     g.head_dim = (int)head_dim;
     g.P = P;
-    g.gqa = (int)(q_heads / kv_heads);
+    set_gqa(g);
     g.f32 = f32 ? 1 : 0;
     g.tile_elems = P * 16 * (f32 ? 2 : 1);
     g.page_elems = (int)kv_heads * g.tile_elems;

@@ -62,7 +62,27 @@ struct Geom {
     int page_elems; // kv_heads * tile_elems
     int ring_rows;  // 0 = full cache; else rows kept by the ring (multiple of 16)
     int f32;        // 1 = the tiles hold f32 (kernels_f32.hip), 0 = bf16
+    // slot / gqa as a product: floor(2^(31 + s) / gqa) + 1, s the bits of gqa - 1 (set_gqa)
+    uint32_t gqa_mul;
+    int gqa_shift;
 };
+inline void set_gqa(Geom &g) {
+    g.gqa = g.q_heads / g.kv_heads;
+    g.gqa_shift = 0;
+    while ((1l << g.gqa_shift) < g.gqa) ++g.gqa_shift;
+    g.gqa_mul = (uint32_t)((1ull << (31 + g.gqa_shift)) / (uint64_t)g.gqa + 1);
+}
+// Query row of a slot, slot / gqa. Exact below 2^31: the product is too large by at most slot * gqa, less than 2^(31 + s). (A division
+// is some thirty instructions, and a chunk's kernel wants five before its first load.)
+__host__ __device__ inline int slot_row(const Geom &g, int slot) {
+    return (int)((uint32_t)(((uint64_t)((uint32_t)slot * 2) * g.gqa_mul) >> 32) >> g.gqa_shift);
+}
+
+// (row, head) of a slot of kv head kvh, counted in heads: where its query and its context lie
+__host__ __device__ inline long context_row(const Geom &g, int kvh, int slot) {
+    const int row = slot_row(g, slot);
+    return (long)row * g.q_heads + kvh * g.gqa + (slot - row * g.gqa);
+}
 
 __host__ __device__ inline int k_index(int P, int r, int d) {
     (void)P;
