@@ -17,6 +17,14 @@ __device__ __forceinline__ uint16_t bf16_bits(float v) {
 __device__ __forceinline__ float bf16_to_f32(uint16_t b) {
     return __uint_as_float(((uint32_t)b) << 16);
 }
+// x and y as two bf16 terms each, hi + lo to 2^-18, x in the low halves; the conversion instruction takes two values (nearest even, as
+// bf16_bits, which is ten instructions for the same pair). For factors of products; stored rows keep bf16_bits, NaN bits included.
+__device__ __forceinline__ void bf16_terms(float x, float y, uint32_t &hi, uint32_t &lo) {
+    typedef __attribute__((ext_vector_type(2))) float f2;
+    typedef __attribute__((ext_vector_type(2))) __bf16 b2;
+    hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{x, y}, b2));
+    lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{x - __uint_as_float(hi << 16), y - __uint_as_float(hi & 0xffff0000u)}, b2));
+}
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 constexpr int DEC_MAX_SPLITS = 512;
@@ -261,14 +269,9 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
         Pre::each(pre_lds, a, rows, n_rows, tid, [&](int r, int c4, float4_t v) __attribute__((always_inline)) {
 #pragma clang fp contract(off)
             if (r < rows) {
-                uint32_t hi[2] = {0, 0}, lo[2] = {0, 0};
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float x = v[i] * a.qscale;
-                    const uint16_t hb = bf16_bits(x);
-                    hi[i >> 1] |= (uint32_t)hb << (16 * (i & 1));
-                    lo[i >> 1] |= (uint32_t)bf16_bits(x - bf16_to_f32(hb)) << (16 * (i & 1));
-                }
+                uint32_t hi[2], lo[2];
+                bf16_terms(v[0] * a.qscale, v[1] * a.qscale, hi[0], lo[0]);
+                bf16_terms(v[2] * a.qscale, v[3] * a.qscale, hi[1], lo[1]);
                 const int at = ((c4 >> 1) * 16 + r) * 2 + (c4 & 1); // 8-byte units: [P/8][16 slots][2]
                 reinterpret_cast<uint2 *>(q_hi)[at] = make_uint2(hi[0], hi[1]);
                 reinterpret_cast<uint2 *>(q_lo)[at] = make_uint2(lo[0], lo[1]);
@@ -337,18 +340,10 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
             uint32_t hi[4], lo[4];
 #pragma unroll
             for (int e2 = 0; e2 < 4; ++e2) {
-                uint32_t h2 = 0, l2 = 0;
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int d = kk * 32 + jj * 8 + e2 * 2 + h;
-                    const float v = (row_ok && d < g.head_dim) ? qv[u][e2 * 2 + h] * a.qscale : 0.0f;
-                    const uint16_t hb = bf16_bits(v);
-                    const uint16_t lb = bf16_bits(v - bf16_to_f32(hb));
-                    h2 |= (uint32_t)hb << (16 * h);
-                    l2 |= (uint32_t)lb << (16 * h);
-                }
-                hi[e2] = h2;
-                lo[e2] = l2;
+                const int d = kk * 32 + jj * 8 + e2 * 2;
+                const float x = row_ok && d < g.head_dim ? qv[u][e2 * 2] * a.qscale : 0.0f;
+                const float y = row_ok && d + 1 < g.head_dim ? qv[u][e2 * 2 + 1] * a.qscale : 0.0f;
+                bf16_terms(x, y, hi[e2], lo[e2]);
             }
             q_hi[idx] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
             q_lo[idx] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
@@ -400,15 +395,18 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
         const float m_safe = m_new == -INFINITY ? 0.0f : m_new;
         const float alpha = fast_exp2(m_run - m_safe);
         float psum = 0.0f;
+        float p[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const float p = fast_exp2(s[i] - m_safe);
-            psum += p;
-            const uint16_t hb = bf16_bits(p);
-            const uint16_t lb = bf16_bits(p - bf16_to_f32(hb));
-            ph[i] = (short)hb;
-            pl[i] = (short)lb;
+            p[i] = fast_exp2(s[i] - m_safe);
+            psum += p[i];
         }
+        uint32_t hi[2], lo[2];
+        bf16_terms(p[0], p[1], hi[0], lo[0]);
+        bf16_terms(p[2], p[3], hi[1], lo[1]);
+        typedef __attribute__((ext_vector_type(2))) uint32_t u2;
+        ph = __builtin_bit_cast(short4_t, u2{hi[0], hi[1]});
+        pl = __builtin_bit_cast(short4_t, u2{lo[0], lo[1]});
         l_run = l_run * alpha + psum;
         // A slot that has seen no key yet holds zeros: no rescale for it (the first page of
         // every wavefront would otherwise walk all its accumulator registers for nothing, which
