@@ -9,16 +9,22 @@ namespace skv {
 // units from its pool's start), which position its first row has, and the first and last
 // position whose rows it may speak for. On full layers entry e is logical page e.
 template <bool RING>
-__device__ __forceinline__ uint32_t entry_tile(const DecodeArgs &a, const ChunkPages &c, int e, int kvh) {
-    int page;
+__device__ __forceinline__ uint32_t entry_place(const DecodeArgs &a, const ChunkPages &c, int e) { // physical page
     if constexpr (RING) {
         int at = c.start + min(e, c.n_old - 1);
         if (at >= c.ring_pages) at -= c.ring_pages;
-        page = e < c.n_old ? a.table[max(at, 0)] : e - c.n_old;
+        const int page = a.table[max(at, 0)];
+        return (uint32_t)(e < c.n_old ? page : e - c.n_old);
     } else {
-        page = a.table[e];
+        return (uint32_t)a.table[e];
     }
-    return (uint32_t)page * (uint32_t)(a.g.page_elems >> 3) + (uint32_t)kvh * (uint32_t)(a.g.tile_elems >> 3);
+}
+__device__ __forceinline__ uint32_t place_tile(const DecodeArgs &a, uint32_t place, int kvh) {
+    return place * (uint32_t)(a.g.page_elems >> 3) + (uint32_t)kvh * (uint32_t)(a.g.tile_elems >> 3);
+}
+template <bool RING>
+__device__ __forceinline__ uint32_t entry_tile(const DecodeArgs &a, const ChunkPages &c, int e, int kvh) {
+    return place_tile(a, entry_place<RING>(a, c, e), kvh);
 }
 template <bool RING>
 __device__ __forceinline__ int entry_pos(const ChunkPages &c, int e) {

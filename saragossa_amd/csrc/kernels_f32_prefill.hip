@@ -52,19 +52,27 @@ __global__ __launch_bounds__(256) void f32_terms_kernel(DecodeArgs a, ChunkPages
     const int hd = a.g.head_dim;
     const long kv_dim = (long)a.g.kv_heads * hd;
     u4 *out = reinterpret_cast<u4 *>(t.terms) + (((size_t)kvh * t.held + blockIdx.x) * 2 + (v ? 1 : 0)) * 3 * PLANE;
+    // (both entries' places are asked for at once)
+    uint32_t place[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) place[h] = entry_place<RING>(a, c, min(2 * pair + h, t.entries - 1));
     const float *tile[2]; // of the pool (an entry of a ring's new rows has none: some tile, not looked at)
     int lo[2], hi[2], pos[2];
     bool own[2]; // every row is the caller's
-    bool fresh = false; // some of the pair's rows are
+    // rows of the entry that are the caller's: none, some, all. The first and the last, nearly every page of a chunk, have paths of their
+    // own: a test per row made V's loads and stores of 4 bytes each behind a branch (512 rows of q32/kv8/hd128 over 512, this launch
+    // 9.5 us -> 8.9; whole chunks over none, 512 29.9 -> 29.3, 50.4 -> 49.6, of q12/kv4/hd96 over 1003 40.1 -> 38.5).
+    enum { NONE, SOME, ALL };
+    int fresh[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const int e = min(2 * pair + h, t.entries - 1); // (past the end: the last page again, all of it left out of V)
         own[h] = RING && e >= c.n_old;
-        tile[h] = reinterpret_cast<const float *>(v ? a.v_pool : a.k_pool) + (own[h] ? 0 : (size_t)entry_tile<RING>(a, c, e, kvh) * 4);
+        tile[h] = reinterpret_cast<const float *>(v ? a.v_pool : a.k_pool) + (own[h] ? 0 : (size_t)place_tile(a, place[h], kvh) * 4);
         pos[h] = entry_pos<RING>(c, e);
         lo[h] = max(t.pos_lo, entry_lo<RING>(c, e));
         hi[h] = 2 * pair + h < t.entries ? min(t.pos_hi, entry_hi<RING>(c, e)) : -1;
-        fresh = fresh || own[h] || (!RING && pos[h] + 15 >= t.new_pos);
+        fresh[h] = own[h] || (!RING && pos[h] >= t.new_pos && pos[h] + 15 <= t.pos_hi) ? ALL : !RING && pos[h] + 15 >= t.new_pos ? SOME : NONE;
     }
     // the caller's row at a position (of an entry that is all the caller's, the nearest one there is)
     const float *rows = (v ? t.v_src : t.k_src) + (long)kvh * hd;
@@ -78,8 +86,11 @@ __global__ __launch_bounds__(256) void f32_terms_kernel(DecodeArgs a, ChunkPages
             const int d = min((i >> 6) * 16 + (i & 15), hd - 1), key = ((i >> 4) & 3) * 4;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                if (!fresh) { // uniform
+                if (fresh[h] == NONE) { // uniform
                     x[h] = *reinterpret_cast<const float4_t *>(tile[h] + i * 4);
+                } else if (fresh[h] == ALL) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) x[h][r] = row_at(pos[h] + key + r)[d];
                 } else {
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
@@ -90,14 +101,18 @@ __global__ __launch_bounds__(256) void f32_terms_kernel(DecodeArgs a, ChunkPages
             }
         } else {
             // dims d0 .. d0 + 7 of a row: two units of its tile, 16 apart
-            const int pg = i / (PLANE / 2), du = i - pg * (PLANE / 2), d0 = (du >> 4) * 8;
+            static_assert(PLANE / 2 % 64 == 0, "a wavefront's units are of one page");
+            const int pg = __builtin_amdgcn_readfirstlane(i / (PLANE / 2)), du = i - pg * (PLANE / 2), d0 = (du >> 4) * 8;
             const float *k = (pg ? tile[1] : tile[0]) + ((du >> 5) * 64 + ((du >> 4) & 1) * 32 + (du & 15)) * 4;
             const int p = (pg ? pos[1] : pos[0]) + (du & 15);
-            const bool nw = fresh && is_new(pg, p);
-            if (!fresh || t.vec) { // uniform
-                const float *row = nw ? row_at(p) : nullptr;
-                x[0] = *reinterpret_cast<const float4_t *>(nw ? row + min(d0, hd - 4) : k);
-                x[1] = *reinterpret_cast<const float4_t *>(nw ? row + min(d0 + 4, hd - 4) : k + 64);
+            const int kind = pg ? fresh[1] : fresh[0];
+            const bool nw = kind == ALL || (kind == SOME && is_new(pg, p));
+            if (kind == NONE) { // uniform
+                x[0] = *reinterpret_cast<const float4_t *>(k);
+                x[1] = *reinterpret_cast<const float4_t *>(k + 64);
+            } else if (kind == ALL && t.vec) {
+                x[0] = *reinterpret_cast<const float4_t *>(row_at(p) + min(d0, hd - 4));
+                x[1] = *reinterpret_cast<const float4_t *>(row_at(p) + min(d0 + 4, hd - 4));
             } else {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) x[e >> 2][e & 3] = *(nw ? row_at(p) + min(d0 + e, hd - 1) : k + (e >> 2) * 64 + (e & 3));
@@ -120,12 +135,15 @@ __global__ __launch_bounds__(256) void f32_terms_kernel(DecodeArgs a, ChunkPages
             const int d = (i >> 6) * 16 + (i & 15), key = ((i >> 4) & 3) * 4;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                if (fresh) {
+                if (fresh[h] == ALL) {
+                    if (d >= hd) x[h] = float4_t{0.f, 0.f, 0.f, 0.f};
+                    // (an entry past the end stands for the last page, which its other half stores)
+                    else if (!RING && hi[h] >= 0) *reinterpret_cast<float4_t *>(const_cast<float *>(tile[h]) + i * 4) = x[h];
+                } else if (fresh[h] == SOME) {
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const bool nw = is_new(h, pos[h] + key + r);
                         if (nw) x[h][r] = d < hd ? x[h][r] : 0.0f;
-                        // (an entry past the end stands for the last page, which its other half stores)
                         if (!RING && nw && d < hd && hi[h] >= 0) const_cast<float *>(tile[h])[i * 4 + r] = x[h][r];
                     }
                 }
