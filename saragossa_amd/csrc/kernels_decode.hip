@@ -92,11 +92,11 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15; // key row inside the tile (A operand) / query slot (B, D)
     const int j = lane >> 4;
-    const int tile = MQ ? tile_z : 0;
     const int q_stride = (!MQ && a.q_head_stride > 0) ? a.q_head_stride : g.head_dim;
     const int G = g.gqa;
     const int C = MQ ? a.n_queries : 1;
     const int n_slots = C * G;
+    const int tile = MQ ? longest_first(n_slots, 16, tile_z) : 0;
     const int rows = min(16, n_slots - tile * 16); // query slots of this workgroup
     // this lane's query slot in the B and D operand layouts
     const int my_slot = min(tile * 16 + n, n_slots - 1);

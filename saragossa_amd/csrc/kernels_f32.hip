@@ -85,7 +85,7 @@ __global__ __launch_bounds__(256) void f32_split_kernel(DecodeArgs a) {
     const int kvh = blockIdx.y;
     const int G = g.gqa;
     const int n_slots = a.n_queries * G;
-    const int slot0 = blockIdx.z * 16;
+    const int slot0 = longest_first(n_slots, 16, blockIdx.z) * 16;
     const int s_last = min(slot0 + 15, n_slots - 1);
     const int my_slot = min(slot0 + n, n_slots - 1);
 

@@ -225,7 +225,7 @@ __global__ __launch_bounds__(WAVES * 64) void f32_prefill_kernel(DecodeArgs a, C
     constexpr int TW = WAVES / HALVES;
     const int half = HALVES > 1 ? wave / TW : 0;
     const int tw = HALVES > 1 ? wave % TW : wave;
-    const int wg_slot0 = blockIdx.z * (TW * TILES * 16);
+    const int wg_slot0 = longest_first(n_slots, TW * TILES * 16, blockIdx.z) * (TW * TILES * 16);
     const int wg_slot1 = min(n_slots, wg_slot0 + TW * TILES * 16) - 1;
 
     auto limit_of = [&](int slot) { return a.q_pos0 + slot_row(a.g, slot); };
