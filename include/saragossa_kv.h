@@ -90,7 +90,8 @@ int32_t skv_flag_sdpa_2pass_enabled(void);        /* RETI_RUST_SDPA_2PASS, utils
 size_t skv_flag_sdpa_2pass_min_len(void);         /* RETI_RUST_SDPA_2PASS_MIN_LEN, utils.rs:270-278 */
 size_t skv_sdpa_2pass_blocks(size_t len);         /* utils.rs:282-286 */
 /* Rows from which this library splits the context of a decode launch: RETI_RUST_SDPA_2PASS_MIN_LEN
- * when it is set (the reference's parse, default 2048 when unparsable), else 128. The reference's
+ * when it is set (the reference's parse, default 2048 when unparsable), else 128 (while it is not set, decode
+ * steps and short chunks stay whole over some pages more where that is faster). The reference's
  * own default (2048, utils.rs:270-278) is what skv_flag_sdpa_2pass_min_len reports; it was tuned
  * for another GPU, and one workgroup per kv head would leave this one idle. */
 size_t skv_effective_split_min_len(void);

@@ -155,6 +155,7 @@ size_t env_usize(const char *name, size_t dflt) {
 // (skv_flags_reload starts a new one), not once per launch.
 struct Tuning {
     size_t split_min_len;   // rows below which the context is not split
+    bool split_min_len_given;
     size_t target_wgs;      // workgroups a decode launch aims for
     size_t min_pages;       // pages per split at least (0 = one per wavefront)
     size_t forced_waves;    // 4 or 8, 0 = by shape
@@ -172,6 +173,7 @@ const Tuning &tuning() {
     const uint64_t epoch = skv_internal_flags_epoch();
     if (epoch != seen) {
         t.split_min_len = skv_effective_split_min_len();
+        t.split_min_len_given = std::getenv("RETI_RUST_SDPA_2PASS_MIN_LEN") != nullptr;
         t.target_wgs = std::max<size_t>(env_usize("SKV_DECODE_WGS", 256), 1);
         t.min_pages = env_usize("SKV_DECODE_MIN_PAGES", 0);
         t.forced_waves = env_usize("SKV_DECODE_WAVES", 0);
@@ -365,6 +367,36 @@ int choose_splits(const skv_layer *L, int n_pages_scan, size_t rows, int waves, 
     return (int)std::max<size_t>(s, 1);
 }
 
+// Contexts of so few pages that one workgroup to a tile of query slots, with no split, is done before the merge of a split would be:
+// a launch less for the host too. Not where the split knobs of decode launches are set. Unsplit, the launch writes the context while other
+// workgroups still read, so the caller sees to it that the context lies over nothing that they read (apart).
+bool may_stay_whole() {
+    const Tuning &t = tuning();
+    return !t.split_min_len_given && t.min_pages == 0 && t.forced_waves == 0;
+}
+bool apart(const float *out, size_t n_out, const float *in, size_t n_in) {
+    const uintptr_t o = reinterpret_cast<uintptr_t>(out), i = reinterpret_cast<uintptr_t>(in);
+    return !in || o >= i + n_in * sizeof(float) || i >= o + n_out * sizeof(float);
+}
+// Decode steps of bf16 layers, eight wavefronts a workgroup. Split / whole, us of GPU time on one MI355X: q32/kv8/hd128 over 150, 250, 380 rows
+// 6.5/5.2, 6.4/5.6, 6.4/6.8; q8/kv8/hd80 6.3/4.9, 6.2/5.0, 6.3/5.9, 500 6.3/6.7; q8/kv2/hd64 5.7/4.5, 5.7/4.6, 5.8/5.2, 500 5.8/5.7; q16/kv2/hd256 7.8/7.1,
+// 7.8/8.1; with the pre-KV step q16/kv8/hd256 over 150 9.6/8.7. Calls in a stream, where the host's two launches take longer than the
+// device: q32/kv8/hd128 over 250 9.1/7.1. (f32 layers, q32/kv8/hd128 over 140, 250 7.6/7.7, 7.6/9.8.)
+bool whole_step(const Geom &g, int n_pages) {
+    return may_stay_whole() && !g.f32 && g.P <= 256 && n_pages <= (g.P <= 96 ? 24 : g.P <= 128 ? 16 : 10);
+}
+// Chunks in the multi-query mode, of `tiles` tiles of all kv heads: the more there are, the fewer splits would share the device. Split / whole, us of GPU
+// time: q32/kv8/hd128, 6 rows (16 tiles) over 250, 500, 700 8.5/6.3, 9.1/8.3, 9.1/10.0, 16 (32) over 500, 700 10.5/8.7, 10.4/10.0, 30 (64) over
+// 250, 700, 1000 12.2/8.1, 12.9/11.4, 13.4/13.5; q8/kv2/hd64, 6 (4) over 500, 700 7.3/7.0, 7.4/8.0; q12/kv4/hd96, 20 (16) over 500, 700
+// 9.8/9.3, 9.7/10.6; q16/kv2/hd256, 6 (6) over 250, 380 11.6/10.5, 11.8/12.8, 16 (16) over 250, 380 15.1/13.2, 14.3/14.7, 48 (48) over 500, 700,
+// 1000 16.0/13.9, 16.5/15.7, 17.0/18.3. f32 layers: q32/kv8/hd128, 30 (64) over 140, 250, 380 12.5/11.8, 16.7/14.9, 18.0/18.1, 6 (16) over 140
+// 10.7/11.1; q16/kv2/hd256, 24 (24) over 140 16.5/18.8.
+bool whole_chunk(const Geom &g, size_t tiles, int n_pages) {
+    if (!may_stay_whole() || g.P > 256) return false;
+    const size_t line = g.f32 ? (g.P <= 128 ? 4 + tiles / 4 : 0) : g.P <= 128 ? 26 + tiles / 2 : 16 + tiles / 3;
+    return (size_t)n_pages <= line;
+}
+
 hipStream_t as_stream(skv_stream s) { return reinterpret_cast<hipStream_t>(s); }
 
 int32_t check_window(const skv_layer *L, size_t window_start) {
@@ -392,7 +424,7 @@ bool wide_f32_heads(const skv_layer *L) { return L->g.f32 && L->g.P > 256; }
 // Arguments of the matrix-core attention kernel for the layer's current length.
 void fill_decode_args(const skv_layer *L, const float *q_dev, float *out_dev, size_t window_start,
                       const float *k_new, const float *v_new, size_t n_queries, size_t target_wgs,
-                      DecodeArgs &a, bool keep_ring = false) {
+                      DecodeArgs &a, bool keep_ring = false, bool whole_ok = false) {
     Geom g = L->g;
     // A ring that has not wrapped is a full layer: every position in its own slot, no page but those in the queries' reach to walk and
     // no position to work out (512 rows of q16/kv8/hd256 on an empty ring of 1056 27.4 -> 23.2 us, over 512 38.6 -> 33.2, f32 over none
@@ -424,6 +456,10 @@ void fill_decode_args(const skv_layer *L, const float *q_dev, float *out_dev, si
     }
     a.waves = choose_waves(L, a.n_pages);
     a.splits = choose_splits(L, a.n_pages, L->len - window_start, a.waves, target_wgs);
+    if (whole_ok && n_queries == 1 && whole_step(g, a.n_pages)) {
+        a.waves = 8;
+        a.splits = 1;
+    }
     a.splits_total = a.splits;
     // scores are multiplied by 1/sqrt(head_dim) (src/decode_resident/kernels.rs:36, 198, 395,
     // 575); log2(e) moves the softmax to base 2.
@@ -643,6 +679,10 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
     if (static_partials && (n_queries != 1 || !uses_flash(L)))
         return fail(SKV_ERR_CONFIG, "decode_step_static: une ligne de requête, noyau matriciel seulement");
     StreamScratch::Lease lease;
+    // the context lies over nothing that the launch reads (see may_stay_whole)
+    const size_t q_dim = (size_t)g.q_heads * g.head_dim, kv_dim = (size_t)g.kv_heads * g.head_dim;
+    const bool out_apart = apart(out_dev, n_queries * q_dim, q_dev, pre && pre->q_head_stride > 0 ? (size_t)g.q_heads * pre->q_head_stride : n_queries * q_dim) &&
+                           apart(out_dev, n_queries * q_dim, k_new, n_queries * kv_dim) && apart(out_dev, n_queries * q_dim, v_new, n_queries * kv_dim);
     if (g.f32 && (uses_flash(L) || n_queries > 1)) {
         // the f32 element's matrix kernels: 16 query slots per workgroup, the context split while
         // that leaves compute units idle; one query row of narrow heads takes the kernel that
@@ -715,6 +755,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
             if (L->g.ring_rows > 0) want = std::min(want, std::max<size_t>((size_t)a.n_pages / 8, 1));
             a.splits = (int)std::min<size_t>((size_t)a.splits, want);
             if (tiles > (size_t)g.kv_heads) a.splits = xcd_splits(a.splits, g.kv_heads, a.n_pages, 4, 16);
+            if (out_apart && whole_chunk(g, tiles, a.n_pages)) a.splits = 1;
             a.splits_total = a.splits;
             if (a.splits > 1) {
                 int32_t rc2 = multi_query_partials(L, s, (size_t)a.splits, n_queries, a, lease);
@@ -757,7 +798,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
         return SKV_OK;
     }
     DecodeArgs a{};
-    fill_decode_args(L, q_dev, out_dev, window_start, k_new, v_new, n_queries, decode_target_wgs(), a);
+    fill_decode_args(L, q_dev, out_dev, window_start, k_new, v_new, n_queries, decode_target_wgs(), a, false, out_apart);
     if (attn_scalar > 0.0f) a.qscale = (1.0f / std::sqrt(attn_scalar)) * 1.4426950408889634f;
     if (pre) {
         a.pre = 1;
@@ -794,6 +835,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
         }
         a.splits = (int)std::min<size_t>((size_t)a.splits, want);
         if (!use_tiles && tiles > (size_t)g.kv_heads) a.splits = xcd_splits(a.splits, g.kv_heads, a.n_pages, a.waves, 10);
+        if (!use_tiles && out_apart && whole_chunk(g, tiles, a.n_pages)) a.splits = 1;
         a.splits_total = a.splits;
         if (a.splits > 1) {
             int32_t rc2 = multi_query_partials(L, s, (size_t)a.splits, n_queries, a, lease);
@@ -1948,6 +1990,22 @@ int32_t skv_decode_step_batch_device(skv_layer *const *seqs, size_t n_seq, skv_s
                                                    : L->len + 1 - skv_window_start(L->len, L->window);
             pages_total += (rows + 15) / 16;
         }
+        // the contexts, all of them, lie over no sequence's rows or queries (see may_stay_whole)
+        bool out_apart = true;
+        {
+            uintptr_t out_lo = UINTPTR_MAX, out_hi = 0;
+            const size_t q_bytes = (size_t)seqs[0]->g.q_heads * seqs[0]->g.head_dim * sizeof(float), kv_bytes = skv_kv_dim(seqs[0]) * sizeof(float);
+            for (size_t i = first; i < first + n; ++i) {
+                const uintptr_t o = reinterpret_cast<uintptr_t>(out_dev[i]);
+                out_lo = std::min(out_lo, o);
+                out_hi = std::max(out_hi, o + q_bytes);
+            }
+            for (size_t i = first; i < first + n; ++i)
+                for (const auto &[in, bytes] : {std::pair<const void *, size_t>{q_dev[i], q_bytes}, {k_dev[i], kv_bytes}, {v_dev[i], kv_bytes}}) {
+                    const uintptr_t at = reinterpret_cast<uintptr_t>(in);
+                    out_apart = out_apart && (at >= out_hi || at + bytes <= out_lo);
+                }
+        }
         DecodeBatchArgs b{};
         size_t floor_before[SKV_MAX_BATCH];
         for (size_t i = 0; i < n; ++i) {
@@ -1963,7 +2021,7 @@ int32_t skv_decode_step_batch_device(skv_layer *const *seqs, size_t n_seq, skv_s
                                                   (size_t)L->g.kv_heads);
             fill_decode_args(L, q_dev[first + i], out_dev[first + i], ws,
                              reinterpret_cast<const float *>(k_dev[first + i]),
-                             reinterpret_cast<const float *>(v_dev[first + i]), 1, share, b.seq[i]);
+                             reinterpret_cast<const float *>(v_dev[first + i]), 1, share, b.seq[i], false, out_apart);
         }
         hipError_t e = launch_decode_batch(b, (int)n, as_stream(stream));
         if (e != hipSuccess) {

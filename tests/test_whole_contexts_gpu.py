@@ -1,0 +1,83 @@
+"""Decode steps and chunks over few pages are attended without a split: on both sides of the lines against the oracle, and with a
+context that lies over what the launch reads, where the split stays."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+import saragossa_amd as skv
+
+pytestmark = pytest.mark.gpu
+
+
+def _layer(state, dims, element, rows, extra, seed):
+    q_heads, kv_heads, head_dim = dims
+    rng = np.random.default_rng(seed)
+    make = state.full_attention_f32 if element == "f32" else state.full_attention_bf16
+    kv = make(rows + extra, q_heads, kv_heads, head_dim)
+    kv.set_block_table(rng.permutation(kv.pages()).astype(np.int32))
+    k, v = (rng.standard_normal((rows + extra, kv_heads * head_dim), dtype=np.float32) for _ in range(2))
+    q = rng.standard_normal((extra, q_heads * head_dim), dtype=np.float32)
+    kv.seed(k[:rows], v[:rows], rows)
+    cache = oracle.LayerKvCache("f32" if element == "f32" else "bf16r")
+    lay = oracle.layout(q_heads, kv_heads, head_dim)
+    cache.append_batch(k[:rows], v[:rows], lay)
+    want = np.stack([oracle.decode_step(cache, k[rows + i], v[rows + i], q[i], lay) for i in range(extra)])
+    return kv, q, k[rows:], v[rows:], want
+
+
+def _stream():
+    return torch.cuda.current_stream().cuda_stream
+
+
+@pytest.mark.parametrize("dims,pages", [((8, 2, 64), 24), ((8, 8, 80), 24), ((16, 4, 128), 16), ((24, 1, 128), 16), ((8, 2, 256), 10)])
+@pytest.mark.parametrize("past", [-1, 0, 1])
+def test_steps_around_the_line(state, dims, pages, past):
+    rows = pages * 16 - 1 + past
+    kv, q, k, v, want = _layer(state, dims, "bf16", rows, 1, rows)
+    qd, kd, vd = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (q, k, v))
+    out = torch.full((1, q.shape[1]), float("nan"), device="cuda")
+    kv.encode_decode_step(_stream(), kd.data_ptr(), 0, vd.data_ptr(), 0, qd.data_ptr(), out.data_ptr())
+    assert np.abs(out.cpu().numpy() - want).max() <= 1e-4
+
+
+@pytest.mark.parametrize("element,tol", [("bf16", 1e-4), ("f32", 2e-5)])
+@pytest.mark.parametrize("dims,chunk,pages", [((8, 2, 64), 5, 29), ((32, 8, 128), 16, 42), ((32, 8, 128), 30, 20), ((16, 2, 256), 6, 18),
+                                              ((16, 2, 256), 40, 29)])
+@pytest.mark.parametrize("past", [0, 1])
+def test_chunks_around_the_line(state, dims, chunk, pages, past, element, tol):
+    rows = pages * 16 - chunk + past
+    kv, q, k, v, want = _layer(state, dims, element, rows, chunk, rows)
+    qd, kd, vd = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (q, k, v))
+    out = torch.full(q.shape, float("nan"), device="cuda")
+    kv.encode_prefill_rows(_stream(), qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), chunk, out.data_ptr())
+    assert np.abs(out.cpu().numpy() - want).max() <= tol
+
+
+@pytest.mark.parametrize("over", ["q", "k", "v"])
+def test_a_step_over_its_own_rows(state, over):
+    """The context lies over the step's query or new row, one head further: what the launch still reads stays whole until it is done."""
+    dims, rows = (32, 8, 128), 200
+    kv, q, k, v, want = _layer(state, dims, "bf16", rows, 1, 7)
+    buf = {n: torch.zeros(6000, device="cuda") for n in "qkv"}
+    for n, a in zip("qkv", (q, k, v)):
+        buf[n][128:128 + a.size] = torch.from_numpy(a.reshape(-1)).cuda()
+    at = {n: b.data_ptr() + 128 * 4 for n, b in buf.items()}
+    kv.encode_decode_step(_stream(), at["k"], 0, at["v"], 0, at["q"], buf[over].data_ptr())
+    assert np.abs(buf[over][:q.size].cpu().numpy() - want[0]).max() <= 1e-4
+
+
+def test_a_batch_over_another_sequences_rows(state):
+    dims, rows = (8, 2, 64), 150
+    seqs = [_layer(state, dims, "bf16", rows + 9 * i, 1, i) for i in range(3)]
+    kd = torch.from_numpy(np.concatenate([s[2] for s in seqs])).cuda()
+    vd = torch.from_numpy(np.concatenate([s[3] for s in seqs])).cuda()
+    qd = torch.from_numpy(np.concatenate([s[1] for s in seqs])).cuda()
+    q_dim, kv_dim = qd.shape[1], kd.shape[1]
+    rest = torch.zeros(2, q_dim, device="cuda")
+    # the first sequence's context over the last ones' queries
+    outs = [qd.data_ptr() + q_dim * 4, rest[0].data_ptr(), rest[1].data_ptr()]
+    skv.encode_decode_step_batch([s[0] for s in seqs], _stream(), [kd.data_ptr() + i * kv_dim * 4 for i in range(3)],
+                                 [vd.data_ptr() + i * kv_dim * 4 for i in range(3)], [qd.data_ptr() + i * q_dim * 4 for i in range(3)], outs)
+    got = np.stack([qd[1].cpu().numpy(), rest[0].cpu().numpy(), rest[1].cpu().numpy()])
+    assert np.abs(got - np.concatenate([s[4] for s in seqs])).max() <= 1e-4
