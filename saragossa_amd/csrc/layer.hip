@@ -157,6 +157,7 @@ struct Tuning {
     size_t split_min_len;   // rows below which the context is not split
     bool split_min_len_given;
     size_t target_wgs;      // workgroups a decode launch aims for
+    bool wgs_given;         // that or prefill_wgs
     size_t min_pages;       // pages per split at least (0 = one per wavefront)
     size_t forced_waves;    // 4 or 8, 0 = by shape
     bool q_vec, fused_append;
@@ -175,6 +176,7 @@ const Tuning &tuning() {
         t.split_min_len = skv_effective_split_min_len();
         t.split_min_len_given = std::getenv("RETI_RUST_SDPA_2PASS_MIN_LEN") != nullptr;
         t.target_wgs = std::max<size_t>(env_usize("SKV_DECODE_WGS", 256), 1);
+        t.wgs_given = std::getenv("SKV_DECODE_WGS") != nullptr || std::getenv("SKV_PREFILL_WGS") != nullptr;
         t.min_pages = env_usize("SKV_DECODE_MIN_PAGES", 0);
         t.forced_waves = env_usize("SKV_DECODE_WAVES", 0);
         t.q_vec = env_usize("SKV_Q_VEC", 1) != 0;
@@ -368,11 +370,11 @@ int choose_splits(const skv_layer *L, int n_pages_scan, size_t rows, int waves, 
 }
 
 // Contexts of so few pages that one workgroup to a tile of query slots, with no split, is done before the merge of a split would be:
-// a launch less for the host too. Not where the split knobs of decode launches are set. Unsplit, the launch writes the context while other
+// a launch less for the host too. Not where a knob of the splits is set. Unsplit, the launch writes the context while other
 // workgroups still read, so the caller sees to it that the context lies over nothing that they read (apart).
 bool may_stay_whole() {
     const Tuning &t = tuning();
-    return !t.split_min_len_given && t.min_pages == 0 && t.forced_waves == 0;
+    return !t.split_min_len_given && !t.wgs_given && t.min_pages == 0 && t.forced_waves == 0;
 }
 bool apart(const float *out, size_t n_out, const float *in, size_t n_in) {
     const uintptr_t o = reinterpret_cast<uintptr_t>(out), i = reinterpret_cast<uintptr_t>(in);

@@ -1,5 +1,7 @@
 """Decode steps and chunks over few pages are attended without a split: on both sides of the lines against the oracle, and with a
 context that lies over what the launch reads, where the split stays."""
+import os
+
 import numpy as np
 import pytest
 import torch
@@ -81,3 +83,28 @@ def test_a_batch_over_another_sequences_rows(state):
                                  [vd.data_ptr() + i * kv_dim * 4 for i in range(3)], [qd.data_ptr() + i * q_dim * 4 for i in range(3)], outs)
     got = np.stack([qd[1].cpu().numpy(), rest[0].cpu().numpy(), rest[1].cpu().numpy()])
     assert np.abs(got - np.concatenate([s[4] for s in seqs])).max() <= 1e-4
+
+
+@pytest.mark.parametrize("knob", ["SKV_DECODE_WGS", "SKV_PREFILL_WGS"])
+@pytest.mark.parametrize("chunk", [1, 16])
+def test_a_given_number_of_workgroups_splits(state, knob, chunk):
+    """Where a knob of the splits is set, to its default here, short contexts are split as they are with any other such knob: bit for bit."""
+    def run(env):
+        saved = {name: os.environ.get(name) for name in env}
+        os.environ.update(env)
+        skv.flags.reload()
+        try:
+            kv, q, k, v, want = _layer(state, (32, 8, 128), "bf16", 220, chunk, 3)
+            qd, kd, vd = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (q, k, v))
+            out = torch.full(q.shape, float("nan"), device="cuda")
+            kv.encode_prefill_rows(_stream(), qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), chunk, out.data_ptr())
+            got = out.cpu().numpy()
+            assert np.abs(got - want).max() <= 1e-4
+            return got
+        finally:
+            for name, was in saved.items():
+                os.environ.pop(name) if was is None else os.environ.__setitem__(name, was)
+            skv.flags.reload()
+    split = run({"RETI_RUST_SDPA_2PASS_MIN_LEN": "128"})
+    assert np.array_equal(run({knob: "256"}), split)
+    assert not np.array_equal(run({}), split)
