@@ -2017,14 +2017,26 @@ int32_t skv_decode_step_batch_device(skv_layer *const *seqs, size_t n_seq, skv_s
             L->len += 1;
             if (L->g.ring_rows > 0 && L->len > (size_t)L->g.ring_rows)
                 L->floor_pos = std::max(L->floor_pos, L->len - (size_t)L->g.ring_rows);
+        }
+        // All contexts stay whole or none does: the merge of one is a launch for all, and a whole one then only walks longer. Batches of two,
+        // each by itself / none, us: q8/kv2/hd64 over 370, 400 rows 7.5/6.3, q16/kv2/hd256 over 150, 400 9.3/8.3, q4/kv1/hd128 over 250, 2000
+        // 7.7/6.9; four of q32/kv8/hd128 over 250, one of them over 600 8.5/8.0.
+        const auto fill = [&](size_t i, bool whole_ok) {
+            const skv_layer *L = seqs[first + i];
             const size_t ws = skv_window_start(L->len - 1, L->window);
             const size_t rows = L->g.ring_rows > 0 ? std::min<size_t>(L->len, (size_t)L->g.ring_rows) : L->len - ws;
             const size_t share = std::max<size_t>(decode_target_wgs() * ((rows + 15) / 16) / std::max<size_t>(pages_total, 1),
                                                   (size_t)L->g.kv_heads);
             fill_decode_args(L, q_dev[first + i], out_dev[first + i], ws,
                              reinterpret_cast<const float *>(k_dev[first + i]),
-                             reinterpret_cast<const float *>(v_dev[first + i]), 1, share, b.seq[i], false, out_apart);
+                             reinterpret_cast<const float *>(v_dev[first + i]), 1, share, b.seq[i], false, whole_ok);
+        };
+        bool split = false;
+        for (size_t i = 0; i < n; ++i) {
+            fill(i, out_apart);
+            split = split || b.seq[i].splits > 1;
         }
+        for (size_t i = 0; split && out_apart && i < n; ++i) fill(i, false);
         hipError_t e = launch_decode_batch(b, (int)n, as_stream(stream));
         if (e != hipSuccess) {
             for (size_t i = 0; i < n; ++i) {

@@ -108,3 +108,28 @@ def test_a_given_number_of_workgroups_splits(state, knob, chunk):
     split = run({"RETI_RUST_SDPA_2PASS_MIN_LEN": "128"})
     assert np.array_equal(run({knob: "256"}), split)
     assert not np.array_equal(run({}), split)
+
+
+def _batch(state, dims, lens, env):
+    saved = {name: os.environ.get(name) for name in env}
+    os.environ.update(env)
+    skv.flags.reload()
+    try:
+        seqs = [_layer(state, dims, "bf16", n, 1, i) for i, n in enumerate(lens)]
+        q, k, v = (torch.from_numpy(np.concatenate([s[i] for s in seqs])).cuda() for i in (1, 2, 3))
+        out = torch.full(q.shape, float("nan"), device="cuda")
+        at = lambda t: [row.data_ptr() for row in t]
+        skv.encode_decode_step_batch([s[0] for s in seqs], _stream(), at(k), at(v), at(q), at(out))
+        got = out.cpu().numpy()
+        assert np.abs(got - np.concatenate([s[4] for s in seqs])).max() <= 1e-4
+        return got
+    finally:
+        for name, was in saved.items():
+            os.environ.pop(name) if was is None else os.environ.__setitem__(name, was)
+        skv.flags.reload()
+
+
+@pytest.mark.parametrize("dims,lens", [((8, 2, 64), [300, 900]), ((8, 2, 64), [900, 300, 90]), ((16, 2, 256), [140, 400])])
+def test_a_batch_stays_whole_together(state, dims, lens):
+    """One context past the line splits the others as well: bit for bit what they are where a knob of the splits is set."""
+    assert np.array_equal(_batch(state, dims, lens, {}), _batch(state, dims, lens, {"RETI_RUST_SDPA_2PASS_MIN_LEN": "128"}))
