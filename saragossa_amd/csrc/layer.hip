@@ -384,8 +384,15 @@ bool apart(const float *out, size_t n_out, const float *in, size_t n_in) {
 // 6.5/5.2, 6.4/5.6, 6.4/6.8; q8/kv8/hd80 6.3/4.9, 6.2/5.0, 6.3/5.9, 500 6.3/6.7; q8/kv2/hd64 5.7/4.5, 5.7/4.6, 5.8/5.2, 500 5.8/5.7; q16/kv2/hd256 7.8/7.1,
 // 7.8/8.1; with the pre-KV step q16/kv8/hd256 over 150 9.6/8.7. Calls in a stream, where the host's two launches take longer than the
 // device: q32/kv8/hd128 over 250 9.1/7.1. (f32 layers, q32/kv8/hd128 over 140, 250 7.6/7.7, 7.6/9.8.)
-bool whole_step(const Geom &g, int n_pages) {
-    return may_stay_whole() && !g.f32 && g.P <= 256 && n_pages <= (g.P <= 96 ? 24 : g.P <= 128 ? 16 : 10);
+// In a batch whose contexts all stay whole the line rises with its workgroups (batch_wgs, sequences times kv heads; 0 = no batch): the more there are,
+// the fewer splits would share the device. Batches, split / whole: q8/kv8/hd80, 4 over 380, 500 rows 7.1/6.3, 7.1/7.3, 8 over 500, 700 8.0/7.6,
+// 8.8/9.0, 16 over 500, 700, 1500 10.0/8.2, 11.6/9.7, 16.5/16.5; q32/kv8/hd128, 4 over 380, 500 7.6/7.3, 7.8/8.5, 8 over 380, 500 9.0/7.7, 9.3/8.9,
+// 16 over 500, 700 12.0/9.7, 14.8/12.1; q16/kv4/hd128, 16 over 500, 700 9.4/9.0, 10.6/10.7; q8/kv8/hd128, 3 over 350 7.0/7.2, 8 over 510 8.7/8.9; q16/kv8/hd256, 4 over
+// 150, 250 8.6/7.5, 8.5/9.0, 8 over 250, 380 10.2/9.4, 11.8/11.5, 16 over 250, 380 12.8/10.7, 15.7/13.5. (f32, q32/kv8/hd128: 8 over 250
+// 10.0/10.6, 16 over 380 16.3/15.1, 16 over 3000 69.8/71.6.)
+bool whole_step(const Geom &g, int n_pages, int batch_wgs) {
+    return may_stay_whole() && !g.f32 && g.P <= 256 &&
+           n_pages <= (g.P <= 96 ? 24 + batch_wgs / 5 : g.P <= 128 ? 16 + batch_wgs / 5 : 10 + std::max(batch_wgs - 32, 0) / 6);
 }
 // Chunks in the multi-query mode, of `tiles` tiles of all kv heads: the more there are, the fewer splits would share the device. Split / whole, us of GPU
 // time: q32/kv8/hd128, 6 rows (16 tiles) over 250, 500, 700 8.5/6.3, 9.1/8.3, 9.1/10.0, 16 (32) over 500, 700 10.5/8.7, 10.4/10.0, 30 (64) over
@@ -426,7 +433,7 @@ bool wide_f32_heads(const skv_layer *L) { return L->g.f32 && L->g.P > 256; }
 // Arguments of the matrix-core attention kernel for the layer's current length.
 void fill_decode_args(const skv_layer *L, const float *q_dev, float *out_dev, size_t window_start,
                       const float *k_new, const float *v_new, size_t n_queries, size_t target_wgs,
-                      DecodeArgs &a, bool keep_ring = false, bool whole_ok = false) {
+                      DecodeArgs &a, bool keep_ring = false, bool whole_ok = false, int batch_wgs = 0) {
     Geom g = L->g;
     // A ring that has not wrapped is a full layer: every position in its own slot, no page but those in the queries' reach to walk and
     // no position to work out (512 rows of q16/kv8/hd256 on an empty ring of 1056 27.4 -> 23.2 us, over 512 38.6 -> 33.2, f32 over none
@@ -458,7 +465,7 @@ void fill_decode_args(const skv_layer *L, const float *q_dev, float *out_dev, si
     }
     a.waves = choose_waves(L, a.n_pages);
     a.splits = choose_splits(L, a.n_pages, L->len - window_start, a.waves, target_wgs);
-    if (whole_ok && n_queries == 1 && whole_step(g, a.n_pages)) {
+    if (whole_ok && n_queries == 1 && whole_step(g, a.n_pages, batch_wgs)) {
         a.waves = 8;
         a.splits = 1;
     }
@@ -2029,7 +2036,7 @@ int32_t skv_decode_step_batch_device(skv_layer *const *seqs, size_t n_seq, skv_s
                                                   (size_t)L->g.kv_heads);
             fill_decode_args(L, q_dev[first + i], out_dev[first + i], ws,
                              reinterpret_cast<const float *>(k_dev[first + i]),
-                             reinterpret_cast<const float *>(v_dev[first + i]), 1, share, b.seq[i], false, whole_ok);
+                             reinterpret_cast<const float *>(v_dev[first + i]), 1, share, b.seq[i], false, whole_ok, (int)n * L->g.kv_heads);
         };
         bool split = false;
         for (size_t i = 0; i < n; ++i) {

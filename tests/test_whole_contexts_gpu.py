@@ -133,3 +133,14 @@ def _batch(state, dims, lens, env):
 def test_a_batch_stays_whole_together(state, dims, lens):
     """One context past the line splits the others as well: bit for bit what they are where a knob of the splits is set."""
     assert np.array_equal(_batch(state, dims, lens, {}), _batch(state, dims, lens, {"RETI_RUST_SDPA_2PASS_MIN_LEN": "128"}))
+
+
+@pytest.mark.parametrize("dims,n_seq,pages", [((8, 2, 64), 3, 25), ((8, 8, 80), 16, 49), ((16, 4, 128), 16, 28), ((8, 2, 256), 16, 10), ((16, 8, 256), 8, 15)])
+def test_batches_around_the_line(state, dims, n_seq, pages):
+    lens = [pages * 16 - 1 - 3 * i for i in range(n_seq)]
+    split = {"RETI_RUST_SDPA_2PASS_MIN_LEN": "128"}
+    below = _batch(state, dims, lens, {})       # all whole
+    lens[-1] = pages * 16
+    above = _batch(state, dims, lens, {})       # one page too many
+    assert np.array_equal(above, _batch(state, dims, lens, split))
+    assert not np.array_equal(below[:-1], above[:-1])
