@@ -251,7 +251,9 @@ int32_t skv_append_batch_device(skv_layer *layer, skv_stream stream, const void 
  * window_start..len. Synchronous. */
 int32_t skv_attention_host(skv_layer *layer, const float *q, size_t n_elems, size_t window_start,
                            float *out);
-/* encode_attention_decode_windowed (attention.rs:738-835): device q and out, async on `stream`. */
+/* encode_attention_decode_windowed (attention.rs:738-835): device q and out, async on `stream`. Here and in the
+ * decode steps below the context may lie over what the same call reads: q_dev (the gated projection), the new row's k_dev or
+ * v_dev. Exactly over q_dev it costs nothing, elsewhere a copy launch where the context is not split. */
 int32_t skv_attention_device(skv_layer *layer, skv_stream stream, const float *q_dev,
                              float *out_dev, size_t window_start);
 /* append + attention of one token in one call (layers.rs:259-288 does the two
@@ -286,7 +288,8 @@ int32_t skv_decode_step_static_device(skv_layer *layer, skv_stream stream, const
  * the layer's sliding window: cached_attention_prefill_rows
  * (src/decoder/attention_ops.rs:976-1017) as one launch on the matrix cores instead of
  * the reference's per-row loop (src/decode_resident/layers.rs:1113-1118). out_dev is
- * [n_rows, q_dim] f32; up to 4096 rows a call it may lie over k_dev or v_dev. */
+ * [n_rows, q_dim] f32; up to 4096 rows a call (f32 ring layers of heads above 256 dims: up to the ring's rows) it may lie
+ * over q_dev, k_dev or v_dev; shifted against q_dev it then takes scratch (above) of its own size, or of a split's. */
 int32_t skv_prefill_chunk_device(skv_layer *layer, skv_stream stream, const float *q_dev,
                                  const void *k_dev, const void *v_dev, size_t n_rows,
                                  float *out_dev);

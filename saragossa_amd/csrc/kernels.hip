@@ -595,4 +595,16 @@ hipError_t launch_gate(const GateArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 
+// A context that was written aside to its place, which may be at any float's address.
+__global__ __launch_bounds__(256) void copy_kernel(float *dst, const float *src, size_t n) {
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) dst[i] = src[i];
+}
+
+hipError_t launch_copy(float *dst, const float *src, size_t n, hipStream_t s) {
+    if (n == 0) return hipSuccess;
+    const size_t blocks = (n + 255) / 256;
+    hipLaunchKernelGGL(copy_kernel, dim3((unsigned)(blocks < 65535 ? blocks : 65535)), dim3(256), 0, s, dst, src, n);
+    return hipGetLastError();
+}
+
 } // namespace skv

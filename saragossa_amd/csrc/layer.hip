@@ -370,15 +370,29 @@ int choose_splits(const skv_layer *L, int n_pages_scan, size_t rows, int waves, 
 }
 
 // Contexts of so few pages that one workgroup to a tile of query slots, with no split, is done before the merge of a split would be:
-// a launch less for the host too. Not where a knob of the splits is set. Unsplit, the launch writes the context while other
-// workgroups still read, so the caller sees to it that the context lies over nothing that they read (apart).
+// a launch less for the host too. Not where a knob of the splits is set, nor where the context lies over what the launch reads.
 bool may_stay_whole() {
     const Tuning &t = tuning();
     return !t.split_min_len_given && !t.wgs_given && t.min_pages == 0 && t.forced_waves == 0;
 }
-bool apart(const float *out, size_t n_out, const float *in, size_t n_in) {
-    const uintptr_t o = reinterpret_cast<uintptr_t>(out), i = reinterpret_cast<uintptr_t>(in);
-    return !in || o >= i + n_in * sizeof(float) || i >= o + n_out * sizeof(float);
+bool overlap(const void *a, size_t a_bytes, const void *b, size_t b_bytes) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return x < y + b_bytes && y < x + a_bytes;
+}
+// Whether the context of n rows lies over queries that workgroups other than the one that writes it may still have to read. An unsplit
+// launch, whose first workgroups write while others have yet to start, then writes elsewhere (see encode_attention); a split one's merge
+// starts behind all reads. Exactly in the queries' place it may lie: a workgroup reads the rows of its own slots alone, and writes
+// them when it has (but for one kernel, see reads_again). head_stride: elements between the heads of the queries (0 = head_dim).
+bool over_queries(const Geom &g, const float *out, const float *q, size_t n, size_t head_stride = 0) {
+    const size_t bytes = n * (size_t)g.q_heads * g.head_dim * sizeof(float);
+    if (out == q && head_stride == 0) return false;
+    return overlap(out, bytes, q, head_stride ? (size_t)g.q_heads * head_stride * sizeof(float) : bytes);
+}
+// The f32 chunk kernel on heads above 128 dims: its plain_slot comes back to a query row after half of the context's columns are stored.
+bool reads_again(const Geom &g, const float *out, const float *q) { return g.f32 && g.P > 128 && out == q; }
+// The same for n K or V rows.
+bool over_rows(const Geom &g, const float *out, const float *rows, size_t n) {
+    return rows && overlap(out, n * (size_t)g.q_heads * g.head_dim * sizeof(float), rows, n * (size_t)g.kv_heads * g.head_dim * sizeof(float));
 }
 // Decode steps of bf16 layers, eight wavefronts a workgroup. Split / whole, us of GPU time on one MI355X: q32/kv8/hd128 over 150, 250, 380 rows
 // 6.5/5.2, 6.4/5.6, 6.4/6.8; q8/kv8/hd80 6.3/4.9, 6.2/5.0, 6.3/5.9, 500 6.3/6.7; q8/kv2/hd64 5.7/4.5, 5.7/4.6, 5.8/5.2, 500 5.8/5.7; q16/kv2/hd256 7.8/7.1,
@@ -490,6 +504,13 @@ bool capturing(hipStream_t s) {
     return status != hipStreamCaptureStatusNone;
 }
 
+int32_t scratch_error(int status, size_t need) {
+    if (status == StreamScratch::REFUSED)
+        return fail(SKV_ERR_DEVICE, "prefill chunk: flux en capture, le tampon du flux est plus petit que les " +
+                                        std::to_string(need) + " o requis (même appel d'abord hors capture)");
+    return fail_hip((hipError_t)status, "prefill chunk: tampon des partiels");
+}
+
 // Split partials of a multi-query launch live in the context's scratch, grown on demand:
 // [kv_heads][n_sets][n_queries * gqa] of (o[head_dim], m, l); in front of them `page_bytes` for
 // pages of the chunk's own rows (*pages, a multiple of 256). The lease is the caller's until it has queued its launches.
@@ -512,11 +533,7 @@ int32_t multi_query_partials(skv_layer *L, hipStream_t s, size_t n_sets, size_t 
                              StreamScratch::Lease &lease, size_t page_bytes = 0, void **pages = nullptr) {
     size_t need = 0;
     const int status = try_partials(L, s, n_sets, n_queries, a, lease, page_bytes, pages, false, &need);
-    if (status == StreamScratch::REFUSED)
-        return fail(SKV_ERR_DEVICE, "prefill chunk: flux en capture, le tampon du flux est plus petit que les " +
-                                        std::to_string(need) + " o requis (même appel d'abord hors capture)");
-    if (status != 0) return fail_hip((hipError_t)status, "prefill chunk: tampon des partiels");
-    return SKV_OK;
+    return status == 0 ? SKV_OK : scratch_error(status, need);
 }
 
 // The layer's pages as the queries of a chunk walk them: from position 0 on on a full layer, from
@@ -688,10 +705,30 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
     if (static_partials && (n_queries != 1 || !uses_flash(L)))
         return fail(SKV_ERR_CONFIG, "decode_step_static: une ligne de requête, noyau matriciel seulement");
     StreamScratch::Lease lease;
-    // the context lies over nothing that the launch reads (see may_stay_whole)
-    const size_t q_dim = (size_t)g.q_heads * g.head_dim, kv_dim = (size_t)g.kv_heads * g.head_dim;
-    const bool out_apart = apart(out_dev, n_queries * q_dim, q_dev, pre && pre->q_head_stride > 0 ? (size_t)g.q_heads * pre->q_head_stride : n_queries * q_dim) &&
-                           apart(out_dev, n_queries * q_dim, k_new, n_queries * kv_dim) && apart(out_dev, n_queries * q_dim, v_new, n_queries * kv_dim);
+    // Whether the context lies over what other workgroups read: the queries (and the gate between them), a step's new row. (A chunk's
+    // rows are stored by a launch in front, or the caller has looked.)
+    const bool over = over_queries(g, out_dev, q_dev, n_queries, pre ? (size_t)pre->q_head_stride : 0) ||
+                      (n_queries == 1 && (over_rows(g, out_dev, k_new, 1) || over_rows(g, out_dev, v_new, 1)));
+    // Such a context of an unsplit launch, and a gated one of any (the merge reads the gate), is written aside and copied behind the launch.
+    float *aside = nullptr;
+    const auto place = [&](int splits, float *&out, bool late = false) -> int32_t {
+        if (!(over || late) || (splits > 1 && !(pre && pre->gate))) return SKV_OK;
+        if (n_queries == 1) {
+            aside = L->out_stage;
+        } else {
+            void *buf = nullptr;
+            const size_t need = n_queries * (size_t)g.q_heads * g.head_dim * sizeof(float);
+            const int status = L->ctx->scratch.get(hip_scratch, s, need, capturing(s), lease, &buf);
+            if (status != 0) return scratch_error(status, need);
+            aside = static_cast<float *>(buf);
+        }
+        out = aside;
+        return SKV_OK;
+    };
+    const auto settle = [&]() -> int32_t {
+        if (aside) SKV_HIP(launch_copy(out_dev, aside, n_queries * (size_t)g.q_heads * g.head_dim, s));
+        return SKV_OK;
+    };
     if (g.f32 && (uses_flash(L) || n_queries > 1)) {
         // the f32 element's matrix kernels: 16 query slots per workgroup, the context split while
         // that leaves compute units idle; one query row of narrow heads takes the kernel that
@@ -735,8 +772,11 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
                     const F32Plan plan = plan_f32_chunk(g, n_queries, first, entries, ring ? entries : a.n_pages, a.splits, most);
                     DecodeArgs b = a;
                     b.splits_total = plan.sets();
-                    if (plan.sets() == 1 || try_partials(L, s, (size_t)plan.sets(), n_queries, b, lease, 0, nullptr, true) == 0)
-                        return run_f32_chunk(plan, b, pages, terms, (int)lo, k_new, v_new, s);
+                    if (plan.sets() == 1 || try_partials(L, s, (size_t)plan.sets(), n_queries, b, lease, 0, nullptr, true) == 0) {
+                        rc = place(plan.sets(), b.out, reads_again(g, out_dev, q_dev));
+                        if (!rc) rc = run_f32_chunk(plan, b, pages, terms, (int)lo, k_new, v_new, s);
+                        return rc ? rc : settle();
+                    }
                 }
                 // no memory for them: the other way needs none
             }
@@ -750,9 +790,11 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
                 int32_t rc2 = multi_query_partials(L, s, (size_t)a.splits, n_queries, a, lease);
                 if (rc2) return rc2;
             }
+            rc = place(a.splits, a.out, reads_again(g, out_dev, q_dev));
+            if (rc) return rc;
             SKV_HIP(launch_f32_prefill(a, pages, nullptr, halves, s));
             if (a.splits > 1) SKV_HIP(launch_merge_rows(a, s));
-            return SKV_OK;
+            return settle();
         }
         if (n_queries > 1) {
             rc = store_rows(); // (a knob that turned between the caller's look at it and this one)
@@ -764,7 +806,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
             if (L->g.ring_rows > 0) want = std::min(want, std::max<size_t>((size_t)a.n_pages / 8, 1));
             a.splits = (int)std::min<size_t>((size_t)a.splits, want);
             if (tiles > (size_t)g.kv_heads) a.splits = xcd_splits(a.splits, g.kv_heads, a.n_pages, 4, 16);
-            if (out_apart && whole_chunk(g, tiles, a.n_pages)) a.splits = 1;
+            if (!over && whole_chunk(g, tiles, a.n_pages)) a.splits = 1;
             a.splits_total = a.splits;
             if (a.splits > 1) {
                 int32_t rc2 = multi_query_partials(L, s, (size_t)a.splits, n_queries, a, lease);
@@ -775,9 +817,11 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
             int32_t rc2 = partials_in(static_partials, SKV_STATIC_SCRATCH_BYTES, a);
             if (rc2) return rc2;
         }
+        rc = place(a.splits, a.out);
+        if (rc) return rc;
         SKV_HIP(launch_f32_split(a, s));
         if (a.splits > 1) SKV_HIP(n_queries > 1 ? launch_merge_rows(a, s) : launch_merge(a, s));
-        return SKV_OK;
+        return settle();
     }
     const bool use_flash = uses_flash(L) || n_queries > 1;
     if (!use_flash) {
@@ -803,11 +847,13 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
         a.window_start = (long)window_start;
         a.inv_scale = 1.0f / std::sqrt(attn_scalar > 0.0f ? attn_scalar : (float)g.head_dim);
         a.g = g;
+        rc = place(1, a.out);
+        if (rc) return rc;
         SKV_HIP(launch_naive(a, s));
-        return SKV_OK;
+        return settle();
     }
     DecodeArgs a{};
-    fill_decode_args(L, q_dev, out_dev, window_start, k_new, v_new, n_queries, decode_target_wgs(), a, false, out_apart);
+    fill_decode_args(L, q_dev, out_dev, window_start, k_new, v_new, n_queries, decode_target_wgs(), a, false, !over);
     if (attn_scalar > 0.0f) a.qscale = (1.0f / std::sqrt(attn_scalar)) * 1.4426950408889634f;
     if (pre) {
         a.pre = 1;
@@ -844,7 +890,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
         }
         a.splits = (int)std::min<size_t>((size_t)a.splits, want);
         if (!use_tiles && tiles > (size_t)g.kv_heads) a.splits = xcd_splits(a.splits, g.kv_heads, a.n_pages, a.waves, 10);
-        if (!use_tiles && out_apart && whole_chunk(g, tiles, a.n_pages)) a.splits = 1;
+        if (!use_tiles && !over && whole_chunk(g, tiles, a.n_pages)) a.splits = 1;
         a.splits_total = a.splits;
         if (a.splits > 1) {
             int32_t rc2 = multi_query_partials(L, s, (size_t)a.splits, n_queries, a, lease);
@@ -855,14 +901,16 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
         int32_t rc2 = partials_in(static_partials, SKV_STATIC_SCRATCH_BYTES, a);
         if (rc2) return rc2;
     }
+    rc = place(a.splits, a.out);
+    if (rc) return rc;
     if (use_tiles) {
         const size_t lo = std::max(window_start, skv_window_start(L->len - n_queries, L->window));
         SKV_HIP(launch_prefill_tiles(a, layer_pages(a.g, lo, L->len), shape, s));
         if (a.splits > 1) SKV_HIP(launch_merge_rows(a, s));
-        return SKV_OK;
+    } else {
+        SKV_HIP(launch_decode(a, s));
     }
-    SKV_HIP(launch_decode(a, s));
-    return SKV_OK;
+    return settle();
 }
 
 void appended(skv_layer *L, size_t n_rows) {
@@ -1395,13 +1443,7 @@ int32_t skv_decode_step_static_device(skv_layer *L, skv_stream stream, const voi
 // Whether a chunk's context is to lie over its K or V rows (a caller's activations that share a buffer): every row
 // then has to be in the cache before the first context is written.
 static bool context_over_rows(const skv_layer *L, size_t c, const float *out, const float *k, const float *v) {
-    const size_t n = c * skv_kv_dim(L) * sizeof(float), m = c * (size_t)L->g.q_heads * L->g.head_dim * sizeof(float);
-    const uintptr_t o = reinterpret_cast<uintptr_t>(out);
-    for (const float *p : {k, v}) {
-        const uintptr_t r = reinterpret_cast<uintptr_t>(p);
-        if (o < r + n && r < o + m) return true;
-    }
-    return false;
+    return over_rows(L->g, out, k, c) || over_rows(L->g, out, v, c);
 }
 
 // A chunk of c > 1 rows on a ring layer (bf16, or f32 where the f32 chunk kernel serves the head_dim). The
@@ -1435,8 +1477,9 @@ static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const flo
     bool made = g.f32 && f32_terms_pay(g, c) && !capturing(s);
     F32Plan plan{};
     const bool halves = g.f32 && f32_halves(g, c * (size_t)g.gqa, walked);
-    // a context over the chunk's own rows is written once they are in the ring: by the merge, so there has to be one
-    const bool over_rows = context_over_rows(L, c, out, k, v);
+    // a context over the chunk's own rows is written once they are in the ring, one over its queries once all are read: by the merge, so
+    // there has to be one
+    const bool late = context_over_rows(L, c, out, k, v) || over_queries(g, out, q, c) || reads_again(g, out, q);
     StreamScratch::Lease lease;
     void *scratch = nullptr;
     int32_t rc = SKV_OK;
@@ -1447,7 +1490,7 @@ static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const flo
         made = most > 0;
         if (made) {
             plan = plan_f32_chunk(g, c, 0, entries, (int)walked, INT32_MAX, most);
-            if (over_rows) plan.splits = std::max(plan.splits, 2);
+            if (late) plan.splits = std::max(plan.splits, 2);
             a.splits = plan.splits;
             a.splits_total = plan.sets();
             made = a.splits_total == 1 || try_partials(L, s, (size_t)a.splits_total, c, a, lease, 0, nullptr, true) == 0;
@@ -1455,7 +1498,7 @@ static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const flo
     }
     if (!made) {
         a.splits = chunk_splits(g, c, (size_t)(g.f32 ? f32_prefill_slots(g.P, halves) : prefill_tile_slots(g.P, shape)), walked);
-        if (over_rows) a.splits = std::max(a.splits, 2);
+        if (late) a.splits = std::max(a.splits, 2);
         a.splits_total = a.splits;
         rc = multi_query_partials(L, s, a.splits > 1 ? (size_t)a.splits : 0, c, a, lease, 2 * pool_bytes, &scratch);
         if (rc) return rc;
@@ -1479,7 +1522,7 @@ static int32_t ring_chunk(skv_layer *L, hipStream_t s, const float *q, const flo
         SKV_HIP(g.f32 ? launch_f32_prefill(a, pages, nullptr, halves, s) : launch_prefill_tiles(a, pages, shape, s));
     }
     if (a.splits_total == 1) return encode_append(L, s, k, v, c);
-    if (over_rows) {
+    if (late) {
         rc = encode_append(L, s, k, v, c);
         if (rc) return rc;
         SKV_HIP(launch_merge_rows(a, s));
@@ -1869,17 +1912,20 @@ static int32_t prekv_step(skv_layer *L, skv_stream stream, const skv_rope *rope,
         SKV_HIP(launch_norm_rope(n, s));
         rc = encode_append(L, s, L->kv_stage, v, 1);
         if (rc) return rc;
-        rc = encode_attention(L, s, L->q_stage, out_dev, skv_window_start(L->len - 1, L->window),
+        // a context over the gate waits aside until all of it is read
+        float *const ctx = gate && over_queries(L->g, out_dev, q, 1, q_head_stride) ? L->out_stage : out_dev;
+        rc = encode_attention(L, s, L->q_stage, ctx, skv_window_start(L->len - 1, L->window),
                               nullptr, nullptr, 1, attn_scalar);
         if (rc || !gate) return rc;
         GateArgs ga{};
-        ga.ctx = out_dev;
+        ga.ctx = ctx;
         ga.gate = gate;
-        ga.out = out_dev;
+        ga.out = ctx;
         ga.heads = L->g.q_heads;
         ga.head_dim = L->g.head_dim;
         ga.gate_head_stride = q_head_stride ? (int)q_head_stride : L->g.head_dim;
         SKV_HIP(launch_gate(ga, s));
+        if (ctx != out_dev) SKV_HIP(launch_copy(out_dev, ctx, (size_t)L->g.q_heads * L->g.head_dim, s));
         return SKV_OK;
     }
     PreKv pre{};

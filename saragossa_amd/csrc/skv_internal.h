@@ -243,6 +243,7 @@ struct GateArgs {
     int heads, head_dim, gate_head_stride;
 };
 hipError_t launch_gate(const GateArgs &a, hipStream_t s);
+hipError_t launch_copy(float *dst, const float *src, size_t n, hipStream_t s);
 hipError_t launch_iota(int32_t *dst, int n, hipStream_t s);
 
 // Measurement aids (a read-only walk of the cache with the decode kernel's pattern; an empty launch).
