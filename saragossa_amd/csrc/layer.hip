@@ -2045,22 +2045,29 @@ int32_t skv_decode_step_batch_device(skv_layer *const *seqs, size_t n_seq, skv_s
                                                    : L->len + 1 - skv_window_start(L->len, L->window);
             pages_total += (rows + 15) / 16;
         }
-        // the contexts, all of them, lie over no sequence's rows or queries (see may_stay_whole)
-        bool out_apart = true;
-        {
-            uintptr_t out_lo = UINTPTR_MAX, out_hi = 0;
-            const size_t q_bytes = (size_t)seqs[0]->g.q_heads * seqs[0]->g.head_dim * sizeof(float), kv_bytes = skv_kv_dim(seqs[0]) * sizeof(float);
+        // Sequences, a bit each, whose context lies over some sequence's queries (but its own, exactly) or rows: see over_queries
+        const auto look = [&]() -> uint32_t {
+            const Geom &g = seqs[0]->g;
+            const size_t q_bytes = (size_t)g.q_heads * g.head_dim * sizeof(float), kv_bytes = (size_t)g.kv_heads * g.head_dim * sizeof(float);
+            uintptr_t lo = UINTPTR_MAX, hi = 0; // of all contexts: what lies outside lies under none
             for (size_t i = first; i < first + n; ++i) {
-                const uintptr_t o = reinterpret_cast<uintptr_t>(out_dev[i]);
-                out_lo = std::min(out_lo, o);
-                out_hi = std::max(out_hi, o + q_bytes);
+                lo = std::min(lo, reinterpret_cast<uintptr_t>(out_dev[i]));
+                hi = std::max(hi, reinterpret_cast<uintptr_t>(out_dev[i]) + q_bytes);
             }
-            for (size_t i = first; i < first + n; ++i)
-                for (const auto &[in, bytes] : {std::pair<const void *, size_t>{q_dev[i], q_bytes}, {k_dev[i], kv_bytes}, {v_dev[i], kv_bytes}}) {
-                    const uintptr_t at = reinterpret_cast<uintptr_t>(in);
-                    out_apart = out_apart && (at >= out_hi || at + bytes <= out_lo);
-                }
-        }
+            uint32_t over = 0;
+            const auto under = [&](const void *in, size_t bytes, const float *own) {
+                const uintptr_t at = reinterpret_cast<uintptr_t>(in);
+                if (at >= hi || at + bytes <= lo) return;
+                for (size_t i = 0; i < n; ++i)
+                    if (out_dev[first + i] != own && overlap(out_dev[first + i], q_bytes, in, bytes)) over |= 1u << i;
+            };
+            for (size_t j = first; j < first + n; ++j) {
+                under(q_dev[j], q_bytes, out_dev[j] == q_dev[j] ? out_dev[j] : nullptr);
+                under(k_dev[j], kv_bytes, nullptr);
+                under(v_dev[j], kv_bytes, nullptr);
+            }
+            return over;
+        };
         DecodeBatchArgs b{};
         size_t floor_before[SKV_MAX_BATCH];
         for (size_t i = 0; i < n; ++i) {
@@ -2084,12 +2091,13 @@ int32_t skv_decode_step_batch_device(skv_layer *const *seqs, size_t n_seq, skv_s
                              reinterpret_cast<const float *>(k_dev[first + i]),
                              reinterpret_cast<const float *>(v_dev[first + i]), 1, share, b.seq[i], false, whole_ok, (int)n * L->g.kv_heads);
         };
+        const uint32_t over = look();
         bool split = false;
         for (size_t i = 0; i < n; ++i) {
-            fill(i, out_apart);
+            fill(i, over == 0);
             split = split || b.seq[i].splits > 1;
         }
-        for (size_t i = 0; split && out_apart && i < n; ++i) fill(i, false);
+        for (size_t i = 0; split && over == 0 && i < n; ++i) fill(i, false);
         hipError_t e = launch_decode_batch(b, (int)n, as_stream(stream));
         if (e != hipSuccess) {
             for (size_t i = 0; i < n; ++i) {

@@ -110,7 +110,7 @@ def test_a_given_number_of_workgroups_splits(state, knob, chunk):
     assert not np.array_equal(run({}), split)
 
 
-def _batch(state, dims, lens, env):
+def _batch(state, dims, lens, env, apart=False):
     saved = {name: os.environ.get(name) for name in env}
     os.environ.update(env)
     skv.flags.reload()
@@ -118,6 +118,9 @@ def _batch(state, dims, lens, env):
         seqs = [_layer(state, dims, "bf16", n, 1, i) for i, n in enumerate(lens)]
         q, k, v = (torch.from_numpy(np.concatenate([s[i] for s in seqs])).cuda() for i in (1, 2, 3))
         out = torch.full(q.shape, float("nan"), device="cuda")
+        if apart: # every sequence's q, k, v and context side by side, as where each has buffers of its own
+            rows = torch.cat([q, k, v, out], dim=1)
+            q, k, v, out = rows.split([q.shape[1], k.shape[1], v.shape[1], out.shape[1]], dim=1)
         at = lambda t: [row.data_ptr() for row in t]
         skv.encode_decode_step_batch([s[0] for s in seqs], _stream(), at(k), at(v), at(q), at(out))
         got = out.cpu().numpy()
@@ -133,6 +136,12 @@ def _batch(state, dims, lens, env):
 def test_a_batch_stays_whole_together(state, dims, lens):
     """One context past the line splits the others as well: bit for bit what they are where a knob of the splits is set."""
     assert np.array_equal(_batch(state, dims, lens, {}), _batch(state, dims, lens, {"RETI_RUST_SDPA_2PASS_MIN_LEN": "128"}))
+
+
+@pytest.mark.parametrize("dims,lens", [((8, 2, 64), [300, 200]), ((16, 2, 256), [140, 90, 60])])
+def test_a_batch_of_buffers_apart_stays_whole(state, dims, lens):
+    """Rows between the contexts but under none of them: bit for bit what the batch is with one tensor of each kind."""
+    assert np.array_equal(_batch(state, dims, lens, {}, apart=True), _batch(state, dims, lens, {}))
 
 
 @pytest.mark.parametrize("dims,n_seq,pages", [((8, 2, 64), 3, 25), ((8, 8, 80), 16, 49), ((16, 4, 128), 16, 28), ((8, 2, 256), 16, 10), ((16, 8, 256), 8, 15)])
