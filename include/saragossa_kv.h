@@ -382,7 +382,8 @@ int32_t skv_attn_gate_device(skv_ctx *ctx, skv_stream stream, const float *ctx_d
  * a batch, with the same result per sequence. All handles must share the head geometry,
  * the element, the window and the context, and be distinct; nothing is modified when one of
  * them is at capacity. (One launch pair on either element up to 16 query heads per kv head,
- * f32 layers up to head_dim 256; other shapes run a launch pair per sequence.) */
+ * f32 layers up to head_dim 256; other shapes run a launch pair per sequence.) A context may lie over its own
+ * sequence's inputs, as in a step; over another's in a batch of up to 16 that is one launch pair. */
 int32_t skv_decode_step_batch_device(skv_layer *const *seqs, size_t n_seq, skv_stream stream,
                                      const void *const *k_dev, const void *const *v_dev,
                                      const float *const *q_dev, float *const *out_dev);

@@ -2098,7 +2098,13 @@ int32_t skv_decode_step_batch_device(skv_layer *const *seqs, size_t n_seq, skv_s
             split = split || b.seq[i].splits > 1;
         }
         for (size_t i = 0; split && over == 0 && i < n; ++i) fill(i, false);
+        // an unsplit context over what other workgroups read is written aside (see encode_attention)
+        for (size_t i = 0; i < n; ++i)
+            if ((over >> i & 1) && b.seq[i].splits == 1) b.seq[i].out = seqs[first + i]->out_stage;
         hipError_t e = launch_decode_batch(b, (int)n, as_stream(stream));
+        for (size_t i = 0; e == hipSuccess && i < n; ++i)
+            if (b.seq[i].out != out_dev[first + i])
+                e = launch_copy(out_dev[first + i], b.seq[i].out, (size_t)seqs[0]->g.q_heads * seqs[0]->g.head_dim, as_stream(stream));
         if (e != hipSuccess) {
             for (size_t i = 0; i < n; ++i) {
                 seqs[first + i]->len -= 1;

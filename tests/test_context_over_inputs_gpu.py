@@ -95,6 +95,30 @@ def test_gated_steps(state, dims, element, rows, lead, fused):
         assert (buf[:q.numel()] - want).abs().max().item() <= 2e-5
 
 
+@pytest.mark.parametrize("dims,element", [((8, 2, 64), "bf16"), ((32, 8, 128), "bf16"), ((4, 2, 512), "bf16"), ((8, 2, 64), "f32")])
+@pytest.mark.parametrize("lens", [[100, 20, 60], [100, 700, 40], [200, 300, 100], [900, 800, 700]])
+@pytest.mark.parametrize("over", ["next query", "in place", "own query", "last rows"])
+@pytest.mark.parametrize("twopass", ["1", "0"])
+def test_batches(state, dims, element, lens, over, twopass):
+    """A sequence's context over the next one's query, over its own, exactly or shifted by a head, or over rows of the last ones"""
+    with _env(RETI_RUST_SDPA_2PASS=twopass):
+        twins = [_twins(state, dims, element, rows, 1) for rows in lens]
+        q, k, v = (torch.cat([t[1][i] for t in twins]) for i in range(3))
+        n, q_dim, kv_dim = len(lens), q.shape[1], k.shape[1]
+        want = torch.zeros(n, q_dim, device="cuda")
+        rows = lambda t: [r.data_ptr() for r in t]
+        skv.encode_decode_step_batch([t[0][1] for t in twins], _stream(), rows(k), rows(v), rows(q), rows(want))
+        shift = {"next query": q_dim, "in place": 0, "own query": dims[2]}.get(over, 0)
+        queries = torch.zeros((n + 1) * q_dim, device="cuda") # contexts `shift` floats behind the queries
+        queries[:n * q_dim] = q.reshape(-1)
+        keys = torch.zeros(n * max(q_dim, kv_dim), device="cuda")
+        keys[:n * kv_dim] = k.reshape(-1)
+        out = queries[shift:shift + n * q_dim] if over != "last rows" else keys[:n * q_dim]
+        at = lambda t, d: [t.data_ptr() + i * d * 4 for i in range(n)]
+        skv.encode_decode_step_batch([t[0][0] for t in twins], _stream(), at(keys, kv_dim), rows(v), at(queries, q_dim), at(out, q_dim))
+        assert (out.reshape(n, q_dim) - want).abs().max().item() <= 2e-5
+
+
 CHUNKS = [  # dims, element, rows in front, rows, window
     ((32, 8, 128), "bf16", 0, 512, 0),      # tile kernel, no split
     ((28, 4, 128), "bf16", 0, 700, 0),      # the same, more workgroups than the device holds
