@@ -404,9 +404,10 @@ bool over_rows(const Geom &g, const float *out, const float *rows, size_t n) {
 // 16 over 500, 700 12.0/9.7, 14.8/12.1; q16/kv4/hd128, 16 over 500, 700 9.4/9.0, 10.6/10.7; q8/kv8/hd128, 3 over 350 7.0/7.2, 8 over 510 8.7/8.9; q16/kv8/hd256, 4 over
 // 150, 250 8.6/7.5, 8.5/9.0, 8 over 250, 380 10.2/9.4, 11.8/11.5, 16 over 250, 380 12.8/10.7, 15.7/13.5. (f32, q32/kv8/hd128: 8 over 250
 // 10.0/10.6, 16 over 380 16.3/15.1, 16 over 3000 69.8/71.6.)
-bool whole_step(const Geom &g, int n_pages, int batch_wgs) {
-    return may_stay_whole() && !g.f32 && g.P <= 256 &&
-           n_pages <= (g.P <= 96 ? 24 + batch_wgs / 5 : g.P <= 128 ? 16 + batch_wgs / 5 : 10 + std::max(batch_wgs - 32, 0) / 6);
+// The line in pages, 0 = none stays whole.
+int whole_step_pages(const Geom &g, int batch_wgs) {
+    if (!may_stay_whole() || g.f32 || g.P > 256) return 0;
+    return g.P <= 96 ? 24 + batch_wgs / 5 : g.P <= 128 ? 16 + batch_wgs / 5 : 10 + std::max(batch_wgs - 32, 0) / 6;
 }
 // Chunks in the multi-query mode, of `tiles` tiles of all kv heads: the more there are, the fewer splits would share the device. Split / whole, us of GPU
 // time: q32/kv8/hd128, 6 rows (16 tiles) over 250, 500, 700 8.5/6.3, 9.1/8.3, 9.1/10.0, 16 (32) over 500, 700 10.5/8.7, 10.4/10.0, 30 (64) over
@@ -444,6 +445,11 @@ bool fused_append_built(const skv_layer *L) { return !L->g.f32 || (L->g.P <= 256
 // head_dim 256; wide f32 heads take the separate norm/rotation launches.
 bool wide_f32_heads(const skv_layer *L) { return L->g.f32 && L->g.P > 256; }
 
+// Pages that a launch of this window walks. ring: the layer is one, and has wrapped.
+int pages_walked(const skv_layer *L, size_t window_start, bool ring) {
+    return ring ? (int)std::min<size_t>((L->len + 15) / 16, (size_t)L->n_pages) : (int)((L->len + 15) / 16 - window_start / 16);
+}
+
 // Arguments of the matrix-core attention kernel for the layer's current length.
 void fill_decode_args(const skv_layer *L, const float *q_dev, float *out_dev, size_t window_start,
                       const float *k_new, const float *v_new, size_t n_queries, size_t target_wgs,
@@ -468,18 +474,17 @@ void fill_decode_args(const skv_layer *L, const float *q_dev, float *out_dev, si
     a.split_base = 0;
     a.window = n_queries > 1 ? (int)L->window : 0; // decode callers pass window_start themselves
     a.window_start = (int)window_start;
+    a.n_pages = pages_walked(L, window_start, g.ring_rows > 0);
     if (g.ring_rows > 0) {
         a.page_first = 0;
-        a.n_pages = (int)std::min<size_t>((L->len + 15) / 16, (size_t)L->n_pages);
         a.ring_t = (int)((L->len - 1) % (size_t)g.ring_rows);
         a.ring_base = (int)(L->len - 1) - a.ring_t;
     } else {
         a.page_first = (int)(window_start / 16);
-        a.n_pages = (int)((L->len + 15) / 16) - a.page_first;
     }
     a.waves = choose_waves(L, a.n_pages);
     a.splits = choose_splits(L, a.n_pages, L->len - window_start, a.waves, target_wgs);
-    if (whole_ok && n_queries == 1 && whole_step(g, a.n_pages, batch_wgs)) {
+    if (whole_ok && n_queries == 1 && a.n_pages <= whole_step_pages(g, batch_wgs)) {
         a.waves = 8;
         a.splits = 1;
     }
@@ -2081,6 +2086,16 @@ int32_t skv_decode_step_batch_device(skv_layer *const *seqs, size_t n_seq, skv_s
         // All contexts stay whole or none does: the merge of one is a launch for all, and a whole one then only walks longer. Batches of two,
         // each by itself / none, us: q8/kv2/hd64 over 370, 400 rows 7.5/6.3, q16/kv2/hd256 over 150, 400 9.3/8.3, q4/kv1/hd128 over 250, 2000
         // 7.7/6.9; four of q32/kv8/hd128 over 250, one of them over 600 8.5/8.0.
+        // (Arguments are filled again only where one had stayed whole. Host time of a call, 16 of q32/kv8/hd128 over 4000 rows, all filled
+        // twice / once: 13.2/11.9.)
+        const int wgs = (int)n * seqs[0]->g.kv_heads, line = whole_step_pages(seqs[0]->g, wgs);
+        uint32_t is_short = 0; // a bit each
+        for (size_t i = 0; i < n; ++i) {
+            const skv_layer *L = seqs[first + i];
+            const bool wrapped = L->g.ring_rows > 0 && L->len > (size_t)L->g.ring_rows;
+            if (pages_walked(L, skv_window_start(L->len - 1, L->window), wrapped) <= line) is_short |= 1u << i;
+        }
+        uint32_t over = is_short ? look() : 0;
         const auto fill = [&](size_t i, bool whole_ok) {
             const skv_layer *L = seqs[first + i];
             const size_t ws = skv_window_start(L->len - 1, L->window);
@@ -2089,16 +2104,18 @@ int32_t skv_decode_step_batch_device(skv_layer *const *seqs, size_t n_seq, skv_s
                                                   (size_t)L->g.kv_heads);
             fill_decode_args(L, q_dev[first + i], out_dev[first + i], ws,
                              reinterpret_cast<const float *>(k_dev[first + i]),
-                             reinterpret_cast<const float *>(v_dev[first + i]), 1, share, b.seq[i], false, whole_ok, (int)n * L->g.kv_heads);
+                             reinterpret_cast<const float *>(v_dev[first + i]), 1, share, b.seq[i], false, whole_ok, wgs);
         };
-        const uint32_t over = look();
-        bool split = false;
+        bool split = false, unsplit = false;
         for (size_t i = 0; i < n; ++i) {
             fill(i, over == 0);
             split = split || b.seq[i].splits > 1;
+            unsplit = unsplit || b.seq[i].splits == 1;
         }
-        for (size_t i = 0; split && over == 0 && i < n; ++i) fill(i, false);
+        for (size_t i = 0; split && over == 0 && i < n; ++i)
+            if (is_short >> i & 1) fill(i, false);
         // an unsplit context over what other workgroups read is written aside (see encode_attention)
+        if (unsplit && !is_short) over = look();
         for (size_t i = 0; i < n; ++i)
             if ((over >> i & 1) && b.seq[i].splits == 1) b.seq[i].out = seqs[first + i]->out_stage;
         hipError_t e = launch_decode_batch(b, (int)n, as_stream(stream));
