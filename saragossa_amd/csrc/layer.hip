@@ -2288,7 +2288,7 @@ int32_t skv_probe_merge_device(skv_layer *L, skv_stream stream, float *out_dev) 
     if (!uses_flash(L)) return fail(SKV_ERR_CONFIG, "probe: noyau matriciel seulement");
     DecodeArgs a{};
     fill_decode_args(L, nullptr, out_dev, skv_window_start(L->len - 1, L->window), nullptr, nullptr, 1,
-                     decode_target_wgs(), a);
+                     decode_target_wgs(), a, false, true);
     if (a.splits > 1) SKV_HIP(launch_merge(a, as_stream(stream)));
     return SKV_OK;
 } catch (...) {

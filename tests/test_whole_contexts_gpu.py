@@ -153,3 +153,15 @@ def test_batches_around_the_line(state, dims, n_seq, pages):
     above = _batch(state, dims, lens, {})       # one page too many
     assert np.array_equal(above, _batch(state, dims, lens, split))
     assert not np.array_equal(below[:-1], above[:-1])
+
+
+@pytest.mark.parametrize("rows,merged", [(150, False), (1000, True)])
+def test_the_probe_of_the_merge_is_the_steps_own(state, rows, merged):
+    """Nothing is launched where the step stays whole."""
+    kv, q, k, v, want = _layer(state, (16, 4, 128), "bf16", rows, 1, rows)
+    qd, kd, vd = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (q, k, v))
+    out = torch.full((1, q.shape[1]), float("nan"), device="cuda")
+    kv.encode_decode_step(_stream(), kd.data_ptr(), 0, vd.data_ptr(), 0, qd.data_ptr(), out.data_ptr())
+    again = torch.full_like(out, 7.0)
+    kv.encode_probe_merge(_stream(), again.data_ptr())
+    assert torch.equal(again, out) if merged else bool((again == 7.0).all())
