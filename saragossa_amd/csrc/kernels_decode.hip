@@ -569,7 +569,8 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, const int
     }
     __syncthreads();
     constexpr int P4 = P / 4;
-    const bool vec_ok = (g.head_dim & 3) == 0;
+    // (partials are aligned where heads are whole units; the context is the caller's, at any float's address)
+    const bool vec_ok = (g.head_dim & 3) == 0 && (a.splits_total > 1 || (reinterpret_cast<uintptr_t>(a.out) & 15) == 0);
     for (int u = tid; u < rows * P4; u += THREADS) {
         const int row = u / P4;
         const int c4 = (u - row * P4) * 4;

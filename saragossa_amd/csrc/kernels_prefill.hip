@@ -735,7 +735,7 @@ __device__ __forceinline__ void merge_rows_of(const DecodeArgs &a, const int kvh
     }
     float *dst = a.out + context_row(g, kvh, slot) * g.head_dim + c4;
     const float inv = 1.0f / lsum;
-    if (vec_ok) {
+    if (vec_ok && (reinterpret_cast<uintptr_t>(a.out) & 15) == 0) {
         *reinterpret_cast<float4_t *>(dst) = float4_t{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
     } else {
 #pragma unroll

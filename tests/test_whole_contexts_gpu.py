@@ -165,3 +165,33 @@ def test_the_probe_of_the_merge_is_the_steps_own(state, rows, merged):
     again = torch.full_like(out, 7.0)
     kv.encode_probe_merge(_stream(), again.data_ptr())
     assert torch.equal(again, out) if merged else bool((again == 7.0).all())
+
+
+@pytest.mark.parametrize("dims,element,rows,chunk,env", [
+    ((32, 8, 128), "bf16", 200, 1, {}),                                      # whole step
+    ((32, 8, 128), "bf16", 2000, 1, {}),                                     # split, merged
+    ((32, 8, 128), "bf16", 200, 16, {}),                                     # whole chunk
+    ((8, 2, 64), "bf16", 2400, 100, {"SKV_PREFILL_TILES": "2"}),             # chunk of splits, merged row by row
+    ((8, 2, 64), "f32", 2400, 100, {"SKV_PREFILL_TILES": "2"}),
+    ((8, 2, 64), "f32", 2400, 1, {}),
+])
+def test_a_context_at_any_floats_address(state, dims, element, rows, chunk, env):
+    """The one at an address of whole 16 bytes, up to the order in which a merge adds its splits: up to 32 of them, 32 roundings of
+    2^-24 of values of about 1."""
+    saved = {name: os.environ.get(name) for name in env}
+    os.environ.update(env)
+    skv.flags.reload()
+    try:
+        got = []
+        for lead in (0, 1, 2, 3):
+            kv, q, k, v, _ = _layer(state, dims, element, rows, chunk, 5)
+            qd, kd, vd = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (q, k, v))
+            buf = torch.full((q.size + 8,), 7.0, device="cuda")
+            kv.encode_prefill_rows(_stream(), qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), chunk, buf.data_ptr() + lead * 4)
+            assert bool((buf[:lead] == 7.0).all() and (buf[lead + q.size:] == 7.0).all())
+            got.append(buf[lead:lead + q.size])
+        assert all((g - got[0]).abs().max().item() <= 2e-6 for g in got)
+    finally:
+        for name, was in saved.items():
+            os.environ.pop(name) if was is None else os.environ.__setitem__(name, was)
+        skv.flags.reload()
