@@ -410,15 +410,36 @@ int whole_step_pages(const Geom &g, int batch_wgs) {
     return g.P <= 96 ? 24 + batch_wgs / 5 : g.P <= 128 ? 16 + batch_wgs / 5 : 10 + std::max(batch_wgs - 32, 0) / 6;
 }
 // Chunks in the multi-query mode, of `tiles` tiles of all kv heads: the more there are, the fewer splits would share the device. Split / whole, us of GPU
-// time: q32/kv8/hd128, 6 rows (16 tiles) over 250, 500, 700 8.5/6.3, 9.1/8.3, 9.1/10.0, 16 (32) over 500, 700 10.5/8.7, 10.4/10.0, 30 (64) over
-// 250, 700, 1000 12.2/8.1, 12.9/11.4, 13.4/13.5; q8/kv2/hd64, 6 (4) over 500, 700 7.3/7.0, 7.4/8.0; q12/kv4/hd96, 20 (16) over 500, 700
-// 9.8/9.3, 9.7/10.6; q16/kv2/hd256, 6 (6) over 250, 380 11.6/10.5, 11.8/12.8, 16 (16) over 250, 380 15.1/13.2, 14.3/14.7, 48 (48) over 500, 700,
-// 1000 16.0/13.9, 16.5/15.7, 17.0/18.3. f32 layers: q32/kv8/hd128, 30 (64) over 140, 250, 380 12.5/11.8, 16.7/14.9, 18.0/18.1, 6 (16) over 140
-// 10.7/11.1; q16/kv2/hd256, 24 (24) over 140 16.5/18.8.
-bool whole_chunk(const Geom &g, size_t tiles, int n_pages) {
+// time: q32/kv8/hd128, 6 rows (16 tiles) over 250, 490 8.5/6.3, 8.5/8.1, 30 (64) over 250, 700, 900 12.2/8.1, 12.9/11.4, 12.6/12.1, 60 (120) over 1300
+// 17.0/15.2; q8/kv2/hd64, 6 (4) over 440 6.9/6.2, 60 (30) over 600 8.8/7.6; q16/kv2/hd256, 48 (48) over 460 14.9/12.7, 90 (90) over 650 20.0/15.1.
+// Tiles of a kv head walk the same pages, on one or two XCDs where kv heads are whole fours (`near`), else on four or eight. Whole, every one of those then asks
+// memory for each page, unless the launch loads shared pages (pages_shared: more than four tiles, never where it appends the rows). There, and where a tile walks
+// alone, the line is lower: q24/kv1/hd128, 6 rows (9 tiles) over 330, 380, 470 8.8/8.1, 8.6/8.2, 8.2/9.5, 12 (18) over 400, 500 8.8/8.8, 8.8/9.6; q16/kv1/hd96, 8
+// (8) over 330, 470 7.9/6.9, 7.4/8.3; q48/kv3/hd256, 16 (48) over 400, 450 16.1/16.3, 16.3/18.1; q32/kv32/hd128, 2 (32) over 490, 590 8.1/8.1, 8.2/9.2; but
+// q32/kv8/hd128, 16 (32) over 560, 610 9.8/8.6, 9.8/9.2, and with shared loads q24/kv1/hd128, 24 (36) over 630 10.5/9.1.
+// f32 layers, four wavefronts a workgroup: a fourth page each is slower than the splits of up to 64 tiles, an eighth than those of 101 to 128, a tenth than those of
+// up to 144. q32/kv8/hd128, 30 rows (64) over 190, 240, 290 11.7/12.3, 15.9/13.9, 16.1/13.8, 60 (120) over 310, 400, 480 17.0/15.2, 17.7/17.9, 18.0/19.2, 90 (184) over 710
+// 28.3/24.9; q8/kv2/hd64, 30 (16) over 100 8.5/7.1; heads of 129 to 256 dims, q16/kv2/hd256, 24 (24) over 140 16.5/18.8.
+// 1052 chunks of bf16 layers and 409 of f32 layers, 1 to 32 kv heads in groups of 1 to 16, at the lines and down to two thirds of them: 1.13 and 1.12 times as fast as
+// split on the average, 0.96 at least. (With 26 + tiles / 2, 16 + tiles / 3 and 4 + tiles / 4 for all, some at the line took up to 1.23 times as long as split.)
+bool whole_chunk(const Geom &g, size_t tiles, int n_pages, bool appends) {
     if (!may_stay_whole() || g.P > 256) return false;
-    const size_t line = g.f32 ? (g.P <= 128 ? 4 + tiles / 4 : 0) : g.P <= 128 ? 26 + tiles / 2 : 16 + tiles / 3;
-    return (size_t)n_pages <= line;
+    const size_t pages = (size_t)n_pages, per_head = tiles / (size_t)g.kv_heads; // tiles that walk the same pages
+    if (g.f32) {
+        if (g.P > 128 || (g.P > 64 && tiles <= 64 && pages > 12 && pages <= 16)) return false;
+        if (g.P > 32 && tiles > 100 && tiles <= 144 && pages > (tiles <= 128 ? 28 : 36)) return false;
+        return pages <= 4 + tiles / 4;
+    }
+    size_t line = g.P <= 128 ? 26 + tiles / 2 : 16 + tiles / 3;
+    if (appends || per_head <= 4) {
+        const bool near = g.kv_heads % 4 == 0;
+        if (g.P <= 96 && (near || per_head <= 2)) line = g.kv_heads > 8 ? 26 + 2 * tiles / 5 : line;
+        else if (g.P <= 96) line = g.P <= 32 ? 26 + tiles / 3 : g.P <= 64 ? 24 + tiles / 4 : 23 + tiles / 5;
+        else if (g.P > 128) line = per_head == 1 ? std::min<size_t>(15 + tiles / 5, 18) : near ? 13 + tiles / 3 : 15 + tiles / 5;
+        else if (near) line = per_head == 1 ? 27 : g.kv_heads > 8 ? 20 + 2 * tiles / 5 : 23 + tiles / 2;
+        else line = per_head <= 2 ? 27 : g.kv_heads <= 2 ? 20 + tiles / 4 : 18 + tiles / 5;
+    }
+    return pages <= line;
 }
 
 hipStream_t as_stream(skv_stream s) { return reinterpret_cast<hipStream_t>(s); }
@@ -811,7 +832,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
             if (L->g.ring_rows > 0) want = std::min(want, std::max<size_t>((size_t)a.n_pages / 8, 1));
             a.splits = (int)std::min<size_t>((size_t)a.splits, want);
             if (tiles > (size_t)g.kv_heads) a.splits = xcd_splits(a.splits, g.kv_heads, a.n_pages, 4, 16);
-            if (!over && whole_chunk(g, tiles, a.n_pages)) a.splits = 1;
+            if (!over && whole_chunk(g, tiles, a.n_pages, false)) a.splits = 1;
             a.splits_total = a.splits;
             if (a.splits > 1) {
                 int32_t rc2 = multi_query_partials(L, s, (size_t)a.splits, n_queries, a, lease);
@@ -895,7 +916,7 @@ int32_t encode_attention(skv_layer *L, hipStream_t s, const float *q_dev, float 
         }
         a.splits = (int)std::min<size_t>((size_t)a.splits, want);
         if (!use_tiles && tiles > (size_t)g.kv_heads) a.splits = xcd_splits(a.splits, g.kv_heads, a.n_pages, a.waves, 10);
-        if (!use_tiles && !over && whole_chunk(g, tiles, a.n_pages)) a.splits = 1;
+        if (!use_tiles && !over && whole_chunk(g, tiles, a.n_pages, k_new != nullptr)) a.splits = 1;
         a.splits_total = a.splits;
         if (a.splits > 1) {
             int32_t rc2 = multi_query_partials(L, s, (size_t)a.splits, n_queries, a, lease);

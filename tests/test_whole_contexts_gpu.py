@@ -43,17 +43,51 @@ def test_steps_around_the_line(state, dims, pages, past):
     assert np.abs(out.cpu().numpy() - want).max() <= 1e-4
 
 
-@pytest.mark.parametrize("element,tol", [("bf16", 1e-4), ("f32", 2e-5)])
-@pytest.mark.parametrize("dims,chunk,pages", [((8, 2, 64), 5, 29), ((32, 8, 128), 16, 42), ((32, 8, 128), 30, 20), ((16, 2, 256), 6, 18),
-                                              ((16, 2, 256), 40, 29)])
-@pytest.mark.parametrize("past", [0, 1])
-def test_chunks_around_the_line(state, dims, chunk, pages, past, element, tol):
-    rows = pages * 16 - chunk + past
-    kv, q, k, v, want = _layer(state, dims, element, rows, chunk, rows)
-    qd, kd, vd = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (q, k, v))
-    out = torch.full(q.shape, float("nan"), device="cuda")
-    kv.encode_prefill_rows(_stream(), qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), chunk, out.data_ptr())
-    assert np.abs(out.cpu().numpy() - want).max() <= tol
+def _chunk(state, dims, element, chunk, pages, env):
+    """A chunk over a context of so many pages with itself: within the element's tolerance of the oracle"""
+    saved = {name: os.environ.get(name) for name in env}
+    os.environ.update(env)
+    skv.flags.reload()
+    try:
+        rows = pages * 16 - chunk - 1
+        kv, q, k, v, want = _layer(state, dims, element, rows, chunk, rows)
+        qd, kd, vd = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (q, k, v))
+        out = torch.full(q.shape, float("nan"), device="cuda")
+        kv.encode_prefill_rows(_stream(), qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), chunk, out.data_ptr())
+        got = out.cpu().numpy()
+        assert np.abs(got - want).max() <= (2e-5 if element == "f32" else 1e-4)
+        return got
+    finally:
+        for name, was in saved.items():
+            os.environ.pop(name) if was is None else os.environ.__setitem__(name, was)
+        skv.flags.reload()
+
+
+@pytest.mark.parametrize("dims,element,chunk,pages,whole", [
+    ((8, 2, 64), "bf16", 5, 28, True), ((8, 2, 64), "bf16", 5, 29, False),          # two tiles a kv head, appended
+    ((8, 2, 64), "bf16", 16, 26, True), ((8, 2, 64), "bf16", 16, 27, False),        # four, on four XCDs
+    ((8, 2, 32), "bf16", 16, 28, True), ((8, 2, 32), "bf16", 16, 29, False),
+    ((16, 1, 96), "bf16", 12, 25, True), ((16, 1, 96), "bf16", 12, 26, False),
+    ((16, 16, 96), "bf16", 3, 32, True), ((16, 16, 96), "bf16", 3, 33, False),      # more than eight kv heads
+    ((32, 8, 128), "bf16", 3, 27, True), ((32, 8, 128), "bf16", 3, 28, False),      # one tile a kv head
+    ((32, 8, 128), "bf16", 16, 39, True), ((32, 8, 128), "bf16", 16, 40, False),    # four, on one XCD
+    ((32, 8, 128), "bf16", 30, 58, True), ((32, 8, 128), "bf16", 30, 59, False),    # eight, rows appended in front
+    ((24, 1, 128), "bf16", 6, 22, True), ((24, 1, 128), "bf16", 6, 23, False),      # nine, on eight XCDs
+    ((36, 3, 128), "bf16", 6, 21, True), ((36, 3, 128), "bf16", 6, 22, False),
+    ((32, 16, 128), "bf16", 10, 32, True), ((32, 16, 128), "bf16", 10, 33, False),
+    ((16, 2, 256), "bf16", 6, 16, True), ((16, 2, 256), "bf16", 6, 17, False),
+    ((16, 8, 256), "bf16", 16, 18, True), ((16, 8, 256), "bf16", 16, 19, False),
+    ((16, 2, 256), "bf16", 40, 29, True), ((16, 2, 256), "bf16", 40, 30, False),
+    ((8, 2, 64), "f32", 48, 10, True), ((8, 2, 64), "f32", 48, 11, False),
+    ((32, 8, 64), "f32", 30, 14, True), ((32, 8, 128), "f32", 30, 12, True), ((32, 8, 128), "f32", 30, 13, False),
+    ((32, 8, 128), "f32", 30, 16, False), ((32, 8, 128), "f32", 30, 17, True), ((32, 8, 128), "f32", 30, 20, True), ((32, 8, 128), "f32", 30, 21, False),
+    ((32, 8, 64), "f32", 60, 28, True), ((32, 8, 64), "f32", 60, 29, False), ((32, 8, 96), "f32", 66, 36, True), ((32, 8, 96), "f32", 66, 37, False),
+    ((16, 2, 256), "f32", 24, 9, False),
+])
+def test_chunks_around_the_line(state, dims, element, chunk, pages, whole):
+    """Whole up to the line, and behind it bit for bit what the chunk is where a knob of the splits is set."""
+    split = _chunk(state, dims, element, chunk, pages, {"RETI_RUST_SDPA_2PASS_MIN_LEN": "128"})
+    assert np.array_equal(_chunk(state, dims, element, chunk, pages, {}), split) != whole
 
 
 @pytest.mark.parametrize("over", ["q", "k", "v"])
