@@ -229,3 +229,76 @@ def test_a_context_at_any_floats_address(state, dims, element, rows, chunk, env)
         for name, was in saved.items():
             os.environ.pop(name) if was is None else os.environ.__setitem__(name, was)
         skv.flags.reload()
+
+
+class _Step:
+    """One step of a kind over a context of so many pages with itself, as often as it is asked for"""
+
+    def __init__(self, state, kind, dims, pages):
+        q_heads, kv_heads, head_dim = dims
+        self.kind, self.rows, self.head_dim = kind, pages * 16 - 1, head_dim
+        self.kv, q, k, v, _ = _layer(state, dims, "bf16", self.rows, 1, pages)
+        rng = np.random.default_rng(pages)
+        if kind == "gated":
+            q = rng.standard_normal((1, 2 * q.size), dtype=np.float32)
+        w = (0.7 + rng.random((2, head_dim))).astype(np.float32)
+        self.q, self.k, self.v, self.w = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (q, k, v, w))
+        self.rope = state.rope_table(self.rows + 1, head_dim, 10000.0)
+        self.out = torch.full((q_heads * head_dim,), float("nan"), device="cuda")
+
+    def __call__(self, stream):
+        self.kv.truncate(self.rows)
+        q, k, v, out = (t.data_ptr() for t in (self.q, self.k, self.v, self.out))
+        if self.kind in ("prekv", "gated"):
+            step = self.kv.encode_decode_step_prekv if self.kind == "prekv" else self.kv.encode_decode_step_gated
+            step(stream, self.rope, self.rows, q, 0, k, 0, v, 0, self.w[0].data_ptr(), self.w[1].data_ptr(), 1e-6, float(self.head_dim), out)
+        else:
+            step = self.kv.encode_decode_step_static if self.kind == "static" else self.kv.encode_decode_step
+            step(stream, k, 0, v, 0, q, out)
+        return self.out
+
+
+LINES = [((8, 2, 32), 24), ((16, 2, 64), 24), ((8, 8, 80), 24), ((32, 8, 128), 16), ((16, 1, 128), 16), ((16, 2, 256), 10)]
+
+
+@pytest.mark.parametrize("kind", ["plain", "static", "prekv", "gated"])
+@pytest.mark.parametrize("dims,pages", LINES)
+@pytest.mark.parametrize("past", [0, 1])
+def test_steps_of_all_kinds_around_the_line(state, kind, dims, pages, past):
+    """Whole up to the line, and behind it bit for bit what the step is where a knob of the splits is set."""
+    step = _Step(state, kind, dims, pages + past)
+    got = step(_stream()).cpu().numpy().copy()
+    os.environ["RETI_RUST_SDPA_2PASS_MIN_LEN"] = "128"
+    skv.flags.reload()
+    try:
+        split = step(_stream()).cpu().numpy()
+    finally:
+        del os.environ["RETI_RUST_SDPA_2PASS_MIN_LEN"]
+        skv.flags.reload()
+    assert np.array_equal(got, split) == bool(past)
+    # (some 24 pages in another order: 24 roundings of 2^-24 of values up to 4)
+    assert np.abs(got - split).max() <= 6e-6
+
+
+@pytest.mark.parametrize("kind", ["plain", "static", "prekv", "gated"])
+@pytest.mark.parametrize("past", [0, 1])
+def test_captured_steps_around_the_line(state, kind, past):
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step = _Step(state, kind, (32, 8, 128), 16 + past)
+        want = step(side.cuda_stream).clone()
+        side.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            step(side.cuda_stream)
+        other = _Step(state, kind, (32, 8, 128), 9)
+        for replay in range(3):
+            other(side.cuda_stream)
+            step.out.fill_(float("nan"))
+            side.synchronize()
+            graph.replay()
+            side.synchronize()
+            assert torch.equal(step.out, want), f"replay {replay}"
+        del graph
+    torch.cuda.synchronize()
