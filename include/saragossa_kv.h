@@ -61,7 +61,8 @@ typedef struct skv_hot skv_hot;
  * stream that is being captured, a call does without.
  * A call on a stream that is being captured is recorded with the lengths of that moment. A chunked-prefill call whose
  * scratch would then have to grow returns SKV_ERR_DEVICE without having queued its attention: run the same call
- * once before the capture, on the same stream. The scratch that a captured call uses stays where it is until the
+ * once before the capture, on the same stream (f32 layers: with SKV_F32_TERMS=0, since a captured call makes no terms and may
+ * want more partials than one that does). The scratch that a captured call uses stays where it is until the
  * context is destroyed; it is also that of the stream's later calls, so replays of such graphs have to be ordered with
  * each other and with chunked-prefill calls on the captured stream, as work on one stream is.
  * Host-side bookkeeping (len, ring position)
@@ -89,9 +90,12 @@ int32_t skv_flag_flash_sdpa_enabled(void);        /* RETI_RUST_FLASH_SDPA, utils
 int32_t skv_flag_sdpa_2pass_enabled(void);        /* RETI_RUST_SDPA_2PASS, utils.rs:260-263 */
 size_t skv_flag_sdpa_2pass_min_len(void);         /* RETI_RUST_SDPA_2PASS_MIN_LEN, utils.rs:270-278 */
 size_t skv_sdpa_2pass_blocks(size_t len);         /* utils.rs:282-286 */
-/* Rows from which this library splits the context of a decode launch: RETI_RUST_SDPA_2PASS_MIN_LEN
- * when it is set (the reference's parse, default 2048 when unparsable), else 128 (while it is not set, decode
- * steps and short chunks stay whole over some pages more where that is faster). The reference's
+/* Rows below which this library never splits the context of a decode launch: RETI_RUST_SDPA_2PASS_MIN_LEN
+ * when it is set (the reference's parse, default 2048 when unparsable), and then it splits from there on; else 128.
+ * While neither it nor SKV_DECODE_WGS, SKV_PREFILL_WGS, SKV_DECODE_MIN_PAGES or SKV_DECODE_WAVES is set, contexts that are
+ * faster whole stay so for longer: steps of bf16 layers up to 384 rows (heads of 97 to 128 dims 256, of 129 to 256 160), in
+ * batches further the more sequences and kv heads they have (16 sequences of 8 kv heads 784, 656, 416), chunks of up to some
+ * hundred rows up to 400 to 1500. The reference's
  * own default (2048, utils.rs:270-278) is what skv_flag_sdpa_2pass_min_len reports; it was tuned
  * for another GPU, and one workgroup per kv head would leave this one idle. */
 size_t skv_effective_split_min_len(void);

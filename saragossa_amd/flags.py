@@ -32,8 +32,9 @@ def sdpa_2pass_blocks(n: int) -> int:
 
 
 def effective_split_min_len() -> int:
-    """Rows from which this library splits a decode launch's context (128 unless
-    RETI_RUST_SDPA_2PASS_MIN_LEN is set; the reference's own default is sdpa_2pass_min_len())."""
+    """Rows below which this library never splits a decode launch's context (128 unless
+    RETI_RUST_SDPA_2PASS_MIN_LEN is set, which then is also where it begins; unset, contexts that are faster whole
+    stay so for longer. The reference's own default is sdpa_2pass_min_len())."""
     return lib().skv_effective_split_min_len()
 
 
